@@ -64,12 +64,13 @@ int psp_version(void);
 #define PSP_CF_PACK(coarsen, log_lanes, log_unroll, segs_sel) \
     (PSP_CF_NATIVE | ((coarsen) - 1) | ((log_lanes) << 3) | ((log_unroll) << 6) | ((segs_sel) << 8))
 typedef struct psp_spmm_plan {
-    int vec;            /* floats per feature load: 4 (N%4==0), 2 (N%2==0) or 1 */
+    int vec;            /* floats every row of X starts at a multiple of: 4 (N%4==0), 2 (N%2==0) or 1.  Loads are 4 floats
+                         * wide from N = 4 on (their alignment is that of one float), 1 float wide below */
     int coarsen;        /* column vectors per lane (the request's CF, 1..8) */
     int lanes_per_row;  /* power of two, 1..64: lanes that share one sparse row */
     int rows_per_wave;  /* 64 / lanes_per_row */
     int unroll;         /* non-zeros whose feature loads are in flight together per lane */
-    int col_tiles;      /* grid.y: ceil(N / (lanes_per_row*coarsen*vec)) */
+    int col_tiles;      /* grid.y: ceil(N / (lanes_per_row*coarsen*4)), N >= 4 */
     int waves_per_block;
     int log_segs_per_wave; /* -1: chosen at launch from the format and the matrix size */
     int even_split;        /* 1: the wavefront's entries are always divided evenly between the lane groups */

@@ -111,8 +111,8 @@ PSP_EXPORT int psp_spmm_plan_for(int N, int CF, int blkWarpNum, psp_spmm_plan *p
     const int stripe_rows = ((blkWarpNum & PSP_BW_STRIPE_MASK) >> PSP_BW_STRIPE_SHIFT) * 256;  // 0: the library option
     blkWarpNum &= ~PSP_BW_STRIPE_MASK;
     PSP_REQUIRE(blkWarpNum == 4 || blkWarpNum == 8, "blkWarpNum must be 4 or 8 (got %d)", blkWarpNum);
-    const int V = (N % 4 == 0) ? 4 : (N % 2 == 0) ? 2 : 1;
-    const int nvec = N / V;
+    const int V = psp_vec_width(N);
+    const int nvec = psp_ceil_div(N, V);
     int C, L, U, logW = -1;
     if (CF & PSP_CF_NATIVE) {
         // native configuration: every field of the wave64 mapping chosen by the caller (the sweep / the decider)
@@ -130,15 +130,15 @@ PSP_EXPORT int psp_spmm_plan_for(int N, int CF, int blkWarpNum, psp_spmm_plan *p
         PSP_REQUIRE(CF >= 1 && CF <= 8, "CF must be 1..8 (got %d)", CF);
         // A lane group owns a tile of 32*CF columns, as the reference's warp does (CF columns per lane of a 32-lane
         // warp, SpMM_kernel.cu:162-165); the remaining columns go to further column tiles (grid.y).  Natively the
-        // 32-column slab is 8 lanes x float4 (16 x float2 / 32 x float when N is not a multiple of 4) and CF is the
-        // number of such vectors per lane, so a wavefront carries 8 rows whatever CF is.
+        // 32-column slab is 8 lanes x 4 floats (fewer than four columns: one lane each) and CF is the number of such
+        // vectors per lane, so a wavefront carries 8 rows whatever CF is.
         C = std::min(CF, nvec);
         L = 32 / V;
         while (L > 1 && (L / 2) * C >= nvec) L >>= 1;  // one tile already covers N: no wider than needed
         U = C == 1 ? 4 : C <= 4 ? 2 : 1;  // feature vectors in flight per lane: U entries x C vectors
         while (U > L) U >>= 1;
     }
-    plan->vec = V;
+    plan->vec = (N % 4 == 0) ? 4 : (N % 2 == 0) ? 2 : 1;
     plan->coarsen = C;
     plan->lanes_per_row = L;
     plan->rows_per_wave = PSP_WAVE / L;

@@ -83,13 +83,14 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
     const int grp = lane >> LOGL;
     const int grp_base = lane - sub;
 
-    int off[C];
+    int off[C], dup[C];  // dup: leading columns of a piece that was moved back to end with the row (psp_vec_col)
     bool live[C];
 #pragma unroll
     for (int i = 0; i < C; i++) {
         const int col = ((i << LOGL) + sub) * V;
         live[i] = col < K;
-        off[i] = live[i] ? col : K - V;
+        off[i] = psp_vec_col<V>(col, K);
+        dup[i] = col - off[i];
     }
 
     // One window: the segments s0 .. s0+nvalid-1 (at most 64), of which only the entries inside [pbeg, pend) count
@@ -123,7 +124,7 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
     const int b0 = min(P1, a0 + q);
     if (a0 >= b0) return;  // the whole group leaves together; nothing below reads other groups' lanes
 
-    // A row(s) of a segment; dead tail vectors are zero so they add nothing to the dot product
+    // A row(s) of a segment; dead tail vectors and repeated columns are zero so they add nothing to the dot product
     auto load_a = [&](int key, float (&dst)[NR][C][V]) {
 #pragma unroll
         for (int r = 0; r < NR; r++)
@@ -135,9 +136,9 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
 #pragma unroll
                     for (int e = 0; e < V; e++) t[e] = 0.0f;
                 }
-                if (live[i]) t = *(const vec_t *)(A + (size_t)(key * NR + r) * (size_t)K + off[i]);
+                if (live[i]) t = psp_load_vec<V>(A + (size_t)(key * NR + r) * (size_t)K + off[i]);
 #pragma unroll
-                for (int e = 0; e < V; e++) dst[r][i][e] = psp_elem<V>(t, e);
+                for (int e = 0; e < V; e++) dst[r][i][e] = e >= dup[i] ? psp_elem<V>(t, e) : 0.0f;
             }
     };
 
@@ -223,7 +224,7 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
                 for (int u = 0; u < U; u++) {
                     const float *br = B + (size_t)ck[u] * (size_t)K;
 #pragma unroll
-                    for (int i = 0; i < C; i++) bv[u][i] = *(const vec_t *)(br + off[i]);
+                    for (int i = 0; i < C; i++) bv[u][i] = psp_load_vec<V>(br + off[i]);
                 }
 #pragma unroll
                 for (int u = 0; u < U; u++)
@@ -355,7 +356,6 @@ static psp_sddmm_kernel_t psp_sddmm_lookup(int logL, int C, int V)
 #define PSP_CASE(L_, C_, U_)                                                               \
     if (logL == L_ && C == C_) {                                                           \
         if (V == 4) return psp_sddmm_kernel<L_, C_, 4, U_, NR, SPLIT, SCALE, BAL>;       \
-        if (V == 2) return psp_sddmm_kernel<L_, C_, 2, U_, NR, SPLIT, SCALE, BAL>;       \
         return psp_sddmm_kernel<L_, C_, 1, U_, NR, SPLIT, SCALE, BAL>;                   \
     }
     PSP_SDDMM_FOR_EACH_LCU(PSP_CASE)

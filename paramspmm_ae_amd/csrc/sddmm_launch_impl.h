@@ -24,13 +24,13 @@ int psp_sddmm_launch(const int *rowPtr, const int *colIdx, const float *val, con
     PSP_REQUIRE(!(BCSR && scale), "sddmm: scale is only supported for csr formats");
     PSP_REQUIRE(!(BCSR && row_max), "sddmm: row maxima are only supported for csr formats");
 
-    const int V = (K % 4 == 0) ? 4 : (K % 2 == 0) ? 2 : 1;
-    const int nvec = K / V;
+    const int V = psp_vec_width(K);
+    const int nvec = psp_ceil_div(K, V);
     int C = psp_ceil_div(nvec, 16);
     if (C > 4) C = 4;
     int logL = 0;
     while ((C << logL) < nvec) logL++;
-    if (logL > 6) return psp_fail(PSP_ERR_RANGE, "sddmm: K = %d is too wide (max %d for this alignment)", K, 256 * V);
+    if (logL > 6) return psp_fail(PSP_ERR_RANGE, "sddmm: K = %d is too wide (max %d)", K, 1024);
     if (logL < 4 && C > 1) C = 1;
 
     psp_sddmm_kernel_t k = scale ? psp_sddmm_lookup<NR, SPLIT, !BCSR>(logL, C, V)

@@ -9,9 +9,9 @@
 //   * the wavefront is cut into R = 64/L groups of L = 2^logL lanes; the range [P0,P1) is divided evenly
 //     between the groups, whatever the row lengths are, so a group walks ceil((P1-P0)/R) entries and
 //     writes a row out whenever it crosses a row end.  Skewed rows therefore cost no idle lanes;
-//   * every lane owns C column vectors of V floats (V = 4 -> global_load_dwordx4); vector i of lane s
-//     covers columns tile*L*C*V + (i*L + s)*V .. +V, so the L lanes of a group read L*V*4 contiguous bytes
-//     of an X row per load;
+//   * every lane owns C column vectors of V floats (V = 4 -> global_load_dwordx4; V = 1 for fewer than four columns);
+//     vector i of lane s covers columns tile*L*C*V + (i*L + s)*V .. +V, so the L lanes of a group read L*V*4
+//     contiguous bytes of an X row per load; the last vector of a row of N % 4 != 0 columns starts at N - 4;
 //   * colIdx / values are read once per L*U entries: lane s of a group takes the U consecutive entries
 //     base + s*U .. in one 4U-byte load per array (a group reads whole 128-byte lines), the pairs are handed
 //     round the group with ds_bpermute, and the next L*U are prefetched while the current ones are consumed;
@@ -31,10 +31,19 @@
 typedef float psp_f32x2 __attribute__((ext_vector_type(2)));
 typedef float psp_f32x4 __attribute__((ext_vector_type(4)));
 
+// Feature rows are loaded and stored in pieces of 4 floats whatever the width: global memory needs 4-byte alignment only,
+// so a row whose length is no multiple of 4 takes the same 16-byte instructions (`mem` carries the alignment).  Its last
+// piece is moved back to end with the row (psp_vec_col): it repeats up to three columns of the piece in front of it.
+// Widths below 4 use single floats.  Before, widths off the multiples of 4 ran on 8- or 4-byte loads with two and four
+// times the lanes or column tiles: Chung-Lu graph of 200 003 rows and 3.0 M entries, N = 47: 167 us.
+typedef float psp_f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int V> struct psp_vec;
-template <> struct psp_vec<1> { typedef float type; };
-template <> struct psp_vec<2> { typedef psp_f32x2 type; };
-template <> struct psp_vec<4> { typedef psp_f32x4 type; };
+template <> struct psp_vec<1> { typedef float type, mem; };
+template <> struct psp_vec<4> { typedef psp_f32x4 type; typedef psp_f32x4_a4 mem; };
+static __host__ __device__ __forceinline__ int psp_vec_width(int N) { return N >= 4 ? 4 : 1; }
+template <int V> __device__ __forceinline__ typename psp_vec<V>::type psp_load_vec(const float *p) { return *(const typename psp_vec<V>::mem *)p; }
+// first column of the piece that starts at column `col` of rows of N columns
+template <int V> __device__ __forceinline__ int psp_vec_col(int col, int N) { return min(col, N - V); }
 
 template <int V> __device__ __forceinline__ float psp_elem(const typename psp_vec<V>::type &v, int e) { return v[e]; }
 template <> __device__ __forceinline__ float psp_elem<1>(const float &v, int) { return v; }
@@ -59,7 +68,7 @@ template <int V> __device__ __forceinline__ void psp_store_vec(float *p, const f
     }
     // Y is written once and not read again by this kernel: the streaming hint keeps it from displacing rows of X
     // in the L2 (measured 1-5 % faster; the same hint on colIdx / val loads is slower, other column tiles re-read them)
-    __builtin_nontemporal_store(t, (typename psp_vec<V>::type *)p);
+    __builtin_nontemporal_store((typename psp_vec<V>::mem)t, (typename psp_vec<V>::mem *)p);
 }
 
 // COUNT consecutive 4-byte words starting at a 4-byte aligned address, fetched in the widest pieces (16, 8, 4 bytes)
@@ -180,7 +189,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                         for (int c = 0; c < C; c++) {
                             const int col = tile_col0 + ((c << logL) + sub) * V;
                             const float z[V] = {};
-                            if (col < N) psp_store_vec<V>(yr + col, z);
+                            if (col < N) psp_store_vec<V>(yr + psp_vec_col<V>(col, N), z);
                         }
                     }
                 }
@@ -241,7 +250,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         for (int i = 0; i < C; i++) {
             const int col = tile_col0 + ((i << logL) + sub) * V;
             live[i] = col < N;
-            off[i] = live[i] ? col : N - V;
+            off[i] = psp_vec_col<V>(col, N);
         }
     }
 
@@ -276,8 +285,11 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                 if (!SPLIT || !shared) {
                     psp_store_vec<V>(yr + off[i], acc[r][i]);
                 } else {
+                    // a piece that was moved back repeats columns of the one in front of it: they get zeros here (a plain
+                    // store may write them twice, both lanes hold the same sum)
+                    const int dup = (int)(blockIdx.y * ((C * V) << logL)) + ((i << logL) + sub) * V - off[i];
 #pragma unroll
-                    for (int e = 0; e < V; e++) unsafeAtomicAdd(yr + off[i] + e, acc[r][i][e]);
+                    for (int e = 0; e < V; e++) unsafeAtomicAdd(yr + off[i] + e, e >= dup ? acc[r][i][e] : 0.0f);
                 }
             }
         }
@@ -421,7 +433,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         _Pragma("unroll") for (int u = 0; u < U; u++)                                                  \
         {                                                                                              \
             const float *xr = X + (size_t)S##_ck[u] * (size_t)N;                                       \
-            _Pragma("unroll") for (int i = 0; i < C; i++) S##_x[u][i] = *(const vec_t *)(xr + off[i]); \
+            _Pragma("unroll") for (int i = 0; i < C; i++) S##_x[u][i] = psp_load_vec<V>(xr + off[i]);  \
         }                                                                                              \
         pos += U;                                                                                      \
         jb++;                                                                                          \
@@ -584,7 +596,6 @@ static psp_spmm_kernel_t psp_spmm_lookup(int C, int V, int U, int lanes_per_row,
         if (act) {                                                              \
             if constexpr (NR <= 2) {                                            \
                 if (V == 4) return psp_spmm_pick<C_, 4, U_, NR, SPLIT, false, true>(single); \
-                if (V == 2) return psp_spmm_pick<C_, 2, U_, NR, SPLIT, false, true>(single); \
                 return psp_spmm_pick<C_, 1, U_, NR, SPLIT, false, true>(single); \
             }                                                                   \
             return nullptr;                                                     \
@@ -596,7 +607,6 @@ static psp_spmm_kernel_t psp_spmm_lookup(int C, int V, int U, int lanes_per_row,
             return nullptr;                                                     \
         }                                                                       \
         if (V == 4) return psp_spmm_pick<C_, 4, U_, NR, SPLIT, false, false>(single); \
-        if (V == 2) return psp_spmm_pick<C_, 2, U_, NR, SPLIT, false, false>(single); \
         return psp_spmm_pick<C_, 1, U_, NR, SPLIT, false, false>(single);       \
     }
     PSP_SPMM_FOR_EACH_CU(PSP_CASE)

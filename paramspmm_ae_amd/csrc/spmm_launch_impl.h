@@ -73,10 +73,10 @@ int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, cons
     }
 
     const int segs_per_block = plan.waves_per_block << logW;
-    psp_spmm_kernel_t k = psp_spmm_lookup<NR, SPLIT>(plan.coarsen, plan.vec, plan.unroll, plan.lanes_per_row, softmax, relu_x != 0);
+    psp_spmm_kernel_t k = psp_spmm_lookup<NR, SPLIT>(plan.coarsen, psp_vec_width(N), plan.unroll, plan.lanes_per_row, softmax, relu_x != 0);
     if (!k)
         return psp_fail(PSP_ERR_ARG, "spmm%s: no kernel for coarsen %d vec %d unroll %d%s", softmax ? " softmax" : "", plan.coarsen,
-                        plan.vec, plan.unroll, softmax ? " (needs N % 4 == 0 and CF <= 4)" : "");
+                        psp_vec_width(N), plan.unroll, softmax ? " (needs N % 4 == 0 and CF <= 4)" : "");
 
     const int align_pct = opt.whole_rows ? (1 << 30) : (plan.even_split ? 0 : opt.align_pct);
     const psp_grid1d g = psp_xcd_grid(psp_ceil_div(nrows, segs_per_block),
