@@ -1,64 +1,13 @@
 // Double-precision SpMM and SDDMM for all six layouts (CSR / 2x1 / 3x1 blocks, plain or row-split).  The reference
 // dispatches its kernels for double as well as float (AT_DISPATCH_FLOATING_TYPES, SpMM_kernel.cu:149, sddmm_kernel.cu
-// :161).  GNN training is single precision, so this path is kept simple rather than tuned: one wavefront per
-// segment, lane groups across the columns taking the segment's entries in turn; the float path's balancing, vector
-// loads and unrolling are not repeated here.
+// :161).  Both run the float path's walks (spmm_kernel.h, sddmm_kernel.h) on pieces of two doubles, one 16-byte load.
 #include "psp_common.h"
+#include "spmm_launch_impl.h"
+#include "sddmm_kernel.h"
 
-// Y[rows_out, N] has been zeroed.  Plain layouts store, row-split layouts add (several segments may share a row).
-// The wavefront is cut into 64 / W groups of W lanes (W = the power of two that covers min(N, 64) columns); the groups
-// take the segment's entries in turn and their partial sums are added across the groups at the end, so narrow
-// feature matrices still use all lanes.
-template <int NR, bool SPLIT>
-__global__ void __launch_bounds__(256)
-spmm_f64_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const double *__restrict__ val,
-                const int *__restrict__ target_row, const double *__restrict__ X, double *__restrict__ Y, int nseg, int N,
-                int logW)
-{
-    const int lane = threadIdx.x & 63;
-    const int s = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (s >= nseg) return;  // wave-uniform
-    const int lb = rowPtr[s], hb = rowPtr[s + 1];
-    if (lb == hb) return;
-    const int key = SPLIT ? target_row[s] : s;
-    const int W = 1 << logW, G = 64 >> logW;
-    const int sub = lane & (W - 1), grp = lane >> logW;
-    for (int c0 = blockIdx.y * W; c0 < N; c0 += gridDim.y * W) {  // wave-uniform
-        const int c = c0 + sub;
-        double acc[NR];
-#pragma unroll
-        for (int r = 0; r < NR; r++) acc[r] = 0.0;
-        if (c < N) {
-            for (int p = lb + grp; p < hb; p += G) {
-                const double x = X[(size_t)colIdx[p] * N + c];
-#pragma unroll
-                for (int r = 0; r < NR; r++) {
-                    const double v = val[(size_t)p * NR + r];
-                    if (NR == 1 || v != 0.0) acc[r] = fma(v, x, acc[r]);  // a zero block entry adds nothing (SpMM_kernel.cu:1399)
-                }
-            }
-        }
-        // the groups' partial sums meet in group 0 (all lanes take part in the exchange)
-#pragma unroll
-        for (int i = 0; i < 6; i++)
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-                const double other = __shfl_xor(acc[r], 1 << i);
-                if ((1 << i) >= W) acc[r] += other;  // wave-uniform
-            }
-        if (grp == 0 && c < N) {
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-                double *y = Y + (size_t)(key * NR + r) * N + c;
-                if (SPLIT) unsafeAtomicAdd(y, acc[r]);
-                else *y = acc[r];
-            }
-        }
-    }
-}
-
-// out[nblk, NR] (out[nnz] for NR = 1); entries whose block value is zero are written as zero.  Groups of W lanes
-// (W covers min(K, 64) columns) take the segment's entries in turn.
+// SDDMM of rows wider than the lane groups' registers hold (K > PSP_SDDMM_F64_MAX_K): one wavefront per segment, groups of
+// W lanes (W covers min(K, 64) columns) take its entries in turn.  out[nblk, NR] (out[nnz] for NR = 1); entries whose block
+// value is zero are written as zero.
 template <int NR, bool SPLIT>
 __global__ void __launch_bounds__(256)
 sddmm_f64_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const double *__restrict__ val_b,
@@ -94,7 +43,7 @@ sddmm_f64_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
     }
 }
 
-// lanes per group: the power of two that covers min(width, 64)
+// lanes per group of that kernel: the power of two that covers min(width, 64)
 static int f64_log_group(int width)
 {
     int logW = 0;
@@ -102,19 +51,41 @@ static int f64_log_group(int width)
     return logW;
 }
 
-template <int NR>
+typedef void (*spmm_f64_kernel_t)(const int *, const int *, const double *, const int *, const double *, double *,
+                                  int, int, int, int, int, int, int, const float *, float *, int, int);
+
+// Mapping: two pieces of two doubles per lane, two entries in flight, lane groups of up to 8 lanes for rows of up to 32
+// doubles (one column tile of 256 bytes) and up to 16 beyond.  Bound by the memory traffic; of thirteen mappings (1 / 2 / 4
+// pieces x 4 ... 32 lanes x 1 ... 4 entries) measured on a mesh, an R-MAT and a block-model graph at N = 16 / 32 / 47 / 100
+// this one is within 12 % of the best nearly everywhere.  Mesh of 2.1 M rows, 2x1 blocks, N = 32: 806 us before (one
+// wavefront per block-row, 8-byte loads, Y cleared by a pass of its own) -> 272 us, 4.5 TB/s of the bytes it cannot do
+// without; CSR 299 us.  Rows of up to 8 doubles: one piece per lane, four entries in flight and groups of four lanes even
+// where fewer would cover the row -- with one lane per row a wavefront's 64 rows were 64 serial chains (N = 3 on the block
+// model: 349 us).
+template <int NR, bool SPLIT>
 static int spmm_f64_launch(const int *rowPtr, const int *colIdx, const double *val, const int *target_row, const double *X,
-                           double *Y, int nseg, int N, hipStream_t st)
+                           double *Y, int nseg, int N, int rows_out, hipStream_t st)
 {
-    const int logW = f64_log_group(N);
-    int col_tiles = psp_ceil_div(N, 1 << logW);
-    if (col_tiles > 64) col_tiles = 64;
-    dim3 grid(psp_ceil_div(nseg, 4), col_tiles, 1), block(256, 1, 1);
-    if (target_row)
-        hipLaunchKernelGGL((spmm_f64_kernel<NR, true>), grid, block, 0, st, rowPtr, colIdx, val, target_row, X, Y, nseg, N, logW);
-    else
-        hipLaunchKernelGGL((spmm_f64_kernel<NR, false>), grid, block, 0, st, rowPtr, colIdx, val, target_row, X, Y, nseg, N, logW);
-    return psp_check_launch("spmm f64 kernel");
+    const int V = N >= 2 ? 2 : 1, nvec = psp_ceil_div(N, V);
+    const int C = nvec <= 4 ? 1 : 2, U = C == 1 ? 4 : 2, widest = nvec <= 16 ? 8 : 16;
+    int L = 4;
+    while (L < widest && L * C < nvec) L <<= 1;
+    spmm_f64_kernel_t k = V == 1 ? psp_spmm_kernel<1, 1, 4, NR, SPLIT, false, false, true, double>
+                        : C == 1 ? psp_spmm_kernel<1, 2, 4, NR, SPLIT, false, false, true, double>
+                                 : psp_spmm_kernel<2, 2, 2, NR, SPLIT, false, false, true, double>;
+    psp_spmm_plan plan;
+    plan.vec = V;
+    plan.coarsen = C;
+    plan.lanes_per_row = L;
+    plan.rows_per_wave = PSP_WAVE / L;
+    plan.unroll = U;
+    plan.col_tiles = psp_ceil_div(nvec, L * C);
+    plan.waves_per_block = 4;
+    plan.log_segs_per_wave = -1;
+    plan.even_split = 0;
+    plan.xcd_stripe_rows = 0;
+    return psp_spmm_enqueue<NR, SPLIT>(k, plan, rowPtr, colIdx, val, target_row, X, Y, nseg, N, rows_out, st, (const float *)nullptr,
+                                       (float *)nullptr, 0);
 }
 
 PSP_EXPORT int psp_spmm_f64(const int *rowPtr, const int *colIdx, const double *val, const int *target_row,
@@ -126,26 +97,51 @@ PSP_EXPORT int psp_spmm_f64(const int *rowPtr, const int *colIdx, const double *
     if (!target_row) PSP_REQUIRE((long long)nseg * vec_size <= rows_out, "spmm_f64: Y has %d rows, the matrix needs %lld",
                                  rows_out, (long long)nseg * vec_size);
     hipStream_t st = (hipStream_t)stream;
-    int rc = psp_zero_f32((float *)Y, (size_t)rows_out * N * 2, st);  // all-zero bits are 0.0 in both precisions
-    if (rc != PSP_OK || nseg == 0 || N == 0) return rc;
-    PSP_REQUIRE(rowPtr && X, "spmm_f64: rowPtr / X is null");
-    if (vec_size == 1) return spmm_f64_launch<1>(rowPtr, colIdx, val, target_row, X, Y, nseg, N, st);
-    if (vec_size == 2) return spmm_f64_launch<2>(rowPtr, colIdx, val, target_row, X, Y, nseg, N, st);
-    return spmm_f64_launch<3>(rowPtr, colIdx, val, target_row, X, Y, nseg, N, st);
+    if (N == 0) return PSP_OK;
+    if (nseg > 0) PSP_REQUIRE(rowPtr && X, "spmm_f64: rowPtr / X is null");
+#define PSP_F64(NR_, SPLIT_) spmm_f64_launch<NR_, SPLIT_>(rowPtr, colIdx, val, target_row, X, Y, nseg, N, rows_out, st)
+    if (vec_size == 1) return target_row ? PSP_F64(1, true) : PSP_F64(1, false);
+    if (vec_size == 2) return target_row ? PSP_F64(2, true) : PSP_F64(2, false);
+    return target_row ? PSP_F64(3, true) : PSP_F64(3, false);
+#undef PSP_F64
 }
 
-template <int NR>
+typedef void (*sddmm_f64_kernel_t)(const int *, const int *, const double *, const int *, const double *, const double *, double *,
+                                   int, int, int, int, int, float *);
+#define PSP_SDDMM_F64_MAX_K 512  // 64 lanes x 4 pieces of two doubles
+
+template <int NR, bool SPLIT>
 static int sddmm_f64_launch(const int *rowPtr, const int *colIdx, const double *val_b, const int *target_row,
                             const double *A, const double *B, double *out, int nseg, int K, hipStream_t st)
 {
-    dim3 grid(psp_ceil_div(nseg, 4), 1, 1), block(256, 1, 1);
-    const int logW = f64_log_group(K);
-    if (target_row)
-        hipLaunchKernelGGL((sddmm_f64_kernel<NR, true>), grid, block, 0, st, rowPtr, colIdx, val_b, target_row, A, B, out, nseg, K,
-                           logW);
-    else
-        hipLaunchKernelGGL((sddmm_f64_kernel<NR, false>), grid, block, 0, st, rowPtr, colIdx, val_b, target_row, A, B, out, nseg, K,
-                           logW);
+    if (K > PSP_SDDMM_F64_MAX_K) {
+        hipLaunchKernelGGL((sddmm_f64_kernel<NR, SPLIT>), dim3(psp_ceil_div(nseg, 4)), dim3(256), 0, st, rowPtr, colIdx, val_b,
+                           target_row, A, B, out, nseg, K, f64_log_group(K));
+        return psp_check_launch("sddmm f64 kernel");
+    }
+    // vectors per lane and lanes per row: as for float (psp_sddmm_launch)
+    const int V = K >= 2 ? 2 : 1, nvec = psp_ceil_div(K, V);
+    // at least four lanes, as above
+    int C = std::min(psp_ceil_div(nvec, 16), 4), logL = 2;
+    while ((C << logL) < nvec) logL++;
+    if (logL < 4) C = 1;
+    sddmm_f64_kernel_t k = nullptr;
+#define PSP_CASE(L_, C_, U_) \
+    if constexpr (L_ >= 2) { \
+        if (V == 2 && logL == L_ && C == C_) k = psp_sddmm_kernel<L_, C_, 2, U_, NR, SPLIT, false, false, double>; \
+    }
+    PSP_SDDMM_FOR_EACH_LCU(PSP_CASE)
+#undef PSP_CASE
+    if (V == 1) k = psp_sddmm_kernel<2, 1, 1, 4, NR, SPLIT, false, false, double>;
+    PSP_REQUIRE(k, "sddmm_f64: no kernel for K = %d", K);
+    const int logR = 6 - logL;
+    int logW = SPLIT ? (logR > 4 ? logR : 4) : logR;
+    while (logW > 0 && (nseg >> logW) < 4096) logW--;
+    if (logW < logR - 1) logW = logR - 1;
+    const int segs_per_block = 4 << logW;
+    const psp_grid1d g = psp_xcd_grid(psp_ceil_div(nseg, segs_per_block), psp_stripe_rows() / segs_per_block);
+    hipLaunchKernelGGL(k, dim3(g.launch), dim3(256), 0, st, rowPtr, colIdx, val_b, target_row, A, B, out, nseg, K, logW, g.real,
+                       g.stripe, (float *)nullptr);
     return psp_check_launch("sddmm f64 kernel");
 }
 
@@ -161,7 +157,9 @@ PSP_EXPORT int psp_sddmm_f64(const int *rowPtr, const int *colIdx, const double 
     PSP_REQUIRE((colIdx != nullptr) == (out != nullptr), "sddmm_f64: colIdx and out must both be given (or both be null for a matrix without entries)");
     PSP_REQUIRE(vec_size == 1 || val_b || !colIdx, "sddmm_f64: block values are null");
     hipStream_t st = (hipStream_t)stream;
-    if (vec_size == 1) return sddmm_f64_launch<1>(rowPtr, colIdx, val_b, target_row, A, B, out, nseg, K, st);
-    if (vec_size == 2) return sddmm_f64_launch<2>(rowPtr, colIdx, val_b, target_row, A, B, out, nseg, K, st);
-    return sddmm_f64_launch<3>(rowPtr, colIdx, val_b, target_row, A, B, out, nseg, K, st);
+#define PSP_F64(NR_, SPLIT_) sddmm_f64_launch<NR_, SPLIT_>(rowPtr, colIdx, val_b, target_row, A, B, out, nseg, K, st)
+    if (vec_size == 1) return target_row ? PSP_F64(1, true) : PSP_F64(1, false);
+    if (vec_size == 2) return target_row ? PSP_F64(2, true) : PSP_F64(2, false);
+    return target_row ? PSP_F64(3, true) : PSP_F64(3, false);
+#undef PSP_F64
 }

@@ -29,6 +29,22 @@ template <int LOGL> __device__ __forceinline__ float psp_group_sum(float v)
     return v;
 }
 
+// the same for double: both halves of a value cross the lanes, then they are added as one number
+template <int LOGL> __device__ __forceinline__ double psp_group_sum(double v)
+{
+#define PSP_DPP_ADD64(CTRL)                                                                            \
+    v += __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true),     \
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true))
+    if constexpr (LOGL >= 1) PSP_DPP_ADD64(0xB1);
+    if constexpr (LOGL >= 2) PSP_DPP_ADD64(0x4E);
+    if constexpr (LOGL >= 3) PSP_DPP_ADD64(0x141);
+    if constexpr (LOGL >= 4) PSP_DPP_ADD64(0x140);
+#undef PSP_DPP_ADD64
+    if constexpr (LOGL >= 5) v += psp_bperm_f((int)((threadIdx.x ^ 16) & 63), v);
+    if constexpr (LOGL >= 6) v += psp_bperm_f((int)((threadIdx.x ^ 32) & 63), v);
+    return v;
+}
+
 // Maximum over aligned groups of 2^LOGL lanes (all lanes of the group active); every lane receives it.
 template <int LOGL> __device__ __forceinline__ float psp_group_max(float v)
 {
@@ -57,25 +73,28 @@ template <int LOGL> __device__ __forceinline__ float psp_group_max(float v)
 // takes consecutive tiles of 2^logW entries, finds the rows that hold them with a 64-ary search in rowPtr and walks
 // them window by window (up to 64 rows at a time, cut at the tile's ends).  Every entry's result is independent, so a
 // row may be cut anywhere, and a hub row of 10^5 entries spreads over a hundred wavefronts instead of pinning one.
-template <int LOGL, int C, int V, int U, int NR, bool SPLIT, bool SCALE, bool BAL = false>
+// T: float, or double in pieces of V = 2 (generic_f64.hip).
+template <int LOGL, int C, int V, int U, int NR, bool SPLIT, bool SCALE, bool BAL = false, typename T = float>
 __global__ void __launch_bounds__(512)
-psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const float *__restrict__ val,
-                 const int *__restrict__ target_row, const float *__restrict__ A, const float *__restrict__ B,
-                 float *__restrict__ out, int nseg, int K, int logW, int tiles, int stripe, float *__restrict__ row_max)
+psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const T *__restrict__ val,
+                 const int *__restrict__ target_row, const T *__restrict__ A, const T *__restrict__ B,
+                 T *__restrict__ out, int nseg, int K, int logW, int tiles, int stripe, float *__restrict__ row_max)
 {
-    typedef typename psp_vec<V>::type vec_t;
+    typedef typename psp_vec<V, T>::type vec_t;
+    typedef T pair_t __attribute__((ext_vector_type(2)));
     constexpr bool BCSR = NR > 1;  // NR rows per stored entry: 1 = CSR, 2 = 2x1 blocks, 3 = 3x1 blocks
     constexpr int L = 1 << LOGL;
     constexpr int R = PSP_WAVE >> LOGL;
     static_assert(U <= L, "unroll must not exceed the group width");
     static_assert(!BAL || !SPLIT, "the entry-balanced walk is for the plain layouts (row-split input is balanced already)");
     __shared__ int2 s_seg[PSP_MAX_WAVES][PSP_WAVE];  // (end offset, A row) of the wavefront's filled segments
-    // CSR results of narrow groups wait here until the group has 32 of them (a 128-byte line of `out`) and then leave
+    // CSR results of narrow groups wait here until the group has a 128-byte line of `out` together and then leave
     // in one burst of stores: a group stores only L floats at a time, and lines written piecemeal are evicted from the
     // L2 half-written by the gather stream (measured: 3x the result's bytes in HBM writes at L = 4).
     // 2x1 blocks hold pairs (16 blocks to a line); 3x1 blocks are stored directly.
-    constexpr int HOLD = (NR <= 2 && LOGL >= 2 && LOGL + NR <= 5) ? ((32 / NR) >> LOGL) : 1;  // chunks held back per group
-    __shared__ __align__(8) float s_hold[HOLD > 1 ? PSP_MAX_WAVES : 1][HOLD > 1 ? HOLD * PSP_WAVE * NR : 1];
+    constexpr int LINE = 128 / sizeof(T);
+    constexpr int HOLD = (NR <= 2 && LOGL >= 2 && ((LINE / NR) >> LOGL) >= 2) ? ((LINE / NR) >> LOGL) : 1;  // chunks held back per group
+    __shared__ __align__(16) T s_hold[HOLD > 1 ? PSP_MAX_WAVES : 1][HOLD > 1 ? HOLD * PSP_WAVE * NR : 1];
 
     const int lane = threadIdx.x & (PSP_WAVE - 1);
     const int wave = threadIdx.x >> 6;
@@ -125,20 +144,20 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
     if (a0 >= b0) return;  // the whole group leaves together; nothing below reads other groups' lanes
 
     // A row(s) of a segment; dead tail vectors and repeated columns are zero so they add nothing to the dot product
-    auto load_a = [&](int key, float (&dst)[NR][C][V]) {
+    auto load_a = [&](int key, T (&dst)[NR][C][V]) {
 #pragma unroll
         for (int r = 0; r < NR; r++)
 #pragma unroll
             for (int i = 0; i < C; i++) {
                 vec_t t;
-                if constexpr (V == 1) t = 0.0f;
+                if constexpr (V == 1) t = (T)0;
                 else {
 #pragma unroll
-                    for (int e = 0; e < V; e++) t[e] = 0.0f;
+                    for (int e = 0; e < V; e++) t[e] = (T)0;
                 }
-                if (live[i]) t = psp_load_vec<V>(A + (size_t)(key * NR + r) * (size_t)K + off[i]);
+                if (live[i]) t = psp_load_vec<V, T>(A + (size_t)(key * NR + r) * (size_t)K + off[i]);
 #pragma unroll
-                for (int e = 0; e < V; e++) dst[r][i][e] = e >= dup[i] ? psp_elem<V>(t, e) : 0.0f;
+                for (int e = 0; e < V; e++) dst[r][i][e] = e >= dup[i] ? psp_elem<V, T>(t, e) : (T)0;
             }
     };
 
@@ -147,7 +166,7 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         if (w_seg[cur + step - 1].x <= a0) cur += step;
     int row_end = w_seg[cur].x;
     int mykey = w_seg[cur].y;
-    float a[NR][C][V], a_nxt[NR][C][V];
+    T a[NR][C][V], a_nxt[NR][C][V];
     load_a(mykey, a);
     {
         const int nk = cur + 1 < PSP_WAVE ? w_seg[cur + 1].y : -1;
@@ -160,27 +179,27 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         if (sub == 0 && m > PSP_F32_LOWEST) psp_atomic_max_f32(row_max + key, m);
         lmax = PSP_F32_LOWEST;
     };
-    const bool want_max = !BCSR && row_max != nullptr;  // uniform
+    const bool want_max = sizeof(T) == 4 && !BCSR && row_max != nullptr;  // uniform
 
     // lane `sub` of the group picks up entry base+sub (column index and, where the format has one, its value); the
     // next chunk's are requested before the current chunk is worked on
-    auto fetch = [&](int base, int &c_out, float (&g_out)[NR]) {
+    auto fetch = [&](int base, int &c_out, T (&g_out)[NR]) {
         const int q = base + sub;
         const int qq = q < b0 ? q : b0 - 1;
         c_out = colIdx[qq];
         if constexpr (NR == 2) {
-            const psp_f32x2 t = ((const psp_f32x2 *)val)[qq];
+            const pair_t t = ((const pair_t *)val)[qq];
             g_out[0] = t[0];
             g_out[1] = t[1];
         } else if constexpr (NR > 2) {
 #pragma unroll
             for (int r = 0; r < NR; r++) g_out[r] = val[(size_t)qq * NR + r];
         } else {
-            g_out[0] = SCALE ? val[qq] : 1.0f;
+            g_out[0] = SCALE ? val[qq] : (T)1;
         }
     };
     int c_cur;
-    float gate[NR];
+    T gate[NR];
     fetch(a0, c_cur, gate);
     int held = 0;         // chunks waiting in s_hold (group-uniform)
     int hold_base = a0;   // entry of the first of them
@@ -190,7 +209,7 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         for (int j = 0; j < HOLD; j++) {
             const int pp = hold_base + (j << LOGL) + sub;
             if (j < held && pp < b0) {
-                if constexpr (NR == 2) ((psp_f32x2 *)out)[pp] = ((const psp_f32x2 *)s_hold[wave])[j * PSP_WAVE + lane];
+                if constexpr (NR == 2) ((pair_t *)out)[pp] = ((const pair_t *)s_hold[wave])[j * PSP_WAVE + lane];
                 else out[pp] = s_hold[wave][j * PSP_WAVE + lane];
             }
         }
@@ -202,13 +221,13 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         const int p = base + sub;
         const bool ok = p < b0;
         int c_nxt = 0;
-        float gate_nxt[NR];
+        T gate_nxt[NR];
 #pragma unroll
-        for (int r = 0; r < NR; r++) gate_nxt[r] = 0.0f;
+        for (int r = 0; r < NR; r++) gate_nxt[r] = (T)0;
         if (base + L < b0) fetch(base + L, c_nxt, gate_nxt);
-        float res[NR];
+        T res[NR];
 #pragma unroll
-        for (int r = 0; r < NR; r++) res[r] = 0.0f;
+        for (int r = 0; r < NR; r++) res[r] = (T)0;
 
         const int cnt = min(L, b0 - base);
         int k = 0;
@@ -222,24 +241,26 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
                 vec_t bv[U][C];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const float *br = B + (size_t)ck[u] * (size_t)K;
+                    const T *br = B + (size_t)ck[u] * (size_t)K;
 #pragma unroll
-                    for (int i = 0; i < C; i++) bv[u][i] = psp_load_vec<V>(br + off[i]);
+                    for (int i = 0; i < C; i++) bv[u][i] = psp_load_vec<V, T>(br + off[i]);
                 }
 #pragma unroll
                 for (int u = 0; u < U; u++)
 #pragma unroll
                     for (int r = 0; r < NR; r++) {
-                        float part = 0.0f;
+                        T part = (T)0;
 #pragma unroll
                         for (int i = 0; i < C; i++)
 #pragma unroll
-                            for (int e = 0; e < V; e++) part = __builtin_fmaf(a[r][i][e], psp_elem<V>(bv[u][i], e), part);
+                            for (int e = 0; e < V; e++) part = psp_fma(a[r][i][e], psp_elem<V, T>(bv[u][i], e), part);
                         part = psp_group_sum<LOGL>(part);
                         // positions past run_end belong to the next row: their dot product with this A row is dropped
                         if (sub == k + u && k + u < run_end) {
                             res[r] = part;
-                            if (!BCSR && want_max) lmax = fmaxf(lmax, SCALE ? part * gate[0] : part);
+                            if constexpr (sizeof(T) == 4) {
+                                if (!BCSR && want_max) lmax = fmaxf(lmax, SCALE ? part * gate[0] : part);
+                            }
                         }
                     }
             }
@@ -264,23 +285,23 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         if (ok) {
             if constexpr (NR == 2 && HOLD == 1) {
                 // entries of a block whose value is zero are padding: written as zero (sddmm_kernel.cu:1103,1115)
-                psp_f32x2 o;
-                o[0] = gate[0] != 0.0f ? res[0] : 0.0f;
-                o[1] = gate[1] != 0.0f ? res[1] : 0.0f;
-                ((psp_f32x2 *)out)[p] = o;
+                pair_t o;
+                o[0] = gate[0] != (T)0 ? res[0] : (T)0;
+                o[1] = gate[1] != (T)0 ? res[1] : (T)0;
+                ((pair_t *)out)[p] = o;
             } else if constexpr (NR > 2) {
 #pragma unroll
-                for (int r = 0; r < NR; r++) out[(size_t)p * NR + r] = gate[r] != 0.0f ? res[r] : 0.0f;
+                for (int r = 0; r < NR; r++) out[(size_t)p * NR + r] = gate[r] != (T)0 ? res[r] : (T)0;
             } else if constexpr (HOLD == 1) {
                 out[p] = SCALE ? res[0] * gate[0] : res[0];
             }
         }
         if constexpr (HOLD > 1) {
             if constexpr (NR == 2) {
-                psp_f32x2 o;  // padding entries of a block (value zero) are written as zero (sddmm_kernel.cu:1103,1115)
-                o[0] = gate[0] != 0.0f ? res[0] : 0.0f;
-                o[1] = gate[1] != 0.0f ? res[1] : 0.0f;
-                ((psp_f32x2 *)s_hold[wave])[held * PSP_WAVE + lane] = o;
+                pair_t o;  // padding entries of a block (value zero) are written as zero (sddmm_kernel.cu:1103,1115)
+                o[0] = gate[0] != (T)0 ? res[0] : (T)0;
+                o[1] = gate[1] != (T)0 ? res[1] : (T)0;
+                ((pair_t *)s_hold[wave])[held * PSP_WAVE + lane] = o;
             } else {
                 s_hold[wave][held * PSP_WAVE + lane] = SCALE ? res[0] * gate[0] : res[0];
             }

@@ -37,30 +37,37 @@ typedef float psp_f32x4 __attribute__((ext_vector_type(4)));
 // Widths below 4 use single floats.  Before, widths off the multiples of 4 ran on 8- or 4-byte loads with two and four
 // times the lanes or column tiles: Chung-Lu graph of 200 003 rows and 3.0 M entries, N = 47: 167 us.
 typedef float psp_f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-template <int V> struct psp_vec;
-template <> struct psp_vec<1> { typedef float type, mem; };
-template <> struct psp_vec<4> { typedef psp_f32x4 type; typedef psp_f32x4_a4 mem; };
+typedef double psp_f64x2 __attribute__((ext_vector_type(2)));
+typedef double psp_f64x2_a8 __attribute__((ext_vector_type(2), aligned(8)));
+template <int V, typename T = float> struct psp_vec;
+template <> struct psp_vec<1, float> { typedef float type, mem; };
+template <> struct psp_vec<4, float> { typedef psp_f32x4 type; typedef psp_f32x4_a4 mem; };
+template <> struct psp_vec<1, double> { typedef double type, mem; };
+template <> struct psp_vec<2, double> { typedef psp_f64x2 type; typedef psp_f64x2_a8 mem; };
 static __host__ __device__ __forceinline__ int psp_vec_width(int N) { return N >= 4 ? 4 : 1; }
-template <int V> __device__ __forceinline__ typename psp_vec<V>::type psp_load_vec(const float *p) { return *(const typename psp_vec<V>::mem *)p; }
+template <int V, typename T> __device__ __forceinline__ typename psp_vec<V, T>::type psp_load_vec(const T *p) { return *(const typename psp_vec<V, T>::mem *)p; }
 // first column of the piece that starts at column `col` of rows of N columns
 template <int V> __device__ __forceinline__ int psp_vec_col(int col, int N) { return min(col, N - V); }
 
-template <int V> __device__ __forceinline__ float psp_elem(const typename psp_vec<V>::type &v, int e) { return v[e]; }
-template <> __device__ __forceinline__ float psp_elem<1>(const float &v, int) { return v; }
+template <int V, typename T = float> __device__ __forceinline__ T psp_elem(const typename psp_vec<V, T>::type &v, int e)
+{
+    if constexpr (V == 1) return v;
+    else return v[e];
+}
 
 // max(x, 0) per element; a NaN stays a NaN, as with torch.relu
-template <int V> __device__ __forceinline__ void psp_relu_vec(typename psp_vec<V>::type &v)
+template <int V, typename T> __device__ __forceinline__ void psp_relu_vec(typename psp_vec<V, T>::type &v)
 {
-    if constexpr (V == 1) v = v < 0.0f ? 0.0f : v;
+    if constexpr (V == 1) v = v < (T)0 ? (T)0 : v;
     else {
 #pragma unroll
-        for (int e = 0; e < V; e++) v[e] = v[e] < 0.0f ? 0.0f : v[e];
+        for (int e = 0; e < V; e++) v[e] = v[e] < (T)0 ? (T)0 : v[e];
     }
 }
 
-template <int V> __device__ __forceinline__ void psp_store_vec(float *p, const float (&a)[V])
+template <int V, typename T> __device__ __forceinline__ void psp_store_vec(T *p, const T (&a)[V])
 {
-    typename psp_vec<V>::type t;
+    typename psp_vec<V, T>::type t;
     if constexpr (V == 1) t = a[0];
     else {
 #pragma unroll
@@ -68,7 +75,7 @@ template <int V> __device__ __forceinline__ void psp_store_vec(float *p, const f
     }
     // Y is written once and not read again by this kernel: the streaming hint keeps it from displacing rows of X
     // in the L2 (measured 1-5 % faster; the same hint on colIdx / val loads is slower, other column tiles re-read them)
-    __builtin_nontemporal_store((typename psp_vec<V>::mem)t, (typename psp_vec<V>::mem *)p);
+    __builtin_nontemporal_store((typename psp_vec<V, T>::mem)t, (typename psp_vec<V, T>::mem *)p);
 }
 
 // COUNT consecutive 4-byte words starting at a 4-byte aligned address, fetched in the widest pieces (16, 8, 4 bytes)
@@ -97,6 +104,18 @@ __device__ __forceinline__ float psp_bperm_f(int src_lane, float v)
 {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(src_lane << 2, __float_as_int(v)));
 }
+__device__ __forceinline__ double psp_bperm_f(int src_lane, double v)
+{
+    return __hiloint2double(psp_bperm_i(src_lane, __double2hiint(v)), psp_bperm_i(src_lane, __double2loint(v)));
+}
+__device__ __forceinline__ float psp_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double psp_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// a stored value from the 4-byte words it was loaded as
+template <typename T> __device__ __forceinline__ T psp_from_words(const int *w)
+{
+    if constexpr (sizeof(T) == 4) return __int_as_float(w[0]);
+    else return __hiloint2double(w[1], w[0]);
+}
 
 #define PSP_MAX_WAVES 8  // blkWarpNum is 4 or 8
 
@@ -115,16 +134,19 @@ __device__ __forceinline__ float psp_bperm_f(int src_lane, float v)
 // configuration from five to four wavefronts per SIMD and made the product 25-45 % slower on the community-ordered
 // graph (341 against 243 us at N = 32, 1018 against 703 at N = 128; the separate pass costs 66 and 256 us).
 // SINGLE: one register set instead of two (the walk below).
-template <int C, int V, int U, int NR, bool SPLIT, bool SM, bool ACT = false, bool SINGLE = false>
+// T: float, or double in pieces of V = 2 (generic_f64.hip).
+template <int C, int V, int U, int NR, bool SPLIT, bool SM, bool ACT = false, bool SINGLE = false, typename T = float>
 __global__ void __launch_bounds__(512)
-psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const float *__restrict__ val,
-                const int *__restrict__ target_row, const float *__restrict__ X, float *__restrict__ Y,
+psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const T *__restrict__ val,
+                const int *__restrict__ target_row, const T *__restrict__ X, T *__restrict__ Y,
                 int nseg, int N, int logL, int logW, int tiles, int stripe, int align_pct,
                 const float *__restrict__ row_max, float *__restrict__ row_sum, int relu_x, int tail_rows)
 {
     static_assert(!SM || NR == 1, "softmax weights exist for the CSR layouts only");
     static_assert(!(SM && ACT), "the softmax-weighted product takes no activation argument");
-    typedef typename psp_vec<V>::type vec_t;
+    static_assert(!SM || sizeof(T) == 4, "softmax weights are single precision");
+    typedef typename psp_vec<V, T>::type vec_t;
+    constexpr int WORDS = sizeof(T) / 4;  // of a stored value
     __shared__ int2 s_seg[PSP_MAX_WAVES][PSP_WAVE];  // (end offset, output row) of the wavefront's segments
     __shared__ float s_m[SM ? PSP_MAX_WAVES : 1][SM ? PSP_WAVE : 1];  // SM: reference maximum of each segment's row
 
@@ -135,8 +157,8 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         const int tile_w = (C * V) << logL;
         const int col0 = blockIdx.y * tile_w;
         const int w = min(tile_w, N - col0);
-        float *yt = Y + (size_t)nseg * NR * (size_t)N + col0;
-        for (int i = threadIdx.x; i < tail_rows * w; i += PSP_WAVE) yt[(size_t)(i / w) * (size_t)N + i % w] = 0.0f;
+        T *yt = Y + (size_t)nseg * NR * (size_t)N + col0;
+        for (int i = threadIdx.x; i < tail_rows * w; i += PSP_WAVE) yt[(size_t)(i / w) * (size_t)N + i % w] = (T)0;
     }
 
     const int tile = psp_xcd_tile(stripe);
@@ -184,12 +206,12 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                     const int tile_col0 = blockIdx.y * ((C * V) << logL);
 #pragma unroll
                     for (int r = 0; r < NR; r++) {
-                        float *yr = Y + (size_t)((s0 + i) * NR + r) * (size_t)N;
+                        T *yr = Y + (size_t)((s0 + i) * NR + r) * (size_t)N;
 #pragma unroll
                         for (int c = 0; c < C; c++) {
                             const int col = tile_col0 + ((c << logL) + sub) * V;
-                            const float z[V] = {};
-                            if (col < N) psp_store_vec<V>(yr + psp_vec_col<V>(col, N), z);
+                            const T z[V] = {};
+                            if (col < N) psp_store_vec<V, T>(yr + psp_vec_col<V>(col, N), z);
                         }
                     }
                 }
@@ -254,13 +276,13 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         }
     }
 
-    float acc[NR][C][V], head[NR][C][V];
+    T acc[NR][C][V], head[NR][C][V];
 #pragma unroll
     for (int r = 0; r < NR; r++)
 #pragma unroll
         for (int i = 0; i < C; i++)
 #pragma unroll
-            for (int e = 0; e < V; e++) acc[r][i][e] = head[r][i][e] = 0.0f;
+            for (int e = 0; e < V; e++) acc[r][i][e] = head[r][i][e] = (T)0;
     float acc_l = 0.0f, head_l = 0.0f, m_cur = 0.0f;  // SM: weight sum of the running row / stashed head, row maximum
 
     // out: a finished row goes to Y; `shared` = other wavefronts add to the same row (row-split formats)
@@ -278,18 +300,18 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         }
 #pragma unroll
         for (int r = 0; r < NR; r++) {
-            float *yr = Y + (size_t)(key * NR + r) * (size_t)N;
+            T *yr = Y + (size_t)(key * NR + r) * (size_t)N;
 #pragma unroll
             for (int i = 0; i < C; i++) {
                 if (!live[i]) continue;
                 if (!SPLIT || !shared) {
-                    psp_store_vec<V>(yr + off[i], acc[r][i]);
+                    psp_store_vec<V, T>(yr + off[i], acc[r][i]);
                 } else {
                     // a piece that was moved back repeats columns of the one in front of it: they get zeros here (a plain
                     // store may write them twice, both lanes hold the same sum)
                     const int dup = (int)(blockIdx.y * ((C * V) << logL)) + ((i << logL) + sub) * V - off[i];
 #pragma unroll
-                    for (int e = 0; e < V; e++) unsafeAtomicAdd(yr + off[i] + e, e >= dup ? acc[r][i][e] : 0.0f);
+                    for (int e = 0; e < V; e++) unsafeAtomicAdd(yr + off[i] + e, e >= dup ? acc[r][i][e] : (T)0);
                 }
             }
         }
@@ -326,10 +348,10 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         const int p0_ = (base) + sub * U;                                                    \
         if (p0_ + U <= b) {                                                                  \
             psp_load_words<U>(colIdx + p0_, c_out);                                          \
-            int w_[U * NR];                                                                  \
-            psp_load_words<U * NR>((const int *)val + (size_t)p0_ * NR, w_);                 \
+            int w_[U * NR * WORDS];                                                          \
+            psp_load_words<U * NR * WORDS>((const int *)val + (size_t)p0_ * (NR * WORDS), w_); \
             _Pragma("unroll") for (int u_ = 0; u_ < U; u_++)                                 \
-                _Pragma("unroll") for (int r_ = 0; r_ < NR; r_++) v_out[u_][r_] = __int_as_float(w_[u_ * NR + r_]); \
+                _Pragma("unroll") for (int r_ = 0; r_ < NR; r_++) v_out[u_][r_] = psp_from_words<T>(w_ + (u_ * NR + r_) * WORDS); \
         } else {                                                                             \
             _Pragma("unroll") for (int u_ = 0; u_ < U; u_++)                                 \
             {                                                                                \
@@ -338,20 +360,20 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                 c_out[u_] = colIdx[pp_];                                                     \
                 _Pragma("unroll") for (int r_ = 0; r_ < NR; r_++)                            \
                 {                                                                            \
-                    const float t_ = val[(size_t)pp_ * NR + r_];                             \
-                    v_out[u_][r_] = ok_ ? t_ : 0.0f;                                         \
+                    const T t_ = val[(size_t)pp_ * NR + r_];                             \
+                    v_out[u_][r_] = ok_ ? t_ : (T)0;                                          \
                 }                                                                            \
             }                                                                                \
         }                                                                                    \
     }
 
     int c_cur[U], c_nxt[U];
-    float v_cur[U][NR], v_nxt[U][NR];
+    T v_cur[U][NR], v_nxt[U][NR];
 #pragma unroll
     for (int u = 0; u < U; u++) {
         c_cur[u] = c_nxt[u] = 0;
 #pragma unroll
-        for (int r = 0; r < NR; r++) v_cur[u][r] = v_nxt[u][r] = 0.0f;
+        for (int r = 0; r < NR; r++) v_cur[u][r] = v_nxt[u][r] = (T)0;
     }
     if (busy) PSP_FETCH(a, c_cur, v_cur);
 
@@ -379,7 +401,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
 #pragma unroll
                 for (int i = 0; i < C; i++)
 #pragma unroll
-                    for (int e = 0; e < V; e++) acc[r][i][e] = 0.0f;
+                    for (int e = 0; e < V; e++) acc[r][i][e] = (T)0;
             acc_l = 0.0f;
             first_run = false;
             mykey = nkey;
@@ -409,7 +431,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
 
 #define PSP_DECLARE(S)      \
     int S##_ck[U], S##_pos; \
-    float S##_vk[U][NR];    \
+    T S##_vk[U][NR];        \
     vec_t S##_x[U][C];
 #define PSP_GATHER(S)                                                                                  \
     {                                                                                                  \
@@ -432,8 +454,8 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         }                                                                                              \
         _Pragma("unroll") for (int u = 0; u < U; u++)                                                  \
         {                                                                                              \
-            const float *xr = X + (size_t)S##_ck[u] * (size_t)N;                                       \
-            _Pragma("unroll") for (int i = 0; i < C; i++) S##_x[u][i] = psp_load_vec<V>(xr + off[i]);  \
+            const T *xr = X + (size_t)S##_ck[u] * (size_t)N;                                       \
+            _Pragma("unroll") for (int i = 0; i < C; i++) S##_x[u][i] = psp_load_vec<V, T>(xr + off[i]); \
         }                                                                                              \
         pos += U;                                                                                      \
         jb++;                                                                                          \
@@ -442,7 +464,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
     {                                                                                                  \
         if (ACT && relu_x) {                                                                           \
             _Pragma("unroll") for (int u = 0; u < U; u++)                                              \
-                _Pragma("unroll") for (int i = 0; i < C; i++) psp_relu_vec<V>(S##_x[u][i]);            \
+                _Pragma("unroll") for (int i = 0; i < C; i++) psp_relu_vec<V, T>(S##_x[u][i]);            \
         }                                                                                              \
         _Pragma("unroll") for (int u = 0; u < U; u++)                                                  \
         {                                                                                              \
@@ -455,10 +477,10 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                 _Pragma("unroll") for (int r = 0; r < NR; r++)                                         \
                 {                                                                                      \
                     /* 2x1 blocks: a zero entry is skipped (SpMM_kernel.cu:1399,1405) */               \
-                    if (NR == 1 || S##_vk[u][r] != 0.0f) {                                             \
+                    if (NR == 1 || S##_vk[u][r] != (T)0) {                                             \
                         _Pragma("unroll") for (int i = 0; i < C; i++)                                  \
                             _Pragma("unroll") for (int e = 0; e < V; e++)                              \
-                                acc[r][i][e] = __builtin_fmaf(S##_vk[u][r], psp_elem<V>(S##_x[u][i], e), acc[r][i][e]); \
+                                acc[r][i][e] = psp_fma(S##_vk[u][r], psp_elem<V, T>(S##_x[u][i], e), acc[r][i][e]); \
                     }                                                                                  \
                 }                                                                                      \
                 if (p1 == row_end && p1 < b) next_segment();                                           \
@@ -549,7 +571,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
             for (int i = 0; i < C; i++)
 #pragma unroll
                 for (int e = 0; e < V; e++) {
-                    const float h = psp_bperm_f(src_c, head[r][i][e]);
+                    const T h = psp_bperm_f(src_c, head[r][i][e]);
                     if (has_tail && (hf & F_HEAD)) acc[r][i][e] += h;
                 }
         if (has_tail && (!(hf & F_HEAD) || (hf & F_CLOSED) || src >= PSP_WAVE)) {

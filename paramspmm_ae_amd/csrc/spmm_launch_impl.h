@@ -3,24 +3,15 @@
 #include <stdlib.h>
 #include "spmm_kernel.h"
 
-template <int NR, bool SPLIT>
-int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, const int *target_row,
-                    const float *X, float *Y, int nrows, int N, int rows_out, int CF, int blkWarpNum,
-                    hipStream_t stream, const float *row_max, float *row_sum, int relu_x)
+// Enqueues kernel `k` with the mapping of `plan`: segments per wavefront, the rows the kernel does not store to, the grid.
+// T = float or double (generic_f64.hip).
+template <int NR, bool SPLIT, typename T, typename KERNEL>
+int psp_spmm_enqueue(KERNEL k, const psp_spmm_plan &plan, const int *rowPtr, const int *colIdx, const T *val, const int *target_row,
+                     const T *X, T *Y, int nrows, int N, int rows_out, hipStream_t stream, const float *row_max, float *row_sum,
+                     int relu_x)
 {
-    psp_spmm_plan plan;
-    int rc = psp_spmm_plan_for(N, CF, blkWarpNum, &plan);
-    if (rc != PSP_OK) return rc;
-    PSP_REQUIRE(nrows >= 0 && rows_out >= 0, "spmm: negative size (rows %d, rows_out %d)", nrows, rows_out);
-    PSP_REQUIRE(Y != nullptr || rows_out == 0, "spmm: Y is null");
-    if (!SPLIT)
-        PSP_REQUIRE((long long)nrows * NR <= rows_out, "spmm: Y has %d rows, the matrix needs %lld", rows_out,
-                    (long long)nrows * NR);
-    if (nrows > 0) {
-        PSP_REQUIRE(rowPtr && X, "spmm: rowPtr / X is null");
-        PSP_REQUIRE(!SPLIT || target_row, "spmm: target_row is null");
-    }
-
+    int rc = PSP_OK;
+    constexpr int WORDS = sizeof(T) / 4;  // Y is cleared by 4-byte words: all-zero bits are 0 in both precisions
     int logL = 0;
     while ((1 << logL) < plan.lanes_per_row) logL++;
     // Segments per wavefront.  Plain input gets one row per lane group on average: rows that are neighbours in
@@ -49,23 +40,22 @@ int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, cons
         // The kernel stores rows that one wavefront holds alone and adds (atomics) to rows shared by several
         // wavefronts.  Large outputs are therefore not cleared as a whole: a pass over the segments clears only
         // the shared rows and the rows without segments.  Small outputs are cheaper to clear outright.
-        if ((long long)rows_out * N >= opt.split_clear_min && nrows > 0)
-            rc = psp_split_clear(rowPtr, target_row, Y, nrows, N, NR, rows_out, logW, stream);
+        if ((long long)rows_out * N * WORDS >= opt.split_clear_min && nrows > 0)
+            rc = psp_split_clear(rowPtr, target_row, (float *)Y, nrows, N * WORDS, NR, rows_out, logW, stream);
         else
-            rc = psp_zero_f32(Y, (size_t)rows_out * N, stream);
+            rc = psp_zero_f32((float *)Y, (size_t)rows_out * N * WORDS, stream);
     } else {
         // rows past the matrix's own: up to PSP_SPMM_TAIL_ROWS_MAX are zeroed by the kernel itself (tail_rows)
         const size_t covered = (size_t)nrows * NR;
         tail_rows = (int)std::min<size_t>((size_t)rows_out - covered, (size_t)PSP_SPMM_TAIL_ROWS_MAX + 1);
         if (tail_rows > PSP_SPMM_TAIL_ROWS_MAX || nrows == 0) {
             tail_rows = 0;
-            rc = psp_zero_f32(Y + covered * N, ((size_t)rows_out - covered) * N, stream);
+            rc = psp_zero_f32((float *)(Y + covered * N), ((size_t)rows_out - covered) * N * WORDS, stream);
         }
     }
     if (rc != PSP_OK) return rc;
     if (nrows == 0) return PSP_OK;
     const bool softmax = row_max != nullptr;
-    PSP_REQUIRE(!(softmax && relu_x), "spmm: the softmax-weighted product takes no activation argument");
     if (softmax && SPLIT) {
         PSP_REQUIRE(row_sum, "spmm softmax: row_sum workspace is null");
         rc = psp_zero_f32(row_sum, (size_t)rows_out, stream);
@@ -73,11 +63,6 @@ int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, cons
     }
 
     const int segs_per_block = plan.waves_per_block << logW;
-    psp_spmm_kernel_t k = psp_spmm_lookup<NR, SPLIT>(plan.coarsen, psp_vec_width(N), plan.unroll, plan.lanes_per_row, softmax, relu_x != 0);
-    if (!k)
-        return psp_fail(PSP_ERR_ARG, "spmm%s: no kernel for coarsen %d vec %d unroll %d%s", softmax ? " softmax" : "", plan.coarsen,
-                        psp_vec_width(N), plan.unroll, softmax ? " (needs N % 4 == 0 and CF <= 4)" : "");
-
     const int align_pct = opt.whole_rows ? (1 << 30) : (plan.even_split ? 0 : opt.align_pct);
     const psp_grid1d g = psp_xcd_grid(psp_ceil_div(nrows, segs_per_block),
                                       (plan.xcd_stripe_rows ? plan.xcd_stripe_rows : opt.stripe_rows) / segs_per_block);
@@ -85,5 +70,31 @@ int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, cons
     hipLaunchKernelGGL(k, grid, block, 0, stream, rowPtr, colIdx, val, target_row, X, Y, nrows, N, logL, logW, g.real, g.stripe, align_pct, row_max, row_sum, relu_x, tail_rows);
     rc = psp_check_launch("spmm kernel");
     if (rc != PSP_OK || !(softmax && SPLIT)) return rc;
-    return psp_row_scale(Y, row_sum, rows_out, N, stream);  // rows that several wavefronts added to
+    if constexpr (WORDS == 1) return psp_row_scale(Y, row_sum, rows_out, N, stream);  // rows that several wavefronts added to
+    return rc;
+}
+
+template <int NR, bool SPLIT>
+int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, const int *target_row,
+                    const float *X, float *Y, int nrows, int N, int rows_out, int CF, int blkWarpNum,
+                    hipStream_t stream, const float *row_max, float *row_sum, int relu_x)
+{
+    psp_spmm_plan plan;
+    int rc = psp_spmm_plan_for(N, CF, blkWarpNum, &plan);
+    if (rc != PSP_OK) return rc;
+    PSP_REQUIRE(nrows >= 0 && rows_out >= 0, "spmm: negative size (rows %d, rows_out %d)", nrows, rows_out);
+    PSP_REQUIRE(Y != nullptr || rows_out == 0, "spmm: Y is null");
+    if (!SPLIT)
+        PSP_REQUIRE((long long)nrows * NR <= rows_out, "spmm: Y has %d rows, the matrix needs %lld", rows_out,
+                    (long long)nrows * NR);
+    PSP_REQUIRE(!(row_max && relu_x), "spmm: the softmax-weighted product takes no activation argument");
+    if (nrows > 0) {
+        PSP_REQUIRE(rowPtr && X, "spmm: rowPtr / X is null");
+        PSP_REQUIRE(!SPLIT || target_row, "spmm: target_row is null");
+    }
+    psp_spmm_kernel_t k = psp_spmm_lookup<NR, SPLIT>(plan.coarsen, psp_vec_width(N), plan.unroll, plan.lanes_per_row, row_max != nullptr, relu_x != 0);
+    if (!k && nrows > 0)
+        return psp_fail(PSP_ERR_ARG, "spmm%s: no kernel for coarsen %d vec %d unroll %d%s", row_max ? " softmax" : "", plan.coarsen,
+                        psp_vec_width(N), plan.unroll, row_max ? " (needs N % 4 == 0 and CF <= 4)" : "");
+    return psp_spmm_enqueue<NR, SPLIT>(k, plan, rowPtr, colIdx, val, target_row, X, Y, nrows, N, rows_out, stream, row_max, row_sum, relu_x);
 }
