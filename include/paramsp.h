@@ -41,9 +41,10 @@ const char *psp_last_error(void);
  *   310: PSP_WINDOW_HALO is 88 (64 before: windowed arrays built by a 300 library do not match these kernels -- build
  *        them again); psp_sddmm_window_f32, psp_attn_window_forward_f32 / _backward_f32, psp_softmax_nll_mean_f32 (+ backward);
  *        option "dense_split";
- *   311: psp_spmm_register_sets (no buffer changed).
+ *   311: psp_spmm_register_sets (no buffer changed);
+ *   312: psp_attn_forward_f32 / _backward_f32 (no buffer changed).
  * The extension modules and the ctypes loader of this package check it when they are imported. */
-#define PSP_ABI_VERSION 311
+#define PSP_ABI_VERSION 312
 int psp_version(void);
 
 /* How a (N, CF, blkWarpNum) request of the Python layer maps onto the wave64 kernels.
@@ -372,6 +373,25 @@ int psp_attn_window_forward_f32(const int *rowPtr_w, const int *colIdx_w, const 
                                 float *Y, int M, int nnz, int K, int rows_out, psp_stream_t stream);
 int psp_attn_window_backward_f32(const int *rowPtr_w, const int *colIdx_w, const float *att, const float *dY, float *G,
                                  float *wsum, int M, int nnz, int K, int rows_out, psp_stream_t stream);
+
+/* The same layer on the PCSR formats (fmt 0 CSR, 1 row-split CSR, 2 2x1 blocks, 3 row-split 2x1 blocks; the arrays are
+ * those of the format's SpMM), any K from 4 to PSP_ATTN_MAX_K, no alignment beyond that of a float.
+ *   forward:  att in the format's entry order (2x1 blocks: [nblk, 2]; val_b says which entries exist, padding reads zero),
+ *             Y[i] = sum_p att[p] X[col(p)].  val_b NULL for fmt 0 / 1.
+ *   backward: G as above; *wsum as above for fmt 0 / 1, for 2x1 blocks sum over the slots of <dY[row], dY[col]> slot[p]
+ *             (slot [nblk, 2], zero at padding: the reference multiplies the slots of a block-row, in block order, with the
+ *             columns of its CSR entries, gnn_conv.py:166-172, so slot[mask[k]] = colIdx_csr[k]).  workspace: psp_attn_workspace_floats(nrows, K) floats
+ *             of device memory (nrows = rows, block-rows or segments of the format), whose shares are added to *wsum in a
+ *             fixed order.
+ * X, dY: one row per column and two per block-row.  blkWarpNum may carry PSP_BW_STRIPE. */
+#define PSP_ATTN_MAX_K 128
+int psp_attn_forward_f32(int fmt, const int *rowPtr, const int *colIdx, const float *val_b, const int *target_row, const float *X,
+                         const float *alpha, float *att, float *Y, int nrows, int K, int rows_out, int blkWarpNum,
+                         psp_stream_t stream);
+int psp_attn_workspace_floats(int nrows, int K);
+int psp_attn_backward_f32(int fmt, const int *rowPtr, const int *colIdx, const float *att, const int *target_row, const float *slot,
+                          const float *dY, float *G, float *wsum, float *workspace, int nrows, int K, int rows_out, int blkWarpNum,
+                          psp_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------
  * DEVICE: softmax over the stored entries of every CSR row (out[p] = exp(e[p]-max_r) / sum_r).

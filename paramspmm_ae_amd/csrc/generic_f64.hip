@@ -52,7 +52,7 @@ static int f64_log_group(int width)
 }
 
 typedef void (*spmm_f64_kernel_t)(const int *, const int *, const double *, const int *, const double *, double *,
-                                  int, int, int, int, int, int, int, const float *, float *, int, int);
+                                  int, int, int, int, int, int, int, const float *, float *, int, int, psp_plain);
 
 // Mapping: two pieces of two doubles per lane, two entries in flight, lane groups of up to 8 lanes for rows of up to 32
 // doubles (one column tile of 256 bytes) and up to 16 beyond.  Bound by the memory traffic; of thirteen mappings (1 / 2 / 4

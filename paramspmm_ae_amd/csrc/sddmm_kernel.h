@@ -9,27 +9,9 @@
 // (the reference stores one float per warp per non-zero).
 #pragma once
 #include "psp_common.h"
-#include "spmm_kernel.h"  // psp_vec
+#include "spmm_kernel.h"  // psp_vec, psp_group_sum
 
-// Sum over aligned groups of 2^LOGL lanes; every lane of the group receives the total.
-template <int LOGL> __device__ __forceinline__ float psp_group_sum(float v)
-{
-    if constexpr (LOGL >= 1)  // lane ^ 1
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
-    if constexpr (LOGL >= 2)  // lane ^ 2
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));
-    if constexpr (LOGL >= 3)  // mirror inside 8 lanes: the partner sits in the other quad
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));
-    if constexpr (LOGL >= 4)  // mirror inside 16 lanes
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true));
-    if constexpr (LOGL >= 5)  // lane ^ 16 inside 32 lanes
-        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
-    if constexpr (LOGL >= 6)  // lane ^ 32
-        v += __int_as_float(__builtin_amdgcn_ds_bpermute((int)((threadIdx.x ^ 32) & 63) << 2, __float_as_int(v)));
-    return v;
-}
-
-// the same for double: both halves of a value cross the lanes, then they are added as one number
+// psp_group_sum (spmm_kernel.h) for double: both halves of a value cross the lanes, then they are added as one number
 template <int LOGL> __device__ __forceinline__ double psp_group_sum(double v)
 {
 #define PSP_DPP_ADD64(CTRL)                                                                            \

@@ -117,7 +117,45 @@ template <typename T> __device__ __forceinline__ T psp_from_words(const int *w)
     else return __hiloint2double(w[1], w[0]);
 }
 
+// Sum over aligned groups of 2^LOGL lanes; every lane of the group receives the total.
+template <int LOGL> __device__ __forceinline__ float psp_group_sum(float v)
+{
+    if constexpr (LOGL >= 1)  // lane ^ 1
+        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
+    if constexpr (LOGL >= 2)  // lane ^ 2
+        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));
+    if constexpr (LOGL >= 3)  // mirror inside 8 lanes: the partner sits in the other quad
+        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));
+    if constexpr (LOGL >= 4)  // mirror inside 16 lanes
+        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true));
+    if constexpr (LOGL >= 5)  // lane ^ 16 inside 32 lanes
+        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
+    if constexpr (LOGL >= 6)  // lane ^ 32
+        v += __int_as_float(__builtin_amdgcn_ds_bpermute((int)((threadIdx.x ^ 32) & 63) << 2, __float_as_int(v)));
+    return v;
+}
+
 #define PSP_MAX_WAVES 8  // blkWarpNum is 4 or 8
+
+// What a product does besides multiplying the stored values by the gathered rows (last template argument of the kernel).
+struct psp_plain {
+    static constexpr int MODE = 0, LOGL = 0;
+};
+// The attention layer of gnn_conv.py:128-180, whose SDDMM and SpMM of a direction gather the same rows of the same matrix:
+// both from one gather.  The whole width lies inside one lane group of 2^LOGL lanes (one column tile).
+//   forward   score[p] = alpha <X_i, X_j> (in every lane of the group after LOGL DPP additions), stored, and Y_i += score[p] X_j.
+//             2x1 blocks: `val` says which entries exist (non-zero); padding scores are zero.
+//   backward  `val` holds the scores: G_i += score[p] dY_j, and every wavefront's share of sum_p <dY_i, dY_j> f(p), the weight
+//             gradient of gnn_conv.py:166-172, lands in wsum[its first segment >> logW].  f(p) = float(j); for 2x1 blocks
+//             slot[p], because the reference pairs the slots of a block-row with the columns of its CSR entries.
+// Every lane group keeps its row i in registers, the next row's is requested one segment ahead.
+template <int LOGL_, bool BACKWARD> struct psp_attention {
+    static constexpr int MODE = BACKWARD ? 2 : 1, LOGL = LOGL_;
+    const float *alpha;  // forward: one float on the device, null = 1
+    float *score;        // forward
+    float *wsum;         // backward
+    const float *slot;   // backward, 2x1 blocks: [nblk, 2], zero at padding
+};
 
 // NR: rows per stored entry (1 = CSR, 2 = 2x1 BCSR, 3 = 3x1 blocks: the reference's vec_spmm, SpMM_kernel.cu:1653-1972).  SPLIT: segments carry an explicit output row.
 // SM (CSR layouts): the stored values are attention scores e; the product is taken with softmax weights,
@@ -135,18 +173,21 @@ template <typename T> __device__ __forceinline__ T psp_from_words(const int *w)
 // graph (341 against 243 us at N = 32, 1018 against 703 at N = 128; the separate pass costs 66 and 256 us).
 // SINGLE: one register set instead of two (the walk below).
 // T: float, or double in pieces of V = 2 (generic_f64.hip).
-template <int C, int V, int U, int NR, bool SPLIT, bool SM, bool ACT = false, bool SINGLE = false, typename T = float>
+template <int C, int V, int U, int NR, bool SPLIT, bool SM, bool ACT = false, bool SINGLE = false, typename T = float, typename XT = psp_plain>
 __global__ void __launch_bounds__(512)
 psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const T *__restrict__ val,
                 const int *__restrict__ target_row, const T *__restrict__ X, T *__restrict__ Y,
                 int nseg, int N, int logL, int logW, int tiles, int stripe, int align_pct,
-                const float *__restrict__ row_max, float *__restrict__ row_sum, int relu_x, int tail_rows)
+                const float *__restrict__ row_max, float *__restrict__ row_sum, int relu_x, int tail_rows, XT xt)
 {
     static_assert(!SM || NR == 1, "softmax weights exist for the CSR layouts only");
     static_assert(!(SM && ACT), "the softmax-weighted product takes no activation argument");
     static_assert(!SM || sizeof(T) == 4, "softmax weights are single precision");
     typedef typename psp_vec<V, T>::type vec_t;
     constexpr int WORDS = sizeof(T) / 4;  // of a stored value
+    constexpr bool FWD = XT::MODE == 1, BWD = XT::MODE == 2, ATT = FWD || BWD;
+    static_assert(!ATT || (SINGLE && !SM && !ACT && sizeof(T) == 4), "the attention forms run on one register set of floats");
+    if constexpr (ATT) logL = XT::LOGL;
     __shared__ int2 s_seg[PSP_MAX_WAVES][PSP_WAVE];  // (end offset, output row) of the wavefront's segments
     __shared__ float s_m[SM ? PSP_MAX_WAVES : 1][SM ? PSP_WAVE : 1];  // SM: reference maximum of each segment's row
 
@@ -161,17 +202,24 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         for (int i = threadIdx.x; i < tail_rows * w; i += PSP_WAVE) yt[(size_t)(i / w) * (size_t)N + i % w] = (T)0;
     }
 
-    const int tile = psp_xcd_tile(stripe);
-    if (tile >= tiles) return;
-
     const int L = 1 << logL, W = 1 << logW;
     const int lane = threadIdx.x & (PSP_WAVE - 1);
     const int wave = threadIdx.x >> 6;
+    const int tile = psp_xcd_tile(stripe);
+    if (tile >= tiles) return;
     const int sub = lane & (L - 1);
     const int grp = lane >> logL;
     const int grp_base = lane - sub;
     const int s0 = (tile * (int)(blockDim.x >> 6) + wave) << logW;  // first segment of this wavefront
     if (s0 >= nseg) return;                                         // wave-uniform
+    // BWD: this wavefront's share of the weight gradient; zero from a wavefront without entries
+    auto report = [&](float sum) {
+        if constexpr (BWD) {
+#pragma unroll
+            for (int d = 1; d < PSP_WAVE; d <<= 1) sum += psp_bperm_f(lane ^ d, sum);
+            if (lane == 0) xt.wsum[s0 >> logW] = sum;
+        }
+    };
     const int nvalid = min(W, nseg - s0);
 
     // ---- segment table of this wavefront: only segments that hold entries, packed to the front ----------
@@ -222,7 +270,10 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int2 *w_seg = s_seg[wave];  // .x = end offset, .y = output row (block-row for NR = 2)
-    if (P0 == P1) return;
+    if (P0 == P1) {
+        report(0.0f);
+        return;
+    }
 
     bool ext_head = false, ext_tail = false;  // the first / last row of this wavefront also has entries elsewhere
     int tr_prev = -1, tr_next = -1;
@@ -283,6 +334,30 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         for (int i = 0; i < C; i++)
 #pragma unroll
             for (int e = 0; e < V; e++) acc[r][i][e] = head[r][i][e] = (T)0;
+    // ATT: row i of the running row, row i of the next one; scores of the entries this lane holds (FWD); lane's share of wsum
+    float ar[NR][C][V], ar_nxt[NR][C][V], keep[U][NR], wsum = 0.0f, alpha = 1.0f;
+    auto load_a = [&](int key, float (&dst)[NR][C][V]) {
+        if constexpr (ATT) {
+            const int tile_w = V << logL;
+#pragma unroll
+            for (int r = 0; r < NR; r++)
+#pragma unroll
+                for (int i = 0; i < C; i++) {
+                    const vec_t t = psp_load_vec<V, T>(X + (size_t)(key * NR + r) * (size_t)N + off[i]);
+                    // dead vectors and the repeated columns of one that was moved back add nothing to the dot product
+                    const int dup = i * tile_w + sub * V - off[i];
+#pragma unroll
+                    for (int e = 0; e < V; e++) dst[r][i][e] = e >= dup ? psp_elem<V, T>(t, e) : 0.0f;
+                }
+        }
+    };
+    // the row that follows segment c's, when the wavefront has one
+    auto load_next_a = [&](int c, int key) {
+        const int nk = c + 1 < PSP_WAVE ? w_seg[c + 1].y : -1;
+        if (nk >= 0 && nk != key) load_a(nk, ar_nxt);
+    };
+    if constexpr (FWD) alpha = xt.alpha ? *xt.alpha : 1.0f;
+
     float acc_l = 0.0f, head_l = 0.0f, m_cur = 0.0f;  // SM: weight sum of the running row / stashed head, row maximum
 
     // out: a finished row goes to Y; `shared` = other wavefronts add to the same row (row-split formats)
@@ -331,6 +406,11 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         row_end = sg.x;
         mykey = sg.y;
         if constexpr (SM) m_cur = s_m[wave][cur];
+        if constexpr (ATT) {
+            load_a(mykey, ar);
+            load_a(mykey, ar_nxt);
+            load_next_a(cur, mykey);
+        }
         const int seg_begin = cur == 0 ? P0 : w_seg[cur - 1].x;
         head_valid = a > seg_begin;
         if constexpr (SPLIT) {
@@ -349,9 +429,10 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         if (p0_ + U <= b) {                                                                  \
             psp_load_words<U>(colIdx + p0_, c_out);                                          \
             int w_[U * NR * WORDS];                                                          \
-            psp_load_words<U * NR * WORDS>((const int *)val + (size_t)p0_ * (NR * WORDS), w_); \
+            if constexpr (!FWD || NR > 1) psp_load_words<U * NR * WORDS>((const int *)val + (size_t)p0_ * (NR * WORDS), w_); \
             _Pragma("unroll") for (int u_ = 0; u_ < U; u_++)                                 \
-                _Pragma("unroll") for (int r_ = 0; r_ < NR; r_++) v_out[u_][r_] = psp_from_words<T>(w_ + (u_ * NR + r_) * WORDS); \
+                _Pragma("unroll") for (int r_ = 0; r_ < NR; r_++)                            \
+                    if constexpr (!FWD || NR > 1) v_out[u_][r_] = psp_from_words<T>(w_ + (u_ * NR + r_) * WORDS); \
         } else {                                                                             \
             _Pragma("unroll") for (int u_ = 0; u_ < U; u_++)                                 \
             {                                                                                \
@@ -406,6 +487,41 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
             first_run = false;
             mykey = nkey;
             if constexpr (SM) m_cur = s_m[wave][cur];
+            if constexpr (ATT) {
+#pragma unroll
+                for (int r = 0; r < NR; r++)
+#pragma unroll
+                    for (int i = 0; i < C; i++)
+#pragma unroll
+                        for (int e = 0; e < V; e++) ar[r][i][e] = ar_nxt[r][i][e];
+            }
+        }
+        if constexpr (ATT) load_next_a(cur, mykey);
+    };
+    // FWD: the scores of the chunk's entries, U consecutive ones per lane, a 128-byte line per group of 8 lanes
+    auto store_scores = [&](int base) {
+        if constexpr (FWD) {
+            const int p0 = base + sub * U;
+            if (p0 + U <= b) {
+                if constexpr ((U * NR) % 4 == 0) {
+#pragma unroll
+                    for (int w = 0; w < U * NR; w += 4) {
+                        psp_f32x4_a4 t;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) t[e] = keep[(w + e) / NR][(w + e) % NR];
+                        *(psp_f32x4_a4 *)(xt.score + (size_t)p0 * NR + w) = t;
+                    }
+                } else {
+#pragma unroll
+                    for (int w = 0; w < U * NR; w++) xt.score[(size_t)p0 * NR + w] = keep[w / NR][w % NR];
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int r = 0; r < NR; r++)
+                        if (p0 + u < b) xt.score[(size_t)(p0 + u) * NR + r] = keep[u][r];
+            }
         }
     };
 
@@ -431,11 +547,13 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
 
 #define PSP_DECLARE(S)      \
     int S##_ck[U], S##_pos; \
+    [[maybe_unused]] float S##_f[U][NR]; \
     T S##_vk[U][NR];        \
     vec_t S##_x[U][C];
 #define PSP_GATHER(S)                                                                                  \
     {                                                                                                  \
         if (jb == L) { /* the chunk is used up: the prefetched one becomes current, the next is requested */ \
+            store_scores(cbase);                                                                       \
             _Pragma("unroll") for (int u = 0; u < U; u++)                                              \
             {                                                                                          \
                 c_cur[u] = c_nxt[u];                                                                   \
@@ -451,6 +569,10 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
         {                                                                                              \
             S##_ck[u] = psp_bperm_i(src, c_cur[u]);                                                    \
             _Pragma("unroll") for (int r = 0; r < NR; r++) S##_vk[u][r] = psp_bperm_f(src, v_cur[u][r]); \
+        }                                                                                              \
+        if constexpr (BWD && NR > 1) {                                                                 \
+            _Pragma("unroll") for (int u = 0; u < U; u++)                                              \
+                _Pragma("unroll") for (int r = 0; r < NR; r++) S##_f[u][r] = xt.slot[(size_t)min(pos + u, b - 1) * NR + r]; \
         }                                                                                              \
         _Pragma("unroll") for (int u = 0; u < U; u++)                                                  \
         {                                                                                              \
@@ -474,6 +596,23 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                     S##_vk[u][0] = __expf(S##_vk[u][0] - m_cur);                                       \
                     acc_l += S##_vk[u][0];                                                             \
                 }                                                                                      \
+                if constexpr (ATT) {                                                                   \
+                    _Pragma("unroll") for (int r = 0; r < NR; r++)                                     \
+                    {                                                                                  \
+                        float d = 0.0f;                                                                \
+                        _Pragma("unroll") for (int i = 0; i < C; i++)                                  \
+                            _Pragma("unroll") for (int e = 0; e < V; e++)                              \
+                                d = __builtin_fmaf(ar[r][i][e], psp_elem<V, T>(S##_x[u][i], e), d);    \
+                        if constexpr (FWD) {                                                           \
+                            d = psp_group_sum<XT::LOGL>(d) * alpha;                                    \
+                            if constexpr (NR > 1) d = S##_vk[u][r] != 0.0f ? d : 0.0f;                 \
+                            S##_vk[u][r] = d;                                                          \
+                            if (sub == jb - 1) keep[u][r] = d;                                         \
+                        } else {                                                                       \
+                            wsum = __builtin_fmaf(d, NR == 1 ? (float)S##_ck[u] : S##_f[u][r], wsum);  \
+                        }                                                                              \
+                    }                                                                                  \
+                }                                                                                      \
                 _Pragma("unroll") for (int r = 0; r < NR; r++)                                         \
                 {                                                                                      \
                     /* 2x1 blocks: a zero entry is skipped (SpMM_kernel.cu:1399,1405) */               \
@@ -495,7 +634,9 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                 PSP_GATHER(A)
                 PSP_CONSUME(A)
             } while (pos < b);
+            store_scores(cbase);
         }
+        report(wsum);
     } else if (busy) {
         PSP_DECLARE(A)
         PSP_DECLARE(B)
@@ -589,7 +730,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
     M_(5, 1) M_(6, 1) M_(7, 1) M_(8, 1)
 
 typedef void (*psp_spmm_kernel_t)(const int *, const int *, const float *, const int *, const float *, float *,
-                                  int, int, int, int, int, int, int, const float *, float *, int, int);
+                                  int, int, int, int, int, int, int, const float *, float *, int, int, psp_plain);
 #define PSP_SPMM_TAIL_ROWS_MAX 16  // more rows than this past the matrix are cleared by a fill launch
 
 // One register set or two (template parameter SINGLE)?  Measured on the block model, the stencil and the R-MAT graph at

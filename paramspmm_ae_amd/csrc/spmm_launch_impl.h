@@ -3,15 +3,9 @@
 #include <stdlib.h>
 #include "spmm_kernel.h"
 
-// Enqueues kernel `k` with the mapping of `plan`: segments per wavefront, the rows the kernel does not store to, the grid.
-// T = float or double (generic_f64.hip).
-template <int NR, bool SPLIT, typename T, typename KERNEL>
-int psp_spmm_enqueue(KERNEL k, const psp_spmm_plan &plan, const int *rowPtr, const int *colIdx, const T *val, const int *target_row,
-                     const T *X, T *Y, int nrows, int N, int rows_out, hipStream_t stream, const float *row_max, float *row_sum,
-                     int relu_x)
+// log2 of the segments per wavefront
+static inline int psp_spmm_log_segs(const psp_spmm_plan &plan, int nrows, bool split)
 {
-    int rc = PSP_OK;
-    constexpr int WORDS = sizeof(T) / 4;  // Y is cleared by 4-byte words: all-zero bits are 0 in both precisions
     int logL = 0;
     while ((1 << logL) < plan.lanes_per_row) logL++;
     // Segments per wavefront.  Plain input gets one row per lane group on average: rows that are neighbours in
@@ -22,17 +16,32 @@ int psp_spmm_enqueue(KERNEL k, const psp_spmm_plan &plan, const int *rowPtr, con
     // 16 beats 8, 32 and 64 at every width).  Small matrices use fewer segments per wavefront so that there are
     // wavefronts for every SIMD.
     const int logR = 6 - logL;
-    int logW = SPLIT ? (logR > 4 ? logR : 4) : logR;
+    int logW = split ? (logR > 4 ? logR : 4) : logR;
     if (plan.log_segs_per_wave >= 0) logW = plan.log_segs_per_wave;  // chosen by a native configuration
     while (logW > 0 && (nrows >> logW) < 4096) logW--;
     if (logW < logR - 1) logW = logR - 1;
     if (logW > 6) logW = 6;
-    const psp_options &opt = psp_opts();
     // whole_rows: every lane group is handed whole segments whatever their lengths, so each element of a plain row
     // is one FMA chain over the row's entries in storage order -- the summation order of the reference's
     // one-warp-per-row kernels (SpMM_kernel.cu:1157-1212), bit for bit -- at the price of the balance between the
     // lane groups.  That needs at least one segment per lane group.
-    if (opt.whole_rows && logW < logR) logW = logR;
+    if (psp_opts().whole_rows && logW < logR) logW = logR;
+    return logW;
+}
+
+// Enqueues kernel `k` with the mapping of `plan`: segments per wavefront, the rows the kernel does not store to, the grid.
+// T = float or double (generic_f64.hip).
+template <int NR, bool SPLIT, typename T, typename KERNEL, typename XT = psp_plain>
+int psp_spmm_enqueue(KERNEL k, const psp_spmm_plan &plan, const int *rowPtr, const int *colIdx, const T *val, const int *target_row,
+                     const T *X, T *Y, int nrows, int N, int rows_out, hipStream_t stream, const float *row_max, float *row_sum,
+                     int relu_x, XT xt = XT())
+{
+    int rc = PSP_OK;
+    constexpr int WORDS = sizeof(T) / 4;  // Y is cleared by 4-byte words: all-zero bits are 0 in both precisions
+    int logL = 0;
+    while ((1 << logL) < plan.lanes_per_row) logL++;
+    const int logW = psp_spmm_log_segs(plan, nrows, SPLIT);
+    const psp_options &opt = psp_opts();
 
     // rows the kernel does not store to must read as zero
     int tail_rows = 0;
@@ -67,7 +76,7 @@ int psp_spmm_enqueue(KERNEL k, const psp_spmm_plan &plan, const int *rowPtr, con
     const psp_grid1d g = psp_xcd_grid(psp_ceil_div(nrows, segs_per_block),
                                       (plan.xcd_stripe_rows ? plan.xcd_stripe_rows : opt.stripe_rows) / segs_per_block);
     dim3 grid(g.launch, plan.col_tiles, 1), block(plan.waves_per_block * PSP_WAVE, 1, 1);
-    hipLaunchKernelGGL(k, grid, block, 0, stream, rowPtr, colIdx, val, target_row, X, Y, nrows, N, logL, logW, g.real, g.stripe, align_pct, row_max, row_sum, relu_x, tail_rows);
+    hipLaunchKernelGGL(k, grid, block, 0, stream, rowPtr, colIdx, val, target_row, X, Y, nrows, N, logL, logW, g.real, g.stripe, align_pct, row_max, row_sum, relu_x, tail_rows, xt);
     rc = psp_check_launch("spmm kernel");
     if (rc != PSP_OK || !(softmax && SPLIT)) return rc;
     if constexpr (WORDS == 1) return psp_row_scale(Y, row_sum, rows_out, N, stream);  // rows that several wavefronts added to

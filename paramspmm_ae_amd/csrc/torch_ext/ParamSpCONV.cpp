@@ -272,6 +272,61 @@ static std::vector<Tensor> attn_window_backward(Tensor dY, Tensor att, Tensor ro
     return {G, wsum};
 }
 
+// ---- the same on the PCSR formats (fmt 0..3) ---------------------------------------------------------------------------
+static bool attn_supported(long K) { return K >= 4 && K <= PSP_ATTN_MAX_K; }
+
+static void check_attn(int fmt, const Tensor &X, const Tensor &rowPtr, const Tensor &colIdx, const Tensor &values,
+                       const Tensor *target_row, int blkWarpNum)
+{
+    TORCH_CHECK(fmt >= 0 && fmt <= 3 && (fmt == 1 || fmt == 3) == (target_row != nullptr), "format code and target_row disagree");
+    check_spmm_args(fmt, X, rowPtr, colIdx, values, target_row);
+    TORCH_CHECK(X.scalar_type() == torch::kFloat32 && attn_supported(X.size(1)), "attn: float32 rows of 4 to ", PSP_ATTN_MAX_K, " columns");
+    TORCH_CHECK((blkWarpNum & ~PSP_BW_STRIPE_MASK) == 4 || (blkWarpNum & ~PSP_BW_STRIPE_MASK) == 8, "blkWarpNum must be 4 or 8");
+    // the kernel reads both rows of a block-row
+    if (fmt == 2) TORCH_CHECK(2 * (rowPtr.size(0) - 1) <= X.size(0), "the dense operand needs two rows per block-row (pad it to an even row count)");
+    if (fmt == 3) TORCH_CHECK(X.size(0) % 2 == 0, "the dense operand needs two rows per block-row (pad it to an even row count)");
+}
+
+// (fmt, X, rowPtr, colIdx, values, target_row | None, alpha | None, blkWarpNum) -> [att in the format's entry order, Y]
+static std::vector<Tensor> attn_forward(int fmt, Tensor X, Tensor rowPtr, Tensor colIdx, Tensor values, c10::optional<Tensor> target_row,
+                                        c10::optional<Tensor> alpha, int blkWarpNum)
+{
+    const Tensor *tr = target_row ? &*target_row : nullptr;
+    check_attn(fmt, X, rowPtr, colIdx, values, tr, blkWarpNum);
+    if (alpha) {
+        need_gpu(*alpha, "alpha");
+        TORCH_CHECK(alpha->scalar_type() == torch::kFloat32 && alpha->numel() == 1, "alpha is one float32 on the device");
+        pspglue::same_device(X, *alpha, "attn");
+    }
+    DeviceGuard guard(X.device());
+    Tensor att = torch::empty_like(values), Y = torch::empty_like(X);
+    ok(psp_attn_forward_f32(fmt, ip(rowPtr), ip(colIdx), fmt >= 2 ? fp(values) : nullptr, tr ? ip(*tr) : nullptr, fp(X),
+                            alpha ? alpha->data_ptr<float>() : nullptr, fpw(att), fpw(Y), (int)rowPtr.size(0) - 1, (int)X.size(1),
+                            (int)X.size(0), blkWarpNum, stream_of(X)));
+    return {att, Y};
+}
+
+// (fmt, dY, att, rowPtr, colIdx, target_row | None, slot | None, blkWarpNum) -> [G, weight-gradient sum as a 1-element tensor]
+static std::vector<Tensor> attn_backward(int fmt, Tensor dY, Tensor att, Tensor rowPtr, Tensor colIdx, c10::optional<Tensor> target_row,
+                                         c10::optional<Tensor> slot, int blkWarpNum)
+{
+    const Tensor *tr = target_row ? &*target_row : nullptr;
+    TORCH_CHECK((fmt >= 2) == slot.has_value(), "attn: 2x1 blocks take the columns of their slots, CSR does not");
+    if (slot) {
+        need_gpu(*slot, "slot");
+        TORCH_CHECK(slot->scalar_type() == torch::kFloat32 && slot->numel() == att.numel(), "attn: slot has one float32 per score");
+        pspglue::same_device(dY, *slot, "attn");
+    }
+    check_attn(fmt, dY, rowPtr, colIdx, att, tr, blkWarpNum);
+    DeviceGuard guard(dY.device());
+    const int nrows = (int)rowPtr.size(0) - 1, K = (int)dY.size(1);
+    Tensor G = torch::empty_like(dY), wsum = torch::empty({1}, dY.options());
+    Tensor ws = torch::empty({(long)psp_attn_workspace_floats(nrows, K)}, dY.options());
+    ok(psp_attn_backward_f32(fmt, ip(rowPtr), ip(colIdx), fp(att), tr ? ip(*tr) : nullptr, slot ? fp(*slot) : nullptr, fp(dY), fpw(G), wsum.data_ptr<float>(),
+                             fpw(ws), nrows, K, (int)dY.size(0), blkWarpNum, stream_of(dY)));
+    return {G, wsum};
+}
+
 static Tensor forward_impl(int fmt, const Tensor &H, const Tensor &W, const Tensor &rowPtr, const Tensor &colIdx,
                            const Tensor &values, const Tensor *target_row, int CF, int blkWarpNum)
 {
@@ -426,6 +481,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("attn_window_backward", &attn_window_backward,
           "attention layer on the windowed layout: (dY, att, rowPtr_w, colIdx_w) -> [G, weight-gradient sum]");
     m.def("attn_window_supported", &attn_window_supported, "is there a fused attention kernel for this width?");
+    m.def("attn_forward", &attn_forward,
+          "attention layer on a PCSR format: (fmt 0..3, X, rowPtr, colIdx, values, target_row | None, alpha | None, blkWarpNum) -> [att, Y]");
+    m.def("attn_backward", &attn_backward,
+          "attention layer on a PCSR format: (fmt 0..3, dY, att, rowPtr, colIdx, target_row | None, slot | None, blkWarpNum) -> [G, weight-gradient sum]");
+    m.def("attn_supported", &attn_supported, "is there a fused attention kernel for this width on the PCSR formats?");
     m.def("window_xw", &window_xw,
           "windowed layout, dense product folded in: (X, W, transW, rowPtr_w, colIdx_w, values_w, relu_input, mask | None, want_raw) -> [Y] or [Y, A f(X)]");
     m.def("window_xw_supported", &window_xw_supported, "widths the folded product exists for");

@@ -47,6 +47,31 @@ def _window_xw(op, Z, weight):
             and Z.dtype == torch.float32 and getattr(op, "fold_dense", True))
 
 
+def _attn_fused(op, X):
+    """Does the attention layer's sparse work run as one launch per direction?  float32 rows of a width the fused kernels
+    have, as many of them as the 2x1 blocks' rows need."""
+    if X.dtype != torch.float32:
+        return False
+    if _fmt(op) == 4:
+        return SpCONV.attn_window_supported(int(X.shape[1]))
+    if op.vec_size not in (1, 2) or not SpCONV.attn_supported(int(X.shape[1])):
+        return False
+    return op.vec_size == 1 or (op.mask is not None and X.shape[0] % 2 == 0)
+
+
+def _slot_columns(op, colIdx):
+    """2x1 blocks: for every slot of the blocks the column the reference's attention-weight gradient multiplies it with
+    (gnn_conv.py:166-172: d_attention[mask] times colIdx in CSR order), zero at padding; made once per operator."""
+    if op.vec_size == 1:
+        return None
+    slots = getattr(op, "_slot_columns", None)
+    if slots is None:
+        slots = torch.zeros(op.val.numel(), device=op.val.device)
+        slots[op.mask] = colIdx.reshape(-1).float()
+        op._slot_columns = slots
+    return slots
+
+
 def _aggregate(op, D):
     """A D through ``op``'s format and configuration."""
     return SpCONV.aggregate(_fmt(op), D, _row_ptr(op), op.colIdx, op.val, op.target_row if op.if_split else None, op.CF,
@@ -227,12 +252,15 @@ class AGNNFunction(torch.autograd.Function):
         # relu_input: X holds pre-activation values; the activation and its backward ride on the dense products
         ctx.relu_input = bool(relu_input)
         X_prime = SpCONV.dense_relu_xw(X, weights) if relu_input else SpCONV.dense_xw(X, weights, False)
-        ctx.fused = (_fmt(ParamSpMM) == 4 and X_prime.dtype == torch.float32
-                     and SpCONV.attn_window_supported(int(X_prime.shape[1])))
+        ctx.fused = _attn_fused(ParamSpMM, X_prime)
         if ctx.fused:
-            # windowed operator: scores (the head's weight multiplied in) and their aggregation in one launch
-            edge_attentions, out = SpCONV.attn_window_forward(X_prime, ParamSpMM.spmm_rowPtr, ParamSpMM.colIdx,
-                                                              attention_w.detach().reshape(-1)[:1])
+            # scores (the head's weight multiplied in) and their aggregation in one launch: both read the same rows
+            alpha = attention_w.detach().reshape(-1)[:1]
+            if _fmt(ParamSpMM) == 4:
+                edge_attentions, out = SpCONV.attn_window_forward(X_prime, ParamSpMM.spmm_rowPtr, ParamSpMM.colIdx, alpha)
+            else:
+                edge_attentions, out = SpCONV.attn_forward(_fmt(ParamSpMM), X_prime, ParamSpMM.rowPtr, ParamSpMM.colIdx, ParamSpMM.val,
+                                                           ParamSpMM.target_row, alpha, _bw(ParamSpMM))
         else:
             if _fmt(ParamSpMM) == 4:
                 edge_attentions = ParamSpMM.AGNN_sddmm(X_prime, attention_w.detach().reshape(-1)[:1])
@@ -253,7 +281,11 @@ class AGNNFunction(torch.autograd.Function):
         d_output = d_output.contiguous()
         if ctx.fused:
             # A_att dY and the reference's sum for the attention weight (below) in one launch
-            d_input_prime, d_attention_w = SpCONV.attn_window_backward(d_output, edge_attentions, op.spmm_rowPtr, op.colIdx)
+            if _fmt(op) == 4:
+                d_input_prime, d_attention_w = SpCONV.attn_window_backward(d_output, edge_attentions, op.spmm_rowPtr, op.colIdx)
+            else:
+                d_input_prime, d_attention_w = SpCONV.attn_backward(_fmt(op), d_output, edge_attentions, op.rowPtr, op.colIdx,
+                                                                    op.target_row, _slot_columns(op, ctx.colIdx), _bw(op))
         else:
             d_input_prime = op.AGNN_spmm(edge_attentions, d_output)
         if not ctx.needs_input_grad[0]:
