@@ -2,6 +2,10 @@
 // (glue in SpCONV/SpCONV.h:43-193): forward A*(H*W), backward [ (A*dY)*W^T, H^T*(A*dY) ].  The dense
 // products are torch::mm (hipBLASLt / rocBLAS under PyTorch-ROCm); the sparse product is libparamsp_hip.so.
 #include "glue_common.h"
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
+#include <torch/csrc/autograd/saved_variable.h>
 
 using namespace pspglue;
 using torch::Tensor;
@@ -410,6 +414,236 @@ static Tensor softmax_nll_mean_backward(Tensor logits, Tensor labels, Tensor gra
     return grad;
 }
 
+// ---- the layers as autograd nodes ----------------------------------------------------------------------------------------
+// One call from Python per layer and direction-free backward: the engine runs apply() without entering the interpreter.  As
+// Python autograd Functions the five layers and the loss of a training step cost some 25 us each of interpreter and binding
+// time, which on a graph of 20 K nodes was more than the GPU needs for the step (305 us per step, GPU busy 185).
+struct Operator {  // what a layer needs of a pcsr_spmm
+    int fmt;       // 0 csr, 1 csr_split, 2 bcsr, 3 bcsr_split, 4 windowed csr
+    Tensor rowPtr, colIdx, val;
+    c10::optional<Tensor> target_row;
+    int CF, bw;
+    bool fold_dense;      // windowed csr: fold a square dense product into the sparse kernel where there is one
+    c10::optional<Tensor> slot;  // 2x1 blocks: columns of the slots (attention weight gradient)
+    const Tensor *tr() const { return target_row ? &*target_row : nullptr; }
+};
+typedef std::shared_ptr<Operator> op_t;
+
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+struct LayerNode : torch::autograd::Node {
+    op_t op;
+    SavedVariable a_, w_, z_;
+    void release_variables() override
+    {
+        a_.reset_data();
+        w_.reset_data();
+        z_.reset_data();
+    }
+    Tensor a() { return a_.unpack(shared_from_this()); }
+    Tensor w() { return w_.unpack(shared_from_this()); }
+    Tensor z() { return z_.unpack(shared_from_this()); }
+    bool wants(size_t i) { return task_should_compute_output(i); }
+};
+
+// the result of `forward` (run without recording), with a node of type N behind it when an input asks for gradients
+template <class N, class F> static Tensor with_node(const op_t &op, std::initializer_list<Tensor> inputs, F forward)
+{
+    const bool record = torch::GradMode::is_enabled() &&
+                        std::any_of(inputs.begin(), inputs.end(), [](const Tensor &t) { return t.requires_grad(); });
+    std::shared_ptr<N> node;
+    if (record) {
+        node = std::shared_ptr<N>(new N(), torch::autograd::deleteNode);
+        torch::autograd::edge_list edges;
+        for (const Tensor &t : inputs) edges.push_back(torch::autograd::impl::gradient_edge(t));
+        node->set_next_edges(std::move(edges));
+        node->op = op;
+    }
+    Tensor out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        out = forward(node.get());
+    }
+    if (record) torch::autograd::set_history(out, node);
+    return out;
+}
+
+static bool folds_dense(const Operator &o, const Tensor &Z, const Tensor &W)
+{
+    return o.fmt == 4 && o.fold_dense && W.size(0) == W.size(1) && W.size(0) == Z.size(1) && window_xw_supported(Z.size(1)) &&
+           Z.scalar_type() == torch::kFloat32;
+}
+
+// A (H W); dH = (A dY) W^T, dW = H^T (A dY) -- A is symmetric (gnn_conv.py:13-107)
+struct GCNFunction : LayerNode {
+    variable_list apply(variable_list &&g) override
+    {
+        if (!g[0].defined()) return {Tensor(), Tensor()};
+        Tensor H = a(), W = w();
+        Tensor AG = aggregate(op->fmt, g[0], op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
+        return {wants(0) ? dense_xw(AG, W, true) : Tensor(), wants(1) ? weight_gradient(H, AG) : Tensor()};
+    }
+};
+static Tensor gcn_layer(op_t op, Tensor H, Tensor W)
+{
+    need_gpu(H, "input");
+    need_gpu(W, "weight");
+    return with_node<GCNFunction>(op, {H, W}, [&](GCNFunction *n) {
+        if (n) n->a_ = SavedVariable(H, false), n->w_ = SavedVariable(W, false);
+        return aggregate(op->fmt, dense_xw(H, W, false), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
+    });
+}
+
+// (A H) W with A H kept for the backward: dW = (A H)^T dY, dH = A (dY W^T) -- the layer that widens its input, and GIN's
+// (gnn_conv.py:202-220)
+struct AggregateFirst : LayerNode {
+    variable_list apply(variable_list &&g) override
+    {
+        if (!g[0].defined()) return {Tensor(), Tensor()};
+        Tensor AH = a(), W = w(), dY = g[0].contiguous(), dH;
+        if (wants(0)) dH = aggregate(op->fmt, dense_xw(dY, W, true), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
+        return {dH, wants(1) ? weight_gradient(AH, dY) : Tensor()};
+    }
+};
+struct GCNAggregateFirstFunction : AggregateFirst {};
+struct GINFunction : AggregateFirst {};
+template <class N> static Tensor aggregate_first_layer(op_t op, Tensor H, Tensor W)
+{
+    need_gpu(H, "input");
+    need_gpu(W, "weight");
+    return with_node<N>(op, {H, W}, [&](N *n) {
+        Tensor AH = aggregate(op->fmt, H, op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
+        if (n) n->a_ = SavedVariable(AH, false), n->w_ = SavedVariable(W, false);
+        return dense_xw(AH, W, false);
+    });
+}
+
+// A (relu(Z) W): dZ = ((A dY) W^T) where Z > 0, dW = relu(Z)^T (A dY)
+struct GCNReLUInputFunction : LayerNode {
+    variable_list apply(variable_list &&g) override
+    {
+        if (!g[0].defined()) return {Tensor(), Tensor()};
+        Tensor Z = a(), W = w(), dY = g[0].contiguous();
+        if (folds_dense(*op, Z, W)) {
+            // one launch delivers A dY (for the weight gradient) and ((A dY) W^T) where Z > 0 (the input gradient)
+            auto r = window_xw(dY, W, true, op->rowPtr, op->colIdx, op->val, false, Z, true);
+            return {r[0], weight_gradient_relu(Z, r[1])};
+        }
+        auto r = relu_input_backward(op->fmt, dY, Z, W, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw);
+        return {r[0], r[1]};
+    }
+};
+static Tensor gcn_relu_layer(op_t op, Tensor Z, Tensor W)
+{
+    return with_node<GCNReLUInputFunction>(op, {Z, W}, [&](GCNReLUInputFunction *n) {
+        if (n) n->a_ = SavedVariable(Z, false), n->w_ = SavedVariable(W, false);
+        // windowed layout, square layer: (A relu(Z)) W in one launch, the dense product in the kernel's epilogue
+        if (folds_dense(*op, Z, W)) return window_xw(Z, W, false, op->rowPtr, op->colIdx, op->val, true, c10::nullopt, false)[0];
+        return relu_input_forward(op->fmt, Z, W, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw);
+    });
+}
+
+// (A relu(Z)) W for a layer that widens its input: the activation is applied as the sparse product gathers the rows of Z,
+// the gradient masked in a pass that follows the backward product
+struct GINReLUInputFunction : LayerNode {
+    variable_list apply(variable_list &&g) override
+    {
+        if (!g[0].defined()) return {Tensor(), Tensor()};
+        Tensor AX = a(), W = w(), Z = z(), dY = g[0].contiguous();
+        return {wants(0) ? aggregate_act_op(op->fmt, dense_xw(dY, W, true), op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw,
+                                            false, Z)
+                         : Tensor(),
+                wants(1) ? weight_gradient(AX, dY) : Tensor()};
+    }
+};
+static Tensor gin_relu_layer(op_t op, Tensor Z, Tensor W)
+{
+    return with_node<GINReLUInputFunction>(op, {Z, W}, [&](GINReLUInputFunction *n) {
+        Tensor AX = aggregate_act_op(op->fmt, Z, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw, true, c10::nullopt);
+        if (n) n->a_ = SavedVariable(AX, false), n->w_ = SavedVariable(W, false), n->z_ = SavedVariable(Z, false);
+        return dense_xw(AX, W, false);
+    });
+}
+
+// The attention layer, its sparse work one launch per direction (gnn_conv.py:128-180): X' = f(X) W, att = alpha <X'_i, X'_j>,
+// out = att-weighted sum of the X' rows; the gradients are the reference's literal formulas
+static std::vector<Tensor> attn_fused_forward(const Operator &o, const Tensor &Xp, const Tensor &alpha)
+{
+    if (o.fmt == 4) return attn_window_forward(Xp, o.rowPtr, o.colIdx, alpha);
+    return attn_forward(o.fmt, Xp, o.rowPtr, o.colIdx, o.val, o.target_row, alpha, o.bw);
+}
+struct AGNNFunction : LayerNode {  // a_ = X, z_ = att
+    bool relu_input = false;
+    std::vector<int64_t> alpha_shape;
+    variable_list apply(variable_list &&g) override
+    {
+        if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+        Tensor X = a(), W = w(), att = z(), dY = g[0].contiguous();
+        auto r = op->fmt == 4 ? attn_window_backward(dY, att, op->rowPtr, op->colIdx)
+                              : attn_backward(op->fmt, dY, att, op->rowPtr, op->colIdx, op->target_row, op->slot, op->bw);
+        Tensor dX, dW;
+        if (wants(0)) dX = relu_input ? dense_xwt_masked(r[0], W, X) : dense_xw(r[0], W, true);
+        if (wants(1)) dW = relu_input ? weight_gradient_relu(X, r[0]) : weight_gradient(X, r[0]);
+        return {dX, dW, r[1].reshape({1, 1}).expand(alpha_shape)};
+    }
+};
+static Tensor agnn_layer(op_t op, Tensor X, Tensor W, Tensor attention_w, bool relu_input)
+{
+    need_gpu(X, "input");
+    need_gpu(W, "weight");
+    return with_node<AGNNFunction>(op, {X, W, attention_w}, [&](AGNNFunction *n) {
+        Tensor Xp = relu_input ? dense_relu_xw(X, W) : dense_xw(X, W, false);
+        auto r = attn_fused_forward(*op, Xp, attention_w.reshape({-1}).narrow(0, 0, 1));
+        if (n) {
+            n->a_ = SavedVariable(X, false), n->w_ = SavedVariable(W, false), n->z_ = SavedVariable(r[0], false);
+            n->relu_input = relu_input;
+            n->alpha_shape = attention_w.sizes().vec();
+        }
+        return r[1];
+    });
+}
+
+struct NllLossMean : LayerNode {  // a_ = labels, z_ = stats
+    int64_t n = 0, C = 0;
+    variable_list apply(variable_list &&g) override
+    {
+        if (!g[0].defined()) return {Tensor(), Tensor()};
+        return {wants(0) ? nll_loss_mean_backward(a(), g[0].contiguous(), z(), n, C) : Tensor(), Tensor()};
+    }
+};
+static Tensor nll_loss_layer(Tensor logp, Tensor labels)
+{
+    return with_node<NllLossMean>(nullptr, {logp, labels}, [&](NllLossMean *n) {
+        auto r = nll_loss_mean(logp, labels);
+        if (n) n->a_ = SavedVariable(labels, false), n->z_ = SavedVariable(r[1], false), n->n = logp.size(0), n->C = logp.size(1);
+        return r[0];
+    });
+}
+struct SoftmaxNllMean : LayerNode {  // a_ = labels, w_ = logits, z_ = stats
+    variable_list apply(variable_list &&g) override
+    {
+        if (!g[0].defined()) return {Tensor(), Tensor()};
+        return {wants(0) ? softmax_nll_mean_backward(w(), a(), g[0].contiguous(), z()) : Tensor(), Tensor()};
+    }
+};
+static Tensor softmax_nll_layer(Tensor logits, Tensor labels)
+{
+    return with_node<SoftmaxNllMean>(nullptr, {logits, labels}, [&](SoftmaxNllMean *n) {
+        auto r = softmax_nll_mean(logits, labels);
+        if (n) n->a_ = SavedVariable(labels, false), n->w_ = SavedVariable(logits, false), n->z_ = SavedVariable(r[1], false);
+        return r[0];
+    });
+}
+
+// the nodes under their own names in Python (type(t.grad_fn).__name__)
+template <class N> static void register_node(const char *name)
+{
+    static PyTypeObject type;
+    torch::autograd::_initFunctionPyTypeObject(type, name, nullptr, nullptr);
+    torch::autograd::registerCppFunction(typeid(N), &type);
+}
+
 #define PSP_CONV(NAME, FMT)                                                                                       \
     static Tensor NAME##_forward(Tensor H, Tensor W, Tensor rowPtr, Tensor colIdx, Tensor values, int CF, int bw)  \
     {                                                                                                             \
@@ -440,6 +674,28 @@ PSP_CONV_SPLIT(bcsr_split_spmm, 3)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     pspglue::check_abi();
+    register_node<GCNFunction>("GCNFunctionBackward");
+    register_node<GCNAggregateFirstFunction>("GCNAggregateFirstFunctionBackward");
+    register_node<GCNReLUInputFunction>("GCNReLUInputFunctionBackward");
+    register_node<GINFunction>("GINFunctionBackward");
+    register_node<GINReLUInputFunction>("GINReLUInputFunctionBackward");
+    register_node<AGNNFunction>("AGNNFunctionBackward");
+    register_node<NllLossMean>("NllLossMeanBackward");
+    register_node<SoftmaxNllMean>("SoftmaxNllMeanBackward");
+    py::class_<Operator, op_t>(m, "Operator", "what a layer needs of a pcsr_spmm")
+        .def(py::init([](int fmt, Tensor rowPtr, Tensor colIdx, Tensor val, c10::optional<Tensor> target_row, int CF, int bw,
+                         bool fold_dense, c10::optional<Tensor> slot) {
+            TORCH_CHECK(fmt >= 0 && fmt <= 4 && (fmt == 1 || fmt == 3) == target_row.has_value(), "format code and target_row disagree");
+            return std::make_shared<Operator>(Operator{fmt, rowPtr, colIdx, val, target_row, CF, bw, fold_dense, slot});
+        }));
+    m.def("gcn_layer", &gcn_layer, "A (H W): (operator, H, W)");
+    m.def("gcn_aggregate_first_layer", &aggregate_first_layer<GCNAggregateFirstFunction>, "(A H) W: (operator, H, W)");
+    m.def("gcn_relu_layer", &gcn_relu_layer, "A (relu(Z) W): (operator, Z, W)");
+    m.def("gin_layer", &aggregate_first_layer<GINFunction>, "(A X) W: (operator, X, W)");
+    m.def("gin_relu_layer", &gin_relu_layer, "(A relu(Z)) W: (operator, Z, W)");
+    m.def("agnn_layer", &agnn_layer, "attention layer: (operator, X, W, attention_w, relu_input)");
+    m.def("nll_loss_layer", &nll_loss_layer, "mean negative log-likelihood: (log-probabilities, int64 labels)");
+    m.def("softmax_nll_layer", &softmax_nll_layer, "nll_loss(log_softmax(logits), labels), mean over the rows");
     m.def("split_csr", &pspglue::split_csr, "row split on the host");
     m.def("split_csr_par", &pspglue::split_csr_par, "row split on the host with a precomputed segment prefix");
     // addition of this build: H^T * G for tall-skinny operands (memory-speed kernel for widths 16..64, else torch::mm)

@@ -1,6 +1,7 @@
-"""GCN / AGNN / GIN layers as autograd Functions over the PCSR operators (same surface and the same forward /
-backward algebra as the reference's gnn_conv.py:13-238).  Layers look their operator up in ``spmm_dict`` by
-output width (gnn_conv.py:121-124)."""
+"""GCN / AGNN / GIN layers as autograd functions over the PCSR operators (same surface and the same forward /
+backward algebra as the reference's gnn_conv.py:13-238).  The functions are nodes of ParamSpCONV: neither direction
+enters the interpreter between two launches.  Layers look their operator up in ``spmm_dict`` by output width
+(gnn_conv.py:121-124)."""
 import math
 
 import torch
@@ -10,23 +11,10 @@ import ParamSpCONV as SpCONV
 
 n_heads = 1
 
-_CONV = {(False, False): "csr_spmm", (True, False): "csr_split_spmm", (False, True): "bcsr_spmm", (True, True): "bcsr_split_spmm"}
-
-
-def _conv_args(op):
-    args = [op.rowPtr, op.colIdx, op.val]
-    if op.if_split:
-        args.append(op.target_row)
-    return args + [op.CF, _bw(op)]
-
 
 def _bw(op):
     """blkWarpNum with the operator's launch flags (the XCD stripe chosen for its format, PCSR.pcsr_spmm.bw_flags)."""
     return op.blkWarpNum | getattr(op, "bw_flags", 0)
-
-
-def _conv_name(op):
-    return _CONV[(bool(op.if_split), op.vec_size != 1)]
 
 
 def _fmt(op):
@@ -40,21 +28,15 @@ def _row_ptr(op):
     return getattr(op, "spmm_rowPtr", op.rowPtr)
 
 
-def _window_xw(op, Z, weight):
-    """Does the layer A (relu(Z) W) run as one windowed launch with the dense product folded in?  A windowed operator, a
-    square weight matrix of a width the kernel has, float32."""
-    return (_fmt(op) == 4 and weight.shape[0] == weight.shape[1] == Z.shape[1] and SpCONV.window_xw_supported(int(Z.shape[1]))
-            and Z.dtype == torch.float32 and getattr(op, "fold_dense", True))
-
-
-def _attn_fused(op, X):
+def _attn_fused(op, X, weights):
     """Does the attention layer's sparse work run as one launch per direction?  float32 rows of a width the fused kernels
     have, as many of them as the 2x1 blocks' rows need."""
-    if X.dtype != torch.float32:
+    if X.dtype != torch.float32 or weights.dtype != torch.float32:
         return False
+    width = int(weights.shape[1])
     if _fmt(op) == 4:
-        return SpCONV.attn_window_supported(int(X.shape[1]))
-    if op.vec_size not in (1, 2) or not SpCONV.attn_supported(int(X.shape[1])):
+        return SpCONV.attn_window_supported(width)
+    if op.vec_size not in (1, 2) or not SpCONV.attn_supported(width):
         return False
     return op.vec_size == 1 or (op.mask is not None and X.shape[0] % 2 == 0)
 
@@ -72,24 +54,15 @@ def _slot_columns(op, colIdx):
     return slots
 
 
-def _aggregate(op, D):
-    """A D through ``op``'s format and configuration."""
-    return SpCONV.aggregate(_fmt(op), D, _row_ptr(op), op.colIdx, op.val, op.target_row if op.if_split else None, op.CF,
-                            _bw(op))
-
-
-class _NllLossMean(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logp, labels):
-        loss, stats = SpCONV.nll_loss_mean(logp, labels)
-        ctx.save_for_backward(labels, stats)
-        ctx.shape = tuple(logp.shape)
-        return loss
-
-    @staticmethod
-    def backward(ctx, grad_loss):
-        labels, stats = ctx.saved_tensors
-        return SpCONV.nll_loss_mean_backward(labels, grad_loss.contiguous(), stats, ctx.shape[0], ctx.shape[1]), None
+def _native(op, slots=None):
+    """The operator as the extension module's layers take it; made once, and again when one of its attributes changes."""
+    k = op.__dict__.get("_native_operator")
+    bw, fold = _bw(op), getattr(op, "fold_dense", True)
+    if (k is None or k[0] is not op.rowPtr or k[1] is not op.colIdx or k[2] is not op.val or k[3] is not op.target_row
+            or k[4] != op.CF or k[5] != bw or k[6] != fold or k[7] is not slots):
+        native = SpCONV.Operator(_fmt(op), _row_ptr(op), op.colIdx, op.val, op.target_row if op.if_split else None, op.CF, bw, fold, slots)
+        k = op._native_operator = (op.rowPtr, op.colIdx, op.val, op.target_row, op.CF, bw, fold, slots, native)
+    return k[-1]
 
 
 def nll_loss_mean(logp, labels):
@@ -100,21 +73,8 @@ def nll_loss_mean(logp, labels):
     int64 labels goes to PyTorch."""
     if (logp.is_cuda and logp.dtype == torch.float32 and logp.dim() == 2 and labels.dtype == torch.int64
             and labels.dim() == 1):
-        return _NllLossMean.apply(logp.contiguous(), labels.contiguous())
+        return SpCONV.nll_loss_layer(logp.contiguous(), labels.contiguous())
     return torch.nn.functional.nll_loss(logp, labels)
-
-
-class _SoftmaxNllMean(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logits, labels):
-        loss, stats = SpCONV.softmax_nll_mean(logits, labels)
-        ctx.save_for_backward(logits, labels, stats)
-        return loss
-
-    @staticmethod
-    def backward(ctx, grad_loss):
-        logits, labels, stats = ctx.saved_tensors
-        return SpCONV.softmax_nll_mean_backward(logits, labels, grad_loss.contiguous(), stats), None
 
 
 def softmax_nll_loss_mean(logits, labels):
@@ -125,36 +85,19 @@ def softmax_nll_loss_mean(logits, labels):
     operators."""
     if (logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2 and labels.dtype == torch.int64
             and labels.dim() == 1 and SpCONV.softmax_nll_supported(int(logits.shape[1]))):
-        return _SoftmaxNllMean.apply(logits.contiguous(), labels.contiguous())
+        return SpCONV.softmax_nll_layer(logits.contiguous(), labels.contiguous())
     return nll_loss_mean(torch.nn.functional.log_softmax(logits, dim=1), labels)
 
 
-class GCNFunction(torch.autograd.Function):
+class GCNFunction(object):
     """forward A(HW); backward dH = (A dY) W^T, dW = H^T (A dY) -- A is symmetric (gnn_conv.py:13-107)."""
 
     @staticmethod
-    def forward(ctx, H, weight, ParamSpMM):
-        ctx.save_for_backward(H, weight)
-        ctx.ParamSpMM = ParamSpMM
-        if _fmt(ParamSpMM) == 4:  # the windowed layout has no named operator of its own: dense product, then A
-            return _aggregate(ParamSpMM, SpCONV.dense_xw(H, weight, False))
-        return getattr(SpCONV, _conv_name(ParamSpMM) + "_forward")(H, weight, *_conv_args(ParamSpMM))
-
-    @staticmethod
-    def backward(ctx, d_output):
-        H, weight = ctx.saved_tensors
-        op = ctx.ParamSpMM
-        if not ctx.needs_input_grad[0]:
-            # the network's first layer: its input holds features, nothing asks for their gradient
-            return None, SpCONV.weight_gradient(H, _aggregate(op, d_output)), None
-        if _fmt(op) == 4:
-            AG = _aggregate(op, d_output.contiguous())
-            return SpCONV.dense_xw(AG, weight, True), SpCONV.weight_gradient(H, AG), None
-        d_input, d_weight = getattr(SpCONV, _conv_name(op) + "_backward")(d_output.contiguous(), H, weight, *_conv_args(op))
-        return d_input, d_weight, None
+    def apply(H, weight, ParamSpMM):
+        return SpCONV.gcn_layer(_native(ParamSpMM), H, weight)
 
 
-class GCNAggregateFirstFunction(torch.autograd.Function):
+class GCNAggregateFirstFunction(object):
     """The same layer computed as (A H) W: for a layer that widens its input (in_features < out_features) the sparse
     product then runs at the input's width.  Backward: dW = (A H)^T dY (A H is kept from the forward pass, so the
     weight gradient needs no sparse product) and dH = A (dY W^T), again at the input's width -- A is symmetric, as in
@@ -162,51 +105,20 @@ class GCNAggregateFirstFunction(torch.autograd.Function):
     width."""
 
     @staticmethod
-    def forward(ctx, H, weight, ParamSpMM):
-        AH = _aggregate(ParamSpMM, H)
-        ctx.save_for_backward(AH, weight)
-        ctx.ParamSpMM = ParamSpMM
-        return SpCONV.dense_xw(AH, weight, False)
-
-    @staticmethod
-    def backward(ctx, d_output):
-        AH, weight = ctx.saved_tensors
-        d_output = d_output.contiguous()
-        d_weight = SpCONV.weight_gradient(AH, d_output)
-        d_input = None
-        if ctx.needs_input_grad[0]:
-            d_input = _aggregate(ctx.ParamSpMM, SpCONV.dense_xw(d_output, weight, True))
-        return d_input, d_weight, None
+    def apply(H, weight, ParamSpMM):
+        return SpCONV.gcn_aggregate_first_layer(_native(ParamSpMM), H, weight)
 
 
-class GCNReLUInputFunction(torch.autograd.Function):
+class GCNReLUInputFunction(object):
     """The GCN layer reading its input through a ReLU, A (relu(Z) W), as one function of the pre-activation values
     Z: forward relu(Z) W with the activation applied as Z is read; backward dZ = ((A dY) W^T) where Z > 0 and
     dW = relu(Z)^T (A dY), again without a pass for the activation.  Five layers with F.relu between them
-    (GNN.py:43-61) are conv1(x), then four of these."""
+    (GNN.py:43-61) are conv1(x), then four of these.  On a windowed operator a square layer of 16 or 32 columns runs
+    the dense product inside the sparse kernel."""
 
     @staticmethod
-    def forward(ctx, Z, weight, ParamSpMM):
-        ctx.save_for_backward(Z, weight)
-        ctx.ParamSpMM = ParamSpMM
-        op = ParamSpMM
-        if _window_xw(op, Z, weight):
-            # windowed layout, square layer: (A relu(Z)) W in one launch, the dense product in the kernel's epilogue
-            return SpCONV.window_xw(Z, weight, False, op.spmm_rowPtr, op.colIdx, op.val, True, None, False)[0]
-        return SpCONV.relu_input_forward(_fmt(op), Z, weight, _row_ptr(op), op.colIdx, op.val,
-                                         op.target_row if op.if_split else None, op.CF, _bw(op))
-
-    @staticmethod
-    def backward(ctx, d_output):
-        Z, weight = ctx.saved_tensors
-        op = ctx.ParamSpMM
-        if _window_xw(op, Z, weight):
-            # one launch delivers A dY (for the weight gradient) and ((A dY) W^T) where Z > 0 (the input gradient)
-            d_input, AG = SpCONV.window_xw(d_output.contiguous(), weight, True, op.spmm_rowPtr, op.colIdx, op.val, False, Z, True)
-            return d_input, SpCONV.weight_gradient_relu(Z, AG), None
-        d_input, d_weight = SpCONV.relu_input_backward(_fmt(op), d_output.contiguous(), Z, weight, _row_ptr(op), op.colIdx, op.val,
-                                                       op.target_row if op.if_split else None, op.CF, _bw(op))
-        return d_input, d_weight, None
+    def apply(Z, weight, ParamSpMM):
+        return SpCONV.gcn_relu_layer(_native(ParamSpMM), Z, weight)
 
 
 class _Layer(torch.nn.Module):
@@ -243,32 +155,34 @@ class GCNConv(_Layer):
         return fn.apply(H, self.weights, self._operator(spmm_dict))
 
 
-class AGNNFunction(torch.autograd.Function):
+class AGNNFunction(object):
     """X' = XW; e = <X'_i, X'_j> per stored entry; attention = e * w; out = SpMM(attention, X')
-    (gnn_conv.py:128-180).  No softmax, as in the reference."""
+    (gnn_conv.py:128-180).  No softmax, as in the reference.  ``relu_input``: X holds pre-activation values; the
+    activation and its backward ride on the dense products."""
+
+    @staticmethod
+    def apply(X, weights, attention_w, ParamSpMM, colIdx, relu_input=False):
+        if _attn_fused(ParamSpMM, X, weights):
+            # scores (the head's weight multiplied in) and their aggregation in one launch per direction
+            native = _native(ParamSpMM, _slot_columns(ParamSpMM, colIdx))
+            return SpCONV.agnn_layer(native, X, weights, attention_w, bool(relu_input))
+        return _AGNNUnfused.apply(X, weights, attention_w, ParamSpMM, colIdx, relu_input)
+
+
+class _AGNNUnfused(torch.autograd.Function):
+    """The layer with its SDDMM and SpMM as separate operators: widths past the fused kernels', double precision."""
 
     @staticmethod
     def forward(ctx, X, weights, attention_w, ParamSpMM, colIdx, relu_input=False):
-        # relu_input: X holds pre-activation values; the activation and its backward ride on the dense products
         ctx.relu_input = bool(relu_input)
         X_prime = SpCONV.dense_relu_xw(X, weights) if relu_input else SpCONV.dense_xw(X, weights, False)
-        ctx.fused = _attn_fused(ParamSpMM, X_prime)
-        if ctx.fused:
-            # scores (the head's weight multiplied in) and their aggregation in one launch: both read the same rows
-            alpha = attention_w.detach().reshape(-1)[:1]
-            if _fmt(ParamSpMM) == 4:
-                edge_attentions, out = SpCONV.attn_window_forward(X_prime, ParamSpMM.spmm_rowPtr, ParamSpMM.colIdx, alpha)
-            else:
-                edge_attentions, out = SpCONV.attn_forward(_fmt(ParamSpMM), X_prime, ParamSpMM.rowPtr, ParamSpMM.colIdx, ParamSpMM.val,
-                                                           ParamSpMM.target_row, alpha, _bw(ParamSpMM))
+        if _fmt(ParamSpMM) == 4:
+            edge_attentions = ParamSpMM.AGNN_sddmm(X_prime, attention_w.detach().reshape(-1)[:1])
         else:
-            if _fmt(ParamSpMM) == 4:
-                edge_attentions = ParamSpMM.AGNN_sddmm(X_prime, attention_w.detach().reshape(-1)[:1])
-            else:
-                edge_feature = ParamSpMM.AGNN_sddmm(X_prime)
-                # csr: [nnz] ; 2x1 blocks: [nblk, 2] -- a single head scales both the same way
-                edge_attentions = (edge_feature * attention_w.reshape(())).contiguous()
-            out = ParamSpMM.AGNN_spmm(edge_attentions, X_prime)
+            edge_feature = ParamSpMM.AGNN_sddmm(X_prime)
+            # csr: [nnz] ; 2x1 blocks: [nblk, 2] -- a single head scales both the same way
+            edge_attentions = (edge_feature * attention_w.reshape(())).contiguous()
+        out = ParamSpMM.AGNN_spmm(edge_attentions, X_prime)
         ctx.save_for_backward(X, weights, edge_attentions)
         ctx.colIdx = colIdx
         ctx.ParamSpMM = ParamSpMM
@@ -279,15 +193,7 @@ class AGNNFunction(torch.autograd.Function):
         op = ctx.ParamSpMM
         X, weights, edge_attentions = ctx.saved_tensors
         d_output = d_output.contiguous()
-        if ctx.fused:
-            # A_att dY and the reference's sum for the attention weight (below) in one launch
-            if _fmt(op) == 4:
-                d_input_prime, d_attention_w = SpCONV.attn_window_backward(d_output, edge_attentions, op.spmm_rowPtr, op.colIdx)
-            else:
-                d_input_prime, d_attention_w = SpCONV.attn_backward(_fmt(op), d_output, edge_attentions, op.rowPtr, op.colIdx,
-                                                                    op.target_row, _slot_columns(op, ctx.colIdx), _bw(op))
-        else:
-            d_input_prime = op.AGNN_spmm(edge_attentions, d_output)
+        d_input_prime = op.AGNN_spmm(edge_attentions, d_output)
         if not ctx.needs_input_grad[0]:
             d_input = None
         elif ctx.relu_input:
@@ -296,8 +202,6 @@ class AGNNFunction(torch.autograd.Function):
             d_input = SpCONV.dense_xw(d_input_prime, weights, True)
         # X^T * d_input_prime (relu(X)^T when the layer reads X through the activation)
         d_weights = SpCONV.weight_gradient_relu(X, d_input_prime) if ctx.relu_input else SpCONV.weight_gradient(X, d_input_prime)
-        if ctx.fused:
-            return d_input, d_weights, d_attention_w.reshape(1, 1).expand(1, n_heads), None, None, None
         d_attention = op.AGNN_sddmm(d_output)
         if d_attention.dim() != 1:
             d_attention = d_attention.view(-1)[op.mask]  # block layout -> CSR slots
@@ -323,8 +227,18 @@ class AGNNConv(_Layer):
         return AGNNFunction.apply(X, self.weights, self.attention_w, self._operator(spmm_dict), colIdx, relu_input)
 
 
-class GINFunction(torch.autograd.Function):
+class GINFunction(object):
     """forward (A X) W; backward dW = (A X)^T dY, dX = A (dY W^T) (gnn_conv.py:202-220)."""
+
+    @staticmethod
+    def apply(X, weight, ParamSpMM):
+        if ParamSpMM.vec_size == 1 or (ParamSpMM.vec_size == 2 and X.shape[0] % 2 == 0):
+            return SpCONV.gin_layer(_native(ParamSpMM), X, weight)
+        return _GINOnOperator.apply(X, weight, ParamSpMM)
+
+
+class _GINOnOperator(torch.autograd.Function):
+    """The same through the operator's own method: 3x1 blocks, and inputs that end inside a block."""
 
     @staticmethod
     def forward(ctx, X, weight, ParamSpMM):
@@ -343,29 +257,14 @@ class GINFunction(torch.autograd.Function):
         return d_input, d_weights, None
 
 
-class GINReLUInputFunction(torch.autograd.Function):
+class GINReLUInputFunction(object):
     """(A relu(Z)) W as one function of the pre-activation values Z, for a layer that widens its input: the activation
     is applied as the sparse product gathers the rows of Z (ParamSpCONV.aggregate_act), the gradient is masked in a pass
     that follows the backward product.  The reference's driver applies F.relu between the layers (GNN.py:63-78)."""
 
     @staticmethod
-    def forward(ctx, Z, weight, ParamSpMM):
-        op = ParamSpMM
-        X_agg = SpCONV.aggregate_act(_fmt(op), Z, _row_ptr(op), op.colIdx, op.val, op.target_row if op.if_split else None, op.CF,
-                                     _bw(op), True, None)
-        ctx.save_for_backward(X_agg, weight, Z)
-        ctx.ParamSpMM = op
-        return SpCONV.dense_xw(X_agg, weight, False)
-
-    @staticmethod
-    def backward(ctx, d_output):
-        X_agg, weights, Z = ctx.saved_tensors
-        op = ctx.ParamSpMM
-        d_output = d_output.contiguous()
-        d_weights = SpCONV.weight_gradient(X_agg, d_output)
-        d_input = SpCONV.aggregate_act(_fmt(op), SpCONV.dense_xw(d_output, weights, True), _row_ptr(op), op.colIdx, op.val,
-                                       op.target_row if op.if_split else None, op.CF, _bw(op), False, Z)
-        return d_input, d_weights, None
+    def apply(Z, weight, ParamSpMM):
+        return SpCONV.gin_relu_layer(_native(ParamSpMM), Z, weight)
 
 
 class GINConv(_Layer):
