@@ -177,7 +177,8 @@ int psp_split_csr_fill_dev(const int *rowPtr, const int *row_split_offset, int n
 /* rowPtr_b[(nrows+1)/2+1]; rowPtr_b[(nrows+1)/2] is nblk.  Input rows must hold strictly ascending columns. */
 int psp_bcsr_offsets_dev(const int *rowPtr, const int *colIdx, int nrows, int *rowPtr_b, int *workspace,
                          int workspace_ints, int *status, psp_stream_t stream);
-/* fills colIdx_b[nblk] and val_b[nblk*2] in the block order of psp_bcsr_build. */
+/* fills colIdx_b[nblk] and val_b[nblk*2] in the block order of psp_bcsr_build; either may be NULL to fill only the other
+ * (the columns alone need no `val`). */
 int psp_bcsr_fill_dev(const int *rowPtr, const int *colIdx, const float *val, int nrows, const int *rowPtr_b,
                       int *colIdx_b, float *val_b, psp_stream_t stream);
 

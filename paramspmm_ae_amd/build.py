@@ -46,13 +46,13 @@ def _ext_command(name):
 
 def build_extensions(force=False):
     os.makedirs(LIB, exist_ok=True)
-    hdr = os.path.join(CSRC, "torch_ext", "glue_common.h")
-    hdr2 = os.path.join(CSRC, "torch_ext", "baseline_rocsparse.h")
+    headers = [os.path.join(CSRC, "torch_ext", h) for h in ("glue_common.h", "baseline_rocsparse.h", "pcsr_load.h")]
+    headers.append(os.path.join(ROOT, "include", "paramsp.h"))
     todo = []
     for name in MODULES:
         src = os.path.join(CSRC, "torch_ext", name + ".cpp")
         out = os.path.join(LIB, name + ".so")
-        newest = max(os.path.getmtime(src), os.path.getmtime(hdr), os.path.getmtime(hdr2), os.path.getmtime(os.path.join(ROOT, "include", "paramsp.h")))
+        newest = max(os.path.getmtime(f) for f in [src] + headers)
         if force or not os.path.exists(out) or os.path.getmtime(out) < newest:
             todo.append(name)
 

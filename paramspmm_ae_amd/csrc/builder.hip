@@ -163,18 +163,6 @@ PSP_EXPORT int psp_split_csr_fill_dev(const int *rowPtr, const int *row_split_of
 }
 
 // ---- BCSR 2x1 -----------------------------------------------------------------------------------------------------
-// position of column c in the ascending range col[lo, hi), or -1
-__device__ __forceinline__ int find_col(const int *__restrict__ col, int lo, int hi, int c)
-{
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        const int v = col[mid];
-        if (v == c) return mid;
-        if (v < c) lo = mid + 1; else hi = mid;
-    }
-    return -1;
-}
-
 // first position in the ascending range col[lo, hi) whose column is not below c[k], for ILP columns at once: the
 // searches have the same depth (`top` = largest power of two not above hi - lo, at least 1), so their loads overlap
 template <int ILP>
@@ -197,81 +185,205 @@ __device__ __forceinline__ int top_power_of_two(int len)
     return top;
 }
 
-// Block-rows with more stored entries than this are built by a whole workgroup (bcsr_long_kernel): walked by a single
-// wavefront, the hub rows of a skewed graph were the tail of the launch (4.5 of 4.8 ms on an R-MAT graph).
-#define BCSR_LONG 2048
+// What a pass over the block-rows does: count their blocks, or write the blocks' columns, their values, or both.  Columns and
+// values can be written by passes of their own because a loader has the columns (and their way back to the host) long
+// before the values have arrived.
+enum { BCSR_COUNT = 0, BCSR_COLS = 1, BCSR_VALS = 2 };
 
-// One wavefront per block-row t (rows 2t and 2t+1).  Blocks: the entries of row 2t in order, then the entries of
-// row 2t+1 whose column row 2t does not hold, in order -- the first-encounter order of the host builder.
-template <bool FILL>
-__global__ void __launch_bounds__(256) bcsr_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
+// Block-rows with more entries than this, or more in their first row than a wavefront's LDS holds, are built by a whole
+// workgroup (bcsr_long_kernel): walked by a single wavefront, the hub rows of a skewed graph were the tail of the launch
+// (4.5 of 4.8 ms on an R-MAT graph).
+#define BCSR_LONG 2048
+#define BCSR_MID 1024
+__device__ __forceinline__ bool bcsr_is_long(int a0, int a1, int b1) { return b1 - a0 > BCSR_LONG || a1 - a0 > BCSR_MID; }
+
+// One wavefront per four consecutive block-rows t (rows 2t and 2t+1).  Blocks: the entries of row 2t in order, then the
+// entries of row 2t+1 whose column row 2t does not hold, in order -- the first-encounter order of the host builder.
+// Rows of up to 64 entries live in registers, one per lane: an entry of row 2t+1 finds its column in row 2t with six
+// ds_bpermutes, and the loads of the four block-rows are in flight together.  Longer ones search row 2t in LDS.  A
+// workgroup is one wavefront: with four of them, half the workgroups of a skewed graph stayed for one slow one.  (One
+// block-row per wavefront with the binary searches in global memory: 378 us for the count and 861 for the fill of an R-MAT
+// graph of 2^20 rows, all of it waiting for dependent loads.)
+template <int WHAT>
+__global__ void __launch_bounds__(64) bcsr_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
                                                    const float *__restrict__ val, int nrows, int nbr,
                                                    int *__restrict__ counts, const int *__restrict__ rowPtr_b,
                                                    int *__restrict__ colIdx_b, float *__restrict__ val_b,
                                                    int *__restrict__ status)
 {
-    const int lane = threadIdx.x & (PSP_WAVE - 1);
-    const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (t >= nbr) return;  // wave-uniform
-    const int a0 = rowPtr[2 * t], a1 = rowPtr[2 * t + 1];
-    const int b1 = (2 * t + 1 < nrows) ? rowPtr[2 * t + 2] : a1;  // odd row count: the last block-row has one row
-    const int len0 = a1 - a0;
-    if (a1 >= a0 && b1 >= a1 && b1 - a0 > BCSR_LONG) return;  // wave-uniform: bcsr_long_kernel takes this block-row
-
-    if (!FILL) {
-        // strictly ascending columns inside both rows?
-        bool bad = a1 < a0 || b1 < a1;
-        for (int p = a0 + lane; p < b1; p += PSP_WAVE)
-            if (p != a0 && p != a1 && colIdx[p] <= colIdx[p - 1]) bad = true;
-        if (bad) atomicOr(status, a1 < a0 || b1 < a1 ? PSP_BUILD_BAD_ROWPTR : PSP_BUILD_UNSORTED);
-        if (a1 < a0 || b1 < a1) {
-            if (lane == 0) counts[t] = 0;
-            return;
-        }
-    } else {
-        const int base = rowPtr_b[t];
-        for (int i = lane; i < len0; i += PSP_WAVE) {
-            const int c = colIdx[a0 + i];
-            const int q = find_col(colIdx, a1, b1, c);
-            colIdx_b[base + i] = c;
-            val_b[2 * (size_t)(base + i)] = val[a0 + i];
-            val_b[2 * (size_t)(base + i) + 1] = q >= 0 ? val[q] : 0.0f;
-        }
+    constexpr bool COUNT = WHAT == BCSR_COUNT, COLS = (WHAT & BCSR_COLS) != 0, VALS = (WHAT & BCSR_VALS) != 0;
+    constexpr int T = 4;
+    __shared__ int s_col[BCSR_MID];
+    __shared__ float s_match[VALS ? BCSR_MID : 1];
+    const int lane = threadIdx.x;
+    const int t0 = blockIdx.x * T;
+    if (t0 >= nbr) return;  // wave-uniform
+    const int ends = rowPtr[min(2 * t0 + min(lane, 2 * T), nrows)];  // lane i: start of row 2 t0 + i
+    int a0[T], a1[T], b1[T], base[T], ca[T], cb[T];
+    float va[T], vb[T];
+    bool small[T];
+#pragma unroll
+    for (int i = 0; i < T; i++) {
+        a0[i] = __builtin_amdgcn_readlane(ends, 2 * i);
+        a1[i] = __builtin_amdgcn_readlane(ends, 2 * i + 1);
+        b1[i] = __builtin_amdgcn_readlane(ends, 2 * i + 2);  // odd row count: the last block-row has one row
+        small[i] = t0 + i < nbr && a1[i] >= a0[i] && b1[i] >= a1[i] && a1[i] - a0[i] <= PSP_WAVE && b1[i] - a1[i] <= PSP_WAVE;
+        const bool ia = small[i] && lane < a1[i] - a0[i], ib = small[i] && lane < b1[i] - a1[i];
+        ca[i] = ia ? colIdx[a0[i] + lane] : 0x7fffffff;
+        cb[i] = ib ? colIdx[a1[i] + lane] : 0x7fffffff;
+        va[i] = VALS && ia ? val[a0[i] + lane] : 0.0f;
+        vb[i] = VALS && ib ? val[a1[i] + lane] : 0.0f;
+        base[i] = !COUNT && t0 + i < nbr ? rowPtr_b[t0 + i] : 0;
     }
-
-    // entries of row 2t+1 that open a block of their own, ranked in order
-    int fresh = 0;
-    for (int p0 = a1; p0 < b1; p0 += PSP_WAVE) {
-        const int p = p0 + lane;
-        bool mine = false;
-        int c = 0;
-        if (p < b1) {
-            c = colIdx[p];
-            mine = find_col(colIdx, a0, a1, c) < 0;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int at[T], found[T];  // entries of row 2t below this lane's column, of its first 63, and the column that follows them
+#pragma unroll
+    for (int i = 0; i < T; i++) at[i] = 0;
+#pragma unroll
+    for (int step = 32; step >= 1; step >>= 1)
+#pragma unroll
+        for (int i = 0; i < T; i++) found[i] = __builtin_amdgcn_ds_bpermute((at[i] + step - 1) << 2, ca[i]), at[i] += found[i] < cb[i] ? step : 0;
+#pragma unroll
+    for (int i = 0; i < T; i++) found[i] = __builtin_amdgcn_ds_bpermute(at[i] << 2, ca[i]);
+#pragma unroll
+    for (int i = 0; i < T; i++) {
+        const int t = t0 + i, na = a1[i] - a0[i], nb = b1[i] - a1[i];
+        if (t >= nbr) break;  // wave-uniform, like every condition on a0, a1, b1
+        if (small[i]) {
+            if (COUNT) {  // strictly ascending columns inside both rows?
+                const int pa = __shfl_up(ca[i], 1), pb = __shfl_up(cb[i], 1);
+                const bool bad = lane > 0 && ((lane < na && ca[i] <= pa) || (lane < nb && cb[i] <= pb));
+                if (__ballot(bad) && lane == 0) atomicOr(status, PSP_BUILD_UNSORTED);
+            }
+            const int pos = at[i];
+            const bool in = lane < nb;
+            const bool hit = found[i] == cb[i] && in;
+            const unsigned long long fresh = __ballot(in && !hit);
+            if (COUNT) {
+                if (lane == 0) counts[t] = na + __popcll(fresh);
+                continue;
+            }
+            const int slot = base[i] + na + __popcll(fresh & below);
+            if (COLS) {
+                if (lane < na) colIdx_b[base[i] + lane] = ca[i];
+                if (in && !hit) colIdx_b[slot] = cb[i];
+            }
+            if (VALS) {
+                // the value of a matched entry goes to the lane that holds its column
+                const unsigned long long hits = __ballot(hit);
+                float m = 0.0f;
+                if (hits) {
+                    s_match[lane] = 0.0f;
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    if (hit) s_match[pos] = vb[i];
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    m = s_match[lane];
+                }
+                if (lane < na) ((float2 *)val_b)[base[i] + lane] = make_float2(va[i], m);
+                if (in && !hit) ((float2 *)val_b)[slot] = make_float2(0.0f, vb[i]);
+            }
+            continue;
         }
-        const unsigned long long m = __ballot(mine);
-        if (FILL && mine) {
-            const int slot = rowPtr_b[t] + len0 + fresh + __popcll(m & ((1ull << lane) - 1ull));
-            colIdx_b[slot] = c;
-            val_b[2 * (size_t)slot] = 0.0f;
-            val_b[2 * (size_t)slot + 1] = val[p];
+        if (na < 0 || nb < 0) {
+            if (COUNT && lane == 0) {
+                atomicOr(status, PSP_BUILD_BAD_ROWPTR);
+                counts[t] = 0;
+            }
+            continue;
         }
-        fresh += __popcll(m);
+        if (bcsr_is_long(a0[i], a1[i], b1[i])) continue;  // bcsr_long_kernel takes this block-row
+        // ILP independent loads and searches per lane and round
+        constexpr int ILP = 4;
+        bool bad = false;
+        for (int p0 = 0; p0 < na; p0 += ILP * PSP_WAVE) {
+            int c[ILP], before[ILP];
+#pragma unroll
+            for (int k = 0; k < ILP; k++) {
+                const int p = p0 + k * PSP_WAVE + lane;
+                c[k] = p < na ? colIdx[a0[i] + p] : 0;
+                before[k] = COUNT && p > 0 && p < na ? colIdx[a0[i] + p - 1] : -1;
+            }
+#pragma unroll
+            for (int k = 0; k < ILP; k++) {
+                const int p = p0 + k * PSP_WAVE + lane;
+                if (p < na) {
+                    if (COUNT && p > 0 && c[k] <= before[k]) bad = true;
+                    s_col[p] = c[k];
+                    if (VALS) s_match[p] = 0.0f;
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int top = top_power_of_two(na);
+        int fresh = 0;
+        for (int q0 = 0; q0 < nb; q0 += ILP * PSP_WAVE) {
+            int c[ILP], before[ILP], pos[ILP];
+            float v[ILP];
+#pragma unroll
+            for (int k = 0; k < ILP; k++) {
+                const int q = q0 + k * PSP_WAVE + lane;
+                c[k] = q < nb ? colIdx[a1[i] + q] : 0x7fffffff;
+                before[k] = COUNT && q > 0 && q < nb ? colIdx[a1[i] + q - 1] : -1;
+                v[k] = VALS && q < nb ? val[a1[i] + q] : 0.0f;
+                pos[k] = 0;
+            }
+            for (int step = top; step >= 1; step >>= 1) {
+#pragma unroll
+                for (int k = 0; k < ILP; k++) {
+                    const int e = max(min(pos[k] + step, na) - 1, 0);  // read without a branch, used where it lies inside the row
+                    if (s_col[e] < c[k] && pos[k] + step <= na) pos[k] += step;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < ILP; k++) {
+                const int q = q0 + k * PSP_WAVE + lane;
+                const bool in = q < nb;
+                if (COUNT && in && q > 0 && c[k] <= before[k]) bad = true;
+                const bool hit = in && pos[k] < na && s_col[min(pos[k], BCSR_MID - 1)] == c[k];
+                const unsigned long long m = __ballot(in && !hit);
+                const int slot = base[i] + na + fresh + __popcll(m & below);
+                if (COLS && in && !hit) colIdx_b[slot] = c[k];
+                if (VALS && in) {
+                    if (hit) s_match[pos[k]] = v[k];
+                    else ((float2 *)val_b)[slot] = make_float2(0.0f, v[k]);
+                }
+                fresh += __popcll(m);
+            }
+        }
+        if (COUNT) {
+            if (__ballot(bad) && lane == 0) atomicOr(status, PSP_BUILD_UNSORTED);
+            if (lane == 0) counts[t] = na + fresh;
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            for (int p = lane; p < na; p += PSP_WAVE) {
+                if (COLS) colIdx_b[base[i] + p] = s_col[p];
+                if (VALS) ((float2 *)val_b)[base[i] + p] = make_float2(val[a0[i] + p], s_match[p]);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the next block-row reuses the wavefront's LDS
+        __builtin_amdgcn_wave_barrier();
     }
-    if (!FILL && lane == 0) counts[t] = len0 + fresh;
 }
 
 // The long block-rows, one workgroup of 1024 lanes at a time.  Workgroup w looks at the block-rows w, w + G, w + 2G, ...
 // (hub rows often sit next to each other; this spreads them over the workgroups), 1024 of them per round: the lanes
 // list the long ones in LDS, then build each together.  Every lane looks up four entries at once, the ranks of the
 // entries that open their own block come from ballots, a prefix over the 16 wavefronts and the running total.
-template <bool FILL>
+template <int WHAT>
 __global__ void __launch_bounds__(1024) bcsr_long_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
                                                          const float *__restrict__ val, int nrows, int nbr,
                                                          int *__restrict__ counts, const int *__restrict__ rowPtr_b,
                                                          int *__restrict__ colIdx_b, float *__restrict__ val_b,
                                                          int *__restrict__ status)
 {
+    constexpr bool FILL = WHAT != BCSR_COUNT, COLS = (WHAT & BCSR_COLS) != 0, VALS = (WHAT & BCSR_VALS) != 0;
     constexpr int ILP = 4, WAVES = 16;
     __shared__ int s_list[1024];
     __shared__ int s_nlist;
@@ -286,7 +398,7 @@ __global__ void __launch_bounds__(1024) bcsr_long_kernel(const int *__restrict__
         if (tt < nbr) {
             const int a0 = rowPtr[2 * mine_t], a1 = rowPtr[2 * mine_t + 1];
             const int b1 = (2 * mine_t + 1 < nrows) ? rowPtr[2 * mine_t + 2] : a1;
-            if (a1 >= a0 && b1 >= a1 && b1 - a0 > BCSR_LONG) s_list[atomicAdd(&s_nlist, 1)] = mine_t;
+            if (a1 >= a0 && b1 >= a1 && bcsr_is_long(a0, a1, b1)) s_list[atomicAdd(&s_nlist, 1)] = mine_t;
         }
         __syncthreads();
         const int nlist = s_nlist;
@@ -297,30 +409,23 @@ __global__ void __launch_bounds__(1024) bcsr_long_kernel(const int *__restrict__
             const int len0 = a1 - a0;
             if (!FILL) {
                 bool bad = false;  // strictly ascending columns inside both rows?
-                for (int p = a0 + tid; p < b1; p += 1024)
-                    if (p != a0 && p != a1 && colIdx[p] <= colIdx[p - 1]) bad = true;
+#pragma unroll 4
+                for (int p = a0 + tid; p < b1; p += 1024) {
+                    const int c = colIdx[p], before = colIdx[max(p - 1, 0)];
+                    if (p != a0 && p != a1 && c <= before) bad = true;
+                }
                 if (bad) atomicOr(status, PSP_BUILD_UNSORTED);
             } else {
+                // row 2t's entries open their blocks; the partner of a block is written below by the entry that finds it
                 const int base = rowPtr_b[t];
-                const int top1 = top_power_of_two(b1 - a1);
-                for (int i0e = 0; i0e < len0; i0e += ILP * 1024) {
-                    int c[ILP], q[ILP];
-#pragma unroll
-                    for (int k = 0; k < ILP; k++) {
-                        const int i = i0e + k * 1024 + tid;
-                        c[k] = i < len0 ? colIdx[a0 + i] : 0;
-                    }
-                    lower_bound_batch<ILP>(colIdx, a1, b1, top1, c, q);
-#pragma unroll
-                    for (int k = 0; k < ILP; k++) {
-                        const int i = i0e + k * 1024 + tid;
-                        if (i < len0) {
-                            const bool hit = q[k] < b1 && colIdx[q[k]] == c[k];
-                            colIdx_b[base + i] = c[k];
-                            val_b[2 * (size_t)(base + i)] = val[a0 + i];
-                            val_b[2 * (size_t)(base + i) + 1] = hit ? val[q[k]] : 0.0f;
-                        }
-                    }
+#pragma unroll 4
+                for (int i = tid; i < len0; i += 1024) {
+                    if (COLS) colIdx_b[base + i] = colIdx[a0 + i];
+                    if (VALS) ((float2 *)val_b)[base + i] = make_float2(val[a0 + i], 0.0f);
+                }
+                if (VALS) {
+                    __threadfence_block();
+                    __syncthreads();
                 }
             }
             // entries of row 2t+1 that open a block of their own, ranked in order
@@ -339,6 +444,7 @@ __global__ void __launch_bounds__(1024) bcsr_long_kernel(const int *__restrict__
 #pragma unroll
                 for (int k = 0; k < ILP; k++) {
                     mine[k] = in[k] && !(lo[k] < a1 && colIdx[lo[k]] == c[k]);
+                    if (VALS && in[k] && !mine[k]) val_b[2 * (size_t)(rowPtr_b[t] + lo[k] - a0) + 1] = val[p0 + k * 1024 + tid];
                     const unsigned long long m = __ballot(mine[k]);
                     if (lane == 0) s_wave[k][wave] = __popcll(m);
                     lo[k] = __popcll(m & ((1ull << lane) - 1ull));  // rank inside the wavefront
@@ -357,9 +463,8 @@ __global__ void __launch_bounds__(1024) bcsr_long_kernel(const int *__restrict__
                     if (FILL && mine[k]) {
                         const int slot = rowPtr_b[t] + len0 + before + ahead + lo[k];
                         const int p = p0 + k * 1024 + tid;
-                        colIdx_b[slot] = c[k];
-                        val_b[2 * (size_t)slot] = 0.0f;
-                        val_b[2 * (size_t)slot + 1] = val[p];
+                        if (COLS) colIdx_b[slot] = c[k];
+                        if (VALS) ((float2 *)val_b)[slot] = make_float2(0.0f, val[p]);
                     }
                     before += chunk_total;
                 }
@@ -372,24 +477,18 @@ __global__ void __launch_bounds__(1024) bcsr_long_kernel(const int *__restrict__
     }
 }
 
-static void launch_bcsr(bool fill, const int *rowPtr, const int *colIdx, const float *val, int nrows, int nbr, int *counts,
+template <int WHAT>
+static void launch_bcsr(const int *rowPtr, const int *colIdx, const float *val, int nrows, int nbr, int *counts,
                         const int *rowPtr_b, int *colIdx_b, float *val_b, int *status, hipStream_t st)
 {
     // about two workgroups of 1024 lanes per CU; a prime (odd) count, because the workgroups take block-rows by index
     // modulo the count and hub rows of generated graphs share their low index bits
     int long_wgs = psp_ceil_div(nbr, 64);
     long_wgs = long_wgs >= 509 ? 509 : (long_wgs | 1);
-    if (fill) {
-        hipLaunchKernelGGL(bcsr_kernel<true>, dim3(psp_ceil_div(nbr, 4)), dim3(256), 0, st, rowPtr, colIdx, val, nrows, nbr,
-                           counts, rowPtr_b, colIdx_b, val_b, status);
-        hipLaunchKernelGGL(bcsr_long_kernel<true>, dim3(long_wgs), dim3(1024), 0, st, rowPtr, colIdx, val, nrows, nbr, counts,
-                           rowPtr_b, colIdx_b, val_b, status);
-    } else {
-        hipLaunchKernelGGL(bcsr_kernel<false>, dim3(psp_ceil_div(nbr, 4)), dim3(256), 0, st, rowPtr, colIdx, val, nrows, nbr,
-                           counts, rowPtr_b, colIdx_b, val_b, status);
-        hipLaunchKernelGGL(bcsr_long_kernel<false>, dim3(long_wgs), dim3(1024), 0, st, rowPtr, colIdx, val, nrows, nbr, counts,
-                           rowPtr_b, colIdx_b, val_b, status);
-    }
+    hipLaunchKernelGGL(bcsr_kernel<WHAT>, dim3(psp_ceil_div(nbr, 4)), dim3(PSP_WAVE), 0, st, rowPtr, colIdx, val, nrows, nbr, counts,
+                       rowPtr_b, colIdx_b, val_b, status);
+    hipLaunchKernelGGL(bcsr_long_kernel<WHAT>, dim3(long_wgs), dim3(1024), 0, st, rowPtr, colIdx, val, nrows, nbr, counts,
+                       rowPtr_b, colIdx_b, val_b, status);
 }
 
 PSP_EXPORT int psp_bcsr_offsets_dev(const int *rowPtr, const int *colIdx, int nrows, int *rowPtr_b, int *workspace,
@@ -399,7 +498,7 @@ PSP_EXPORT int psp_bcsr_offsets_dev(const int *rowPtr, const int *colIdx, int nr
     const int nbr = (nrows + 1) / 2;
     hipStream_t st = (hipStream_t)stream;
     if (nbr > 0) {  // colIdx may be null for a matrix without entries (the host cannot tell, rowPtr is on the device)
-        launch_bcsr(false, rowPtr, colIdx, nullptr, nrows, nbr, rowPtr_b, nullptr, nullptr, nullptr, status, st);
+        launch_bcsr<BCSR_COUNT>(rowPtr, colIdx, nullptr, nrows, nbr, rowPtr_b, nullptr, nullptr, nullptr, status, st);
     }
     return exclusive_scan(rowPtr_b, rowPtr_b, nbr, workspace, workspace_ints, status, st);
 }
@@ -410,7 +509,10 @@ PSP_EXPORT int psp_bcsr_fill_dev(const int *rowPtr, const int *colIdx, const flo
     PSP_REQUIRE(rowPtr && rowPtr_b && nrows >= 0, "bcsr_fill_dev: bad input");
     const int nbr = (nrows + 1) / 2;
     if (nbr == 0) return PSP_OK;  // the entry arrays may be null when rowPtr_b says there are no blocks
-    launch_bcsr(true, rowPtr, colIdx, val, nrows, nbr, nullptr, rowPtr_b, colIdx_b, val_b, nullptr, (hipStream_t)stream);
+    hipStream_t st = (hipStream_t)stream;
+    if (colIdx_b && val_b) launch_bcsr<BCSR_COLS | BCSR_VALS>(rowPtr, colIdx, val, nrows, nbr, nullptr, rowPtr_b, colIdx_b, val_b, nullptr, st);
+    else if (colIdx_b) launch_bcsr<BCSR_COLS>(rowPtr, colIdx, val, nrows, nbr, nullptr, rowPtr_b, colIdx_b, val_b, nullptr, st);
+    else if (val_b) launch_bcsr<BCSR_VALS>(rowPtr, colIdx, val, nrows, nbr, nullptr, rowPtr_b, colIdx_b, val_b, nullptr, st);
     return psp_check_launch("bcsr fill kernel");
 }
 

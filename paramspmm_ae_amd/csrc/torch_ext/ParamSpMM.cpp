@@ -1,6 +1,7 @@
 // Python module `ParamSpMM`: the binding surface of the reference's SpMM/SpMM.cpp:891-926, backed by
 // libparamsp_hip.so.  Argument order, tensor requirements and return types follow the reference bindings.
 #include "glue_common.h"
+#include "pcsr_load.h"
 #include "baseline_rocsparse.h"
 
 using namespace pspglue;
@@ -338,6 +339,8 @@ static py::dict spmm_plan(int N, int CF, int blkWarpNum)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     pspglue::check_abi();
+    m.def("load_formats", &pspglue::load_formats,
+          "host CSR arrays to every format on the device and the host: (rowPtr, colIdx, val, ncols, granularity, granularity_b)");
     m.def("window_build", &window_build, "windowed CSR of a CSR matrix: (rowPtr, colIdx, values) -> [rowPtr_w, colIdx_w, values_w]");
     m.def("window_spmm", &window_spmm, "windowed CSR SpMM (HIP, gfx950): (X, rowPtr_w, colIdx_w, values_w, variant)");
     m.def("window_plan", &window_plan, "(N, variant) -> tile width, rows per workgroup, LDS bytes of the windowed kernel");

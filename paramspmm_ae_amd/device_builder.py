@@ -20,7 +20,11 @@ def _stream():
 
 
 def _check_status(status, what):
-    flags = int(status.item())  # synchronises with the builder kernels
+    raise_for(int(status.item()), what)  # synchronises with the builder kernels
+
+
+def raise_for(flags, what):
+    """The exception a builder's PSP_BUILD_* flags stand for, if any are set."""
     if flags & 4:
         raise ValueError("%s: rowPtr decreases, does not start at 0 or does not end at the entry count" % what)
     if flags & 8:

@@ -30,30 +30,45 @@ def _stat_block(rowPtr, colIdx, num_nodes, num_edges):
     unbiased std)."""
     row_nnz = rowPtr[1:] - rowPtr[:-1]
     occupied = row_nnz != 0
-    real_nrow = torch.sum(occupied)
-    nonempty_rate = real_nrow / num_nodes
-    avg_degree = num_edges / num_nodes
-    cov = row_nnz.float().std() / avg_degree
-    if nonempty_rate < 0.98:
-        real_avg_degree = (num_edges / real_nrow).item()
-        real_cov = torch.std(row_nnz[occupied].float()) / real_avg_degree
-    else:
-        real_avg_degree, real_cov = avg_degree, cov
     last = (rowPtr[1:] - 1)[occupied].long()
     first = rowPtr[:-1][occupied].long()
     width = colIdx[last] - colIdx[first]
+    return _statistics(num_nodes, num_edges, row_nnz, torch.sum(occupied), torch.max(row_nnz), row_nnz.float().std(),
+                       lambda: torch.std(row_nnz[occupied].float()), torch.max(width), torch.sum(width))
+
+
+def _real_avg_degree(num_nodes, num_edges, real_nrow):
+    """(non-empty rate, mean row length over the non-empty rows unless nearly all rows are)."""
+    rate = real_nrow / num_nodes
+    return rate, (num_edges / real_nrow).item() if rate < 0.98 else num_edges / num_nodes
+
+
+def _statistics(num_nodes, num_edges, row_nnz, real_nrow, max_row_nnz, std, std_occupied, max_bw, sum_bw):
+    nonempty_rate, real_avg_degree = _real_avg_degree(num_nodes, num_edges, real_nrow)
+    avg_degree = num_edges / num_nodes
+    cov = std / avg_degree
     return {
         "row_nnz": row_nnz,
-        "max_row_nnz": torch.max(row_nnz),
+        "max_row_nnz": max_row_nnz,
         "real_nrow": real_nrow,
         "nonempty_rate": nonempty_rate,
         "avg_degree": avg_degree,
         "COV": cov,
         "real_avg_degree": real_avg_degree,
-        "real_COV": real_cov,
-        "max_bw": torch.max(width),
-        "avg_bw": torch.sum(width) / real_nrow,
+        "real_COV": std_occupied() / real_avg_degree if nonempty_rate < 0.98 else cov,
+        "max_bw": max_bw,
+        "avg_bw": sum_bw / real_nrow,
     }
+
+
+def _granularity(real_avg_degree, manual_granularity, is_avg_granularity):
+    """Segment length of a row split (graph_input.py:89-102, 117-129): average, manual, or the next multiple of 32 above
+    the mean row length."""
+    if is_avg_granularity:
+        return int(real_avg_degree)
+    if manual_granularity is not None:
+        return manual_granularity
+    return math.ceil(real_avg_degree / 32) * 32
 
 
 class csr_data(object):
@@ -165,13 +180,7 @@ class csr_data(object):
         return int(row_split_nnz.sum()) / self.real_nrow, row_split_nnz
 
     def _choose_granularity(self, manual_granularity, is_avg_granularity):
-        # graph_input.py:89-102 / 117-129: average, manual, or the next multiple of 32 above the mean row length
-        if is_avg_granularity:
-            g = int(self.real_avg_degree)
-        elif manual_granularity is not None:
-            g = manual_granularity
-        else:
-            g = math.ceil(self.real_avg_degree / 32) * 32
+        g = _granularity(self.real_avg_degree, manual_granularity, is_avg_granularity)
         self.split_granularity = g
         self.split_ratio, self.row_split_nnz = self.split_ratio_comp(g)
 
@@ -190,6 +199,11 @@ class csr_data(object):
         self.real_avg_degree = (self.num_edges / self.real_nrow).item()
         self._choose_granularity(manual_granularity, is_avg_granularity)
 
+    def _adopt_split(self, rowPtr_split, target_row, host_rowPtr_split, host_target_row):
+        self.rowPtr_split, self.target_row = host_rowPtr_split, host_target_row
+        self._keep_device("rowPtr_split", rowPtr_split)
+        self._keep_device("target_row", target_row)
+
     def get_split(self, verbose=True, build_on="auto"):
         if self.split_granularity is None:
             raise ValueError("split_granularity is None, must be init first")
@@ -198,9 +212,7 @@ class csr_data(object):
             from . import device_builder
 
             rs, tr = device_builder.split_csr_device(self.on_device("rowPtr", "cuda"), self.split_granularity)
-            self.rowPtr_split, self.target_row = device_builder.to_host(rs, tr)
-            self._keep_device("rowPtr_split", rs)
-            self._keep_device("target_row", tr)
+            self._adopt_split(rs, tr, *device_builder.to_host(rs, tr))
         else:
             import ParamSpMM  # the extension module of this build (lib/ParamSpMM.so)
 
@@ -208,15 +220,18 @@ class csr_data(object):
             offsets[1:] = self.row_split_nnz.cumsum(dim=0).to(torch.int32)
             self.rowPtr_split, self.target_row = ParamSpMM.split_csr_par(self.rowPtr, offsets, self.split_granularity)
         if verbose:
-            print(
-                "get_split -> split time: (ms): {:.3f} split_gran: {} \n split_ratio: {} avg_nnz: {} split_rows: {}".format(
-                    (time.perf_counter() - t0) * 1e3,
-                    self.split_granularity,
-                    self.split_ratio,
-                    self.real_avg_degree,
-                    self.target_row.shape[0],
-                )
+            self.print_split((time.perf_counter() - t0) * 1e3)
+
+    def print_split(self, ms):
+        print(
+            "get_split -> {}split_gran: {} \n split_ratio: {} avg_nnz: {} split_rows: {}".format(
+                "" if ms is None else "split time: (ms): {:.3f} ".format(ms),
+                self.split_granularity,
+                self.split_ratio,
+                self.real_avg_degree,
+                self.target_row.shape[0],
             )
+        )
 
     def print_info(self):
         if self.csr_flag:
@@ -378,6 +393,86 @@ class graph_input(object):
         self.mtx_edges = nnz
         self.density = nnz / (n * n)
         self.csr_data = csr_data(rowPtr, colIdx, val, n, nnz, True)
+        native = blk_size == 2 and nnz > 0 and _use_device(build_on) and self._load_native(manual_granularity, is_avg_granularity, build_on)
+        if not native:
+            self._load_stepwise(rowPtr, colIdx, val, manual_granularity, is_avg_granularity, blk_size, build_on)
+
+        self.mask = None
+        if if_mask:
+            import ParamSDDMM
+
+            if not torch.cuda.is_available():
+                raise RuntimeError("if_mask=True runs genmask on the GPU and no GPU is available")
+            dev = torch.device("cuda")
+            mask = ParamSDDMM.genmask(
+                self.bcsr_data.on_device("rowPtr", dev), self.csr_data.on_device("rowPtr", dev),
+                self.bcsr_data.on_device("val", dev), self.mtx_edges
+            )
+            self.mask = mask.to(torch.int64)
+
+        self.loaded_flag = True
+        self.reordered_flag = True
+        self.bcsr_flag = True
+        if native:
+            self.csr_split_flag = self.bcsr_split_flag = True
+        else:
+            self.get_split_csr(build_on)
+            self.get_split_bcsr(build_on)
+        if self.verbose:
+            print("data format all preprocess (ms): {:.3f}".format((time.perf_counter() - t0) * 1e3))
+        return self
+
+    def _load_native(self, manual_granularity, is_avg_granularity, build_on):
+        """Every format of ``self.csr_data`` in one native call (ParamSpMM.load_formats): transfers both ways, statistics,
+        2x1 blocks and both row splits.  False: the rows are not strictly ascending and the host builder has to take over."""
+        import ParamSpMM
+
+        from . import device_builder
+
+        c, n, nnz = self.csr_data, self.mtx_nodes, self.mtx_edges
+
+        def granularity(real_nrow):
+            return _granularity(_real_avg_degree(n, nnz, torch.tensor(real_nrow))[1], manual_granularity, is_avg_granularity)
+
+        def granularity_b(real_nrow, nblk):
+            return _granularity((float(nblk) / torch.tensor(real_nrow)).item(), manual_granularity, is_avg_granularity)
+
+        got = ParamSpMM.load_formats(c.rowPtr, c.colIdx, c.val, (n + 1) // 2 * 2, granularity, granularity_b)
+        device_builder.raise_for(got["flags"] & ~2, "load_from_csr")
+        for k in ("rowPtr", "colIdx", "val"):
+            c._keep_device(k, got[k])
+        if got["flags"]:
+            if build_on == "device":
+                device_builder.raise_for(got["flags"], "bcsr")
+            return False
+        stats = _statistics(n, nnz, got["row_nnz"], torch.tensor(got["real_nrow"]), torch.tensor(got["max_row_nnz"], dtype=torch.int32),
+                            torch.tensor(got["std"], dtype=torch.float32), lambda: torch.tensor(got["std_occupied"], dtype=torch.float32),
+                            torch.tensor(got["max_bw"], dtype=torch.int32), torch.tensor(got["sum_bw"]))
+        for k, v in stats.items():
+            setattr(c, k, v)
+        c.split_granularity, segments, c.row_split_nnz = got["split_stats"]
+        c.split_ratio = segments / c.real_nrow
+        c._adopt_split(*got["split"])
+        on_gpu, host = got["blocks"][:3], got["blocks"][3:]
+        nblk = host[1].numel()
+        b = csr_data(*(t.numpy() for t in host), (n + 1) // 2, float(nblk), False)
+        for k, t in zip(("rowPtr", "colIdx", "val"), on_gpu):
+            b._keep_device(k, t)
+        b.row_nnz, real_nrow, b.split_granularity, segments, b.row_split_nnz = got["blocks_stats"]
+        b.real_nrow = torch.tensor(real_nrow)
+        b.real_avg_degree = (b.num_edges / b.real_nrow).item()
+        b.split_ratio = segments / b.real_nrow
+        b._adopt_split(*got["blocks_split"])
+        self.bcsr_data = b
+        self.pack_rate = nnz / (2 * nblk)  # graph_input.py:274
+        if self.verbose:
+            c.print_split(None)
+            b.print_split(None)
+        return True
+
+    def _load_stepwise(self, rowPtr, colIdx, val, manual_granularity, is_avg_granularity, blk_size, build_on):
+        """The same one builder at a time: host builders, 3x1 blocks, rows that are not strictly ascending."""
+        n, nnz = self.mtx_nodes, self.mtx_edges
         self.csr_data.init_info(is_avg_granularity=is_avg_granularity, manual_granularity=manual_granularity)
 
         on_gpu = []
@@ -396,28 +491,6 @@ class graph_input(object):
             self.bcsr_data._keep_device(k, t)
         self.bcsr_data.init_info(is_avg_granularity=is_avg_granularity, manual_granularity=manual_granularity)
         self.pack_rate = nnz / (blk_size * nblk) if nblk else 0.0  # graph_input.py:274
-
-        self.mask = None
-        if if_mask:
-            import ParamSDDMM
-
-            if not torch.cuda.is_available():
-                raise RuntimeError("if_mask=True runs genmask on the GPU and no GPU is available")
-            dev = torch.device("cuda")
-            mask = ParamSDDMM.genmask(
-                self.bcsr_data.on_device("rowPtr", dev), self.csr_data.on_device("rowPtr", dev),
-                self.bcsr_data.on_device("val", dev), self.mtx_edges
-            )
-            self.mask = mask.to(torch.int64)
-
-        self.loaded_flag = True
-        self.reordered_flag = True
-        self.bcsr_flag = True
-        self.get_split_csr(build_on)
-        self.get_split_bcsr(build_on)
-        if self.verbose:
-            print("data format all preprocess (ms): {:.3f}".format((time.perf_counter() - t0) * 1e3))
-        return self
 
     def permute_rows(self, t):
         """a per-vertex tensor in the order the graph was loaded in (identity without ``reorder``)"""
