@@ -432,7 +432,7 @@ int psp_gemm_atb_f32(const float *A, const float *B, float *C, long long n, int 
 /* Same product without atomics: every workgroup stores its partial product in the caller's workspace and a second
  * kernel adds them in a fixed order (so results repeat bit for bit, and the 20-60 us the contended atomics take are
  * saved).  workspace: psp_gemm_atb_workspace_floats(n, K1, K2) floats of device memory, contents irrelevant on
- * entry; 0 means the shape runs the atomic kernel and needs none. */
+ * entry; 0 for widths there is no kernel for. */
 long long psp_gemm_atb_workspace_floats(long long n, int K1, int K2);
 int psp_gemm_atb_ws_f32(const float *A, const float *B, float *C, long long n, int K1, int K2, float *workspace,
                         long long workspace_floats, psp_stream_t stream);
@@ -444,8 +444,7 @@ int psp_gemm_atb_ws_act_f32(const float *A, const float *B, float *C, long long 
 /* ---------------------------------------------------------------------------------------------
  * DEVICE: Y[n,K2] = X[n,K1] * W (transW = 0, W is [K1,K2] row-major) or X * W^T (transW != 0, W is [K2,K1]) for
  * tall-skinny X and a small weight matrix: torch::mm(H, W) and torch::mm(AG, W.t()) of the fused GCN layer
- * (SpCONV/SpCONV.h:43-71).  Supported widths: K2 in {16, 32} with K1 in {16, 32, 48, 64} (and 128 with K2 = 16): one
- * lane per row, FMAs; K2 in {64, 128} with K1 in {16, 32, 64, 128}: fp32 matrix cores (v_mfma_f32_16x16x4_f32), W in
+ * (SpCONV/SpCONV.h:43-71).  Supported widths: multiples of 16 up to 128.  fp32 matrix cores (v_mfma_f32_16x16x4_f32), W in
  * LDS.  psp_gemm_xw_supported tells.  Y is overwritten; X and Y 16-byte aligned.  Deterministic (no atomics, one
  * fixed summation order per output element).
  * ------------------------------------------------------------------------------------------- */

@@ -2,88 +2,27 @@
 // H^T * (A dY) of the fused GCN layer (SpCONV/SpCONV.h:70 calls torch::mm(H.t(), AG)).  The product is a
 // reduction over n with a tiny output; a general GEMM picks tiles for large outputs and runs it 20-40 times
 // slower than the memory traffic allows.  HBM-bound up to about 64 x 64: 4 n (K1 + K2) bytes.
-// Two kernels:
-//   psp_atb_mfma_kernel  the matrix cores (v_mfma_f32_16x16x4_f32) fed straight from coalesced loads, for the shapes
-//                        whose accumulators fit a wavefront (or a workgroup's four); partial products either meet in
-//                        a caller's workspace and are added by psp_atb_reduce_kernel in a fixed order, or go to C
-//                        with atomics.
-//   psp_atb_kernel       the remaining shapes: every workgroup streams a band of rows through LDS, keeps a
-//                        K1/16 x K2/16 register tile per lane (vector FMAs) and adds its partial product to C with
-//                        fp32 atomics.
+// The matrix cores (v_mfma_f32_16x16x4_f32) are fed straight from coalesced loads; partial products either meet in a
+// caller's workspace and are added by psp_atb_reduce_kernel in a fixed order, or go to C with atomics.
 #include "psp_common.h"
 #include "spmm_kernel.h"
 #include "bf16_split.h"
 
-// RELU_A (both kernels): A enters the product as max(a, 0) -- the weight gradient of a layer whose input is the
-// activation of the previous layer's output, without that activation ever being stored.
-template <int K1, int K2, bool RELU_A>
-__global__ void __launch_bounds__(256)
-psp_atb_kernel(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, long long n,
-               long long rows_per_block)
-{
-    constexpr int RM = K1 / 16, RN = K2 / 16;
-    constexpr int ATB_ROWS = (K1 + K2 > 128) ? 32 : 64;  // at most 32 KB of LDS per workgroup
-    __shared__ float sA[ATB_ROWS][K1];
-    __shared__ float sB[ATB_ROWS][K2];
-    const int t = threadIdx.x;
-    const int ti = t >> 4, tj = t & 15;
-    float acc[RM][RN];
-#pragma unroll
-    for (int a = 0; a < RM; a++)
-#pragma unroll
-        for (int b = 0; b < RN; b++) acc[a][b] = 0.0f;
-
-    const long long r_begin = (long long)blockIdx.x * rows_per_block;
-    const long long r_end = r_begin + rows_per_block < n ? r_begin + rows_per_block : n;
-    for (long long base = r_begin; base < r_end; base += ATB_ROWS) {
-        // stage ATB_ROWS rows of A and B; rows past the end contribute zeros
-        for (int v = t; v < ATB_ROWS * K1 / 4; v += 256) {
-            const int r = v / (K1 / 4), c4 = v % (K1 / 4);
-            psp_f32x4 x = {0.f, 0.f, 0.f, 0.f};
-            if (base + r < r_end) x = *(const psp_f32x4 *)(A + (base + r) * K1 + c4 * 4);
-            if constexpr (RELU_A) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) x[e] = x[e] < 0.0f ? 0.0f : x[e];
-            }
-            *(psp_f32x4 *)&sA[r][c4 * 4] = x;
-        }
-        for (int v = t; v < ATB_ROWS * K2 / 4; v += 256) {
-            const int r = v / (K2 / 4), c4 = v % (K2 / 4);
-            psp_f32x4 x = {0.f, 0.f, 0.f, 0.f};
-            if (base + r < r_end) x = *(const psp_f32x4 *)(B + (base + r) * K2 + c4 * 4);
-            *(psp_f32x4 *)&sB[r][c4 * 4] = x;
-        }
-        __syncthreads();
-#pragma unroll 8
-        for (int r = 0; r < ATB_ROWS; r++) {
-            float av[RM], bv[RN];
-#pragma unroll
-            for (int a = 0; a < RM; a++) av[a] = sA[r][ti + 16 * a];
-#pragma unroll
-            for (int b = 0; b < RN; b++) bv[b] = sB[r][tj + 16 * b];
-#pragma unroll
-            for (int a = 0; a < RM; a++)
-#pragma unroll
-                for (int b = 0; b < RN; b++) acc[a][b] = __builtin_fmaf(av[a], bv[b], acc[a][b]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < RM; a++)
-#pragma unroll
-        for (int b = 0; b < RN; b++) unsafeAtomicAdd(&C[(ti + 16 * a) * K2 + tj + 16 * b], acc[a][b]);
-}
-
-// The same product on the matrix cores.  v_mfma_f32_16x16x4_f32 contracts four rows at a time; operand lane l holds
+// RELU_A: A enters the product as max(a, 0) -- the weight gradient of a layer whose input is the activation of the
+// previous layer's output, without that activation ever being stored.
+//
+// v_mfma_f32_16x16x4_f32 contracts four rows at a time; operand lane l holds
 // one element of row l / 16 of the four, for output index l % 16.  Which column of A (of B) an output index stands for
-// is free as long as the epilogue knows, so a lane loads V consecutive floats of its row (V = 4, 2 or 1) and feeds
-// them to V different tiles: tile m, index i is column (m / V) * 16 V + V i + (m % V).  One wave-wide load is then a
-// contiguous kilobyte (V = 4) that fills four tiles' operands, with no staging and no repeated loads.
+// is free as long as the epilogue knows, so a lane loads V consecutive floats of its row (V = 4, the last piece less) and
+// feeds them to V different tiles (psp_atb_col).  One wave-wide load is then a contiguous kilobyte (V = 4) that fills four
+// tiles' operands, with no staging and no repeated loads.
 // Wavefronts take U-group chunks round-robin, so the whole grid reads one contiguous window at a time.
-//   JSPLIT = 1 (up to sixteen 16x16 output tiles): each wavefront owns its chunks and all tiles; the workgroup's four
-//              partial products are added in LDS.
-//   JSPLIT = 4 (wider outputs, K2 a multiple of 64): the four wavefronts of a workgroup share their chunks and own a
-//              quarter of B's columns each; A is loaded by all four (the repeats are L1 / L2 hits).
+//   JSPLIT = 1: each wavefront owns its chunks and all tiles; the workgroup's four partial products are added in LDS.  From
+//              17 tiles on a wavefront takes a SIMD's registers alone and one workgroup fills a CU; the matrix cores are kept
+//              busy by the chunk in flight.  At 10^6 rows: 80 x 80 258 us (vector FMAs on LDS tiles, atomics) -> 160, 96 x 96
+//              317 -> 240, 112 x 112 403 -> 290; 64 x 128 194 (JSPLIT = 4) -> 183, 128 x 64 227 -> 185.
+//   JSPLIT = 4 (56 tiles and more, K2 = 128): the four wavefronts of a workgroup share their chunks and own a quarter of
+//              B's columns each; A is loaded by all four (the repeats are L1 / L2 hits).
 typedef float psp_mfma_acc __attribute__((ext_vector_type(4)));
 
 template <int V> __device__ __forceinline__ void psp_atb_load(const float *p, float *out)
@@ -91,6 +30,10 @@ template <int V> __device__ __forceinline__ void psp_atb_load(const float *p, fl
     if (V == 4) {
         const psp_f32x4 x = *(const psp_f32x4 *)p;
         out[0] = x[0], out[1] = x[1], out[2] = x[2], out[3] = x[3];
+    } else if (V == 3) {
+        typedef float f32x3 __attribute__((ext_vector_type(3), aligned(4)));
+        const f32x3 x = *(const f32x3 *)p;
+        out[0] = x[0], out[1] = x[1], out[2] = x[2];
     } else if (V == 2) {
         const psp_f32x2 x = *(const psp_f32x2 *)p;
         out[0] = x[0], out[1] = x[1];
@@ -98,18 +41,28 @@ template <int V> __device__ __forceinline__ void psp_atb_load(const float *p, fl
         out[0] = *p;
     }
 }
-// column of a (sub)matrix that index i of tile m stands for
-template <int V> __device__ __forceinline__ int psp_atb_col(int m, int i) { return (m / V) * 16 * V + V * i + (m % V); }
+// R tiles are loaded in pieces of four (16 bytes per lane) and a last one of R % 4: column that index i of tile m stands for
+template <int R> __device__ __forceinline__ int psp_atb_col(int m, int i)
+{
+    constexpr int N4 = R / 4 * 4, REM = R % 4;
+    return m < N4 ? (m / 4) * 64 + 4 * i + m % 4 : N4 * 16 + REM * i + (m - N4);
+}
+template <int R> __device__ __forceinline__ void psp_atb_load_row(const float *row, int c, float (&out)[R])
+{
+    constexpr int N4 = R / 4 * 4, REM = R % 4;
+#pragma unroll
+    for (int m = 0; m < N4; m += 4) psp_atb_load<4>(row + m * 16 + 4 * c, out + m);
+    if constexpr (REM > 0) psp_atb_load<REM>(row + N4 * 16 + REM * c, out + N4);
+}
 
 template <int K1, int K2, int JSPLIT, bool RELU_A>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, K1 * K2 / JSPLIT > 16 * 256 ? 1 : 2)
 psp_atb_mfma_kernel(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, long long n,
                     float *__restrict__ partial)
 {
     constexpr int RM = K1 / 16, RN = K2 / 16, RNW = RN / JSPLIT;
-    constexpr int VA = RM % 4 == 0 ? 4 : RM % 2 == 0 ? 2 : 1, VB = RNW % 4 == 0 ? 4 : RNW % 2 == 0 ? 2 : 1;
-    constexpr int U = (RM + RNW <= 2) ? 8 : (RM + RNW <= 4) ? 4 : 2;
-    static_assert(RN % JSPLIT == 0 && RM * RNW <= 16, "tile split does not fit the register budget");
+    constexpr int U = (RM + RNW <= 2) ? 8 : (RM + RNW <= 4 || RM * RNW > 16) ? 4 : 2;
+    static_assert(RN % JSPLIT == 0, "tile split");
     __shared__ float red[JSPLIT == 1 ? RM * RN * 256 : 1];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int kk = lane >> 4, c = lane & 15;
@@ -130,14 +83,12 @@ psp_atb_mfma_kernel(const float *__restrict__ A, const float *__restrict__ B, fl
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const long long row = (g + u) * 4 + kk;
-#pragma unroll
-            for (int t = 0; t < RM / VA; t++) psp_atb_load<VA>(A + row * K1 + t * 16 * VA + VA * c, &fa[u][t * VA]);
+            psp_atb_load_row<RM>(A + row * K1, c, fa[u]);
             if constexpr (RELU_A) {
 #pragma unroll
                 for (int m = 0; m < RM; m++) fa[u][m] = fa[u][m] < 0.0f ? 0.0f : fa[u][m];
             }
-#pragma unroll
-            for (int t = 0; t < RNW / VB; t++) psp_atb_load<VB>(B + row * K2 + col0 + t * 16 * VB + VB * c, &fb[u][t * VB]);
+            psp_atb_load_row<RNW>(B + row * K2 + col0, c, fb[u]);
         }
     };
     auto multiply = [&](const float (&fa)[U][RM], const float (&fb)[U][RNW]) {
@@ -184,11 +135,11 @@ psp_atb_mfma_kernel(const float *__restrict__ A, const float *__restrict__ B, fl
             const long long row = (gt + u) * 4 + kk;
 #pragma unroll
             for (int m = 0; m < RM; m++) {
-                a0[u][m] = row < n ? A[row * K1 + psp_atb_col<VA>(m, c)] : 0.f;
+                a0[u][m] = row < n ? A[row * K1 + psp_atb_col<RM>(m, c)] : 0.f;
                 if (RELU_A) a0[u][m] = a0[u][m] < 0.0f ? 0.0f : a0[u][m];
             }
 #pragma unroll
-            for (int q = 0; q < RNW; q++) b0[u][q] = row < n ? B[row * K2 + col0 + psp_atb_col<VB>(q, c)] : 0.f;
+            for (int q = 0; q < RNW; q++) b0[u][q] = row < n ? B[row * K2 + col0 + psp_atb_col<RNW>(q, c)] : 0.f;
         }
         multiply(a0, b0);
     }
@@ -215,7 +166,7 @@ psp_atb_mfma_kernel(const float *__restrict__ A, const float *__restrict__ B, fl
         for (int e = threadIdx.x; e < RM * RN * 256; e += 256) {
             const int l = e & 63, v = (e >> 6) & 3, tile = e >> 8;
             const int m = tile / RN, q = tile % RN;
-            float *d = &dst[psp_atb_col<VA>(m, 4 * (l >> 4) + v) * K2 + psp_atb_col<VB>(q, l & 15)];
+            float *d = &dst[psp_atb_col<RM>(m, 4 * (l >> 4) + v) * K2 + psp_atb_col<RNW>(q, l & 15)];
             if (partial) *d = red[e];
             else unsafeAtomicAdd(d, red[e]);
         }
@@ -226,7 +177,7 @@ psp_atb_mfma_kernel(const float *__restrict__ A, const float *__restrict__ B, fl
             for (int q = 0; q < RNW; q++)
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
-                    float *d = &dst[psp_atb_col<VA>(m, 4 * kk + v) * K2 + col0 + psp_atb_col<VB>(q, c)];
+                    float *d = &dst[psp_atb_col<RM>(m, 4 * kk + v) * K2 + col0 + psp_atb_col<RNW>(q, c)];
                     if (partial) *d = acc[m][q][v];
                     else unsafeAtomicAdd(d, acc[m][q][v]);
                 }
@@ -362,19 +313,7 @@ psp_atb_reduce_kernel(const float *__restrict__ partial, float *__restrict__ C, 
     }
 }
 
-typedef void (*psp_atb_kernel_t)(const float *, const float *, float *, long long, long long);
 typedef void (*psp_atb_mfma_kernel_t)(const float *, const float *, float *, long long, float *);
-
-static psp_atb_kernel_t atb_lookup(int K1, int K2, bool relu_a = false)
-{
-#define ATB_CASE(a, b) \
-    if (K1 == a && K2 == b) return relu_a ? psp_atb_kernel<a, b, true> : psp_atb_kernel<a, b, false>;
-#define ATB_ROW(a) ATB_CASE(a, 16) ATB_CASE(a, 32) ATB_CASE(a, 48) ATB_CASE(a, 64) ATB_CASE(a, 80) ATB_CASE(a, 96) ATB_CASE(a, 112) ATB_CASE(a, 128)
-    ATB_ROW(16) ATB_ROW(32) ATB_ROW(48) ATB_ROW(64) ATB_ROW(80) ATB_ROW(96) ATB_ROW(112) ATB_ROW(128)
-#undef ATB_ROW
-#undef ATB_CASE
-    return nullptr;
-}
 
 // *jsplit receives the kernel's JSPLIT
 static psp_atb_mfma_kernel_t atb_mfma_lookup(int K1, int K2, int *jsplit, bool relu_a = false)
@@ -384,58 +323,51 @@ static psp_atb_mfma_kernel_t atb_mfma_lookup(int K1, int K2, int *jsplit, bool r
     if (K1 == a && K2 == b) return relu_a ? psp_atb_mfma_kernel<a, b, 1, true> : psp_atb_mfma_kernel<a, b, 1, false>;
     ATB_MFMA(16, 16) ATB_MFMA(16, 32) ATB_MFMA(16, 48) ATB_MFMA(16, 64) ATB_MFMA(16, 80) ATB_MFMA(16, 96) ATB_MFMA(16, 112) ATB_MFMA(16, 128)
     ATB_MFMA(32, 16) ATB_MFMA(32, 32) ATB_MFMA(32, 48) ATB_MFMA(32, 64) ATB_MFMA(32, 80) ATB_MFMA(32, 96) ATB_MFMA(32, 112) ATB_MFMA(32, 128)
-    ATB_MFMA(48, 16) ATB_MFMA(48, 32) ATB_MFMA(48, 48) ATB_MFMA(48, 64) ATB_MFMA(48, 80)
-    ATB_MFMA(64, 16) ATB_MFMA(64, 32) ATB_MFMA(64, 48) ATB_MFMA(64, 64)
-    ATB_MFMA(80, 16) ATB_MFMA(80, 32) ATB_MFMA(80, 48)
-    ATB_MFMA(96, 16) ATB_MFMA(96, 32) ATB_MFMA(112, 16) ATB_MFMA(112, 32) ATB_MFMA(128, 16) ATB_MFMA(128, 32)
+#define ATB_ROW(a) ATB_MFMA(a, 16) ATB_MFMA(a, 32) ATB_MFMA(a, 48) ATB_MFMA(a, 64) ATB_MFMA(a, 80) ATB_MFMA(a, 96) ATB_MFMA(a, 112)
+    ATB_ROW(48) ATB_ROW(64) ATB_ROW(80) ATB_ROW(96) ATB_ROW(112) ATB_ROW(128)
+    ATB_MFMA(48, 128) ATB_MFMA(64, 128) ATB_MFMA(80, 128) ATB_MFMA(96, 128)
+#undef ATB_ROW
 #undef ATB_MFMA
     *jsplit = 4;
 #define ATB_MFMA4(a, b) \
     if (K1 == a && K2 == b) return relu_a ? psp_atb_mfma_kernel<a, b, 4, true> : psp_atb_mfma_kernel<a, b, 4, false>;
-    ATB_MFMA4(64, 128) ATB_MFMA4(80, 64) ATB_MFMA4(96, 64) ATB_MFMA4(112, 64) ATB_MFMA4(128, 64)
-    ATB_MFMA4(80, 128) ATB_MFMA4(96, 128) ATB_MFMA4(112, 128) ATB_MFMA4(128, 128)
+    ATB_MFMA4(112, 128) ATB_MFMA4(128, 128)
 #undef ATB_MFMA4
     return nullptr;
 }
 
-// Workgroups of the MFMA kernel: about four per CU, fewer when there are not that many 8-group chunks.
+// Workgroups of the MFMA kernel: about four per CU (wide outputs: one), fewer when there are not that many 8-group chunks.
 static long long atb_mfma_grid(long long n, int jsplit, int E)
 {
     const long long chunks = ((n + 3) / 4 + 7) / 8;
-    const long long max_wgs = 1024;
+    const long long max_wgs = jsplit == 1 && E > 4096 ? 256 : 1024;  // from 17 tiles on one workgroup fills a CU
     long long wgs = jsplit == 1 ? (chunks + 3) / 4 : chunks;
     if (wgs > max_wgs) wgs = max_wgs;
     return wgs < 1 ? 1 : wgs;
 }
 
-PSP_EXPORT int psp_gemm_atb_supported(int K1, int K2) { return atb_lookup(K1, K2) != nullptr; }
+PSP_EXPORT int psp_gemm_atb_supported(int K1, int K2)
+{
+    int jsplit;
+    return atb_mfma_lookup(K1, K2, &jsplit) != nullptr;
+}
 
 static int atb_atomic(const float *A, const float *B, float *C, long long n, int K1, int K2, bool relu_a, hipStream_t stream)
 {
     PSP_REQUIRE(n >= 0 && K1 >= 1 && K2 >= 1, "gemm_atb: bad size");
-    psp_atb_kernel_t k = atb_lookup(K1, K2, relu_a);
-    PSP_REQUIRE(k != nullptr, "gemm_atb: K1 and K2 must be multiples of 16 up to 128 (got %d, %d)", K1, K2);
+    int jsplit = 1;
+    psp_atb_mfma_kernel_t km = atb_mfma_lookup(K1, K2, &jsplit, relu_a);
+    PSP_REQUIRE(km != nullptr, "gemm_atb: K1 and K2 must be multiples of 16 up to 128 (got %d, %d)", K1, K2);
     PSP_REQUIRE(C != nullptr && (n == 0 || (A && B)), "gemm_atb: null pointer");
     int rc = psp_zero_f32(C, (size_t)K1 * K2, stream);
     if (rc != PSP_OK || n == 0) return rc;
-    int jsplit = 1;
-    if (psp_atb_mfma_kernel_t km = atb_mfma_lookup(K1, K2, &jsplit, relu_a)) {
-        long long wgs = atb_mfma_grid(n, jsplit, K1 * K2);
-        if (K1 == 128 && K2 == 128 && psp_opts().dense_split) {
-            km = relu_a ? psp_atb_split_kernel<true> : psp_atb_split_kernel<false>;
-            wgs = wgs < ATB_SPLIT_WGS ? wgs : ATB_SPLIT_WGS;
-        }
-        hipLaunchKernelGGL(km, dim3((unsigned)wgs), dim3(256), 0, stream, A, B, C, n, (float *)nullptr);
-        return psp_check_launch("gemm_atb mfma kernel");
+    long long wgs = atb_mfma_grid(n, jsplit, K1 * K2);
+    if (K1 == 128 && K2 == 128 && psp_opts().dense_split) {
+        km = relu_a ? psp_atb_split_kernel<true> : psp_atb_split_kernel<false>;
+        wgs = wgs < ATB_SPLIT_WGS ? wgs : ATB_SPLIT_WGS;
     }
-    // about 8 workgroups per CU, each on a contiguous band of whole 64-row tiles
-    const int ATB_ROWS = 64;
-    long long blocks = (n + ATB_ROWS - 1) / ATB_ROWS;
-    if (blocks > 2048) blocks = 2048;
-    long long rows_per_block = ((n + blocks - 1) / blocks + ATB_ROWS - 1) / ATB_ROWS * ATB_ROWS;
-    blocks = (n + rows_per_block - 1) / rows_per_block;
-    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), 0, stream, A, B, C, n, rows_per_block);
-    return psp_check_launch("gemm_atb kernel");
+    hipLaunchKernelGGL(km, dim3((unsigned)wgs), dim3(256), 0, stream, A, B, C, n, (float *)nullptr);
+    return psp_check_launch("gemm_atb mfma kernel");
 }
 
 PSP_EXPORT int psp_gemm_atb_f32(const float *A, const float *B, float *C, long long n, int K1, int K2,
@@ -456,7 +388,7 @@ PSP_EXPORT int psp_gemm_atb_ws_act_f32(const float *A, const float *B, float *C,
 {
     int jsplit = 1;
     psp_atb_mfma_kernel_t km = atb_mfma_lookup(K1, K2, &jsplit, relu_a != 0);
-    if (!km || n <= 0) return atb_atomic(A, B, C, n, K1, K2, relu_a != 0, (hipStream_t)stream);  // shapes of the LDS-tiled kernel; n = 0
+    if (!km || n <= 0) return atb_atomic(A, B, C, n, K1, K2, relu_a != 0, (hipStream_t)stream);  // n = 0, widths there is no kernel for
     PSP_REQUIRE(A && B && C, "gemm_atb_ws: null pointer");
     long long wgs = atb_mfma_grid(n, jsplit, K1 * K2);
     PSP_REQUIRE(workspace && workspace_floats >= wgs * K1 * K2, "gemm_atb_ws: the workspace holds %lld floats, %lld needed",

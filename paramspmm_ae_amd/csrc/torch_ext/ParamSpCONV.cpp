@@ -32,11 +32,27 @@ static Tensor aggregate(int fmt, const Tensor &D, const Tensor &rowPtr, const Te
     return Y;
 }
 
+// Rows from which the library's dense kernels are used (PyTorch's GEMM below): they cost one launch with the activation
+// or the mask folded in, where PyTorch needs one for each.
+constexpr long kDenseRows = 1024;
+
+// Where a product's result is the activation of a ReLU network (GCN, GIN), another order of its sum puts some element on the
+// other side of zero, which drops or adds a whole term of the gradient: a training run would not repeat the figures it gave
+// before.  Those products stay with the order that each shape has always had: the library's (ascending k up to 32 columns,
+// see dense_xw.hip) at the shapes below from 16384 rows on, PyTorch's GEMM elsewhere.  Gradients (X W^T and the weight
+// gradient) and the attention layer have no such step behind them and take the library's kernel at every shape.
+enum class Order { any, kept };
+static bool kept_order_is_ours(long n, long K1, long K2)
+{
+    const bool pow2 = K1 == 16 || K1 == 32 || K1 == 64 || K1 == 128;
+    return n >= 16384 && (K2 <= 32 ? K1 <= 64 || (K1 == 128 && K2 == 16) : (K2 == 64 || K2 == 128) && pow2);
+}
+
 // H^T * AG.  For narrow layers the product is a reduction over ~10^6 rows into a tiny matrix, which the library
 // streams at memory speed; everything else goes to torch::mm.
 static Tensor weight_gradient(const Tensor &H, const Tensor &AG)
 {
-    const bool narrow = H.dim() == 2 && AG.dim() == 2 && H.size(0) == AG.size(0) && H.size(0) >= 16384 &&
+    const bool narrow = H.dim() == 2 && AG.dim() == 2 && H.size(0) == AG.size(0) && H.size(0) >= kDenseRows &&
                         H.scalar_type() == torch::kFloat32 && AG.scalar_type() == torch::kFloat32 &&
                         psp_gemm_atb_supported((int)H.size(1), (int)AG.size(1));
     if (!narrow) return torch::mm(H.t(), AG);
@@ -51,15 +67,15 @@ static Tensor weight_gradient(const Tensor &H, const Tensor &AG)
     return dW;
 }
 
-// X * W (or X * W^T): the library's one-lane-per-row kernel for narrow layers on many rows, torch::mm otherwise
-static Tensor dense_xw(const Tensor &X, const Tensor &W, bool transW)
+// X * W (or X * W^T): the library's kernel for narrow layers on many rows, torch::mm otherwise
+static Tensor dense_xw(const Tensor &X, const Tensor &W, bool transW, Order order)
 {
     const long K1 = X.dim() == 2 ? X.size(1) : -1;
     const bool shapes = X.dim() == 2 && W.dim() == 2 && W.size(transW ? 1 : 0) == K1;
     const long K2 = shapes ? W.size(transW ? 0 : 1) : -1;
-    const bool narrow = shapes && X.size(0) >= 16384 && X.scalar_type() == torch::kFloat32 &&
+    const bool narrow = shapes && X.size(0) >= kDenseRows && X.scalar_type() == torch::kFloat32 &&
                         W.scalar_type() == torch::kFloat32 && X.is_cuda() && W.is_cuda() &&
-                        psp_gemm_xw_supported((int)K1, (int)K2);
+                        psp_gemm_xw_supported((int)K1, (int)K2) && (order == Order::any || kept_order_is_ours(X.size(0), K1, K2));
     if (!narrow) return torch::mm(X, transW ? W.t() : W);
     Tensor Xc = X.contiguous(), Wc = W.contiguous();
     DeviceGuard guard(Xc.device());
@@ -70,12 +86,13 @@ static Tensor dense_xw(const Tensor &X, const Tensor &W, bool transW)
 
 // The same two products with the ReLU between two layers folded in (psp_gemm_xw_act_f32 / psp_gemm_atb_ws_act_f32);
 // shapes the library does not cover apply the activation with PyTorch and multiply with torch::mm.
-static Tensor dense_relu_xw(const Tensor &Z, const Tensor &W)
+static Tensor dense_relu_xw(const Tensor &Z, const Tensor &W, Order order)
 {
     const long K1 = Z.dim() == 2 ? Z.size(1) : -1;
     const bool shapes = Z.dim() == 2 && W.dim() == 2 && W.size(0) == K1;
-    const bool narrow = shapes && Z.size(0) >= 16384 && Z.scalar_type() == torch::kFloat32 && W.scalar_type() == torch::kFloat32 &&
-                        psp_gemm_xw_supported((int)K1, (int)W.size(1));
+    const bool narrow = shapes && Z.size(0) >= kDenseRows && Z.scalar_type() == torch::kFloat32 && W.scalar_type() == torch::kFloat32 &&
+                        psp_gemm_xw_supported((int)K1, (int)W.size(1)) &&
+                        (order == Order::any || kept_order_is_ours(Z.size(0), K1, W.size(1)));
     if (!narrow) return torch::mm(torch::relu(Z), W);
     Tensor Zc = Z.contiguous(), Wc = W.contiguous();
     DeviceGuard guard(Zc.device());
@@ -89,7 +106,7 @@ static Tensor dense_xwt_masked(const Tensor &AG, const Tensor &W, const Tensor &
     const long K1 = AG.dim() == 2 ? AG.size(1) : -1;
     const bool shapes = AG.dim() == 2 && W.dim() == 2 && W.size(1) == K1 && Z.dim() == 2 && Z.size(0) == AG.size(0) &&
                         Z.size(1) == W.size(0);
-    const bool narrow = shapes && AG.size(0) >= 16384 && AG.scalar_type() == torch::kFloat32 && W.scalar_type() == torch::kFloat32 &&
+    const bool narrow = shapes && AG.size(0) >= kDenseRows && AG.scalar_type() == torch::kFloat32 && W.scalar_type() == torch::kFloat32 &&
                         Z.scalar_type() == torch::kFloat32 && psp_gemm_xw_supported((int)K1, (int)W.size(0));
     if (!narrow) return at::threshold_backward(torch::mm(AG, W.t()), Z, 0);  // what F.relu's backward runs
     Tensor Gc = AG.contiguous(), Wc = W.contiguous(), Zc = Z.contiguous();
@@ -101,7 +118,7 @@ static Tensor dense_xwt_masked(const Tensor &AG, const Tensor &W, const Tensor &
 // relu(Z)^T * AG
 static Tensor weight_gradient_relu(const Tensor &Z, const Tensor &AG)
 {
-    const bool narrow = Z.dim() == 2 && AG.dim() == 2 && Z.size(0) == AG.size(0) && Z.size(0) >= 16384 &&
+    const bool narrow = Z.dim() == 2 && AG.dim() == 2 && Z.size(0) == AG.size(0) && Z.size(0) >= kDenseRows &&
                         Z.scalar_type() == torch::kFloat32 && AG.scalar_type() == torch::kFloat32 &&
                         psp_gemm_atb_supported((int)Z.size(1), (int)AG.size(1));
     if (!narrow) return torch::mm(torch::relu(Z).t(), AG);
@@ -124,7 +141,7 @@ static Tensor relu_input_forward(int fmt, Tensor Z, Tensor W, Tensor rowPtr, Ten
     need_gpu(Z, "input");
     need_gpu(W, "weight");
     TORCH_CHECK(fmt >= 0 && fmt <= 4 && (fmt == 1 || fmt == 3) == target_row.has_value(), "format code and target_row disagree");
-    return aggregate(fmt, dense_relu_xw(Z, W), rowPtr, colIdx, values, target_row ? &*target_row : nullptr, CF, bw);
+    return aggregate(fmt, dense_relu_xw(Z, W, Order::kept), rowPtr, colIdx, values, target_row ? &*target_row : nullptr, CF, bw);
 }
 // [dZ, dW] = [ ((A dY) W^T) where Z > 0,  relu(Z)^T (A dY) ]
 static std::vector<Tensor> relu_input_backward(int fmt, Tensor dY, Tensor Z, Tensor W, Tensor rowPtr, Tensor colIdx,
@@ -336,7 +353,7 @@ static Tensor forward_impl(int fmt, const Tensor &H, const Tensor &W, const Tens
 {
     need_gpu(H, "input");
     need_gpu(W, "weight");
-    return aggregate(fmt, dense_xw(H, W, false), rowPtr, colIdx, values, target_row, CF, blkWarpNum);
+    return aggregate(fmt, dense_xw(H, W, false, Order::kept), rowPtr, colIdx, values, target_row, CF, blkWarpNum);
 }
 
 static std::vector<Tensor> backward_impl(int fmt, const Tensor &dY, const Tensor &H, const Tensor &W, const Tensor &rowPtr,
@@ -348,7 +365,7 @@ static std::vector<Tensor> backward_impl(int fmt, const Tensor &dY, const Tensor
     // the reference multiplies by A, not A^T (SpCONV/SpCONV.h:67-71): exact for the symmetric matrices its
     // loaders build
     Tensor AG = aggregate(fmt, dY, rowPtr, colIdx, values, target_row, CF, blkWarpNum);
-    return {dense_xw(AG, W, true), weight_gradient(H, AG)};
+    return {dense_xw(AG, W, true, Order::any), weight_gradient(H, AG)};
 }
 
 // ---- mean NLL loss of the training step (an addition of this build; F.nll_loss in GNN.py:131-146) ----------
@@ -482,7 +499,7 @@ struct GCNFunction : LayerNode {
         if (!g[0].defined()) return {Tensor(), Tensor()};
         Tensor H = a(), W = w();
         Tensor AG = aggregate(op->fmt, g[0], op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
-        return {wants(0) ? dense_xw(AG, W, true) : Tensor(), wants(1) ? weight_gradient(H, AG) : Tensor()};
+        return {wants(0) ? dense_xw(AG, W, true, Order::any) : Tensor(), wants(1) ? weight_gradient(H, AG) : Tensor()};
     }
 };
 static Tensor gcn_layer(op_t op, Tensor H, Tensor W)
@@ -491,7 +508,7 @@ static Tensor gcn_layer(op_t op, Tensor H, Tensor W)
     need_gpu(W, "weight");
     return with_node<GCNFunction>(op, {H, W}, [&](GCNFunction *n) {
         if (n) n->a_ = SavedVariable(H, false), n->w_ = SavedVariable(W, false);
-        return aggregate(op->fmt, dense_xw(H, W, false), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
+        return aggregate(op->fmt, dense_xw(H, W, false, Order::kept), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
     });
 }
 
@@ -502,7 +519,7 @@ struct AggregateFirst : LayerNode {
     {
         if (!g[0].defined()) return {Tensor(), Tensor()};
         Tensor AH = a(), W = w(), dY = g[0].contiguous(), dH;
-        if (wants(0)) dH = aggregate(op->fmt, dense_xw(dY, W, true), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
+        if (wants(0)) dH = aggregate(op->fmt, dense_xw(dY, W, true, Order::any), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
         return {dH, wants(1) ? weight_gradient(AH, dY) : Tensor()};
     }
 };
@@ -515,7 +532,7 @@ template <class N> static Tensor aggregate_first_layer(op_t op, Tensor H, Tensor
     return with_node<N>(op, {H, W}, [&](N *n) {
         Tensor AH = aggregate(op->fmt, H, op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
         if (n) n->a_ = SavedVariable(AH, false), n->w_ = SavedVariable(W, false);
-        return dense_xw(AH, W, false);
+        return dense_xw(AH, W, false, Order::kept);
     });
 }
 
@@ -551,7 +568,7 @@ struct GINReLUInputFunction : LayerNode {
     {
         if (!g[0].defined()) return {Tensor(), Tensor()};
         Tensor AX = a(), W = w(), Z = z(), dY = g[0].contiguous();
-        return {wants(0) ? aggregate_act_op(op->fmt, dense_xw(dY, W, true), op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw,
+        return {wants(0) ? aggregate_act_op(op->fmt, dense_xw(dY, W, true, Order::any), op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw,
                                             false, Z)
                          : Tensor(),
                 wants(1) ? weight_gradient(AX, dY) : Tensor()};
@@ -562,7 +579,7 @@ static Tensor gin_relu_layer(op_t op, Tensor Z, Tensor W)
     return with_node<GINReLUInputFunction>(op, {Z, W}, [&](GINReLUInputFunction *n) {
         Tensor AX = aggregate_act_op(op->fmt, Z, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw, true, c10::nullopt);
         if (n) n->a_ = SavedVariable(AX, false), n->w_ = SavedVariable(W, false), n->z_ = SavedVariable(Z, false);
-        return dense_xw(AX, W, false);
+        return dense_xw(AX, W, false, Order::kept);
     });
 }
 
@@ -583,7 +600,7 @@ struct AGNNFunction : LayerNode {  // a_ = X, z_ = att
         auto r = op->fmt == 4 ? attn_window_backward(dY, att, op->rowPtr, op->colIdx)
                               : attn_backward(op->fmt, dY, att, op->rowPtr, op->colIdx, op->target_row, op->slot, op->bw);
         Tensor dX, dW;
-        if (wants(0)) dX = relu_input ? dense_xwt_masked(r[0], W, X) : dense_xw(r[0], W, true);
+        if (wants(0)) dX = relu_input ? dense_xwt_masked(r[0], W, X) : dense_xw(r[0], W, true, Order::any);
         if (wants(1)) dW = relu_input ? weight_gradient_relu(X, r[0]) : weight_gradient(X, r[0]);
         return {dX, dW, r[1].reshape({1, 1}).expand(alpha_shape)};
     }
@@ -593,7 +610,7 @@ static Tensor agnn_layer(op_t op, Tensor X, Tensor W, Tensor attention_w, bool r
     need_gpu(X, "input");
     need_gpu(W, "weight");
     return with_node<AGNNFunction>(op, {X, W, attention_w}, [&](AGNNFunction *n) {
-        Tensor Xp = relu_input ? dense_relu_xw(X, W) : dense_xw(X, W, false);
+        Tensor Xp = relu_input ? dense_relu_xw(X, W, Order::any) : dense_xw(X, W, false, Order::any);
         auto r = attn_fused_forward(*op, Xp, attention_w.reshape({-1}).narrow(0, 0, 1));
         if (n) {
             n->a_ = SavedVariable(X, false), n->w_ = SavedVariable(W, false), n->z_ = SavedVariable(r[0], false);
@@ -707,14 +724,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("dense_xw", [](Tensor X, Tensor W, bool transW) {
         need_gpu(X, "X");
         need_gpu(W, "W");
-        return dense_xw(X, W, transW);
+        return dense_xw(X, W, transW, transW ? Order::any : Order::kept);
     }, "X * W (transW false) or X * W^T for tall-skinny X: (X, W, transW)");
     // the dense products of a layer that reads its input through a ReLU, for layers that place them around their
     // own sparse operators (the attention layer): max(Z, 0) * W, (G * W^T) where Z > 0, max(Z, 0)^T * G
     m.def("dense_relu_xw", [](Tensor Z, Tensor W) {
         need_gpu(Z, "Z");
         need_gpu(W, "W");
-        return dense_relu_xw(Z, W);
+        return dense_relu_xw(Z, W, Order::kept);
     }, "max(Z, 0) * W: (Z, W)");
     m.def("dense_xwt_masked", [](Tensor G, Tensor W, Tensor Z) {
         need_gpu(G, "G");

@@ -23,9 +23,10 @@ def graph():
 @pytest.mark.parametrize("vec,split", [(1, False), (1, True), (2, False), (2, True)])
 @pytest.mark.parametrize("K", [4, 16, 17, 32, 33, 47, 64, 65, 100, 128])
 def test_attention_forward_backward(graph, vec, split, K):
-    import ParamSpCONV as SpCONV
     from paramspmm_ae_amd.gnn_conv import _slot_columns
     from paramspmm_ae_amd.PCSR import pcsr_spmm
+
+    import ParamSpCONV as SpCONV
 
     g, n = graph, graph.mtx_nodes
     op = pcsr_spmm(g, vec_size=vec, if_split=split)
