@@ -193,23 +193,27 @@ int psp_fill_f32(float *p, size_t n, float value, hipStream_t stream)
     return psp_check_launch("fill");
 }
 
+// One lane per row reads the sums; the few rows that have one are then scaled by sixteen lanes each.  With sixteen lanes on every
+// row the kernel took 23 us for 2^20 rows of which one in nine has a sum.
 __global__ void __launch_bounds__(256) psp_row_scale_kernel(float *__restrict__ Y, const float *__restrict__ s, int rows, int N)
 {
-    // 16 lanes per row: almost every row has s == 0 and costs one load
-    const long long g = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    const int sub = threadIdx.x & 15;
-    if (g >= rows) return;
-    const float w = s[g];
-    if (w == 0.0f) return;
-    const float inv = 1.0f / w;
-    float *yr = Y + g * N;
-    for (int c = sub; c < N; c += 16) yr[c] *= inv;
+    const int row = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & (PSP_WAVE - 1), sub = lane & 15;
+    const float w = row < rows ? s[row] : 0.0f;
+    unsigned mine = (unsigned)(__ballot(w != 0.0f) >> (lane - sub)) & 0xffffu;  // rows of these sixteen lanes
+    while (mine) {
+        const int i = __ffs((int)mine) - 1;
+        mine &= mine - 1;
+        const float inv = 1.0f / psp_bperm_f(lane - sub + i, w);
+        float *yr = Y + (size_t)(row - sub + i) * (size_t)N;
+        for (int c = sub; c < N; c += 16) yr[c] *= inv;
+    }
 }
 
 int psp_row_scale(float *Y, const float *s, int rows, int N, hipStream_t stream)
 {
     if (rows == 0 || N == 0) return PSP_OK;
-    hipLaunchKernelGGL(psp_row_scale_kernel, dim3(psp_ceil_div((long long)rows * 16, 256)), dim3(256), 0, stream, Y, s, rows, N);
+    hipLaunchKernelGGL(psp_row_scale_kernel, dim3(psp_ceil_div(rows, 256)), dim3(256), 0, stream, Y, s, rows, N);
     return psp_check_launch("row scale");
 }
 

@@ -128,11 +128,11 @@ static int sddmm_f64_launch(const int *rowPtr, const int *colIdx, const double *
     sddmm_f64_kernel_t k = nullptr;
 #define PSP_CASE(L_, C_, U_) \
     if constexpr (L_ >= 2) { \
-        if (V == 2 && logL == L_ && C == C_) k = psp_sddmm_kernel<L_, C_, 2, U_, NR, SPLIT, false, false, double>; \
+        if (V == 2 && logL == L_ && C == C_) k = psp_sddmm_kernel<L_, C_, 2, U_, NR, SPLIT, false, false, false, double>; \
     }
     PSP_SDDMM_FOR_EACH_LCU(PSP_CASE)
 #undef PSP_CASE
-    if (V == 1) k = psp_sddmm_kernel<2, 1, 1, 4, NR, SPLIT, false, false, double>;
+    if (V == 1) k = psp_sddmm_kernel<2, 1, 1, 4, NR, SPLIT, false, false, false, double>;
     PSP_REQUIRE(k, "sddmm_f64: no kernel for K = %d", K);
     const int logR = 6 - logL;
     int logW = SPLIT ? (logR > 4 ? logR : 4) : logR;

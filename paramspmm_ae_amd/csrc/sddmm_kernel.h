@@ -11,6 +11,8 @@
 #include "psp_common.h"
 #include "spmm_kernel.h"  // psp_vec, psp_group_sum
 
+template <int I> struct psp_int { static constexpr int value = I; };
+
 // psp_group_sum (spmm_kernel.h) for double: both halves of a value cross the lanes, then they are added as one number
 template <int LOGL> __device__ __forceinline__ double psp_group_sum(double v)
 {
@@ -43,12 +45,19 @@ template <int LOGL> __device__ __forceinline__ float psp_group_max(float v)
 
 // val: bcsr -> [nblk,2] block values (gate); csr -> optional per-entry scale (may be null when !SCALE)
 //
+// The gathers bind it: the rows of B come from wherever the columns point, and what counts is how many of them are under
+// way.  So a group walks its entries U at a time whatever rows they belong to, with the next U requested before the
+// current U are multiplied (two register sets), and changes its A row between two entries where one ends.  The walk by
+// rows before this one stopped at every row's end, which on short rows left half of each step empty and nothing under way
+// across it.  U = 2 up to 128 columns: 4 cost 10-16 registers and one to two wavefronts per SIMD (10^6 rows of 21 entries, plain, K = 32 /
+// 64 / 128: by rows 236 / 428 / 784 us, U = 4 224 / 395 / 733, U = 2 198 / 357 / 667); U = 1 with four vectors per lane.
+//
 // The walk is the one of the SpMM kernel: a wavefront owns W = 2^logW consecutive segments, their stored entries
 // are divided evenly between the 64/L lane groups, and a group reloads its A row (prefetched one segment ahead)
 // whenever it crosses into another row.  Every stored entry is written exactly once, so `out` needs no clearing.
 //
-// row_max (CSR layouts, may be null): the largest result of every row is also raised into row_max[row] (atomic
-// max, once per lane group and row; the caller has filled the array with the lowest float).  The attention
+// MAX (CSR layouts): the largest result of every row is also raised into row_max[row] (atomic
+// max, once per row and window; the caller has filled the array with the lowest float).  The attention
 // pipeline's softmax-weighted SpMM takes its reference maxima from there instead of sweeping the entries again.
 //
 // BAL (plain layouts): the launch is a fixed grid of wavefronts that divide the *stored entries* between them -- each
@@ -56,7 +65,7 @@ template <int LOGL> __device__ __forceinline__ float psp_group_max(float v)
 // them window by window (up to 64 rows at a time, cut at the tile's ends).  Every entry's result is independent, so a
 // row may be cut anywhere, and a hub row of 10^5 entries spreads over a hundred wavefronts instead of pinning one.
 // T: float, or double in pieces of V = 2 (generic_f64.hip).
-template <int LOGL, int C, int V, int U, int NR, bool SPLIT, bool SCALE, bool BAL = false, typename T = float>
+template <int LOGL, int C, int V, int U, int NR, bool SPLIT, bool SCALE, bool BAL = false, bool MAX = false, typename T = float>
 __global__ void __launch_bounds__(512)
 psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, const T *__restrict__ val,
                  const int *__restrict__ target_row, const T *__restrict__ A, const T *__restrict__ B,
@@ -77,6 +86,9 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
     constexpr int LINE = 128 / sizeof(T);
     constexpr int HOLD = (NR <= 2 && LOGL >= 2 && ((LINE / NR) >> LOGL) >= 2) ? ((LINE / NR) >> LOGL) : 1;  // chunks held back per group
     __shared__ __align__(16) T s_hold[HOLD > 1 ? PSP_MAX_WAVES : 1][HOLD > 1 ? HOLD * PSP_WAVE * NR : 1];
+
+    static_assert(!MAX || (sizeof(T) == 4 && !BCSR), "row maxima exist for the CSR layouts in single precision");
+    __shared__ float s_max[MAX ? PSP_MAX_WAVES : 1][MAX ? PSP_WAVE : 1];  // largest result so far of each filled segment
 
     const int lane = threadIdx.x & (PSP_WAVE - 1);
     const int wave = threadIdx.x >> 6;
@@ -109,6 +121,7 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         const unsigned long long fmask = __ballot(filled);
         const int slot = __popcll(fmask & ((1ull << lane) - 1ull));
         s_seg[wave][lane] = make_int2(P1, -1);
+        if constexpr (MAX) s_max[wave][lane] = PSP_F32_LOWEST;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         if (filled) s_seg[wave][slot] = make_int2(e, SPLIT ? target_row[s0 + lane] : s0 + lane);
@@ -156,12 +169,13 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
     }
 
     float lmax = PSP_F32_LOWEST;  // largest result among this lane's entries of the current row
-    auto emit_row_max = [&](int key) {
+    auto emit_row_max = [&](int slot) {
         const float m = psp_group_max<LOGL>(lmax);
-        if (sub == 0 && m > PSP_F32_LOWEST) psp_atomic_max_f32(row_max + key, m);
+        if constexpr (MAX) {
+            if (sub == 0) __hip_atomic_fetch_max(&s_max[wave][slot], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
         lmax = PSP_F32_LOWEST;
     };
-    const bool want_max = sizeof(T) == 4 && !BCSR && row_max != nullptr;  // uniform
 
     // lane `sub` of the group picks up entry base+sub (column index and, where the format has one, its value); the
     // next chunk's are requested before the current chunk is worked on
@@ -199,10 +213,40 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         held = 0;
     };
 
+    constexpr int STEPS = L / U;
+    static_assert(STEPS == 1 || STEPS % 2 == 0, "the two register sets alternate through a chunk");
+    vec_t bv[2][U][C];
+    auto gather = [&](int k, int cols, vec_t (&dst)[U][C]) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const T *br = B + (size_t)psp_bperm_i(grp_base + k + u, cols) * (size_t)K;
+#pragma unroll
+            for (int i = 0; i < C; i++) dst[u][i] = psp_load_vec<V, T>(br + off[i]);
+        }
+    };
+    // the current row is finished: go to the next filled segment, whose A row was requested one segment ago
+    auto next_row = [&]() {
+        const int2 nx = w_seg[++cur];
+        row_end = nx.x;
+        if (nx.y != mykey) {
+            if constexpr (MAX) emit_row_max(cur - 1);  // the group is converged here: the condition is group-uniform
+            mykey = nx.y;
+#pragma unroll
+            for (int r = 0; r < NR; r++)
+#pragma unroll
+                for (int i = 0; i < C; i++)
+#pragma unroll
+                    for (int e = 0; e < V; e++) a[r][i][e] = a_nxt[r][i][e];
+        }
+        const int nk = cur + 1 < PSP_WAVE ? w_seg[cur + 1].y : -1;
+        if (nk >= 0 && nk != mykey) load_a(nk, a_nxt);
+    };
+    gather(0, c_cur, bv[0]);
+
     for (int base = a0; base < b0; base += L) {
         const int p = base + sub;
         const bool ok = p < b0;
-        int c_nxt = 0;
+        int c_nxt = c_cur;
         T gate_nxt[NR];
 #pragma unroll
         for (int r = 0; r < NR; r++) gate_nxt[r] = (T)0;
@@ -211,57 +255,46 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
 #pragma unroll
         for (int r = 0; r < NR; r++) res[r] = (T)0;
 
-        const int cnt = min(L, b0 - base);
-        int k = 0;
-        while (k < cnt) {
-            // the current row's entries inside this chunk: positions [k, run_end)
-            const int run_end = min(cnt, row_end - base);
-            for (; k < run_end; k += U) {
-                int ck[U];
+        // U entries at a time, the next U entries' rows of B on the way meanwhile (from the next chunk's columns at the end)
+        auto step = [&](const int st, auto set_) {
+            constexpr int SET = decltype(set_)::value;
+            if (base + st * U >= b0) return;
+            if (base + (st + 1) * U < b0) {
+                if (st + 1 < STEPS) gather((st + 1) * U, c_cur, bv[1 - SET]);
+                else gather(0, c_nxt, bv[1 - SET]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < U; u++) ck[u] = psp_bperm_i(grp_base + min(k + u, L - 1), c_cur);
-                vec_t bv[U][C];
+            for (int u = 0; u < U; u++) {
+                const int e_ = base + st * U + u;
+                if (e_ == row_end && e_ < b0) next_row();
 #pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const T *br = B + (size_t)ck[u] * (size_t)K;
+                for (int r = 0; r < NR; r++) {
+                    T part = (T)0;
 #pragma unroll
-                    for (int i = 0; i < C; i++) bv[u][i] = psp_load_vec<V, T>(br + off[i]);
+                    for (int i = 0; i < C; i++)
+#pragma unroll
+                        for (int e = 0; e < V; e++) part = psp_fma(a[r][i][e], psp_elem<V, T>(bv[SET][u][i], e), part);
+                    part = psp_group_sum<LOGL>(part);
+                    if (sub == st * U + u && e_ < b0) {
+                        res[r] = part;
+                        if constexpr (MAX) lmax = fmaxf(lmax, SCALE ? part * gate[0] : part);
+                    }
                 }
+            }
+            if constexpr (STEPS == 1) {
 #pragma unroll
                 for (int u = 0; u < U; u++)
 #pragma unroll
-                    for (int r = 0; r < NR; r++) {
-                        T part = (T)0;
-#pragma unroll
-                        for (int i = 0; i < C; i++)
-#pragma unroll
-                            for (int e = 0; e < V; e++) part = psp_fma(a[r][i][e], psp_elem<V, T>(bv[u][i], e), part);
-                        part = psp_group_sum<LOGL>(part);
-                        // positions past run_end belong to the next row: their dot product with this A row is dropped
-                        if (sub == k + u && k + u < run_end) {
-                            res[r] = part;
-                            if constexpr (sizeof(T) == 4) {
-                                if (!BCSR && want_max) lmax = fmaxf(lmax, SCALE ? part * gate[0] : part);
-                            }
-                        }
-                    }
+                    for (int i = 0; i < C; i++) bv[0][u][i] = bv[1][u][i];
             }
-            k = run_end;
-            if (base + k == row_end && base + k < b0) {
-                const int2 nx = w_seg[++cur];
-                row_end = nx.x;
-                if (nx.y != mykey) {
-                    if (want_max) emit_row_max(mykey);  // the group is converged here: the condition is group-uniform
-                    mykey = nx.y;
-#pragma unroll
-                    for (int r = 0; r < NR; r++)
-#pragma unroll
-                        for (int i = 0; i < C; i++)
-#pragma unroll
-                            for (int e = 0; e < V; e++) a[r][i][e] = a_nxt[r][i][e];
-                }
-                const int nk = cur + 1 < PSP_WAVE ? w_seg[cur + 1].y : -1;
-                if (nk >= 0 && nk != mykey) load_a(nk, a_nxt);
+        };
+        if constexpr (STEPS == 1) step(0, psp_int<0>());
+        else {
+#pragma unroll(LOGL >= 5 ? 1 : STEPS)  // (wide groups: 2 x 16 or 2 x 32 copies of the body would not fit the instruction cache)
+            for (int st = 0; st < STEPS; st += 2) {
+                step(st, psp_int<0>());
+                step(st + 1, psp_int<1>());
             }
         }
         if (ok) {
@@ -294,15 +327,41 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         for (int r = 0; r < NR; r++) gate[r] = gate_nxt[r];
     }
     if constexpr (HOLD > 1) release();
-    if (want_max) emit_row_max(mykey);
+    if constexpr (MAX) emit_row_max(cur);
     };  // run_window
 
+    // The window's row maxima leave together, one per lane (a row's segments are neighbours in the table: their first takes the
+    // maximum of all), because neighbouring rows' atomics then share a request: one atomic per row and lane group, sent
+    // as each row closed, took up to a third of the kernel (10^6 rows of 21 entries, K = 32: 309 us, like this 281, without maxima
+    // 247).  Stores for the rows that no other wavefront touches made it slower, not faster (atomics act behind the L2, and
+    // lines that see both kinds go back and forth).
+    auto flush_max = [&](const int tabW) {
+        if constexpr (MAX) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int key = s_seg[wave][lane].y;
+            float m = s_max[wave][lane];
+            bool first = true;
+            if constexpr (SPLIT) {
+                first = lane == 0 || s_seg[wave][lane > 0 ? lane - 1 : 0].y != key;
+                for (int d = 1; d < tabW; d <<= 1) {
+                    const int k_ = psp_bperm_i((lane + d) & (PSP_WAVE - 1), key);
+                    const float m_ = psp_bperm_f((lane + d) & (PSP_WAVE - 1), m);
+                    if (lane + d < PSP_WAVE && k_ == key) m = fmaxf(m, m_);
+                }
+            }
+            if (first && key >= 0 && m > PSP_F32_LOWEST) psp_atomic_max_f32(row_max + key, m);
+        }
+    };
     if constexpr (!BAL) {
         const int tile = psp_xcd_tile(stripe);
         if (tile >= tiles) return;
         const int s0 = (tile * (int)(blockDim.x >> 6) + wave) << logW;
         if (s0 >= nseg) return;  // wave-uniform
-        run_window(s0, min(1 << logW, nseg - s0), rowPtr[s0], 0x7fffffff, 1 << logW);
+        const int nvalid = min(1 << logW, nseg - s0);
+        run_window(s0, nvalid, rowPtr[s0], 0x7fffffff, 1 << logW);
+        flush_max(1 << logW);
     } else {
         // Tiles of 2^logW stored entries.  Each XCD (workgroups are dealt to them round-robin) owns one contiguous
         // eighth of the tiles and its wavefronts take them in turn, so at any time an XCD works on a run of
@@ -334,6 +393,7 @@ psp_sddmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
         while (pbeg < e1 && s0 < nseg) {  // wave-uniform
             const int nvalid = min(PSP_WAVE, nseg - s0);
             run_window(s0, nvalid, pbeg, e1, PSP_WAVE);
+            flush_max(PSP_WAVE);
             // the next window's table overwrites this one's: every group has finished reading it here
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -350,16 +410,16 @@ typedef void (*psp_sddmm_kernel_t)(const int *, const int *, const float *, cons
 // (LOGL, C, U) triples that exist.  C grows only once the group is 16 lanes wide (DPP-only reduction);
 // beyond 64 vectors the group widens to 32 and 64 lanes.
 #define PSP_SDDMM_FOR_EACH_LCU(M_) \
-    M_(0, 1, 1) M_(1, 1, 2) M_(2, 1, 4) M_(3, 1, 4) M_(4, 1, 4) \
-    M_(4, 2, 4) M_(4, 3, 2) M_(4, 4, 2) M_(5, 4, 2) M_(6, 4, 2)
+    M_(0, 1, 1) M_(1, 1, 1) M_(2, 1, 2) M_(3, 1, 2) M_(4, 1, 2) \
+    M_(4, 2, 2) M_(4, 3, 2) M_(4, 4, 1) M_(5, 4, 1) M_(6, 4, 2)
 
-template <int NR, bool SPLIT, bool SCALE, bool BAL = false>
+template <int NR, bool SPLIT, bool SCALE, bool BAL = false, bool MAX = false>
 static psp_sddmm_kernel_t psp_sddmm_lookup(int logL, int C, int V)
 {
 #define PSP_CASE(L_, C_, U_)                                                               \
     if (logL == L_ && C == C_) {                                                           \
-        if (V == 4) return psp_sddmm_kernel<L_, C_, 4, U_, NR, SPLIT, SCALE, BAL>;       \
-        return psp_sddmm_kernel<L_, C_, 1, U_, NR, SPLIT, SCALE, BAL>;                   \
+        if (V == 4) return psp_sddmm_kernel<L_, C_, 4, U_, NR, SPLIT, SCALE, BAL, MAX>;       \
+        return psp_sddmm_kernel<L_, C_, 1, U_, NR, SPLIT, SCALE, BAL, MAX>;                   \
     }
     PSP_SDDMM_FOR_EACH_LCU(PSP_CASE)
 #undef PSP_CASE

@@ -1,6 +1,20 @@
 // Host launcher shared by the four SDDMM translation units.
 #pragma once
 #include "sddmm_kernel.h"
+#include <map>
+#include <mutex>
+#include <utility>
+
+// Workgroups of `waves` wavefronts that fit a CU (asked once per kernel and size; races write the same value)
+static inline int psp_sddmm_per_cu(psp_sddmm_kernel_t k, int waves)
+{
+    static std::mutex lock;
+    static std::map<std::pair<psp_sddmm_kernel_t, int>, int> known;
+    std::lock_guard<std::mutex> hold(lock);
+    int &n = known[{k, waves}];
+    if (n == 0 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)k, waves * PSP_WAVE, 0) != hipSuccess || n < 1)) n = 1;
+    return n;
+}
 
 template <int NR, bool SPLIT>
 int psp_sddmm_launch(const int *rowPtr, const int *colIdx, const float *val, const int *target_row,
@@ -33,17 +47,22 @@ int psp_sddmm_launch(const int *rowPtr, const int *colIdx, const float *val, con
     if (logL > 6) return psp_fail(PSP_ERR_RANGE, "sddmm: K = %d is too wide (max %d)", K, 1024);
     if (logL < 4 && C > 1) C = 1;
 
-    psp_sddmm_kernel_t k = scale ? psp_sddmm_lookup<NR, SPLIT, !BCSR>(logL, C, V)
-                                 : psp_sddmm_lookup<NR, SPLIT, false>(logL, C, V);
-    if constexpr (!SPLIT) {
-        if (balanced)
-            k = scale ? psp_sddmm_lookup<NR, false, !BCSR, true>(logL, C, V) : psp_sddmm_lookup<NR, false, false, true>(logL, C, V);
-    }
+    auto pick = [&](auto bal_) {
+        constexpr bool BAL = !SPLIT && decltype(bal_)::value != 0;
+        if constexpr (!BCSR) {
+            if (row_max)
+                return scale ? psp_sddmm_lookup<NR, SPLIT, true, BAL, true>(logL, C, V) : psp_sddmm_lookup<NR, SPLIT, false, BAL, true>(logL, C, V);
+        }
+        return scale ? psp_sddmm_lookup<NR, SPLIT, !BCSR, BAL>(logL, C, V) : psp_sddmm_lookup<NR, SPLIT, false, BAL>(logL, C, V);
+    };
+    psp_sddmm_kernel_t k = balanced ? pick(psp_int<1>()) : pick(psp_int<0>());
     if (!k) return psp_fail(PSP_ERR_ARG, "sddmm: no kernel for logL %d coarsen %d vec %d", logL, C, V);
     if (balanced) {
-        // A fixed grid that fills the GPU once; its wavefronts divide the stored entries between them in tiles of 256
-        // (the entry count is on the device, in rowPtr): each XCD takes one contiguous eighth of the tiles.
-        const int wgs = 256 * 32 / blkWarpNum;
+        // A grid that fills the GPU once; its wavefronts divide the stored entries between them in tiles of 256
+        // (the entry count is on the device, in rowPtr): each XCD takes one contiguous eighth of the tiles.  "Once" is what the
+        // kernel's registers allow: workgroups that start when others have ended would work through their full share alone
+        // (10^6 rows of 21 entries, K = 32: 287 us with eight wavefronts per SIMD launched where six fit, 247 with six).
+        const int wgs = 256 * psp_sddmm_per_cu(k, blkWarpNum);
         dim3 grid(wgs, 1, 1), block(blkWarpNum * PSP_WAVE, 1, 1);
         hipLaunchKernelGGL(k, grid, block, 0, stream, rowPtr, colIdx, BCSR ? val : scale, target_row, A, B, out, nrows, K,
                            8, wgs, wgs / PSP_XCDS, row_max);
@@ -51,9 +70,10 @@ int psp_sddmm_launch(const int *rowPtr, const int *colIdx, const float *val, con
     }
 
     // segments per wavefront: as for SpMM (one per lane group for plain input, 16 for row-split input, fewer for
-    // small matrices)
+    // small matrices); groups of 32 and 64 lanes get two, so that the second row is on its way while the first is worked on
+    // (K = 300, five entries per row: 985 -> 685 us)
     const int logR = 6 - logL;
-    int logW = SPLIT ? (logR > 4 ? logR : 4) : logR;
+    int logW = SPLIT ? (logR > 4 ? logR : 4) : (logL >= 5 ? logR + 1 : logR);
     while (logW > 0 && (nrows >> logW) < 4096) logW--;
     if (logW < logR - 1) logW = logR - 1;
     const int segs_per_block = blkWarpNum << logW;
