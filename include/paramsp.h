@@ -43,8 +43,9 @@ const char *psp_last_error(void);
  *        option "dense_split";
  *   311: psp_spmm_register_sets (no buffer changed);
  *   312: psp_attn_forward_f32 / _backward_f32 (no buffer changed).
+ *   313: psp_spmm_window_grad_f32 (no buffer changed).
  * The extension modules and the ctypes loader of this package check it when they are imported. */
-#define PSP_ABI_VERSION 312
+#define PSP_ABI_VERSION 313
 int psp_version(void);
 
 /* How a (N, CF, blkWarpNum) request of the Python layer maps onto the wave64 kernels.
@@ -348,6 +349,17 @@ int psp_spmm_window_f32(const int *rowPtr_w, const int *colIdx_w, const float *v
 int psp_spmm_window_xw_f32(const int *rowPtr_w, const int *colIdx_w, const float *val_w, const float *X, const float *W,
                            int transW, float *Y, float *Y_raw, int M, int nnz, int N, int rows_out, int relu_x,
                            const float *mask, psp_stream_t stream);
+
+/* Backward of a layer on the windowed layout, weight gradient included: with G the gradient of the layer's output and Z its
+ * input, dW[KZ, N] = f(Z)^T (A G) (f = max(., 0) when relu_z) and, with W[KZ, N], KZ = N, dZ = ((A G) W^T) where Z > 0; without
+ * W, dZ (may be null) receives A G itself.  A G need not be stored for the product.  Z[M, KZ] row-major, 16-byte aligned;
+ * the widths there are: psp_spmm_window_grad_supported (N = 16: KZ 16, and 32 without W; N = 32: KZ = 32).  workspace:
+ * psp_spmm_window_grad_workspace_floats(...) floats, contents irrelevant on entry.  Repeats bit for bit. */
+int psp_spmm_window_grad_supported(int N, int KZ, int dense);
+long long psp_spmm_window_grad_workspace_floats(int M, int N, int KZ, int dense);
+int psp_spmm_window_grad_f32(const int *rowPtr_w, const int *colIdx_w, const float *val_w, const float *G, const float *Z, int KZ,
+                             int relu_z, const float *W, float *dZ, float *dW, float *workspace, long long workspace_floats,
+                             int M, int nnz, int N, int rows_out, psp_stream_t stream);
 
 /* SDDMM over the same layout: out[p] = alpha <A[row(p), :], B[col(p), :]> for every stored entry, in the layout's entry
  * order (out is parallel to colIdx_w).  The B rows of a block's window sit in LDS; only remote entries gather.

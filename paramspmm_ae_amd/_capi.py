@@ -101,6 +101,9 @@ SIGNATURES = {
     "psp_attn_forward_f32": [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "psp_attn_workspace_floats": [_i, _i],
     "psp_attn_backward_f32": [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
+    "psp_spmm_window_grad_supported": [_i, _i, _i],
+    "psp_spmm_window_grad_workspace_floats": [_i, _i, _i, _i],
+    "psp_spmm_window_grad_f32": [_vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, ctypes.c_longlong, _i, _i, _i, _i, _vp],
     "psp_spmm_window_xw_f32": [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp],
     "psp_gemm_xw_supported": [_i, _i],
     "psp_gemm_xw_f32": [_vp, _vp, _vp, ctypes.c_longlong, _i, _i, _i, _vp],
@@ -122,7 +125,7 @@ for _name, _args in SIGNATURES.items():
 lib.psp_last_error.argtypes = []
 lib.psp_last_error.restype = ctypes.c_char_p
 
-ABI_VERSION = 312  # PSP_ABI_VERSION of include/paramsp.h: the struct layouts and buffer sizes this module assumes
+ABI_VERSION = 313  # PSP_ABI_VERSION of include/paramsp.h: the struct layouts and buffer sizes this module assumes
 if lib.psp_version() < ABI_VERSION:
     raise ImportError("%s is version %d, this package needs %d: rebuild it (paramspmm_ae_amd/build_param.sh)"
                       % (LIB_PATH, lib.psp_version(), ABI_VERSION))

@@ -313,6 +313,12 @@ psp_atb_reduce_kernel(const float *__restrict__ partial, float *__restrict__ C, 
     }
 }
 
+int psp_sum_partials(const float *partial, float *C, int P, int E, hipStream_t stream)
+{
+    hipLaunchKernelGGL(psp_atb_reduce_kernel, dim3((unsigned)((E + 15) / 16)), dim3(1024), 0, stream, partial, C, P, E);
+    return psp_check_launch("partial sums");
+}
+
 typedef void (*psp_atb_mfma_kernel_t)(const float *, const float *, float *, long long, float *);
 
 // *jsplit receives the kernel's JSPLIT
@@ -401,9 +407,7 @@ PSP_EXPORT int psp_gemm_atb_ws_act_f32(const float *A, const float *B, float *C,
     hipLaunchKernelGGL(km, dim3((unsigned)wgs), dim3(256), 0, st, A, B, C, n, workspace);
     int rc = psp_check_launch("gemm_atb mfma kernel");
     if (rc != PSP_OK) return rc;
-    hipLaunchKernelGGL(psp_atb_reduce_kernel, dim3((unsigned)((K1 * K2 + 15) / 16)), dim3(1024), 0, st, workspace, C, (int)wgs,
-                       K1 * K2);
-    return psp_check_launch("gemm_atb reduce kernel");
+    return psp_sum_partials(workspace, C, (int)wgs, K1 * K2, st);
 }
 
 PSP_EXPORT int psp_gemm_atb_ws_f32(const float *A, const float *B, float *C, long long n, int K1, int K2,

@@ -35,9 +35,15 @@
 // W sits in LDS (transposed on the way in for W^T); a lane group gathers its row of A f(X) with DPP moves and each lane
 // forms its four output columns (N multiply-adds per column).  The row of A f(X) itself can be stored as well (Y_raw:
 // the backward pass needs A dY for the weight gradient and (A dY) W^T for the input gradient).  Measured and dropped:
-// the same product on the matrix cores (the block's 64 rows parked in LDS, one 16 x 16 tile per wavefront):
-// the extra barrier per block and the 4-byte stores of the tile layout cost more than the multiply-adds they replace
-// (GCN epoch, hidden 16 / 32: 1.71 / 2.60 ms against 1.61 / 2.49).
+// the same product on the matrix cores, with the block's 64 rows parked in LDS and a barrier (GCN epoch, hidden 16 / 32: 1.71 /
+// 2.60 ms against 1.61 / 2.49) or with a wavefront's own rows and none (92 us against 92 at 16 columns, 156 against 158 at 32).
+// KZ (backward of a layer whose input is Z [M, KZ], KZ = TN or 2 TN, one column tile): the weight gradient f(Z)^T (A X), a KZ x TN
+// matrix summed over all rows, is formed while the rows of A X are in registers.  A wavefront parks its rows and their Z in LDS,
+// reads both back in the operand layout of v_mfma_f32_16x16x4_f32 (four rows a step; no barrier, a wavefront reads only what
+// it wrote) and keeps the product in accumulators for the whole run; the workgroups' products meet in `part` and are added in a
+// fixed order.  Z is the mask of EPI at the same time, and (A X) W^T comes off the same staged rows.  The separate kernel for
+// the gradient read A X and Z again and had A X written for it: 10^6 rows of 20 entries, square layer of 16 columns 122 + 27 us ->
+// 112 + 7; 32-column Z and no (A X) W^T 96 + 40 -> 113 + 7.
 // relu_x applies max(x, 0) to X as it enters (once per window element rather than once per gather); mask keeps an
 // output element only where mask > 0, read where the row is stored -- the two halves of a ReLU folded into the
 // product, as psp_spmm_act_f32 offers for the other formats.
@@ -45,15 +51,20 @@
 
 #include "window_common.h"
 
-template <int C, int LOGL, int PSPW_THREADS, bool EPI = false>
-__global__ void __launch_bounds__(PSPW_THREADS)
+// KZ: row strides of a wavefront's Z and A X rows in LDS: the four rows of a step lie on different banks (A X is also read with
+// four columns of all rows, for which 36 has no conflicts; at 16 columns a stride of 20 would, but spilled a register: same time).
+constexpr int pspw_z_stride(int kz) { return kz == 32 ? 48 : 16; }
+constexpr int pspw_g_stride(int tn) { return tn == 32 ? 36 : 16; }
+
+template <int C, int LOGL, int PSPW_THREADS, bool EPI = false, int KZ = 0>
+// (four wavefronts per SIMD: what the registers of the variants without a weight gradient allow)
+__global__ void __launch_bounds__(PSPW_THREADS, KZ > 0 ? 4 : 1)
 psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__ colIdx, const float *__restrict__ val,
                        const float *__restrict__ X, float *__restrict__ Y, const float *__restrict__ mask, int M, int N,
                        int nnz, int nruns, int stripe, int run, int relu_x, const float *__restrict__ W, int transW,
-                       float *__restrict__ Y_raw)
+                       float *__restrict__ Y_raw, const float *__restrict__ Z, int relu_z, float *__restrict__ part)
 {
     constexpr int L = 1 << LOGL;
-    static_assert(!EPI || C == 1, "the dense epilogue exists for one vector per lane (one column tile of 16 or 32)");
     constexpr int TN = L * C * 4;                  // columns per tile
     constexpr int RB = PSPW_BLOCK;                 // rows per step
     constexpr int RPG = RB * L / PSPW_THREADS;     // rows per lane group
@@ -65,6 +76,10 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
     constexpr int FPT = RB * V4 / PSPW_THREADS;    // pieces per lane when 64 rows enter
     static_assert(RPG >= 1 && RB * V4 % PSPW_THREADS == 0, "shape");
     static_assert(UR <= L, "one lane per prefetched remote entry");
+    constexpr int ZV = KZ > 0 ? KZ / TN : 1;                          // 16-byte pieces of a Z row per lane
+    constexpr int WROWS = PSP_WAVE / L;                                  // rows of a block per wavefront
+    constexpr int ZS = pspw_z_stride(KZ), GS = pspw_g_stride(TN);
+    static_assert(!(EPI || KZ > 0) || (C == 1 && RPG == 1 && KZ % TN == 0), "epilogues: one column tile, one row per lane group");
     // [RING + 1][TN]: the ring and one row of zeros, which the padding of a row's entry registers points at (value 0
     // times a zero, so the summing loop needs no predicate and a padding slot can never bring an Inf or NaN in)
     extern __shared__ __align__(16) float s_x[];
@@ -87,6 +102,13 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
             s_w[idx] = transW ? W[j_ * TN + k_] : W[idx];
         }
     }
+
+    float *s_z = s_w + (EPI ? TN * TN : 0) + (tid >> 6) * (WROWS * (ZS + GS)), *s_g = s_z + WROWS * ZS;  // this wavefront's rows
+    psp_f32x4 dw[KZ > 0 ? KZ / 16 : 1][TN / 16];
+#pragma unroll
+    for (int i = 0; i < (KZ > 0 ? KZ / 16 : 1); i++)
+#pragma unroll
+        for (int h = 0; h < TN / 16; h++) dw[i][h] = (psp_f32x4){0.f, 0.f, 0.f, 0.f};
 
     bool live[C];
     int off[C];
@@ -203,6 +225,12 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
     for (int j = j0; j < j1; j++) {
         // loads for the blocks that follow (past the end of the run they read clamped addresses and are not used)
         int a2[RPG], m2[RPG], b2[RPG];
+        psp_f32x4 z[ZV];
+        if constexpr (KZ > 0) {
+#pragma unroll
+            for (int i = 0; i < ZV; i++)
+                z[i] = *(const psp_f32x4 *)(Z + (size_t)min(j * RB + grp, M - 1) * (size_t)KZ + (i * L + sub) * 4);
+        }
         load_pairs(an, mn, cln, vln, crn, vrn);
         load_bounds(j + 2, a2, m2, b2);
         fill_load((j + 1) * RB + PSPW_HALO, w);  // the rows that enter with block j + 1
@@ -324,7 +352,64 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
                 }
             }
             const int r = j * RB + grp * RPG + k;
-            if constexpr (EPI) {
+            if constexpr (KZ > 0) {
+                const int row = (tid & (PSP_WAVE - 1)) >> LOGL;
+                const int mr = tid & 15, mq = (tid & (PSP_WAVE - 1)) >> 4;
+#pragma unroll
+                for (int i = 0; i < ZV; i++) {
+                    psp_f32x4 f = z[i];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) f[e] = r >= M || (relu_z && f[e] < 0.0f) ? 0.0f : f[e];
+                    *(psp_f32x4 *)(s_z + row * ZS + (i * L + sub) * 4) = f;
+                }
+                *(psp_f32x4 *)(s_g + row * GS + sub * 4) = acc[k][0];  // (rows past the matrix are empty: zero)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                for (int st = 0; st < WROWS / 4; st++) {
+                    float fa[KZ / 16], fb[TN / 16];
+#pragma unroll
+                    for (int i = 0; i < KZ / 16; i++) fa[i] = s_z[(4 * st + mq) * ZS + 16 * i + mr];
+#pragma unroll
+                    for (int h = 0; h < TN / 16; h++) fb[h] = s_g[(4 * st + mq) * GS + 16 * h + mr];
+#pragma unroll
+                    for (int i = 0; i < KZ / 16; i++)
+#pragma unroll
+                        for (int h = 0; h < TN / 16; h++) dw[i][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i], fb[h], dw[i][h], 0, 0, 0);
+                }
+                if constexpr (EPI) {
+                    // the product with the staged matrix, transposed so that a lane ends up with four columns of one row (the
+                    // upper half of the tile repeats the rows of a wavefront that has eight); k ascending in every sum
+                    asm volatile("" ::: "memory");  // W is read again in every block: kept in registers it would cost a wavefront per SIMD
+                    const int orow = mr & (WROWS - 1), oat = j * RB + (tid >> 6) * WROWS + orow;
+                    psp_f32x4 o[TN / 16];
+#pragma unroll
+                    for (int h = 0; h < TN / 16; h++) o[h] = (psp_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int st = 0; st < TN / 4; st++) {
+                        const float gk = s_g[orow * GS + 4 * st + mq];
+#pragma unroll
+                        for (int h = 0; h < TN / 16; h++)
+                            o[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_w[(4 * st + mq) * TN + 16 * h + mr], gk, o[h], 0, 0, 0);
+                    }
+                    if (oat < M && mr < WROWS) {
+#pragma unroll
+                        for (int h = 0; h < TN / 16; h++) {
+                            const size_t at = (size_t)oat * (size_t)N + 16 * h + 4 * mq;
+                            const psp_f32x4 mk = *(const psp_f32x4 *)(s_z + orow * ZS + 16 * h + 4 * mq);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) o[h][e] = mk[e] > 0.0f ? o[h][e] : 0.0f;
+                            __builtin_nontemporal_store(o[h], (psp_f32x4 *)(Y + at));
+                        }
+                    }
+                }
+                // the next block's rows overwrite these: in program order, after the reads
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
+            if constexpr (EPI && KZ == 0) {
                 // the row of A f(X) is complete: store it if asked, then multiply it by the staged matrix (every lane
                 // of the wavefront takes part in the DPP moves; N == TN here, so every lane has columns)
                 const psp_f32x4 raw = acc[k][0];
@@ -343,13 +428,13 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
                 }
                 acc[k][0] = o;
             }
-            if (r < M) {
+            if (r < M && (KZ == 0 || (!EPI && Y != nullptr))) {
 #pragma unroll
                 for (int i = 0; i < C; i++) {
                     if (!live[i]) continue;
                     const size_t at = (size_t)r * (size_t)N + tile_col0 + off[i];
                     psp_f32x4 y = acc[k][i];
-                    if (mask) {
+                    if (KZ == 0 && mask) {
                         const psp_f32x4 mk = *(const psp_f32x4 *)(mask + at);
 #pragma unroll
                         for (int e = 0; e < 4; e++) y[e] = mk[e] > 0.0f ? y[e] : 0.0f;
@@ -372,6 +457,24 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
         }
         to_ring(a, m, cl, vl);
         __syncthreads();
+    }
+    if constexpr (KZ > 0) {
+        // the ring is free: the wavefronts' products meet there
+        const int lane = tid & (PSP_WAVE - 1);
+        float *mine = s_x + (tid >> 6) * (KZ * TN);
+#pragma unroll
+        for (int i = 0; i < KZ / 16; i++)
+#pragma unroll
+            for (int h = 0; h < TN / 16; h++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) mine[(16 * i + 4 * (lane >> 4) + e) * TN + 16 * h + (lane & 15)] = dw[i][h][e];
+        __syncthreads();
+        for (int idx = tid; idx < KZ * TN; idx += PSPW_THREADS) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int v = 0; v < PSPW_THREADS / PSP_WAVE; v++) sum += s_x[v * (KZ * TN) + idx];
+            part[(size_t)run_id * (KZ * TN) + idx] = sum;
+        }
     }
 }
 
@@ -455,16 +558,23 @@ PSP_EXPORT int psp_window_build_dev(const int *rowPtr, const int *colIdx, const 
 
 // ---- launch -----------------------------------------------------------------------------------------------------------
 typedef void (*pspw_kernel_t)(const int *, const int *, const float *, const float *, float *, const float *, int, int,
-                              int, int, int, int, int, const float *, int, float *);
+                              int, int, int, int, int, const float *, int, float *, const float *, int, float *);
 
 struct pspw_variant {
     pspw_kernel_t fn;
     int tn, threads;
 };
 
-// one row of a block per lane group: 64 groups of 4 lanes, or 64 groups of 8 lanes in a workgroup of 512
-static pspw_variant pspw_lookup(int variant, bool epilogue = false)
+// one row of a block per lane group: 64 groups of 4 lanes, or 64 groups of 8 lanes in a workgroup of 512.  kz: width of the
+// matrix whose weight gradient is formed with the product, 0 = none
+static pspw_variant pspw_lookup(int variant, bool epilogue = false, int kz = 0)
 {
+    if (kz != 0) {
+        if (variant == 1 && kz == 16) return {epilogue ? psp_spmm_window_kernel<1, 2, 256, true, 16> : psp_spmm_window_kernel<1, 2, 256, false, 16>, 16, 256};
+        if (variant == 1 && kz == 32 && !epilogue) return {psp_spmm_window_kernel<1, 2, 256, false, 32>, 16, 256};
+        if (variant == 2 && kz == 32) return {epilogue ? psp_spmm_window_kernel<1, 3, 512, true, 32> : psp_spmm_window_kernel<1, 3, 512, false, 32>, 32, 512};
+        return {nullptr, 0, 0};
+    }
     if (epilogue) {
         switch (variant) {
         case 1: return {psp_spmm_window_kernel<1, 2, 256, true>, 16, 256};
@@ -492,44 +602,89 @@ PSP_EXPORT int psp_spmm_window_plan(int N, int variant, int *tile_cols, int *row
     return variant;
 }
 
-static int pspw_launch(const int *rowPtr_w, const int *colIdx_w, const float *val_w, const float *X, float *Y, int M, int nnz,
-                       int N, int rows_out, int variant, int relu_x, const float *mask, const float *W, int transW,
-                       float *Y_raw, hipStream_t st)
+// Z with its width (0: no weight gradient), the gradient, and the workspace that the workgroups' shares of it meet in
+struct pspw_grad {
+    const float *Z;
+    int kz, relu_z;
+    float *dW, *ws;
+    long long ws_floats;
+};
+
+// LDS bytes, blocks per workgroup and number of workgroups of a launch
+static int pspw_shape(int M, int N, int v, int tn, int lds, bool epi, int kz, const pspw_variant &k, int *lds_out, int *run, int *nruns)
 {
-    const bool epi = W != nullptr;
-    int tn = 0, rb = 0, lds = 0;
-    const int v = psp_spmm_window_plan(N, variant, &tn, &rb, &lds);
-    if (v < 0) return v;
-    PSP_REQUIRE(M >= 0 && nnz >= 0 && rows_out >= M, "spmm_window: Y has %d rows, the matrix %d (%d entries)", rows_out, M, nnz);
-    PSP_REQUIRE((((size_t)X | (size_t)Y | (size_t)mask | (size_t)Y_raw) & 15) == 0, "spmm_window: X, Y and mask must be 16-byte aligned");
-    if (epi) {
-        PSP_REQUIRE(N == tn && (N == 16 || N == 32), "spmm_window: the dense epilogue exists for N = 16 and 32 (got %d)", N);
-        lds += tn * tn * 4;
-    }
-    if (nnz == 0) {  // (the kernel clamps its loads to entry nnz - 1)
-        const int rc = psp_zero_f32(Y, (size_t)rows_out * N, st);
-        return rc != PSP_OK || !Y_raw ? rc : psp_zero_f32(Y_raw, (size_t)rows_out * N, st);
-    }
-    int rc = psp_zero_f32(Y + (size_t)M * N, ((size_t)rows_out - (size_t)M) * N, st);  // rows past the matrix
-    if (rc == PSP_OK && Y_raw) rc = psp_zero_f32(Y_raw + (size_t)M * N, ((size_t)rows_out - (size_t)M) * N, st);
-    if (rc != PSP_OK || M == 0) return rc;
-    PSP_REQUIRE(rowPtr_w && colIdx_w && val_w && X && Y, "spmm_window: null pointer");
-    const pspw_variant k = pspw_lookup(v, epi);
-    const int key = v + (epi ? 4 : 0);
-    static bool lds_raised[8];
+    if (epi) lds += tn * tn * 4;
+    if (kz) lds += k.threads / PSP_WAVE * (k.threads == 256 ? 16 : 8) * (pspw_z_stride(kz) + pspw_g_stride(tn)) * 4;
+    const int key = v + (epi ? 4 : 0) + (kz == 0 ? 0 : (kz == tn ? 8 : 16));
+    static bool lds_raised[24];
     if (lds > 48 * 1024 && !lds_raised[key]) {
         const hipError_t e = hipFuncSetAttribute((const void *)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return psp_fail(PSP_ERR_LAUNCH, "spmm_window: %d bytes of LDS refused: %s", lds, hipGetErrorString(e));
         lds_raised[key] = true;
     }
-    const int nblocks = psp_ceil_div(M, rb), tiles = psp_ceil_div(N, tn);
-    const int run = pspw_run_length(nblocks, tiles, key, (const void *)k.fn, k.threads, lds);
-    const int nruns = psp_ceil_div(nblocks, run);
+    const int nblocks = psp_ceil_div(M, PSPW_BLOCK);
+    *lds_out = lds;
+    *run = pspw_run_length(nblocks, psp_ceil_div(N, tn), key, (const void *)k.fn, k.threads, lds);
+    *nruns = psp_ceil_div(nblocks, *run);
+    return PSP_OK;
+}
+
+static int pspw_launch(const int *rowPtr_w, const int *colIdx_w, const float *val_w, const float *X, float *Y, int M, int nnz,
+                       int N, int rows_out, int variant, int relu_x, const float *mask, const float *W, int transW,
+                       float *Y_raw, hipStream_t st, pspw_grad gr = pspw_grad())
+{
+    const bool epi = W != nullptr;
+    int tn = 0, lds = 0;
+    const int v = psp_spmm_window_plan(N, variant, &tn, nullptr, &lds);
+    if (v < 0) return v;
+    PSP_REQUIRE(M >= 0 && nnz >= 0 && rows_out >= M, "spmm_window: Y has %d rows, the matrix %d (%d entries)", rows_out, M, nnz);
+    PSP_REQUIRE((((size_t)X | (size_t)Y | (size_t)mask | (size_t)Y_raw | (size_t)gr.Z) & 15) == 0, "spmm_window: X, Y and mask must be 16-byte aligned");
+    if (epi) PSP_REQUIRE(N == tn && (N == 16 || N == 32), "spmm_window: the dense epilogue exists for N = 16 and 32 (got %d)", N);
+    int rc = PSP_OK;
+    if (nnz == 0) {  // (the kernel clamps its loads to entry nnz - 1)
+        if (Y) rc = psp_zero_f32(Y, (size_t)rows_out * N, st);
+        if (rc == PSP_OK && Y_raw) rc = psp_zero_f32(Y_raw, (size_t)rows_out * N, st);
+        return rc != PSP_OK || !gr.kz ? rc : psp_zero_f32(gr.dW, (size_t)gr.kz * N, st);
+    }
+    if (Y) rc = psp_zero_f32(Y + (size_t)M * N, ((size_t)rows_out - (size_t)M) * N, st);  // rows past the matrix
+    if (rc == PSP_OK && Y_raw) rc = psp_zero_f32(Y_raw + (size_t)M * N, ((size_t)rows_out - (size_t)M) * N, st);
+    if (rc != PSP_OK || M == 0) return rc;
+    PSP_REQUIRE(rowPtr_w && colIdx_w && val_w && X && (Y || gr.kz), "spmm_window: null pointer");
+    const pspw_variant k = pspw_lookup(v, epi, gr.kz);
+    PSP_REQUIRE(k.fn, "spmm_window: no weight gradient of %d x %d", gr.kz, N);
+    int run = 0, nruns = 0;
+    rc = pspw_shape(M, N, v, tn, lds, epi, gr.kz, k, &lds, &run, &nruns);
+    if (rc != PSP_OK) return rc;
+    PSP_REQUIRE(gr.kz == 0 || (gr.Z && gr.dW && gr.ws && gr.ws_floats >= (long long)nruns * gr.kz * N),
+                "spmm_window: the weight gradient needs Z, dW and %lld floats of workspace", (long long)nruns * gr.kz * N);
     const psp_grid1d g = psp_xcd_grid(nruns, 1);  // long runs: neighbouring runs share two halo windows, nothing to keep in one L2
-    dim3 grid(g.launch, tiles, 1), block(k.threads, 1, 1);
+    dim3 grid(g.launch, psp_ceil_div(N, tn), 1), block(k.threads, 1, 1);
     hipLaunchKernelGGL(k.fn, grid, block, lds, st, rowPtr_w, colIdx_w, val_w, X, Y, mask, M, N, nnz, nruns, g.stripe, run,
-                       relu_x != 0, W, transW != 0, Y_raw);
-    return psp_check_launch("spmm window kernel");
+                       relu_x != 0, W, transW != 0, Y_raw, gr.Z, gr.relu_z, gr.ws);
+    rc = psp_check_launch("spmm window kernel");
+    return rc != PSP_OK || !gr.kz ? rc : psp_sum_partials(gr.ws, gr.dW, nruns, gr.kz * N, st);
+}
+
+PSP_EXPORT int psp_spmm_window_grad_supported(int N, int KZ, int dense) { return (N == 16 || N == 32) && pspw_lookup(N / 16, dense != 0, KZ).fn != nullptr; }
+
+PSP_EXPORT long long psp_spmm_window_grad_workspace_floats(int M, int N, int KZ, int dense)
+{
+    PSP_REQUIRE(M >= 0 && psp_spmm_window_grad_supported(N, KZ, dense), "spmm_window_grad: no weight gradient of %d x %d", KZ, N);
+    int tn = 0, lds = 0, run = 0, nruns = 0;
+    const int v = psp_spmm_window_plan(N, 0, &tn, nullptr, &lds);
+    if (v < 0) return v;
+    const int rc = pspw_shape(M, N, v, tn, lds, dense != 0, KZ, pspw_lookup(v, dense != 0, KZ), &lds, &run, &nruns);
+    return rc != PSP_OK ? rc : (long long)nruns * KZ * N;
+}
+
+PSP_EXPORT int psp_spmm_window_grad_f32(const int *rowPtr_w, const int *colIdx_w, const float *val_w, const float *G, const float *Z,
+                                        int KZ, int relu_z, const float *W, float *dZ, float *dW, float *workspace,
+                                        long long workspace_floats, int M, int nnz, int N, int rows_out, psp_stream_t stream)
+{
+    PSP_REQUIRE(psp_spmm_window_grad_supported(N, KZ, W != nullptr), "spmm_window_grad: no weight gradient of %d x %d", KZ, N);
+    PSP_REQUIRE(dW && (!W || dZ), "spmm_window_grad: null pointer");
+    return pspw_launch(rowPtr_w, colIdx_w, val_w, G, dZ, M, nnz, N, rows_out, 0, 0, nullptr, W, 1, nullptr, (hipStream_t)stream,
+                       pspw_grad{Z, KZ, relu_z != 0, dW, workspace, workspace_floats});
 }
 
 PSP_EXPORT int psp_spmm_window_f32(const int *rowPtr_w, const int *colIdx_w, const float *val_w, const float *X, float *Y,

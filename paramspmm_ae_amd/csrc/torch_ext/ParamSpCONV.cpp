@@ -239,6 +239,36 @@ static std::vector<Tensor> window_xw(Tensor X, Tensor W, bool transW, Tensor row
     return {Y};
 }
 
+// Backward on the windowed layout with the weight gradient formed in the sparse kernel (psp_spmm_window_grad_f32): dW = f(Z)^T (A G)
+// and, with W, dZ = ((A G) W^T) where Z > 0, else A G when want_ag.  Returns {dW, dZ or A G or nothing}.
+static bool window_grad_supported(const Tensor &G, const Tensor &Z, bool dense)
+{
+    return G.dim() == 2 && Z.dim() == 2 && G.size(0) == Z.size(0) && G.scalar_type() == torch::kFloat32 && Z.scalar_type() == torch::kFloat32 &&
+           psp_spmm_window_grad_supported((int)G.size(1), (int)Z.size(1), dense ? 1 : 0);
+}
+static std::vector<Tensor> window_grad(Tensor G, Tensor Z, bool relu_z, const Tensor *W, bool want_ag, Tensor rowPtr_w, Tensor colIdx_w,
+                                       Tensor values_w)
+{
+    Tensor Gc = G.contiguous(), Zc = Z.contiguous(), Wc;
+    check_spmm_args(4, Gc, rowPtr_w, colIdx_w, values_w, nullptr);
+    pspglue::same_device(Gc, Zc, "window_grad");
+    if (W) {
+        Wc = W->contiguous();
+        need_f32(Wc, "weight", 2);
+        pspglue::same_device(Gc, Wc, "window_grad");
+    }
+    DeviceGuard guard(Gc.device());
+    const int M = pspglue::fmt_rows(4, rowPtr_w), N = (int)Gc.size(1), KZ = (int)Zc.size(1);
+    TORCH_CHECK(Gc.size(0) >= M && Zc.size(0) >= M && (!W || (Wc.size(0) == KZ && Wc.size(1) == N)), "window_grad: shapes");
+    const long long ws_floats = psp_spmm_window_grad_workspace_floats(M, N, KZ, W ? 1 : 0);
+    Tensor dW = torch::empty({KZ, N}, Gc.options()), ws = torch::empty({(long)ws_floats}, Gc.options()), Y;
+    if (W || want_ag) Y = torch::empty_like(Gc);
+    ok(psp_spmm_window_grad_f32(ip(rowPtr_w), ip(colIdx_w), fp(values_w), fp(Gc), fp(Zc), KZ, relu_z ? 1 : 0, W ? fp(Wc) : nullptr,
+                                Y.defined() ? fpw(Y) : nullptr, fpw(dW), fpw(ws), ws_floats, M, (int)colIdx_w.size(0), N,
+                                (int)Gc.size(0), stream_of(Gc)));
+    return {dW, Y};
+}
+
 // ---- attention layer on the windowed layout: SDDMM and SpMM of a direction in one launch ---------------------------------
 static bool attn_window_supported(long K) { return K >= 4 && K % 4 == 0 && K <= PSP_ATTN_WINDOW_MAX_K; }
 
@@ -498,6 +528,10 @@ struct GCNFunction : LayerNode {
     {
         if (!g[0].defined()) return {Tensor(), Tensor()};
         Tensor H = a(), W = w();
+        if (op->fmt == 4 && wants(1) && window_grad_supported(g[0], H, false)) {
+            auto r = window_grad(g[0], H, false, nullptr, wants(0), op->rowPtr, op->colIdx, op->val);
+            return {wants(0) ? dense_xw(r[1], W, true, Order::any) : Tensor(), r[0]};
+        }
         Tensor AG = aggregate(op->fmt, g[0], op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
         return {wants(0) ? dense_xw(AG, W, true, Order::any) : Tensor(), wants(1) ? weight_gradient(H, AG) : Tensor()};
     }
@@ -543,9 +577,13 @@ struct GCNReLUInputFunction : LayerNode {
         if (!g[0].defined()) return {Tensor(), Tensor()};
         Tensor Z = a(), W = w(), dY = g[0].contiguous();
         if (folds_dense(*op, Z, W)) {
-            // one launch delivers A dY (for the weight gradient) and ((A dY) W^T) where Z > 0 (the input gradient)
-            auto r = window_xw(dY, W, true, op->rowPtr, op->colIdx, op->val, false, Z, true);
-            return {r[0], weight_gradient_relu(Z, r[1])};
+            // one launch delivers ((A dY) W^T) where Z > 0 (the input gradient) and the weight gradient
+            auto r = window_grad(dY, Z, true, &W, false, op->rowPtr, op->colIdx, op->val);
+            return {r[1], r[0]};
+        }
+        if (op->fmt == 4 && window_grad_supported(dY, Z, false)) {
+            auto r = window_grad(dY, Z, true, nullptr, true, op->rowPtr, op->colIdx, op->val);
+            return {dense_xwt_masked(r[1], W, Z), r[0]};
         }
         auto r = relu_input_backward(op->fmt, dY, Z, W, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw);
         return {r[0], r[1]};

@@ -97,7 +97,7 @@ static int pspw_run_length(int nblocks, int tiles, int slot_key, const void *ker
         return e ? atoi(e) : 0;
     }();
     if (forced > 0) return forced;
-    static int slots_of[16];  // workgroups the current GPU holds at once, per kernel of the including file (0 = not asked yet)
+    static int slots_of[24];  // workgroups the current GPU holds at once, per kernel of the including file (0 = not asked yet)
     if (slots_of[slot_key] == 0) {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
