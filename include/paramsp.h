@@ -44,8 +44,9 @@ const char *psp_last_error(void);
  *   311: psp_spmm_register_sets (no buffer changed);
  *   312: psp_attn_forward_f32 / _backward_f32 (no buffer changed).
  *   313: psp_spmm_window_grad_f32 (no buffer changed).
+ *   314: psp_sum_partials_f32, psp_dense_grad_f32 (no buffer changed).
  * The extension modules and the ctypes loader of this package check it when they are imported. */
-#define PSP_ABI_VERSION 313
+#define PSP_ABI_VERSION 314
 int psp_version(void);
 
 /* How a (N, CF, blkWarpNum) request of the Python layer maps onto the wave64 kernels.
@@ -354,7 +355,8 @@ int psp_spmm_window_xw_f32(const int *rowPtr_w, const int *colIdx_w, const float
  * input, dW[KZ, N] = f(Z)^T (A G) (f = max(., 0) when relu_z) and, with W[KZ, N], KZ = N, dZ = ((A G) W^T) where Z > 0; without
  * W, dZ (may be null) receives A G itself.  A G need not be stored for the product.  Z[M, KZ] row-major, 16-byte aligned;
  * the widths there are: psp_spmm_window_grad_supported (N = 16: KZ 16, and 32 without W; N = 32: KZ = 32).  workspace:
- * psp_spmm_window_grad_workspace_floats(...) floats, contents irrelevant on entry.  Repeats bit for bit. */
+ * psp_spmm_window_grad_workspace_floats(...) floats, contents irrelevant on entry; with dW null the
+ * partial sums stay there and the call returns how many (see psp_sum_partials_f32).  Repeats bit for bit. */
 int psp_spmm_window_grad_supported(int N, int KZ, int dense);
 long long psp_spmm_window_grad_workspace_floats(int M, int N, int KZ, int dense);
 int psp_spmm_window_grad_f32(const int *rowPtr_w, const int *colIdx_w, const float *val_w, const float *G, const float *Z, int KZ,
@@ -452,6 +454,24 @@ int psp_gemm_atb_ws_f32(const float *A, const float *B, float *C, long long n, i
  * output through a ReLU (GNN.py:43-61 applies F.relu between the layers) without that activation being stored. */
 int psp_gemm_atb_ws_act_f32(const float *A, const float *B, float *C, long long n, int K1, int K2, int relu_a,
                             float *workspace, long long workspace_floats, psp_stream_t stream);
+/* C null: the workgroups' partial products stay in the workspace, K1 * K2 floats each; the call returns how many (n > 0,
+ * supported widths).  psp_sum_partials_f32 adds them -- those of several products in one launch -- in the same fixed order. */
+#define PSP_SUM_JOBS_MAX 8
+typedef struct psp_partial_sum {
+    const float *partial; /* [count, elements] */
+    float *C;             /* [elements] */
+    int count, elements;
+} psp_partial_sum;
+int psp_sum_partials_f32(const psp_partial_sum *sums, int n, psp_stream_t stream);
+
+/* ---------------------------------------------------------------------------------------------
+ * DEVICE: both gradients of a layer relu(Z) W in one launch, from the gradient G[n,K2] of its product: dZ[n,K1] = (G W^T)
+ * where Z > 0, dW[K1,K2] = max(Z, 0)^T G, W[K1,K2] row-major; n > 0, G, Z and dZ 16-byte aligned, widths:
+ * psp_dense_grad_supported (multiples of 16 up to 64).  Workspace and dW null as in psp_gemm_atb_ws_act_f32. */
+int psp_dense_grad_supported(int K1, int K2);
+long long psp_dense_grad_workspace_floats(long long n, int K1, int K2);
+int psp_dense_grad_f32(const float *G, const float *Z, const float *W, float *dZ, float *dW, long long n, int K1, int K2,
+                       float *workspace, long long workspace_floats, psp_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------
  * DEVICE: Y[n,K2] = X[n,K1] * W (transW = 0, W is [K1,K2] row-major) or X * W^T (transW != 0, W is [K2,K1]) for

@@ -17,7 +17,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .decider import SpMMDecider, DEFAULT_PICKLE_PATH
-from .gnn_conv import AGNNConv, GCNConv, GINConv, nll_loss_mean, softmax_nll_loss_mean
+from .gnn_conv import AGNNConv, GCNConv, GINConv, network_loss, nll_loss_mean, softmax_nll_loss_mean
 from .graph_input import graph_input
 from .PCSR import pcsr_spmm
 
@@ -124,8 +124,13 @@ _FUSED_ADAM = os.environ.get("PSP_FUSED_ADAM", "1") != "0"
 def loss_of_step(model, labels):
     """F.nll_loss(model(), labels) of the reference's training step (GNN.py:131-146).  The networks end in a
     log-softmax; with ``model.fuse_loss`` (the default) it is folded into the loss -- one pass over the logits instead
-    of a softmax, a loss and their two backward passes."""
+    of a softmax, a loss and their two backward passes -- and plain GCN and GIN networks run as one autograd node with it
+    (gnn_conv.network_loss)."""
     if getattr(model, "fuse_loss", True) and hasattr(model, "logits"):
+        if type(model) in (Net_5layers, GIN) and model.fuse_relu and "logits" not in model.__dict__:
+            loss = network_loss((model.conv1, model.conv2, model.conv3, model.conv4, model.conv5), model.spmm_dict, model.x, labels)
+            if loss is not None:
+                return loss
         return softmax_nll_loss_mean(model.logits(), labels)
     return nll_loss_mean(model(), labels)
 

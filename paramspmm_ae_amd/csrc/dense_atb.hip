@@ -3,10 +3,11 @@
 // reduction over n with a tiny output; a general GEMM picks tiles for large outputs and runs it 20-40 times
 // slower than the memory traffic allows.  HBM-bound up to about 64 x 64: 4 n (K1 + K2) bytes.
 // The matrix cores (v_mfma_f32_16x16x4_f32) are fed straight from coalesced loads; partial products either meet in a
-// caller's workspace and are added by psp_atb_reduce_kernel in a fixed order, or go to C with atomics.
+// caller's workspace and are added by psp_sum_partials_kernel in a fixed order, or go to C with atomics.
 #include "psp_common.h"
 #include "spmm_kernel.h"
 #include "bf16_split.h"
+#include "dense_tiles.h"
 
 // RELU_A: A enters the product as max(a, 0) -- the weight gradient of a layer whose input is the activation of the
 // previous layer's output, without that activation ever being stored.
@@ -23,38 +24,6 @@
 //              317 -> 240, 112 x 112 403 -> 290; 64 x 128 194 (JSPLIT = 4) -> 183, 128 x 64 227 -> 185.
 //   JSPLIT = 4 (56 tiles and more, K2 = 128): the four wavefronts of a workgroup share their chunks and own a quarter of
 //              B's columns each; A is loaded by all four (the repeats are L1 / L2 hits).
-typedef float psp_mfma_acc __attribute__((ext_vector_type(4)));
-
-template <int V> __device__ __forceinline__ void psp_atb_load(const float *p, float *out)
-{
-    if (V == 4) {
-        const psp_f32x4 x = *(const psp_f32x4 *)p;
-        out[0] = x[0], out[1] = x[1], out[2] = x[2], out[3] = x[3];
-    } else if (V == 3) {
-        typedef float f32x3 __attribute__((ext_vector_type(3), aligned(4)));
-        const f32x3 x = *(const f32x3 *)p;
-        out[0] = x[0], out[1] = x[1], out[2] = x[2];
-    } else if (V == 2) {
-        const psp_f32x2 x = *(const psp_f32x2 *)p;
-        out[0] = x[0], out[1] = x[1];
-    } else {
-        out[0] = *p;
-    }
-}
-// R tiles are loaded in pieces of four (16 bytes per lane) and a last one of R % 4: column that index i of tile m stands for
-template <int R> __device__ __forceinline__ int psp_atb_col(int m, int i)
-{
-    constexpr int N4 = R / 4 * 4, REM = R % 4;
-    return m < N4 ? (m / 4) * 64 + 4 * i + m % 4 : N4 * 16 + REM * i + (m - N4);
-}
-template <int R> __device__ __forceinline__ void psp_atb_load_row(const float *row, int c, float (&out)[R])
-{
-    constexpr int N4 = R / 4 * 4, REM = R % 4;
-#pragma unroll
-    for (int m = 0; m < N4; m += 4) psp_atb_load<4>(row + m * 16 + 4 * c, out + m);
-    if constexpr (REM > 0) psp_atb_load<REM>(row + N4 * 16 + REM * c, out + N4);
-}
-
 template <int K1, int K2, int JSPLIT, bool RELU_A>
 __global__ void __launch_bounds__(256, K1 * K2 / JSPLIT > 16 * 256 ? 1 : 2)
 psp_atb_mfma_kernel(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, long long n,
@@ -292,12 +261,20 @@ psp_atb_split_kernel(const float *__restrict__ A, const float *__restrict__ B, f
 // C[e] = sum over the P workgroup slots of partial[p][e].  A workgroup of 1024 lanes takes 16 elements; lane t adds the
 // slots t / 16, t / 16 + 64, ... of element t % 16 (all loads independent, so one memory latency covers them), then
 // the 64 sums of an element meet in LDS.
-__global__ void __launch_bounds__(1024)
-psp_atb_reduce_kernel(const float *__restrict__ partial, float *__restrict__ C, int P, int E)
+// Several sums share a launch (the weight gradients of a training step: a launch each took 5-7 us of mostly latency).
+struct psp_sum_jobs {
+    psp_partial_sum job[PSP_SUM_JOBS_MAX];
+    int first_block[PSP_SUM_JOBS_MAX + 1];  // blocks of 16 elements
+};
+__global__ void __launch_bounds__(1024) psp_sum_partials_kernel(psp_sum_jobs jobs)
 {
     __shared__ float part[64][17];
+    int j = 0;
+    while ((int)blockIdx.x >= jobs.first_block[j + 1]) j++;
+    const float *partial = jobs.job[j].partial;
+    const int P = jobs.job[j].count, E = jobs.job[j].elements;
     const int el = threadIdx.x & 15, sg = threadIdx.x >> 4;
-    const int e = blockIdx.x * 16 + el;
+    const int e = ((int)blockIdx.x - jobs.first_block[j]) * 16 + el;
     float s = 0.f;
     if (e < E) {
 #pragma unroll 16
@@ -309,14 +286,29 @@ psp_atb_reduce_kernel(const float *__restrict__ partial, float *__restrict__ C, 
         float t = 0.f;
 #pragma unroll
         for (int g = 0; g < 64; g++) t += part[g][threadIdx.x];
-        C[e] = t;
+        jobs.job[j].C[e] = t;
     }
 }
 
-int psp_sum_partials(const float *partial, float *C, int P, int E, hipStream_t stream)
+PSP_EXPORT int psp_sum_partials_f32(const psp_partial_sum *sums, int n, psp_stream_t stream)
 {
-    hipLaunchKernelGGL(psp_atb_reduce_kernel, dim3((unsigned)((E + 15) / 16)), dim3(1024), 0, stream, partial, C, P, E);
-    return psp_check_launch("partial sums");
+    PSP_REQUIRE(n >= 0 && (sums || n == 0), "sum_partials: null pointer or negative count");
+    for (int at = 0; at < n; at += PSP_SUM_JOBS_MAX) {
+        psp_sum_jobs jobs;
+        int m = 0, blocks = 0;
+        for (; m < PSP_SUM_JOBS_MAX && at + m < n; m++) {
+            const psp_partial_sum &s = sums[at + m];
+            PSP_REQUIRE(s.partial && s.C && s.count >= 1 && s.elements >= 1, "sum_partials: sum %d is empty", at + m);
+            jobs.job[m] = s;
+            jobs.first_block[m] = blocks;
+            blocks += (s.elements + 15) / 16;
+        }
+        for (int i = m; i <= PSP_SUM_JOBS_MAX; i++) jobs.first_block[i] = blocks;
+        hipLaunchKernelGGL(psp_sum_partials_kernel, dim3((unsigned)blocks), dim3(1024), 0, (hipStream_t)stream, jobs);
+        const int rc = psp_check_launch("partial sums");
+        if (rc != PSP_OK) return rc;
+    }
+    return PSP_OK;
 }
 
 typedef void (*psp_atb_mfma_kernel_t)(const float *, const float *, float *, long long, float *);
@@ -395,7 +387,7 @@ PSP_EXPORT int psp_gemm_atb_ws_act_f32(const float *A, const float *B, float *C,
     int jsplit = 1;
     psp_atb_mfma_kernel_t km = atb_mfma_lookup(K1, K2, &jsplit, relu_a != 0);
     if (!km || n <= 0) return atb_atomic(A, B, C, n, K1, K2, relu_a != 0, (hipStream_t)stream);  // n = 0, widths there is no kernel for
-    PSP_REQUIRE(A && B && C, "gemm_atb_ws: null pointer");
+    PSP_REQUIRE(A && B, "gemm_atb_ws: null pointer");
     long long wgs = atb_mfma_grid(n, jsplit, K1 * K2);
     PSP_REQUIRE(workspace && workspace_floats >= wgs * K1 * K2, "gemm_atb_ws: the workspace holds %lld floats, %lld needed",
                 workspace_floats, wgs * K1 * K2);
@@ -407,7 +399,9 @@ PSP_EXPORT int psp_gemm_atb_ws_act_f32(const float *A, const float *B, float *C,
     hipLaunchKernelGGL(km, dim3((unsigned)wgs), dim3(256), 0, st, A, B, C, n, workspace);
     int rc = psp_check_launch("gemm_atb mfma kernel");
     if (rc != PSP_OK) return rc;
-    return psp_sum_partials(workspace, C, (int)wgs, K1 * K2, st);
+    if (!C) return (int)wgs;
+    const psp_partial_sum sum = {workspace, C, (int)wgs, K1 * K2};
+    return psp_sum_partials_f32(&sum, 1, stream);
 }
 
 PSP_EXPORT int psp_gemm_atb_ws_f32(const float *A, const float *B, float *C, long long n, int K1, int K2,

@@ -37,11 +37,9 @@
 // to the GPU and every wavefront walks blocks of 32 rows with the next block's loads in flight.
 #include "psp_common.h"
 #include "bf16_split.h"
+#include "dense_tiles.h"
 #include <cstdlib>
 
-typedef float psp_f32x4 __attribute__((ext_vector_type(4)));
-
-#define XWW_STRIDE(K2) (((K2) + 63) / 64 * 64 + 4)
 #define XWW_ROWS 32  // rows per wavefront and step: two MFMA row blocks share every operand read from LDS
 
 // 4 x 4 transpose between the four 16-lane rows of a wavefront and the four elements of v: element e of row q <-> element q of

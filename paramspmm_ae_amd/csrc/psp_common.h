@@ -70,8 +70,6 @@ int psp_fill_f32(float *p, size_t n, float value, hipStream_t stream);
 
 // Y[r, :] /= s[r] for every row with s[r] != 0 (rows of the softmax-weighted row-split SpMM that several
 // wavefronts accumulated without normalising)
-// C[e] = sum over p < P of partial[p][e] (E elements each), in a fixed order (dense_atb.hip)
-int psp_sum_partials(const float *partial, float *C, int P, int E, hipStream_t stream);
 int psp_row_scale(float *Y, const float *s, int rows, int N, hipStream_t stream);
 
 #define PSP_F32_LOWEST (-3.402823466e+38f)

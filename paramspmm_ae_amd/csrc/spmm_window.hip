@@ -644,7 +644,10 @@ static int pspw_launch(const int *rowPtr_w, const int *colIdx_w, const float *va
     if (nnz == 0) {  // (the kernel clamps its loads to entry nnz - 1)
         if (Y) rc = psp_zero_f32(Y, (size_t)rows_out * N, st);
         if (rc == PSP_OK && Y_raw) rc = psp_zero_f32(Y_raw, (size_t)rows_out * N, st);
-        return rc != PSP_OK || !gr.kz ? rc : psp_zero_f32(gr.dW, (size_t)gr.kz * N, st);
+        if (rc != PSP_OK || !gr.kz) return rc;
+        if (gr.dW) return psp_zero_f32(gr.dW, (size_t)gr.kz * N, st);
+        rc = psp_zero_f32(gr.ws, (size_t)gr.kz * N, st);
+        return rc != PSP_OK ? rc : 1;
     }
     if (Y) rc = psp_zero_f32(Y + (size_t)M * N, ((size_t)rows_out - (size_t)M) * N, st);  // rows past the matrix
     if (rc == PSP_OK && Y_raw) rc = psp_zero_f32(Y_raw + (size_t)M * N, ((size_t)rows_out - (size_t)M) * N, st);
@@ -655,14 +658,17 @@ static int pspw_launch(const int *rowPtr_w, const int *colIdx_w, const float *va
     int run = 0, nruns = 0;
     rc = pspw_shape(M, N, v, tn, lds, epi, gr.kz, k, &lds, &run, &nruns);
     if (rc != PSP_OK) return rc;
-    PSP_REQUIRE(gr.kz == 0 || (gr.Z && gr.dW && gr.ws && gr.ws_floats >= (long long)nruns * gr.kz * N),
-                "spmm_window: the weight gradient needs Z, dW and %lld floats of workspace", (long long)nruns * gr.kz * N);
+    PSP_REQUIRE(gr.kz == 0 || (gr.Z && gr.ws && gr.ws_floats >= (long long)nruns * gr.kz * N),
+                "spmm_window: the weight gradient needs Z and %lld floats of workspace", (long long)nruns * gr.kz * N);
     const psp_grid1d g = psp_xcd_grid(nruns, 1);  // long runs: neighbouring runs share two halo windows, nothing to keep in one L2
     dim3 grid(g.launch, psp_ceil_div(N, tn), 1), block(k.threads, 1, 1);
     hipLaunchKernelGGL(k.fn, grid, block, lds, st, rowPtr_w, colIdx_w, val_w, X, Y, mask, M, N, nnz, nruns, g.stripe, run,
                        relu_x != 0, W, transW != 0, Y_raw, gr.Z, gr.relu_z, gr.ws);
     rc = psp_check_launch("spmm window kernel");
-    return rc != PSP_OK || !gr.kz ? rc : psp_sum_partials(gr.ws, gr.dW, nruns, gr.kz * N, st);
+    if (rc != PSP_OK || !gr.kz) return rc;
+    if (!gr.dW) return nruns;
+    const psp_partial_sum sum = {gr.ws, gr.dW, nruns, gr.kz * N};
+    return psp_sum_partials_f32(&sum, 1, st);
 }
 
 PSP_EXPORT int psp_spmm_window_grad_supported(int N, int KZ, int dense) { return (N == 16 || N == 32) && pspw_lookup(N / 16, dense != 0, KZ).fn != nullptr; }
@@ -682,7 +688,7 @@ PSP_EXPORT int psp_spmm_window_grad_f32(const int *rowPtr_w, const int *colIdx_w
                                         long long workspace_floats, int M, int nnz, int N, int rows_out, psp_stream_t stream)
 {
     PSP_REQUIRE(psp_spmm_window_grad_supported(N, KZ, W != nullptr), "spmm_window_grad: no weight gradient of %d x %d", KZ, N);
-    PSP_REQUIRE(dW && (!W || dZ), "spmm_window_grad: null pointer");
+    PSP_REQUIRE((dW || workspace) && (!W || dZ), "spmm_window_grad: null pointer");
     return pspw_launch(rowPtr_w, colIdx_w, val_w, G, dZ, M, nnz, N, rows_out, 0, 0, nullptr, W, 1, nullptr, (hipStream_t)stream,
                        pspw_grad{Z, KZ, relu_z != 0, dW, workspace, workspace_floats});
 }

@@ -48,22 +48,51 @@ static bool kept_order_is_ours(long n, long K1, long K2)
     return n >= 16384 && (K2 <= 32 ? K1 <= 64 || (K1 == 128 && K2 == 16) : (K2 == 64 || K2 == 128) && pow2);
 }
 
+// Weight gradients leave their kernels as partial products of the workgroups.  The sums of everything one backward call forms
+// share a launch (psp_sum_partials_f32): flush() before the gradients are handed out.
+struct PartialSums {
+    std::vector<psp_partial_sum> jobs;
+    std::vector<Tensor> held;  // workspaces and results, until the launch
+    psp_stream_t stream = nullptr;
+    void add(const Tensor &ws, Tensor &dW, int count)
+    {
+        jobs.push_back({fp(ws), fpw(dW), count, (int)dW.numel()});
+        held.push_back(ws);
+        held.push_back(dW);
+        stream = stream_of(ws);
+    }
+    void flush()
+    {
+        if (jobs.empty()) return;
+        DeviceGuard guard(held[0].device());
+        ok(psp_sum_partials_f32(jobs.data(), (int)jobs.size(), stream));
+        jobs.clear();
+        held.clear();
+    }
+};
+static int ok_count(int rc)
+{
+    ok(rc);
+    return rc;
+}
+
 // H^T * AG.  For narrow layers the product is a reduction over ~10^6 rows into a tiny matrix, which the library
 // streams at memory speed; everything else goes to torch::mm.
-static Tensor weight_gradient(const Tensor &H, const Tensor &AG)
+static Tensor weight_gradient(const Tensor &H, const Tensor &AG, PartialSums *sums = nullptr, bool relu = false)
 {
     const bool narrow = H.dim() == 2 && AG.dim() == 2 && H.size(0) == AG.size(0) && H.size(0) >= kDenseRows &&
                         H.scalar_type() == torch::kFloat32 && AG.scalar_type() == torch::kFloat32 &&
                         psp_gemm_atb_supported((int)H.size(1), (int)AG.size(1));
-    if (!narrow) return torch::mm(H.t(), AG);
+    if (!narrow) return torch::mm((relu ? torch::relu(H) : H).t(), AG);
     Tensor Hc = H.contiguous(), Gc = AG.contiguous();
     DeviceGuard guard(Hc.device());
     Tensor dW = torch::empty({Hc.size(1), Gc.size(1)}, Hc.options());
     // partial products of the workgroups go through a workspace and are added in a fixed order (no atomics)
     const long long ws_floats = psp_gemm_atb_workspace_floats(Hc.size(0), (int)Hc.size(1), (int)Gc.size(1));
     Tensor ws = torch::empty({(long)ws_floats}, Hc.options());
-    ok(psp_gemm_atb_ws_f32(fp(Hc), fp(Gc), fpw(dW), Hc.size(0), (int)Hc.size(1), (int)Gc.size(1), fpw(ws), ws_floats,
-                           stream_of(Hc)));
+    const int count = ok_count(psp_gemm_atb_ws_act_f32(fp(Hc), fp(Gc), sums ? nullptr : fpw(dW), Hc.size(0), (int)Hc.size(1),
+                                                       (int)Gc.size(1), relu ? 1 : 0, fpw(ws), ws_floats, stream_of(Hc)));
+    if (sums) sums->add(ws, dW, count);
     return dW;
 }
 
@@ -116,20 +145,28 @@ static Tensor dense_xwt_masked(const Tensor &AG, const Tensor &W, const Tensor &
     return Y;
 }
 // relu(Z)^T * AG
-static Tensor weight_gradient_relu(const Tensor &Z, const Tensor &AG)
+static Tensor weight_gradient_relu(const Tensor &Z, const Tensor &AG, PartialSums *sums = nullptr)
 {
-    const bool narrow = Z.dim() == 2 && AG.dim() == 2 && Z.size(0) == AG.size(0) && Z.size(0) >= kDenseRows &&
-                        Z.scalar_type() == torch::kFloat32 && AG.scalar_type() == torch::kFloat32 &&
-                        psp_gemm_atb_supported((int)Z.size(1), (int)AG.size(1));
-    if (!narrow) return torch::mm(torch::relu(Z).t(), AG);
-    Tensor Zc = Z.contiguous(), Gc = AG.contiguous();
-    DeviceGuard guard(Zc.device());
-    Tensor dW = torch::empty({Zc.size(1), Gc.size(1)}, Zc.options());
-    const long long ws_floats = psp_gemm_atb_workspace_floats(Zc.size(0), (int)Zc.size(1), (int)Gc.size(1));
-    Tensor ws = torch::empty({(long)ws_floats}, Zc.options());
-    ok(psp_gemm_atb_ws_act_f32(fp(Zc), fp(Gc), fpw(dW), Zc.size(0), (int)Zc.size(1), (int)Gc.size(1), 1, fpw(ws), ws_floats,
-                               stream_of(Zc)));
-    return dW;
+    return weight_gradient(Z, AG, sums, true);
+}
+// {(AG * W^T) where Z > 0, relu(Z)^T * AG}: one launch where the library has the pair (psp_dense_grad_f32)
+static std::pair<Tensor, Tensor> dense_grads_relu(const Tensor &AG, const Tensor &W, const Tensor &Z, PartialSums *sums)
+{
+    const bool pair = AG.dim() == 2 && W.dim() == 2 && Z.dim() == 2 && Z.size(0) == AG.size(0) && Z.size(1) == W.size(0) &&
+                      AG.size(1) == W.size(1) && AG.size(0) >= kDenseRows && AG.scalar_type() == torch::kFloat32 &&
+                      W.scalar_type() == torch::kFloat32 && Z.scalar_type() == torch::kFloat32 &&
+                      psp_dense_grad_supported((int)W.size(0), (int)W.size(1));
+    if (!pair) return {dense_xwt_masked(AG, W, Z), weight_gradient_relu(Z, AG, sums)};
+    Tensor Gc = AG.contiguous(), Wc = W.contiguous(), Zc = Z.contiguous();
+    DeviceGuard guard(Gc.device());
+    const int K1 = (int)Wc.size(0), K2 = (int)Wc.size(1);
+    Tensor dZ = torch::empty_like(Zc), dW = torch::empty_like(Wc);
+    const long long ws_floats = psp_dense_grad_workspace_floats(Gc.size(0), K1, K2);
+    Tensor ws = torch::empty({(long)ws_floats}, Gc.options());
+    const int count = ok_count(psp_dense_grad_f32(fp(Gc), fp(Zc), fp(Wc), fpw(dZ), sums ? nullptr : fpw(dW), Gc.size(0), K1, K2, fpw(ws),
+                                                  ws_floats, stream_of(Gc)));
+    if (sums) sums->add(ws, dW, count);
+    return {dZ, dW};
 }
 
 // GCN layer that reads its input through a ReLU: A * (relu(Z) * W).  fmt: 0 csr, 1 csr_split, 2 bcsr, 3 bcsr_split.
@@ -151,7 +188,8 @@ static std::vector<Tensor> relu_input_backward(int fmt, Tensor dY, Tensor Z, Ten
     need_gpu(W, "weight");
     TORCH_CHECK(fmt >= 0 && fmt <= 4 && (fmt == 1 || fmt == 3) == target_row.has_value(), "format code and target_row disagree");
     Tensor AG = aggregate(fmt, dY, rowPtr, colIdx, values, target_row ? &*target_row : nullptr, CF, bw);
-    return {dense_xwt_masked(AG, W, Z), weight_gradient_relu(Z, AG)};
+    auto r = dense_grads_relu(AG, W, Z, nullptr);
+    return {r.first, r.second};
 }
 
 // A * D alone, for callers that place the sparse product on the narrower side of the layer: (A H) W costs a sparse
@@ -240,14 +278,14 @@ static std::vector<Tensor> window_xw(Tensor X, Tensor W, bool transW, Tensor row
 }
 
 // Backward on the windowed layout with the weight gradient formed in the sparse kernel (psp_spmm_window_grad_f32): dW = f(Z)^T (A G)
-// and, with W, dZ = ((A G) W^T) where Z > 0, else A G when want_ag.  Returns {dW, dZ or A G or nothing}.
+// and, with W, dZ = ((A G) W^T) where Z > 0, else A G when want_ag.  Returns {dW (whole after sums.flush()), dZ or A G or nothing}.
 static bool window_grad_supported(const Tensor &G, const Tensor &Z, bool dense)
 {
     return G.dim() == 2 && Z.dim() == 2 && G.size(0) == Z.size(0) && G.scalar_type() == torch::kFloat32 && Z.scalar_type() == torch::kFloat32 &&
            psp_spmm_window_grad_supported((int)G.size(1), (int)Z.size(1), dense ? 1 : 0);
 }
 static std::vector<Tensor> window_grad(Tensor G, Tensor Z, bool relu_z, const Tensor *W, bool want_ag, Tensor rowPtr_w, Tensor colIdx_w,
-                                       Tensor values_w)
+                                       Tensor values_w, PartialSums &sums)
 {
     Tensor Gc = G.contiguous(), Zc = Z.contiguous(), Wc;
     check_spmm_args(4, Gc, rowPtr_w, colIdx_w, values_w, nullptr);
@@ -263,9 +301,10 @@ static std::vector<Tensor> window_grad(Tensor G, Tensor Z, bool relu_z, const Te
     const long long ws_floats = psp_spmm_window_grad_workspace_floats(M, N, KZ, W ? 1 : 0);
     Tensor dW = torch::empty({KZ, N}, Gc.options()), ws = torch::empty({(long)ws_floats}, Gc.options()), Y;
     if (W || want_ag) Y = torch::empty_like(Gc);
-    ok(psp_spmm_window_grad_f32(ip(rowPtr_w), ip(colIdx_w), fp(values_w), fp(Gc), fp(Zc), KZ, relu_z ? 1 : 0, W ? fp(Wc) : nullptr,
-                                Y.defined() ? fpw(Y) : nullptr, fpw(dW), fpw(ws), ws_floats, M, (int)colIdx_w.size(0), N,
-                                (int)Gc.size(0), stream_of(Gc)));
+    const int count = ok_count(psp_spmm_window_grad_f32(ip(rowPtr_w), ip(colIdx_w), fp(values_w), fp(Gc), fp(Zc), KZ, relu_z ? 1 : 0,
+                                                        W ? fp(Wc) : nullptr, Y.defined() ? fpw(Y) : nullptr, nullptr, fpw(ws), ws_floats,
+                                                        M, (int)colIdx_w.size(0), N, (int)Gc.size(0), stream_of(Gc)));
+    sums.add(ws, dW, count);
     return {dW, Y};
 }
 
@@ -495,7 +534,7 @@ struct LayerNode : torch::autograd::Node {
 };
 
 // the result of `forward` (run without recording), with a node of type N behind it when an input asks for gradients
-template <class N, class F> static Tensor with_node(const op_t &op, std::initializer_list<Tensor> inputs, F forward)
+template <class N, class F> static Tensor with_node(const op_t &op, at::ArrayRef<Tensor> inputs, F forward)
 {
     const bool record = torch::GradMode::is_enabled() &&
                         std::any_of(inputs.begin(), inputs.end(), [](const Tensor &t) { return t.requires_grad(); });
@@ -522,102 +561,94 @@ static bool folds_dense(const Operator &o, const Tensor &Z, const Tensor &W)
            Z.scalar_type() == torch::kFloat32;
 }
 
-// A (H W); dH = (A dY) W^T, dW = H^T (A dY) -- A is symmetric (gnn_conv.py:13-107)
-struct GCNFunction : LayerNode {
-    variable_list apply(variable_list &&g) override
-    {
-        if (!g[0].defined()) return {Tensor(), Tensor()};
-        Tensor H = a(), W = w();
-        if (op->fmt == 4 && wants(1) && window_grad_supported(g[0], H, false)) {
-            auto r = window_grad(g[0], H, false, nullptr, wants(0), op->rowPtr, op->colIdx, op->val);
-            return {wants(0) ? dense_xw(r[1], W, true, Order::any) : Tensor(), r[0]};
-        }
-        Tensor AG = aggregate(op->fmt, g[0], op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
-        return {wants(0) ? dense_xw(AG, W, true, Order::any) : Tensor(), wants(1) ? weight_gradient(H, AG) : Tensor()};
-    }
+// The layers without attention, each direction once: for nodes of their own and for a whole network's.
+enum Layer {
+    kGCN = 0,             // A (H W); dH = (A dY) W^T, dW = H^T (A dY) -- A is symmetric (gnn_conv.py:13-107)
+    kAggregateFirst = 1,  // (A H) W with A H kept: dW = (A H)^T dY, dH = A (dY W^T) -- the layer that widens its input, and
+                          // GIN's (gnn_conv.py:202-220)
+    kGCNReLU = 2,         // A (relu(Z) W): dZ = ((A dY) W^T) where Z > 0, dW = relu(Z)^T (A dY)
+    kGINReLU = 3          // (A relu(Z)) W for a layer that widens its input: the activation is applied as the sparse product
+                          // gathers the rows of Z, the gradient masked in a pass that follows the backward product
 };
-static Tensor gcn_layer(op_t op, Tensor H, Tensor W)
+// kept: what the backward needs besides the input and the weights (A H; undefined for the kinds that keep nothing)
+static Tensor layer_forward(int kind, const Operator &o, const Tensor &in, const Tensor &W, Tensor &kept)
 {
-    need_gpu(H, "input");
+    need_gpu(in, "input");
     need_gpu(W, "weight");
-    return with_node<GCNFunction>(op, {H, W}, [&](GCNFunction *n) {
-        if (n) n->a_ = SavedVariable(H, false), n->w_ = SavedVariable(W, false);
-        return aggregate(op->fmt, dense_xw(H, W, false, Order::kept), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
-    });
-}
-
-// (A H) W with A H kept for the backward: dW = (A H)^T dY, dH = A (dY W^T) -- the layer that widens its input, and GIN's
-// (gnn_conv.py:202-220)
-struct AggregateFirst : LayerNode {
-    variable_list apply(variable_list &&g) override
-    {
-        if (!g[0].defined()) return {Tensor(), Tensor()};
-        Tensor AH = a(), W = w(), dY = g[0].contiguous(), dH;
-        if (wants(0)) dH = aggregate(op->fmt, dense_xw(dY, W, true, Order::any), op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
-        return {dH, wants(1) ? weight_gradient(AH, dY) : Tensor()};
+    switch (kind) {
+    case kGCN: return aggregate(o.fmt, dense_xw(in, W, false, Order::kept), o.rowPtr, o.colIdx, o.val, o.tr(), o.CF, o.bw);
+    case kAggregateFirst:
+        kept = aggregate(o.fmt, in, o.rowPtr, o.colIdx, o.val, o.tr(), o.CF, o.bw);
+        return dense_xw(kept, W, false, Order::kept);
+    case kGCNReLU:
+        // windowed layout, square layer: (A relu(Z)) W in one launch, the dense product in the kernel's epilogue
+        if (folds_dense(o, in, W)) return window_xw(in, W, false, o.rowPtr, o.colIdx, o.val, true, c10::nullopt, false)[0];
+        return relu_input_forward(o.fmt, in, W, o.rowPtr, o.colIdx, o.val, o.target_row, o.CF, o.bw);
+    default:
+        kept = aggregate_act_op(o.fmt, in, o.rowPtr, o.colIdx, o.val, o.target_row, o.CF, o.bw, true, c10::nullopt);
+        return dense_xw(kept, W, false, Order::kept);
     }
-};
-struct GCNAggregateFirstFunction : AggregateFirst {};
-struct GINFunction : AggregateFirst {};
-template <class N> static Tensor aggregate_first_layer(op_t op, Tensor H, Tensor W)
-{
-    need_gpu(H, "input");
-    need_gpu(W, "weight");
-    return with_node<N>(op, {H, W}, [&](N *n) {
-        Tensor AH = aggregate(op->fmt, H, op->rowPtr, op->colIdx, op->val, op->tr(), op->CF, op->bw);
-        if (n) n->a_ = SavedVariable(AH, false), n->w_ = SavedVariable(W, false);
-        return dense_xw(AH, W, false, Order::kept);
-    });
 }
-
-// A (relu(Z) W): dZ = ((A dY) W^T) where Z > 0, dW = relu(Z)^T (A dY)
-struct GCNReLUInputFunction : LayerNode {
-    variable_list apply(variable_list &&g) override
-    {
-        if (!g[0].defined()) return {Tensor(), Tensor()};
-        Tensor Z = a(), W = w(), dY = g[0].contiguous();
-        if (folds_dense(*op, Z, W)) {
+// {gradient of the input, of the weights (whole after sums.flush())}, either undefined when not wanted; `in` may be undefined
+// for kAggregateFirst
+static std::pair<Tensor, Tensor> layer_backward(int kind, const Operator &o, const Tensor &g, const Tensor &in, const Tensor &W,
+                                                const Tensor &kept, bool want_in, bool want_w, PartialSums &sums)
+{
+    Tensor dY = g.contiguous(), dIn, dW;
+    if (kind == kGCN || kind == kGCNReLU) {
+        const bool relu = kind == kGCNReLU;
+        if (relu && folds_dense(o, in, W)) {
             // one launch delivers ((A dY) W^T) where Z > 0 (the input gradient) and the weight gradient
-            auto r = window_grad(dY, Z, true, &W, false, op->rowPtr, op->colIdx, op->val);
+            auto r = window_grad(dY, in, true, &W, false, o.rowPtr, o.colIdx, o.val, sums);
             return {r[1], r[0]};
         }
-        if (op->fmt == 4 && window_grad_supported(dY, Z, false)) {
-            auto r = window_grad(dY, Z, true, nullptr, true, op->rowPtr, op->colIdx, op->val);
-            return {dense_xwt_masked(r[1], W, Z), r[0]};
+        Tensor AG;
+        if (o.fmt == 4 && want_w && window_grad_supported(dY, in, false)) {
+            auto r = window_grad(dY, in, relu, nullptr, want_in, o.rowPtr, o.colIdx, o.val, sums);
+            dW = r[0], AG = r[1];
+        } else {
+            AG = aggregate(o.fmt, dY, o.rowPtr, o.colIdx, o.val, o.tr(), o.CF, o.bw);
+            if (relu && want_in && want_w) return dense_grads_relu(AG, W, in, &sums);
+            if (want_w) dW = weight_gradient(in, AG, &sums, relu);
         }
-        auto r = relu_input_backward(op->fmt, dY, Z, W, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw);
-        return {r[0], r[1]};
+        if (want_in) dIn = relu ? dense_xwt_masked(AG, W, in) : dense_xw(AG, W, true, Order::any);
+        return {dIn, dW};
     }
-};
-static Tensor gcn_relu_layer(op_t op, Tensor Z, Tensor W)
-{
-    return with_node<GCNReLUInputFunction>(op, {Z, W}, [&](GCNReLUInputFunction *n) {
-        if (n) n->a_ = SavedVariable(Z, false), n->w_ = SavedVariable(W, false);
-        // windowed layout, square layer: (A relu(Z)) W in one launch, the dense product in the kernel's epilogue
-        if (folds_dense(*op, Z, W)) return window_xw(Z, W, false, op->rowPtr, op->colIdx, op->val, true, c10::nullopt, false)[0];
-        return relu_input_forward(op->fmt, Z, W, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw);
-    });
+    if (want_in) {
+        Tensor D = dense_xw(dY, W, true, Order::any);
+        dIn = kind == kGINReLU ? aggregate_act_op(o.fmt, D, o.rowPtr, o.colIdx, o.val, o.target_row, o.CF, o.bw, false, in)
+                               : aggregate(o.fmt, D, o.rowPtr, o.colIdx, o.val, o.tr(), o.CF, o.bw);
+    }
+    if (want_w) dW = weight_gradient(kept, dY, &sums);
+    return {dIn, dW};
 }
 
-// (A relu(Z)) W for a layer that widens its input: the activation is applied as the sparse product gathers the rows of Z,
-// the gradient masked in a pass that follows the backward product
-struct GINReLUInputFunction : LayerNode {
+template <int KIND> struct PlainLayer : LayerNode {  // a_ = input (kAggregateFirst: none), z_ = kept
     variable_list apply(variable_list &&g) override
     {
         if (!g[0].defined()) return {Tensor(), Tensor()};
-        Tensor AX = a(), W = w(), Z = z(), dY = g[0].contiguous();
-        return {wants(0) ? aggregate_act_op(op->fmt, dense_xw(dY, W, true, Order::any), op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw,
-                                            false, Z)
-                         : Tensor(),
-                wants(1) ? weight_gradient(AX, dY) : Tensor()};
+        constexpr bool in = KIND != kAggregateFirst, keeps = KIND == kAggregateFirst || KIND == kGINReLU;
+        PartialSums sums;
+        auto r = layer_backward(KIND, *op, g[0], in ? a() : Tensor(), w(), keeps ? z() : Tensor(), wants(0), wants(1), sums);
+        sums.flush();
+        return {r.first, r.second};
     }
 };
-static Tensor gin_relu_layer(op_t op, Tensor Z, Tensor W)
+struct GCNFunction : PlainLayer<kGCN> {};
+struct GCNAggregateFirstFunction : PlainLayer<kAggregateFirst> {};
+struct GCNReLUInputFunction : PlainLayer<kGCNReLU> {};
+struct GINFunction : PlainLayer<kAggregateFirst> {};
+struct GINReLUInputFunction : PlainLayer<kGINReLU> {};
+template <class N, int KIND> static Tensor plain_layer(op_t op, Tensor H, Tensor W)
 {
-    return with_node<GINReLUInputFunction>(op, {Z, W}, [&](GINReLUInputFunction *n) {
-        Tensor AX = aggregate_act_op(op->fmt, Z, op->rowPtr, op->colIdx, op->val, op->target_row, op->CF, op->bw, true, c10::nullopt);
-        if (n) n->a_ = SavedVariable(AX, false), n->w_ = SavedVariable(W, false), n->z_ = SavedVariable(Z, false);
-        return dense_xw(AX, W, false, Order::kept);
+    return with_node<N>(op, {H, W}, [&](N *n) {
+        Tensor kept, out = layer_forward(KIND, *op, H, W, kept);
+        if (n) {
+            if (KIND != kAggregateFirst) n->a_ = SavedVariable(H, false);
+            n->w_ = SavedVariable(W, false);
+            if (kept.defined()) n->z_ = SavedVariable(kept, false);
+        }
+        return out;
     });
 }
 
@@ -638,8 +669,12 @@ struct AGNNFunction : LayerNode {  // a_ = X, z_ = att
         auto r = op->fmt == 4 ? attn_window_backward(dY, att, op->rowPtr, op->colIdx)
                               : attn_backward(op->fmt, dY, att, op->rowPtr, op->colIdx, op->target_row, op->slot, op->bw);
         Tensor dX, dW;
-        if (wants(0)) dX = relu_input ? dense_xwt_masked(r[0], W, X) : dense_xw(r[0], W, true, Order::any);
-        if (wants(1)) dW = relu_input ? weight_gradient_relu(X, r[0]) : weight_gradient(X, r[0]);
+        if (relu_input && wants(0) && wants(1)) {
+            std::tie(dX, dW) = dense_grads_relu(r[0], W, X, nullptr);
+        } else {
+            if (wants(0)) dX = relu_input ? dense_xwt_masked(r[0], W, X) : dense_xw(r[0], W, true, Order::any);
+            if (wants(1)) dW = weight_gradient(X, r[0], nullptr, relu_input);
+        }
         return {dX, dW, r[1].reshape({1, 1}).expand(alpha_shape)};
     }
 };
@@ -691,6 +726,70 @@ static Tensor softmax_nll_layer(Tensor logits, Tensor labels)
     });
 }
 
+// A training step's network and loss, nll_loss(log_softmax(layers(x)), labels), as one node.  On a graph of 20 K nodes the step is
+// bound by the host: six nodes cost the engine some 80 us, and each layer's weight gradient a launch for its sum.
+struct NetworkLoss : LayerNode {  // a_ = labels, w_ = logits, z_ = stats
+    struct Part {
+        int kind;
+        op_t op;
+        SavedVariable in, w, kept;
+    };
+    std::vector<Part> parts;
+    void release_variables() override
+    {
+        LayerNode::release_variables();
+        for (Part &p : parts) p.in.reset_data(), p.w.reset_data(), p.kept.reset_data();
+    }
+    variable_list apply(variable_list &&g) override
+    {
+        variable_list out(1 + parts.size());
+        if (!g[0].defined()) return out;
+        auto self = shared_from_this();
+        size_t lowest = 0;  // the lowest input (x, then the weights) that asks for its gradient
+        while (lowest < out.size() && !wants(lowest)) lowest++;
+        if (lowest == out.size()) return out;
+        Tensor d = softmax_nll_mean_backward(w(), a(), g[0].contiguous(), z());
+        PartialSums sums;
+        for (size_t l = parts.size(); l-- > 0 && lowest <= l + 1;) {
+            Part &p = parts[l];
+            const bool keeps = p.kind == kAggregateFirst || p.kind == kGINReLU;
+            std::tie(d, out[l + 1]) = layer_backward(p.kind, *p.op, d, p.kind == kAggregateFirst ? Tensor() : p.in.unpack(self), p.w.unpack(self),
+                                                     keeps ? p.kept.unpack(self) : Tensor(), lowest <= l, wants(l + 1), sums);
+            if (!wants(l + 1)) out[l + 1] = Tensor();
+        }
+        if (wants(0)) out[0] = d;
+        sums.flush();
+        return out;
+    }
+};
+static Tensor network_loss(std::vector<int> kinds, std::vector<op_t> ops, Tensor x, std::vector<Tensor> weights, Tensor labels)
+{
+    const size_t L = weights.size();
+    TORCH_CHECK(L > 0 && kinds.size() == L && ops.size() == L, "network_loss: one kind, operator and weight matrix per layer");
+    for (int k : kinds) TORCH_CHECK(k >= kGCN && k <= kGINReLU, "network_loss: unknown kind of layer");
+    std::vector<Tensor> inputs{x};
+    inputs.insert(inputs.end(), weights.begin(), weights.end());
+    return with_node<NetworkLoss>(nullptr, inputs, [&](NetworkLoss *n) {
+        Tensor h = x;
+        if (n) n->parts.reserve(L);
+        for (size_t l = 0; l < L; l++) {
+            Tensor kept, out = layer_forward(kinds[l], *ops[l], h, weights[l], kept);
+            if (n) {
+                n->parts.emplace_back();
+                NetworkLoss::Part &p = n->parts.back();
+                p.kind = kinds[l], p.op = ops[l];
+                p.w = SavedVariable(weights[l], false);
+                if (kinds[l] != kAggregateFirst) p.in = SavedVariable(h, false);
+                if (kept.defined()) p.kept = SavedVariable(kept, false);
+            }
+            h = out;
+        }
+        auto r = softmax_nll_mean(h, labels);
+        if (n) n->a_ = SavedVariable(labels, false), n->w_ = SavedVariable(h, false), n->z_ = SavedVariable(r[1], false);
+        return r[0];
+    });
+}
+
 // the nodes under their own names in Python (type(t.grad_fn).__name__)
 template <class N> static void register_node(const char *name)
 {
@@ -737,20 +836,23 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     register_node<AGNNFunction>("AGNNFunctionBackward");
     register_node<NllLossMean>("NllLossMeanBackward");
     register_node<SoftmaxNllMean>("SoftmaxNllMeanBackward");
+    register_node<NetworkLoss>("NetworkLossBackward");
     py::class_<Operator, op_t>(m, "Operator", "what a layer needs of a pcsr_spmm")
         .def(py::init([](int fmt, Tensor rowPtr, Tensor colIdx, Tensor val, c10::optional<Tensor> target_row, int CF, int bw,
                          bool fold_dense, c10::optional<Tensor> slot) {
             TORCH_CHECK(fmt >= 0 && fmt <= 4 && (fmt == 1 || fmt == 3) == target_row.has_value(), "format code and target_row disagree");
             return std::make_shared<Operator>(Operator{fmt, rowPtr, colIdx, val, target_row, CF, bw, fold_dense, slot});
         }));
-    m.def("gcn_layer", &gcn_layer, "A (H W): (operator, H, W)");
-    m.def("gcn_aggregate_first_layer", &aggregate_first_layer<GCNAggregateFirstFunction>, "(A H) W: (operator, H, W)");
-    m.def("gcn_relu_layer", &gcn_relu_layer, "A (relu(Z) W): (operator, Z, W)");
-    m.def("gin_layer", &aggregate_first_layer<GINFunction>, "(A X) W: (operator, X, W)");
-    m.def("gin_relu_layer", &gin_relu_layer, "(A relu(Z)) W: (operator, Z, W)");
+    m.def("gcn_layer", &plain_layer<GCNFunction, kGCN>, "A (H W): (operator, H, W)");
+    m.def("gcn_aggregate_first_layer", &plain_layer<GCNAggregateFirstFunction, kAggregateFirst>, "(A H) W: (operator, H, W)");
+    m.def("gcn_relu_layer", &plain_layer<GCNReLUInputFunction, kGCNReLU>, "A (relu(Z) W): (operator, Z, W)");
+    m.def("gin_layer", &plain_layer<GINFunction, kAggregateFirst>, "(A X) W: (operator, X, W)");
+    m.def("gin_relu_layer", &plain_layer<GINReLUInputFunction, kGINReLU>, "(A relu(Z)) W: (operator, Z, W)");
     m.def("agnn_layer", &agnn_layer, "attention layer: (operator, X, W, attention_w, relu_input)");
     m.def("nll_loss_layer", &nll_loss_layer, "mean negative log-likelihood: (log-probabilities, int64 labels)");
     m.def("softmax_nll_layer", &softmax_nll_layer, "nll_loss(log_softmax(logits), labels), mean over the rows");
+    m.def("network_loss", &network_loss,
+          "nll_loss(log_softmax(layers(x)), labels): (kinds 0 gcn, 1 aggregate first, 2 gcn of relu, 3 aggregate first of relu; operators, x, weights, labels)");
     m.def("split_csr", &pspglue::split_csr, "row split on the host");
     m.def("split_csr_par", &pspglue::split_csr_par, "row split on the host with a precomputed segment prefix");
     // addition of this build: H^T * G for tall-skinny operands (memory-speed kernel for widths 16..64, else torch::mm)

@@ -5,6 +5,7 @@ enters the interpreter between two launches.  Layers look their operator up in `
 import math
 
 import torch
+from torch.nn.modules import module as _module
 
 import paramspmm_ae_amd  # noqa: F401
 import ParamSpCONV as SpCONV
@@ -148,11 +149,15 @@ class GCNConv(_Layer):
         A layer that widens its input is computed as (A H) W when ``spmm_dict`` also holds an operator for the input's
         width (the reference's layers look up the output's width only, gnn_conv.py:121-124, and always compute
         A (H W))."""
+        fn, op = self.choose(H.shape[0], spmm_dict, relu_input)
+        return fn.apply(H, self.weights, op)
+
+    def choose(self, rows, spmm_dict, relu_input):
+        """(function, operator) of a forward pass over ``rows`` rows"""
         in_w, out_w = self.weights.shape
         if self.aggregate_first and not relu_input and in_w < out_w and in_w in spmm_dict:
-            return GCNAggregateFirstFunction.apply(H, self.weights, spmm_dict[in_w])
-        fn = GCNReLUInputFunction if relu_input else GCNFunction
-        return fn.apply(H, self.weights, self._operator(spmm_dict))
+            return GCNAggregateFirstFunction, spmm_dict[in_w]
+        return GCNReLUInputFunction if relu_input else GCNFunction, self._operator(spmm_dict)
 
 
 class AGNNFunction(object):
@@ -275,16 +280,51 @@ class GINConv(_Layer):
         pass.  A layer that does not widen its input is evaluated as A (relu(X) W) -- the same product, the sparse
         part at the narrower width -- with the activation and its backward folded into the dense products, like the
         GCN layer; a widening layer applies the activation inside the sparse product."""
+        fn, op = self.choose(X.shape[0], spmm_dict, relu_input)
+        if relu_input and fn in (GINFunction, _GINOnOperator):
+            X = torch.relu(X)
+        return fn.apply(X, self.weights, op)
+
+    def choose(self, rows, spmm_dict, relu_input):
+        """(function, operator) of a forward pass over ``rows`` rows; functions without ReLU in their name take an
+        activated input"""
         in_w, out_w = self.weights.shape
         if relu_input and in_w >= out_w:
             op = self._operator(spmm_dict)
             if op.vec_size in (1, 2):
-                return GCNReLUInputFunction.apply(X, self.weights, op)
+                return GCNReLUInputFunction, op
         # the sparse product runs at the input's width: take the operator configured for that width when there is
         # one (the reference's layers look up the output's width only, gnn_conv.py:223-226)
         op = spmm_dict[in_w] if self.operator_of_input_width and in_w in spmm_dict else self._operator(spmm_dict)
         if relu_input and op.vec_size in (1, 2):
-            return GINReLUInputFunction.apply(X, self.weights, op)
-        if relu_input:
-            X = torch.relu(X)
-        return GINFunction.apply(X, self.weights, op)
+            return GINReLUInputFunction, op
+        return GINFunction if op.vec_size == 1 or (op.vec_size == 2 and rows % 2 == 0) else _GINOnOperator, op
+
+
+# kinds of ParamSpCONV.network_loss
+_NETWORK_KIND = {GCNFunction: 0, GCNAggregateFirstFunction: 1, GINFunction: 1, GCNReLUInputFunction: 2, GINReLUInputFunction: 3}
+
+
+def network_loss(convs, spmm_dict, x, labels):
+    """Layers ``convs`` with ReLU between them on ``x``, log-softmax and mean NLL loss as one autograd node, or None where
+    some part of it has to run by itself: subclasses and layers with hooks, operators a layer's native form does not take,
+    losses softmax_nll_loss_mean leaves to PyTorch."""
+    if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and labels.is_cuda and labels.dtype == torch.int64
+            and labels.dim() == 1 and labels.is_contiguous() and not _module._has_any_global_hook()):
+        return None
+    kinds, ops, weights = [], [], []
+    for conv in convs:
+        w = conv.weights
+        if (type(conv) not in (GCNConv, GINConv) or conv._forward_hooks or conv._forward_pre_hooks or conv._backward_hooks
+                or conv._backward_pre_hooks or "forward" in conv.__dict__ or w.dtype != torch.float32):
+            return None
+        fn, op = conv.choose(x.shape[0], spmm_dict, bool(kinds))
+        kind = _NETWORK_KIND.get(fn)
+        if kind is None or (kinds and kind < 2):
+            return None
+        kinds.append(kind)
+        ops.append(_native(op))
+        weights.append(w)
+    if not SpCONV.softmax_nll_supported(w.shape[1]):
+        return None
+    return SpCONV.network_loss(kinds, ops, x, weights, labels)
