@@ -467,7 +467,7 @@ int psp_sum_partials_f32(const psp_partial_sum *sums, int n, psp_stream_t stream
 /* ---------------------------------------------------------------------------------------------
  * DEVICE: both gradients of a layer relu(Z) W in one launch, from the gradient G[n,K2] of its product: dZ[n,K1] = (G W^T)
  * where Z > 0, dW[K1,K2] = max(Z, 0)^T G, W[K1,K2] row-major; n > 0, G, Z and dZ 16-byte aligned, widths:
- * psp_dense_grad_supported (multiples of 16 up to 64).  Workspace and dW null as in psp_gemm_atb_ws_act_f32. */
+ * psp_dense_grad_supported (multiples of 16, K1 K2 up to about 80 x 80).  Workspace and dW null as in psp_gemm_atb_ws_act_f32. */
 int psp_dense_grad_supported(int K1, int K2);
 long long psp_dense_grad_workspace_floats(long long n, int K1, int K2);
 int psp_dense_grad_f32(const float *G, const float *Z, const float *W, float *dZ, float *dW, long long n, int K1, int K2,

@@ -3,22 +3,27 @@
 // in one launch.  The two products read the same two matrices; as launches of their own (dense_xw.hip, dense_atb.hip) they
 // read them twice, and on a graph of 10^4 rows each costs its 3-4 us of launch and latency whatever it does.
 // HBM-bound: 4 n (2 K1 + K2) bytes.  Both products, one after the other -> this kernel, with the sum of the partial products:
-// 20 K rows 16 x 16 13.5 -> 8.2 us, 10^6 rows 16 x 16 54 -> 37, 48 x 48 197 -> 155, 64 x 64 302 -> 215 (memory: 160).
+// 20 K rows 16 x 16 13.5 -> 8.2 us, 10^6 rows 16 x 16 54 -> 37, 48 x 48 197 -> 150, 64 x 64 302 -> 212
+// (memory: 160), 128 x 16 355 -> 249 (227).
 #include "psp_common.h"
 #include "dense_tiles.h"
 
-// A wavefront takes 32 rows at a time and loads them twice, in the layouts of the two products (both are described in the
+// A wavefront takes 16 rows at a time and loads them twice, in the layouts of the two products (both are described in the
 // files named above): the second load of a row follows the first at once and finds it in the CU's L1 or the L2.  Everything a
-// block needs is requested before its first MFMA; two to four workgroups per CU (as many as the registers allow) keep the
-// memory busy while others multiply.  The workgroups' parts of dW go to `partial` (K1 x K2 each) and are added afterwards in a fixed order.
+// step needs is requested before its first MFMA; as many workgroups per CU as the registers allow keep the memory busy while
+// others multiply.  Steps of 32 rows keep fewer of them: 10^6 rows 48 x 48 155 us against 150, 64 x 64 215 against 212, 200 K rows
+// 64 x 64 58 against 52; only at 16 x 16, where the registers do not limit, they are faster (37 against 43).
+// The workgroups' parts of dW go to `partial` (K1 x K2 each) and are added afterwards in a fixed order.
 // n > 0; rows past n are loaded from row n - 1, enter dW as zeros and are not stored.
-constexpr int psp_dense_grad_wgs(int K1, int K2) { return K1 + K2 <= 48 ? 4 : K1 + K2 <= 64 ? 3 : 2; }  // per CU
+constexpr int psp_dense_grad_wgs(int K1, int K2) { return K1 + K2 > 144 ? 2 : K1 + K2 > 80 ? 3 : 4; }  // per CU
+constexpr int psp_dense_grad_halves(int K1, int K2) { return K1 + K2 <= 32 ? 2 : 1; }  // 16 rows each, per step
 template <int K1, int K2>
 __global__ void __launch_bounds__(256, psp_dense_grad_wgs(K1, K2))
 psp_dense_grad_kernel(const float *__restrict__ G, const float *__restrict__ Z, const float *__restrict__ W,
                       float *__restrict__ dZ, float *__restrict__ partial, long long n, long long nblocks)
 {
     constexpr int RM = K1 / 16, RN = K2 / 16;  // column tiles of Z and of G
+    constexpr int H = psp_dense_grad_halves(K1, K2), U = 4 * H;
     constexpr int TQ = (RM + 3) / 4;
     constexpr int S = XWW_STRIDE(K1);
     constexpr int LDS = K2 * S > RM * RN * 256 ? K2 * S : RM * RN * 256;
@@ -39,12 +44,12 @@ psp_dense_grad_kernel(const float *__restrict__ G, const float *__restrict__ Z, 
         for (int t = 0; t < RN; t++) dw[m][t] = psp_mfma_acc{0.f, 0.f, 0.f, 0.f};
 
     for (long long blk = (long long)blockIdx.x * 4 + w; blk < nblocks; blk += (long long)gridDim.x * 4) {
-        const long long row0 = blk * 32;
-        const bool whole = row0 + 32 <= n;
-        psp_f32x4 g4[2][RN], z4[2][RM];     // of row 16 h + r: columns 16 t + 4 q ..
-        float az[8][RM], bg[8][RN];         // of row 4 u + q: psp_atb_col of r
+        const long long row0 = blk * (16 * H);
+        const bool whole = row0 + 16 * H <= n;
+        psp_f32x4 g4[H][RN], z4[H][RM];     // of row 16 h + r: columns 16 t + 4 q ..
+        float az[U][RM], bg[U][RN];         // of row 4 u + q: psp_atb_col of r
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < H; h++) {
             const long long row = min(row0 + 16 * h + r, n - 1);
 #pragma unroll
             for (int t = 0; t < RN; t++) g4[h][t] = ((const psp_f32x4 *)(G + row * K2) + q)[4 * t];
@@ -52,16 +57,16 @@ psp_dense_grad_kernel(const float *__restrict__ G, const float *__restrict__ Z, 
             for (int t = 0; t < RM; t++) z4[h][t] = ((const psp_f32x4 *)(Z + row * K1) + q)[4 * t];
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < U; u++) {
             const long long row = min(row0 + 4 * u + q, n - 1);
             psp_atb_load_row<RM>(Z + row * K1, r, az[u]);
             psp_atb_load_row<RN>(G + row * K2, r, bg[u]);
         }
         __builtin_amdgcn_sched_barrier(0);  // the loads stay in front of the products
 
-        psp_mfma_acc acc[2][RM];
+        psp_mfma_acc acc[H][RM];
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+        for (int h = 0; h < H; h++)
 #pragma unroll
             for (int j = 0; j < RM; j++) acc[h][j] = psp_mfma_acc{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -75,11 +80,11 @@ psp_dense_grad_kernel(const float *__restrict__ G, const float *__restrict__ Z, 
 #pragma unroll
                 for (int j = 0; j < RM; j++)
 #pragma unroll
-                    for (int h = 0; h < 2; h++)
+                    for (int h = 0; h < H; h++)
                         acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[j / 4][j % 4], g4[h][t][e], acc[h][j], 0, 0, 0);
             }
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < H; h++) {
             const long long row = row0 + 16 * h + r;
             if (row >= n) continue;
             psp_f32x4 *out = (psp_f32x4 *)(dZ + row * K1) + q;
@@ -92,7 +97,7 @@ psp_dense_grad_kernel(const float *__restrict__ G, const float *__restrict__ Z, 
             }
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < U; u++) {
             const bool in = whole || row0 + 4 * u + q < n;
 #pragma unroll
             for (int m = 0; m < RM; m++) az[u][m] = !in || az[u][m] < 0.0f ? 0.0f : az[u][m];  // NaN stays NaN
@@ -128,20 +133,25 @@ psp_dense_grad_kernel(const float *__restrict__ G, const float *__restrict__ Z, 
 
 typedef void (*psp_dense_grad_kernel_t)(const float *, const float *, const float *, float *, float *, long long, long long);
 
-// Widths up to 64: there the two products' matrix-core time stays below the memory time of one of them.
+// Up to 25 tiles, K1 K2 <= 80 x 80: the accumulators of 96 x 96 leave one wavefront per SIMD, and the two fp32 products need as
+// long on the matrix cores as the memory system for the rows (10^6 rows 478 us as two launches, 416 as one; 200 K rows 114, 120).
 static psp_dense_grad_kernel_t dense_grad_lookup(int K1, int K2)
 {
 #define DG(a, b) \
     if (K1 == a && K2 == b) return psp_dense_grad_kernel<a, b>;
-#define DG_ROW(a) DG(a, 16) DG(a, 32) DG(a, 48) DG(a, 64)
-    DG_ROW(16) DG_ROW(32) DG_ROW(48) DG_ROW(64)
+#define DG_ROW(a) DG(a, 16) DG(a, 32) DG(a, 48)
+    DG_ROW(16) DG_ROW(32) DG_ROW(48) DG_ROW(64) DG_ROW(80) DG_ROW(96) DG_ROW(112) DG_ROW(128)
+#define DG_WIDE(a) DG(a, 64) DG(a, 80)
+    DG_WIDE(16) DG_WIDE(32) DG_WIDE(48) DG_WIDE(64) DG_WIDE(80)
+    DG(96, 64) DG(16, 96) DG(16, 112) DG(16, 128) DG(32, 96) DG(32, 112) DG(32, 128) DG(48, 96) DG(48, 112) DG(48, 128) DG(64, 96)
+#undef DG_WIDE
 #undef DG_ROW
 #undef DG
     return nullptr;
 }
 static long long dense_grad_grid(long long n, int K1, int K2)
 {
-    const long long wgs = (n + 127) / 128, most = 256 * psp_dense_grad_wgs(K1, K2);
+    const long long wgs = (n + 63) / 64, most = 256 * psp_dense_grad_wgs(K1, K2);
     return wgs < most ? wgs : most;
 }
 
@@ -160,9 +170,9 @@ PSP_EXPORT int psp_dense_grad_f32(const float *G, const float *Z, const float *W
     PSP_REQUIRE(n > 0 && G && Z && W && dZ && workspace, "dense_grad: null pointer or no rows");
     PSP_REQUIRE((((size_t)G | (size_t)Z | (size_t)dZ) & 15) == 0, "dense_grad: G, Z and dZ must be 16-byte aligned");
     PSP_REQUIRE(n / 128 < 0x7fffffffLL, "dense_grad: too many rows");
-    const long long grid = dense_grad_grid(n, K1, K2);
+    const long long grid = dense_grad_grid(n, K1, K2), rows = 16 * psp_dense_grad_halves(K1, K2);
     PSP_REQUIRE(workspace_floats >= grid * K1 * K2, "dense_grad: the workspace holds %lld floats, %lld needed", workspace_floats, grid * K1 * K2);
-    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, G, Z, W, dZ, workspace, n, (n + 31) / 32);
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, G, Z, W, dZ, workspace, n, (n + rows - 1) / rows);
     const int rc = psp_check_launch("dense_grad kernel");
     if (rc != PSP_OK) return rc;
     if (!dW) return (int)grid;

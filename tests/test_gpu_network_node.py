@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n", [1024, 1025, 1055, 4097, 140000])
-@pytest.mark.parametrize("k1,k2", [(16, 16), (16, 48), (32, 32), (48, 16), (64, 32), (64, 64)])
+@pytest.mark.parametrize("k1,k2", [(16, 16), (16, 48), (32, 32), (48, 16), (64, 32), (64, 64), (80, 80), (128, 16), (16, 128)])
 def test_dense_grads_of_one_kernel(n, k1, k2):
     import paramspmm_ae_amd  # noqa: F401
     import ParamSpCONV as S
