@@ -533,9 +533,18 @@ struct LayerNode : torch::autograd::Node {
     bool wants(size_t i) { return task_should_compute_output(i); }
 };
 
+// The nodes have no forward-mode derivative.  What runs inside with_node is out of autograd's sight, so a tangent would be
+// dropped, which says that the derivative is zero: refused as an autograd.Function without a jvp refuses it.
+static void refuse_tangents(at::ArrayRef<Tensor> inputs)
+{
+    for (const Tensor &t : inputs)
+        TORCH_CHECK_NOT_IMPLEMENTED(!t._fw_grad(0).defined(), "ParamSpCONV: the layers and losses have no forward-mode derivative");
+}
+
 // the result of `forward` (run without recording), with a node of type N behind it when an input asks for gradients
 template <class N, class F> static Tensor with_node(const op_t &op, at::ArrayRef<Tensor> inputs, F forward)
 {
+    refuse_tangents(inputs);
     const bool record = torch::GradMode::is_enabled() &&
                         std::any_of(inputs.begin(), inputs.end(), [](const Tensor &t) { return t.requires_grad(); });
     std::shared_ptr<N> node;

@@ -1,0 +1,71 @@
+"""What a layer or a loss does under autograd modes that its native node does not serve: it says so, and never returns a result
+whose derivative is silently missing."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fwd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def graph():
+    from paramspmm_ae_amd import synth
+    from paramspmm_ae_amd.graph_input import graph_input
+
+    r, c, n = synth.sbm(1200, 20, 6, 2, seed=5)
+    g = graph_input("g", "")
+    g.verbose = False
+    return g.load_from_csr(*synth.to_gcn_csr(r, c, n)[:3], if_mask=True)
+
+
+def _ops(graph, window=False):
+    from paramspmm_ae_amd.PCSR import pcsr_spmm
+
+    op = pcsr_spmm(graph=graph, vec_size=1, if_split=False, CF=0 if window else 1, window=window)
+    return {d: op for d in (16, 32)}
+
+
+def _layers(graph, window):
+    """(name, function of one tensor, that tensor): every layer and loss, as a function of its input and of its weights"""
+    from paramspmm_ae_amd import gnn_conv as G
+
+    ops, n = _ops(graph, window), graph.mtx_nodes
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    X, W, aw = (torch.randn(*s, device="cuda", generator=gen) for s in ((n, 16), (16, 16), (1, 1)))
+    labels = torch.randint(0, 16, (n,), device="cuda", generator=gen)
+    col = graph.csr_data.on_device("colIdx", "cuda").unsqueeze(-1)
+    for f in (G.GCNFunction, G.GCNAggregateFirstFunction, G.GCNReLUInputFunction, G.GINFunction, G.GINReLUInputFunction):
+        yield f.__name__, lambda x, f=f: f.apply(x, W, ops[16]), X
+        yield f.__name__ + " weights", lambda w, f=f: f.apply(X, w, ops[16]), W
+    for relu in (False, True):
+        yield "AGNN", lambda x: G.AGNNFunction.apply(x, W, aw, ops[16], col, relu), X
+        yield "AGNN weights", lambda w: G.AGNNFunction.apply(X, w, aw, ops[16], col, relu), W
+        yield "AGNN attention weight", lambda a: G.AGNNFunction.apply(X, W, a, ops[16], col, relu), aw
+    yield "nll", lambda x: G.nll_loss_mean(x, labels), torch.log_softmax(X, 1)
+    yield "softmax nll", lambda x: G.softmax_nll_loss_mean(x, labels), X
+
+
+@pytest.mark.parametrize("window", [False, True])
+def test_tangents_are_refused(graph, window):
+    for name, f, at in _layers(graph, window):
+        print("case", name, flush=True)
+        f(at)
+        with fwd.dual_level():
+            for record in (False, True):
+                with torch.set_grad_enabled(record), pytest.raises(NotImplementedError):
+                    f(fwd.make_dual(at, torch.ones_like(at)))
+            f(at)  # no tangent: as outside
+
+
+def test_tangent_of_a_whole_network_is_refused(graph):
+    from paramspmm_ae_amd import GNN
+
+    model = GNN.build_model("GCN", graph, _ops(graph), 16, 32, 16)
+    labels = torch.randint(0, 16, graph.y.shape, device="cuda")
+    x = model.x
+    with fwd.dual_level():
+        model.x = fwd.make_dual(x, torch.ones_like(x))
+        with pytest.raises(NotImplementedError):
+            GNN.loss_of_step(model, labels)
+    model.x = x
+    GNN.loss_of_step(model, labels).backward()
