@@ -76,6 +76,14 @@ static int ok_count(int rc)
     return rc;
 }
 
+// The rows of a dense kernel's operand.  Those kernels read 16 bytes at a time and their entry points refuse other starts; a
+// contiguous view into a flat buffer may start on any element and is copied.
+static Tensor rows16(const Tensor &t)
+{
+    Tensor c = t.contiguous();
+    return (reinterpret_cast<uintptr_t>(c.const_data_ptr()) & 15) == 0 ? c : c.clone();
+}
+
 // H^T * AG.  For narrow layers the product is a reduction over ~10^6 rows into a tiny matrix, which the library
 // streams at memory speed; everything else goes to torch::mm.
 static Tensor weight_gradient(const Tensor &H, const Tensor &AG, PartialSums *sums = nullptr, bool relu = false)
@@ -84,7 +92,7 @@ static Tensor weight_gradient(const Tensor &H, const Tensor &AG, PartialSums *su
                         H.scalar_type() == torch::kFloat32 && AG.scalar_type() == torch::kFloat32 &&
                         psp_gemm_atb_supported((int)H.size(1), (int)AG.size(1));
     if (!narrow) return torch::mm((relu ? torch::relu(H) : H).t(), AG);
-    Tensor Hc = H.contiguous(), Gc = AG.contiguous();
+    Tensor Hc = rows16(H), Gc = rows16(AG);
     DeviceGuard guard(Hc.device());
     Tensor dW = torch::empty({Hc.size(1), Gc.size(1)}, Hc.options());
     // partial products of the workgroups go through a workspace and are added in a fixed order (no atomics)
@@ -106,7 +114,7 @@ static Tensor dense_xw(const Tensor &X, const Tensor &W, bool transW, Order orde
                         W.scalar_type() == torch::kFloat32 && X.is_cuda() && W.is_cuda() &&
                         psp_gemm_xw_supported((int)K1, (int)K2) && (order == Order::any || kept_order_is_ours(X.size(0), K1, K2));
     if (!narrow) return torch::mm(X, transW ? W.t() : W);
-    Tensor Xc = X.contiguous(), Wc = W.contiguous();
+    Tensor Xc = rows16(X), Wc = W.contiguous();
     DeviceGuard guard(Xc.device());
     Tensor Y = torch::empty({Xc.size(0), K2}, Xc.options());
     ok(psp_gemm_xw_f32(fp(Xc), fp(Wc), fpw(Y), Xc.size(0), (int)K1, (int)K2, transW ? 1 : 0, stream_of(Xc)));
@@ -123,7 +131,7 @@ static Tensor dense_relu_xw(const Tensor &Z, const Tensor &W, Order order)
                         psp_gemm_xw_supported((int)K1, (int)W.size(1)) &&
                         (order == Order::any || kept_order_is_ours(Z.size(0), K1, W.size(1)));
     if (!narrow) return torch::mm(torch::relu(Z), W);
-    Tensor Zc = Z.contiguous(), Wc = W.contiguous();
+    Tensor Zc = rows16(Z), Wc = W.contiguous();
     DeviceGuard guard(Zc.device());
     Tensor Y = torch::empty({Zc.size(0), Wc.size(1)}, Zc.options());
     ok(psp_gemm_xw_act_f32(fp(Zc), fp(Wc), fpw(Y), Zc.size(0), (int)K1, (int)Wc.size(1), 0, 1, nullptr, stream_of(Zc)));
@@ -138,7 +146,7 @@ static Tensor dense_xwt_masked(const Tensor &AG, const Tensor &W, const Tensor &
     const bool narrow = shapes && AG.size(0) >= kDenseRows && AG.scalar_type() == torch::kFloat32 && W.scalar_type() == torch::kFloat32 &&
                         Z.scalar_type() == torch::kFloat32 && psp_gemm_xw_supported((int)K1, (int)W.size(0));
     if (!narrow) return at::threshold_backward(torch::mm(AG, W.t()), Z, 0);  // what F.relu's backward runs
-    Tensor Gc = AG.contiguous(), Wc = W.contiguous(), Zc = Z.contiguous();
+    Tensor Gc = rows16(AG), Wc = W.contiguous(), Zc = rows16(Z);
     DeviceGuard guard(Gc.device());
     Tensor Y = torch::empty({Gc.size(0), Wc.size(0)}, Gc.options());
     ok(psp_gemm_xw_act_f32(fp(Gc), fp(Wc), fpw(Y), Gc.size(0), (int)K1, (int)Wc.size(0), 1, 0, fp(Zc), stream_of(Gc)));
@@ -157,7 +165,7 @@ static std::pair<Tensor, Tensor> dense_grads_relu(const Tensor &AG, const Tensor
                       W.scalar_type() == torch::kFloat32 && Z.scalar_type() == torch::kFloat32 &&
                       psp_dense_grad_supported((int)W.size(0), (int)W.size(1));
     if (!pair) return {dense_xwt_masked(AG, W, Z), weight_gradient_relu(Z, AG, sums)};
-    Tensor Gc = AG.contiguous(), Wc = W.contiguous(), Zc = Z.contiguous();
+    Tensor Gc = rows16(AG), Wc = W.contiguous(), Zc = rows16(Z);
     DeviceGuard guard(Gc.device());
     const int K1 = (int)Wc.size(0), K2 = (int)Wc.size(1);
     Tensor dZ = torch::empty_like(Zc), dW = torch::empty_like(Wc);
@@ -287,7 +295,7 @@ static bool window_grad_supported(const Tensor &G, const Tensor &Z, bool dense)
 static std::vector<Tensor> window_grad(Tensor G, Tensor Z, bool relu_z, const Tensor *W, bool want_ag, Tensor rowPtr_w, Tensor colIdx_w,
                                        Tensor values_w, PartialSums &sums)
 {
-    Tensor Gc = G.contiguous(), Zc = Z.contiguous(), Wc;
+    Tensor Gc = rows16(G), Zc = rows16(Z), Wc;
     check_spmm_args(4, Gc, rowPtr_w, colIdx_w, values_w, nullptr);
     pspglue::same_device(Gc, Zc, "window_grad");
     if (W) {
