@@ -107,7 +107,8 @@ int psp_spmm_register_sets(int unroll, int lanes_per_row);
  *                      order, which is the summation order of the reference's one-warp-per-row kernels
  *                      (SpMM/SpMM_kernel.cu:1157-1212, 1362-1440): results repeat the sequential chain bit for bit.
  *                      Default 0: rows may be cut between lane groups and summed piecewise (faster on skewed rows).
- *   "dense_split"      1 (default): the dense layer products (the gemm_xw and gemm_atb entry points) at 128 x 128 form
+ *   "dense_split"      1 (default): the dense layer products (the gemm_xw and gemm_atb entry points) at 128 x 128 and
+ *                      from 16384 rows on form
  *                      every fp32 product from the three bf16 terms of each operand (six bf16 matrix-core products,
  *                      fp32 accumulation: error 2^-23 of |x||w| per product, the rounding level of fp32) and are
  *                      bound by their memory traffic; an infinite input (or one within a bf16 rounding step of

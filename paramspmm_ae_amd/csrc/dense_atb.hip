@@ -360,7 +360,7 @@ static int atb_atomic(const float *A, const float *B, float *C, long long n, int
     int rc = psp_zero_f32(C, (size_t)K1 * K2, stream);
     if (rc != PSP_OK || n == 0) return rc;
     long long wgs = atb_mfma_grid(n, jsplit, K1 * K2);
-    if (K1 == 128 && K2 == 128 && psp_opts().dense_split) {
+    if (K1 == 128 && K2 == 128 && n >= PSP_SPLIT_MIN_ROWS && psp_opts().dense_split) {
         km = relu_a ? psp_atb_split_kernel<true> : psp_atb_split_kernel<false>;
         wgs = wgs < ATB_SPLIT_WGS ? wgs : ATB_SPLIT_WGS;
     }
@@ -391,7 +391,7 @@ PSP_EXPORT int psp_gemm_atb_ws_act_f32(const float *A, const float *B, float *C,
     long long wgs = atb_mfma_grid(n, jsplit, K1 * K2);
     PSP_REQUIRE(workspace && workspace_floats >= wgs * K1 * K2, "gemm_atb_ws: the workspace holds %lld floats, %lld needed",
                 workspace_floats, wgs * K1 * K2);
-    if (K1 == 128 && K2 == 128 && psp_opts().dense_split) {
+    if (K1 == 128 && K2 == 128 && n >= PSP_SPLIT_MIN_ROWS && psp_opts().dense_split) {
         km = relu_a ? psp_atb_split_kernel<true> : psp_atb_split_kernel<false>;
         wgs = wgs < ATB_SPLIT_WGS ? wgs : ATB_SPLIT_WGS;  // (uses the first slots of the workspace)
     }

@@ -360,7 +360,7 @@ PSP_EXPORT int psp_gemm_xw_act_f32(const float *X, const float *W, float *Y, lon
     PSP_REQUIRE((((size_t)X | (size_t)Y | (size_t)mask) & 15) == 0, "gemm_xw: X, Y and mask must be 16-byte aligned");
     PSP_REQUIRE((n + 255) / 256 <= 0x7fffffffLL, "gemm_xw: too many rows");
     const long long nblocks = (n + XWW_ROWS - 1) / XWW_ROWS;
-    if (K1 == 128 && K2 == 128 && psp_opts().dense_split) {
+    if (K1 == 128 && K2 == 128 && n >= PSP_SPLIT_MIN_ROWS && psp_opts().dense_split) {
         psp_xw_kernel_t ks = mask ? psp_xw_split_kernel<false, true>
                                        : (relu_x ? psp_xw_split_kernel<true, false> : psp_xw_split_kernel<false, false>);
         const int lds = (K1 / 32) * (K2 / 16) * 3 * 64 * 16;  // 96 KB: one workgroup of eight wavefronts per CU

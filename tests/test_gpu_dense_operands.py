@@ -64,3 +64,31 @@ def test_first_layer_on_a_windowed_operator_takes_an_unaligned_input(k1, k2):
     for a in got[1:]:
         for x, y in zip(a, got[0]):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("n", [1024, 4097, 16383, 16384])
+def test_128_wide_products_of_few_rows_are_plain_fp32(n):
+    """Below 16384 rows: no larger an error than PyTorch's fp32 product allows, and infinities as IEEE arithmetic has them (the
+    bf16 split of 16384 rows and more gives NaN there)."""
+    import paramspmm_ae_amd  # noqa: F401
+    import ParamSpCONV as S
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    Z, G, W = (torch.randn(*s, device="cuda", generator=gen) for s in ((n, 128), (n, 128), (128, 128)))
+    Zd, Gd, Wd = (t.cpu().double() for t in (Z, G, W))
+    for got, want, size, terms in ((S.dense_relu_xw(Z, W), Zd.relu() @ Wd, Zd.relu() @ Wd.abs(), 128),
+                                   (S.dense_xw(G, W, True), Gd @ Wd.t(), Gd.abs() @ Wd.abs().t(), 128),
+                                   (S.dense_xwt_masked(G, W, Z), (Gd @ Wd.t()) * (Zd > 0), Gd.abs() @ Wd.abs().t(), 128),
+                                   (S.weight_gradient(Z, G), Zd.t() @ Gd, Zd.abs().t() @ Gd.abs(), n),
+                                   (S.weight_gradient_relu(Z, G), Zd.relu().t() @ Gd, Zd.relu().t() @ Gd.abs(), n)):
+        # a sum of m terms has at most m roundings of 2^-24 of the terms' sizes; they are random, so some ten sqrt(m) bound it
+        assert bool(((got.cpu().double() - want).abs() <= 10 * terms ** 0.5 * 2.0 ** -24 * size).all())
+    if n >= 16384:
+        return
+    G[5, 3] = float("inf")
+    for got, want in ((S.dense_xw(G, W, True), G.cpu() @ W.cpu().t()),
+                      (S.weight_gradient(Z, G), Z.cpu().t() @ G.cpu()),
+                      (S.dense_xwt_masked(G, W, Z), torch.where(Z.cpu() > 0, G.cpu() @ W.cpu().t(), 0.0))):
+        got = got.cpu()
+        assert bool(want.isinf().any()) and not bool(want.isnan().any())
+        assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[want.isinf()], want[want.isinf()]) and not bool(got.isnan().any())
