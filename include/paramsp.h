@@ -259,7 +259,9 @@ int psp_spmm_vec_split_f32(const int *rowPtr_bs, const int *colIdx_b, const floa
  *   relu_x != 0: Y = A * max(X, 0) -- the product reads the previous layer's output through the ReLU, applied to the
  *   rows as they are gathered (no activated copy of X is written);
  *   mask != NULL ([rows_out, N], 16-byte aligned like Y): Y = (A * X) where mask > 0, else 0 -- the gradient with respect
- *   to the pre-activation values a layer was given; a pass over Y that follows the product on the same stream. */
+ *   to the pre-activation values a layer was given; a pass over Y that follows the product on the same stream.  Here and
+ *   wherever this file says "where mask > 0" or "where Z > 0", an element is zeroed where the mask is at most 0: one that
+ *   is not a number lets the gradient pass, as F.relu's backward does. */
 int psp_spmm_act_f32(int fmt, const int *rowPtr, const int *colIdx, const float *val, const int *target_row,
                      const float *X, float *Y, int nseg, int N, int rows_out, int CF, int blkWarpNum, int relu_x,
                      const float *mask, psp_stream_t stream);

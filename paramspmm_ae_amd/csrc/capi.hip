@@ -844,7 +844,7 @@ PSP_EXPORT int psp_spmm_vec_split_f32(const int *rowPtr_bs, const int *colIdx_b,
                                     (hipStream_t)stream, nullptr, nullptr);
 }
 
-// Y[i] = Y[i] where mask[i] > 0, else 0 (float4 pieces; n a multiple of 4 is not required)
+// Y[i] = 0 where mask[i] <= 0 (float4 pieces; n a multiple of 4 is not required)
 __global__ void __launch_bounds__(256) psp_mask_kernel(float *__restrict__ Y, const float *__restrict__ mask, size_t n)
 {
     const size_t n4 = n / 4;
@@ -852,11 +852,11 @@ __global__ void __launch_bounds__(256) psp_mask_kernel(float *__restrict__ Y, co
         psp_f32x4 y = ((const psp_f32x4 *)Y)[i];
         const psp_f32x4 m = __builtin_nontemporal_load((const psp_f32x4 *)mask + i);
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = m[e] > 0.0f ? y[e] : 0.0f;
+        for (int e = 0; e < 4; e++) y[e] = psp_relu_grad(y[e], m[e]);
         ((psp_f32x4 *)Y)[i] = y;
     }
     const size_t t = n4 * 4 + (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) Y[t] = mask[t] > 0.0f ? Y[t] : 0.0f;
+    if (t < n) Y[t] = psp_relu_grad(Y[t], mask[t]);
 }
 
 PSP_EXPORT int psp_spmm_act_f32(int fmt, const int *rowPtr, const int *colIdx, const float *val, const int *target_row,

@@ -92,7 +92,7 @@ psp_dense_grad_kernel(const float *__restrict__ G, const float *__restrict__ Z, 
             for (int j = 0; j < RM; j++) {
                 psp_f32x4 o = acc[h][j];
 #pragma unroll
-                for (int c = 0; c < 4; c++) o[c] = z4[h][j][c] > 0.0f ? o[c] : 0.0f;
+                for (int c = 0; c < 4; c++) o[c] = psp_relu_grad(o[c], z4[h][j][c]);
                 out[4 * j] = o;
             }
         }

@@ -153,7 +153,7 @@ psp_xw_kernel(const float *__restrict__ X, const float *__restrict__ W, float *_
                 if constexpr (MASK) {
                     const psp_f32x4 m = mr[4 * j];
 #pragma unroll
-                    for (int c = 0; c < 4; c++) o[c] = m[c] > 0.0f ? o[c] : 0.0f;
+                    for (int c = 0; c < 4; c++) o[c] = psp_relu_grad(o[c], m[c]);
                 }
                 yr[4 * j] = o;
             }
@@ -290,7 +290,7 @@ psp_xw_split_kernel(const float *__restrict__ X, const float *__restrict__ W, fl
                 if constexpr (MASK) {
                     const psp_f32x4 m = mr[4 * j];
 #pragma unroll
-                    for (int c = 0; c < 4; c++) o[c] = m[c] > 0.0f ? o[c] : 0.0f;
+                    for (int c = 0; c < 4; c++) o[c] = psp_relu_grad(o[c], m[c]);
                 }
                 yr[4 * j] = o;
             }

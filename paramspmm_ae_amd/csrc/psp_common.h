@@ -75,6 +75,9 @@ int psp_row_scale(float *Y, const float *s, int rows, int N, hipStream_t stream)
 #define PSP_F32_LOWEST (-3.402823466e+38f)
 
 #ifdef __HIPCC__
+// Gradient of max(z, 0) applied to g: zero where z <= 0, and where z is not a number the gradient passes, as F.relu's does.
+__device__ __forceinline__ float psp_relu_grad(float g, float z) { return z <= 0.0f ? 0.0f : g; }
+
 // float maximum through the integer atomics: the order of non-negative floats is that of their bit patterns read
 // as signed integers, the order of negative floats is the reverse of their patterns read as unsigned
 __device__ __forceinline__ void psp_atomic_max_f32(float *addr, float v)

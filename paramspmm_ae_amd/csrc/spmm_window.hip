@@ -399,7 +399,7 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
                             const size_t at = (size_t)oat * (size_t)N + 16 * h + 4 * mq;
                             const psp_f32x4 mk = *(const psp_f32x4 *)(s_z + orow * ZS + 16 * h + 4 * mq);
 #pragma unroll
-                            for (int e = 0; e < 4; e++) o[h][e] = mk[e] > 0.0f ? o[h][e] : 0.0f;
+                            for (int e = 0; e < 4; e++) o[h][e] = psp_relu_grad(o[h][e], mk[e]);
                             __builtin_nontemporal_store(o[h], (psp_f32x4 *)(Y + at));
                         }
                     }
@@ -437,7 +437,7 @@ psp_spmm_window_kernel(const int *__restrict__ rowPtr_w, const int *__restrict__
                     if (KZ == 0 && mask) {
                         const psp_f32x4 mk = *(const psp_f32x4 *)(mask + at);
 #pragma unroll
-                        for (int e = 0; e < 4; e++) y[e] = mk[e] > 0.0f ? y[e] : 0.0f;
+                        for (int e = 0; e < 4; e++) y[e] = psp_relu_grad(y[e], mk[e]);
                     }
                     __builtin_nontemporal_store(y, (psp_f32x4 *)(Y + at));
                 }
