@@ -56,13 +56,13 @@ def _slot_columns(op, colIdx):
 
 
 def _native(op, slots=None):
-    """The operator as the extension module's layers take it; made once, and again when one of its attributes changes."""
+    """The operator as the extension module's layers take it; made once, and again when anything it is made of changes."""
+    arrays = (_row_ptr(op), op.colIdx, op.val, op.target_row if op.if_split else None)
+    numbers = (_fmt(op), op.CF, _bw(op), getattr(op, "fold_dense", True))
     k = op.__dict__.get("_native_operator")
-    bw, fold = _bw(op), getattr(op, "fold_dense", True)
-    if (k is None or k[0] is not op.rowPtr or k[1] is not op.colIdx or k[2] is not op.val or k[3] is not op.target_row
-            or k[4] != op.CF or k[5] != bw or k[6] != fold or k[7] is not slots):
-        native = SpCONV.Operator(_fmt(op), _row_ptr(op), op.colIdx, op.val, op.target_row if op.if_split else None, op.CF, bw, fold, slots)
-        k = op._native_operator = (op.rowPtr, op.colIdx, op.val, op.target_row, op.CF, bw, fold, slots, native)
+    if k is None or k[1] != numbers or k[2] is not slots or any(a is not b for a, b in zip(k[0], arrays)):
+        native = SpCONV.Operator(numbers[0], *arrays, *numbers[1:], slots)
+        k = op._native_operator = (arrays, numbers, slots, native)
     return k[-1]
 
 
