@@ -396,8 +396,8 @@ int psp_attn_window_backward_f32(const int *rowPtr_w, const int *colIdx_w, const
  * those of the format's SpMM), any K from 4 to PSP_ATTN_MAX_K, no alignment beyond that of a float.
  *   forward:  att in the format's entry order (2x1 blocks: [nblk, 2]; val_b says which entries exist, padding reads zero),
  *             Y[i] = sum_p att[p] X[col(p)].  val_b NULL for fmt 0 / 1.
- *   backward: G as above; *wsum as above for fmt 0 / 1, for 2x1 blocks sum over the slots of <dY[row], dY[col]> slot[p]
- *             (slot [nblk, 2], zero at padding: the reference multiplies the slots of a block-row, in block order, with the
+ *   backward: G as above; *wsum as above for fmt 0 / 1 with slot NULL, else sum over the scores of <dY[row], dY[col]> slot[p]
+ *             (one float per score; for 2x1 blocks, which always take it, [nblk, 2], zero at padding: the reference multiplies the slots of a block-row, in block order, with the
  *             columns of its CSR entries, gnn_conv.py:166-172, so slot[mask[k]] = colIdx_csr[k]).  workspace: psp_attn_workspace_floats(nrows, K) floats
  *             of device memory (nrows = rows, block-rows or segments of the format), whose shares are added to *wsum in a
  *             fixed order.

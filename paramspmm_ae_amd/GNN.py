@@ -247,7 +247,7 @@ def build_model(net, graph, operators, hidden, num_features, num_classes, num_la
     graph.init_feat_embedding(num_features, 2)
     graph.init_labels(num_classes, 2)
     if net == "AGNN":
-        colIdx = graph.csr_data.colIdx.to(device).unsqueeze(-1)
+        colIdx = graph.csr_data.on_device("colIdx", device).unsqueeze(-1)  # the array the operators hold
         return AGNN(num_classes, num_features, graph.x, operators, hidden, colIdx, num_layers).to(device)
     return GIN(num_classes, num_features, graph.x, operators, hidden).to(device)
 

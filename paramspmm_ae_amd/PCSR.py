@@ -182,6 +182,7 @@ class pcsr_spmm(object):
             self.target_row = fmt.on_device("target_row", device) if if_split else None
             if vec_size != 1 and getattr(graph, "mask", None) is not None:
                 self.mask = graph.mask.to(device)
+                self.csr_colIdx = graph.csr_data.on_device("colIdx", device)  # the columns that ``mask`` leads to
         self.vec_size = vec_size
         self.if_split = if_split
         self.CF = CF

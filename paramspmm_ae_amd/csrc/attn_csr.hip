@@ -48,14 +48,14 @@ static psp_spmm_plan attn_plan(int K, int blkWarpNum)
     return p;
 }
 
-template <int NR, bool SPLIT, bool BWD>
+template <int NR, bool SPLIT, bool BWD, bool SLOT>
 static int attn_enqueue(const psp_spmm_plan &p, const int *rowPtr, const int *colIdx, const float *val, const int *target_row,
                         const float *X, float *Y, int nrows, int K, int rows_out, const float *alpha, float *score, float *wsum,
                         const float *slot, hipStream_t st)
 {
 #define PSP_ATTN(LOGL_, C_, U_)                                                                                                   \
     {                                                                                                                             \
-        typedef psp_attention<LOGL_, BWD> xt_t;                                                                                   \
+        typedef psp_attention<LOGL_, BWD, SLOT> xt_t;                                                                             \
         return psp_spmm_enqueue<NR, SPLIT>(psp_spmm_kernel<C_, 4, U_, NR, SPLIT, false, false, true, float, xt_t>, p, rowPtr, colIdx, \
                                            val, target_row, X, Y, nrows, K, rows_out, st, (const float *)nullptr, (float *)nullptr, 0, \
                                            xt_t{alpha, score, wsum, slot});                                                       \
@@ -83,8 +83,9 @@ static int attn_launch(bool bwd, int fmt, const int *rowPtr, const int *colIdx, 
     if (nrows > 0) PSP_REQUIRE(rowPtr && X && (!split || target_row), "attn: null pointer");
     const psp_spmm_plan p = attn_plan(K, blkWarpNum);
 #define PSP_GO(NR_, SPLIT_)                                                                                                  \
-    return bwd ? attn_enqueue<NR_, SPLIT_, true>(p, rowPtr, colIdx, val, target_row, X, Y, nrows, K, rows_out, alpha, score, wsum, slot, st) \
-               : attn_enqueue<NR_, SPLIT_, false>(p, rowPtr, colIdx, val, target_row, X, Y, nrows, K, rows_out, alpha, score, wsum, slot, st)
+    return !bwd ? attn_enqueue<NR_, SPLIT_, false, false>(p, rowPtr, colIdx, val, target_row, X, Y, nrows, K, rows_out, alpha, score, wsum, slot, st) \
+         : NR_ > 1 || slot ? attn_enqueue<NR_, SPLIT_, true, true>(p, rowPtr, colIdx, val, target_row, X, Y, nrows, K, rows_out, alpha, score, wsum, slot, st) \
+                           : attn_enqueue<NR_, SPLIT_, true, (NR_ > 1)>(p, rowPtr, colIdx, val, target_row, X, Y, nrows, K, rows_out, alpha, score, wsum, slot, st)
     if (fmt == 0) PSP_GO(1, false);
     if (fmt == 1) PSP_GO(1, true);
     if (fmt == 2) PSP_GO(2, false);

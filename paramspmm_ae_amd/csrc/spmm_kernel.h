@@ -140,21 +140,23 @@ template <int LOGL> __device__ __forceinline__ float psp_group_sum(float v)
 // What a product does besides multiplying the stored values by the gathered rows (last template argument of the kernel).
 struct psp_plain {
     static constexpr int MODE = 0, LOGL = 0;
+    static constexpr bool SLOT = false;
 };
 // The attention layer of gnn_conv.py:128-180, whose SDDMM and SpMM of a direction gather the same rows of the same matrix:
 // both from one gather.  The whole width lies inside one lane group of 2^LOGL lanes (one column tile).
 //   forward   score[p] = alpha <X_i, X_j> (in every lane of the group after LOGL DPP additions), stored, and Y_i += score[p] X_j.
 //             2x1 blocks: `val` says which entries exist (non-zero); padding scores are zero.
 //   backward  `val` holds the scores: G_i += score[p] dY_j, and every wavefront's share of sum_p <dY_i, dY_j> f(p), the weight
-//             gradient of gnn_conv.py:166-172, lands in wsum[its first segment >> logW].  f(p) = float(j); for 2x1 blocks
-//             slot[p], because the reference pairs the slots of a block-row with the columns of its CSR entries.
+//             gradient of gnn_conv.py:166-172, lands in wsum[its first segment >> logW].  f(p) = slot[p] (SLOT), else float(j).
+//             2x1 blocks always take the slots: the reference pairs the slots of a block-row with the columns of its CSR entries.
 // Every lane group keeps its row i in registers, the next row's is requested one segment ahead.
-template <int LOGL_, bool BACKWARD> struct psp_attention {
+template <int LOGL_, bool BACKWARD, bool SLOT_> struct psp_attention {
     static constexpr int MODE = BACKWARD ? 2 : 1, LOGL = LOGL_;
+    static constexpr bool SLOT = SLOT_;
     const float *alpha;  // forward: one float on the device, null = 1
     float *score;        // forward
     float *wsum;         // backward
-    const float *slot;   // backward, 2x1 blocks: [nblk, 2], zero at padding
+    const float *slot;   // SLOT: one float per score; 2x1 blocks [nblk, 2], zero at padding
 };
 
 // NR: rows per stored entry (1 = CSR, 2 = 2x1 BCSR, 3 = 3x1 blocks: the reference's vec_spmm, SpMM_kernel.cu:1653-1972).  SPLIT: segments carry an explicit output row.
@@ -186,6 +188,8 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
     typedef typename psp_vec<V, T>::type vec_t;
     constexpr int WORDS = sizeof(T) / 4;  // of a stored value
     constexpr bool FWD = XT::MODE == 1, BWD = XT::MODE == 2, ATT = FWD || BWD;
+    static_assert(!XT::SLOT || BWD, "the slots' columns belong to the weight gradient");
+    static_assert(!(BWD && NR > 1) || XT::SLOT, "2x1 blocks take the columns of their slots");
     static_assert(!ATT || (SINGLE && !SM && !ACT && sizeof(T) == 4), "the attention forms run on one register set of floats");
     if constexpr (ATT) logL = XT::LOGL;
     __shared__ int2 s_seg[PSP_MAX_WAVES][PSP_WAVE];  // (end offset, output row) of the wavefront's segments
@@ -570,7 +574,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
             S##_ck[u] = psp_bperm_i(src, c_cur[u]);                                                    \
             _Pragma("unroll") for (int r = 0; r < NR; r++) S##_vk[u][r] = psp_bperm_f(src, v_cur[u][r]); \
         }                                                                                              \
-        if constexpr (BWD && NR > 1) {                                                                 \
+        if constexpr (XT::SLOT) {                                                                      \
             _Pragma("unroll") for (int u = 0; u < U; u++)                                              \
                 _Pragma("unroll") for (int r = 0; r < NR; r++) S##_f[u][r] = xt.slot[(size_t)min(pos + u, b - 1) * NR + r]; \
         }                                                                                              \
@@ -609,7 +613,7 @@ psp_spmm_kernel(const int *__restrict__ rowPtr, const int *__restrict__ colIdx, 
                             S##_vk[u][r] = d;                                                          \
                             if (sub == jb - 1) keep[u][r] = d;                                         \
                         } else {                                                                       \
-                            wsum = __builtin_fmaf(d, NR == 1 ? (float)S##_ck[u] : S##_f[u][r], wsum);  \
+                            wsum = __builtin_fmaf(d, XT::SLOT ? S##_f[u][r] : (float)S##_ck[u], wsum); \
                         }                                                                              \
                     }                                                                                  \
                 }                                                                                      \

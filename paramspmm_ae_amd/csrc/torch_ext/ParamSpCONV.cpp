@@ -404,12 +404,13 @@ static std::vector<Tensor> attn_forward(int fmt, Tensor X, Tensor rowPtr, Tensor
     return {att, Y};
 }
 
-// (fmt, dY, att, rowPtr, colIdx, target_row | None, slot | None, blkWarpNum) -> [G, weight-gradient sum as a 1-element tensor]
+// (fmt, dY, att, rowPtr, colIdx, target_row | None, slot | None, blkWarpNum) -> [G, weight-gradient sum as a 1-element tensor];
+// slot: what each score's dot product is multiplied with (CSR: None for the entry's own column)
 static std::vector<Tensor> attn_backward(int fmt, Tensor dY, Tensor att, Tensor rowPtr, Tensor colIdx, c10::optional<Tensor> target_row,
                                          c10::optional<Tensor> slot, int blkWarpNum)
 {
     const Tensor *tr = target_row ? &*target_row : nullptr;
-    TORCH_CHECK((fmt >= 2) == slot.has_value(), "attn: 2x1 blocks take the columns of their slots, CSR does not");
+    TORCH_CHECK(fmt < 2 || slot.has_value(), "attn: 2x1 blocks take the columns of their slots");
     if (slot) {
         need_gpu(*slot, "slot");
         TORCH_CHECK(slot->scalar_type() == torch::kFloat32 && slot->numel() == att.numel(), "attn: slot has one float32 per score");
@@ -518,7 +519,7 @@ struct Operator {  // what a layer needs of a pcsr_spmm
     c10::optional<Tensor> target_row;
     int CF, bw;
     bool fold_dense;      // windowed csr: fold a square dense product into the sparse kernel where there is one
-    c10::optional<Tensor> slot;  // 2x1 blocks: columns of the slots (attention weight gradient)
+    c10::optional<Tensor> slot;  // attention weight gradient: a column per score, where it is not the entry's own
     const Tensor *tr() const { return target_row ? &*target_row : nullptr; }
 };
 typedef std::shared_ptr<Operator> op_t;

@@ -42,16 +42,30 @@ def _attn_fused(op, X, weights):
     return op.vec_size == 1 or (op.mask is not None and X.shape[0] % 2 == 0)
 
 
+def _is_own(op, colIdx):
+    """Is ``colIdx`` the very array that the operator's columns come from (a view of it, as [nnz, 1]), or None?"""
+    own = op.colIdx if op.vec_size == 1 else getattr(op, "csr_colIdx", None)
+    return own is not None and (colIdx is None or colIdx.dtype == own.dtype and colIdx.numel() == own.numel()
+                                and colIdx.data_ptr() == own.data_ptr())
+
+
 def _slot_columns(op, colIdx):
-    """2x1 blocks: for every slot of the blocks the column the reference's attention-weight gradient multiplies it with
-    (gnn_conv.py:166-172: d_attention[mask] times colIdx in CSR order), zero at padding; made once per operator."""
-    if op.vec_size == 1:
+    """For every score the column the reference's attention-weight gradient multiplies it with (gnn_conv.py:166-172:
+    d_attention[mask] times the caller's colIdx in CSR order; 2x1 blocks: zero at padding).  None where that is the entry's own
+    column: CSR operators that are given their own array, and the windowed layout, whose entries have an order of their own.  The
+    slots of an operator's own columns are made once; other columns are taken as they are at every call."""
+    if _fmt(op) == 4:
         return None
-    slots = getattr(op, "_slot_columns", None)
-    if slots is None:
-        slots = torch.zeros(op.val.numel(), device=op.val.device)
-        slots[op.mask] = colIdx.reshape(-1).float()
-        op._slot_columns = slots
+    own = _is_own(op, colIdx)
+    if op.vec_size == 1:
+        return None if own else colIdx.reshape(-1).float()
+    k = op.__dict__.get("_own_slot_columns")
+    if own and k is not None and k[0] is op.csr_colIdx and k[1] is op.mask:
+        return k[2]
+    slots = torch.zeros(op.val.numel(), device=op.val.device)
+    slots[op.mask] = (op.csr_colIdx if own else colIdx).reshape(-1).float()
+    if own:
+        op._own_slot_columns = (op.csr_colIdx, op.mask, slots)
     return slots
 
 
@@ -213,12 +227,16 @@ class _AGNNUnfused(torch.autograd.Function):
         # the reference's literal formula for the attention weight gradient (gnn_conv.py:172):
         # mm(d_attention[1, nnz] expanded to n_heads rows, colIdx.float()[nnz, 1])^T.  Every row of the product is the
         # same dot product over the nnz entries; as a GEMM it takes 20 ms on 2*10^7 entries (a 1 x nnz x 1 problem),
-        # as a dot product some tens of microseconds.  The float copy of colIdx is made once per operator.
-        # A windowed operator keeps its entries in its own order inside the rows: its colIdx is the one that matches.
-        col_f = getattr(op, "_colIdx_as_float", None)
-        if col_f is None or col_f.numel() != ctx.colIdx.numel():
-            col_f = (op.colIdx if _fmt(op) == 4 else ctx.colIdx).reshape(-1).to(d_attention.dtype)
-            op._colIdx_as_float = col_f
+        # as a dot product some tens of microseconds.  A windowed operator keeps its entries in its own order inside the rows:
+        # its colIdx is the one that matches.  The float copy of an operator's own columns is made once.
+        col = op.colIdx if _fmt(op) == 4 or ctx.colIdx is None else ctx.colIdx
+        k = op.__dict__.get("_own_columns_as_float")
+        if k is not None and k[0] is op.colIdx and k[1].dtype == d_attention.dtype and k[1].numel() == col.numel() and _is_own(op, col):
+            col_f = k[1]
+        else:
+            col_f = col.reshape(-1).to(d_attention.dtype)
+            if _is_own(op, col):
+                op._own_columns_as_float = (op.colIdx, col_f)
         d_attention_w = torch.dot(d_attention, col_f).reshape(1, 1).expand(1, n_heads)
         return d_input, d_weights, d_attention_w, None, None, None
 

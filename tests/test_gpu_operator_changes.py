@@ -1,4 +1,5 @@
-"""An operator whose attributes are replaced between two calls: the layers use what it holds now."""
+"""An operator whose attributes are replaced between two calls: the layers use what it holds now, and an attention layer multiplies
+its weight gradient with the columns that it is given."""
 import pytest
 import torch
 
@@ -39,3 +40,33 @@ def test_layers_follow_the_operators_format(graph):
     win.rowPtr_w = win.rowPtr_w.clone()
     assert G._native(win) is not was
     assert torch.allclose(G.GCNFunction.apply(X, W, win), want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("width", [16, 144])  # one launch per direction; separate operators
+@pytest.mark.parametrize("config", [(1, False), (1, True), (2, False), (2, True)])
+def test_attention_weight_gradient_uses_the_columns_it_is_given(graph, width, config):
+    from paramspmm_ae_amd import gnn_conv as G
+    from paramspmm_ae_amd.PCSR import pcsr_spmm
+
+    op, n, c = pcsr_spmm(graph, vec_size=config[0], if_split=config[1]), graph.mtx_nodes, graph.csr_data
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    X, dY = (torch.randn(n, width, device="cuda", generator=gen) for _ in range(2))
+    W, aw = torch.randn(width, width, device="cuda", generator=gen) / width, torch.ones(1, 1, device="cuda").requires_grad_()
+    own = c.on_device("colIdx", "cuda")
+    d = dY.cpu().double()
+    rows = torch.repeat_interleave(torch.arange(n), c.row_nnz.long())
+    # the reference's scores in the order of its mask: a row's slots of the 2x1 blocks in block order
+    at = c.colIdx.long() if config[0] == 1 else op.colIdx.cpu().long()[op.mask.cpu() // 2]
+    dots = (d[rows] * d[at]).sum(1)
+    changed = own.clone()
+    changed[::3] += 7
+    inplace = own.clone()
+    for k, col in enumerate((own.unsqueeze(-1), own.clone(), changed, own.unsqueeze(-1), changed.long().unsqueeze(-1), inplace, inplace)):
+        if k == 6:
+            inplace += 3  # the same tensor, other contents
+        print("case", config, width, k, flush=True)
+        got, = torch.autograd.grad(G.AGNNFunction.apply(X, W, aw, op, col, False), [aw], dY)
+        w = col.reshape(-1).cpu().double()
+        # the sums run in fp32: width products per dot, nnz terms; 1e-5 of the terms' sizes is some ten times their random error
+        size = ((d[rows].abs() * d[at].abs()).sum(1) * w).sum()
+        assert abs(float(got) - float((dots * w).sum())) <= 1e-5 * float(size)
