@@ -49,17 +49,22 @@ static bool kept_order_is_ours(long n, long K1, long K2)
 }
 
 // Weight gradients leave their kernels as partial products of the workgroups.  The sums of everything one backward call forms
-// share a launch (psp_sum_partials_f32): flush() before the gradients are handed out.
+// share a launch (psp_sum_partials_f32): flush() before the gradients are handed out.  What a launch less saves, some 5 us,
+// counts where the workspaces are small; past kHeldBytes they are summed and given back at once (64 MB a layer at 128 x 128).
 struct PartialSums {
+    static constexpr size_t kHeldBytes = (size_t)32 << 20;
     std::vector<psp_partial_sum> jobs;
     std::vector<Tensor> held;  // workspaces and results, until the launch
+    size_t held_bytes = 0;
     psp_stream_t stream = nullptr;
     void add(const Tensor &ws, Tensor &dW, int count)
     {
         jobs.push_back({fp(ws), fpw(dW), count, (int)dW.numel()});
         held.push_back(ws);
         held.push_back(dW);
+        held_bytes += ws.nbytes();
         stream = stream_of(ws);
+        if (held_bytes > kHeldBytes) flush();
     }
     void flush()
     {
@@ -68,6 +73,7 @@ struct PartialSums {
         ok(psp_sum_partials_f32(jobs.data(), (int)jobs.size(), stream));
         jobs.clear();
         held.clear();
+        held_bytes = 0;
     }
 };
 static int ok_count(int rc)
@@ -745,18 +751,23 @@ static Tensor softmax_nll_layer(Tensor logits, Tensor labels)
 }
 
 // A training step's network and loss, nll_loss(log_softmax(layers(x)), labels), as one node.  On a graph of 20 K nodes the step is
-// bound by the host: six nodes cost the engine some 80 us, and each layer's weight gradient a launch for its sum.
+// bound by the host: six nodes cost the engine some 80 us, and each layer's weight gradient a launch for its sum.  In a backward
+// pass that does not keep the graph, what a layer saved is given back when its gradients are launched, as nodes of their own
+// would do (10^6 rows, hidden 128: every layer's input or kept product is 512 MB).
 struct NetworkLoss : LayerNode {  // a_ = labels, w_ = logits, z_ = stats
     struct Part {
         int kind;
         op_t op;
         SavedVariable in, w, kept;
+        void release() { in.reset_data(), w.reset_data(), kept.reset_data(); }
     };
     std::vector<Part> parts;
+    bool last_pass = false;
+    void will_release_variables() override { last_pass = true; }
     void release_variables() override
     {
         LayerNode::release_variables();
-        for (Part &p : parts) p.in.reset_data(), p.w.reset_data(), p.kept.reset_data();
+        for (Part &p : parts) p.release();
     }
     variable_list apply(variable_list &&g) override
     {
@@ -767,12 +778,14 @@ struct NetworkLoss : LayerNode {  // a_ = labels, w_ = logits, z_ = stats
         while (lowest < out.size() && !wants(lowest)) lowest++;
         if (lowest == out.size()) return out;
         Tensor d = softmax_nll_mean_backward(w(), a(), g[0].contiguous(), z());
+        if (last_pass) LayerNode::release_variables();
         PartialSums sums;
         for (size_t l = parts.size(); l-- > 0 && lowest <= l + 1;) {
             Part &p = parts[l];
             const bool keeps = p.kind == kAggregateFirst || p.kind == kGINReLU;
             std::tie(d, out[l + 1]) = layer_backward(p.kind, *p.op, d, p.kind == kAggregateFirst ? Tensor() : p.in.unpack(self), p.w.unpack(self),
                                                      keeps ? p.kept.unpack(self) : Tensor(), lowest <= l, wants(l + 1), sums);
+            if (last_pass) p.release();
             if (!wants(l + 1)) out[l + 1] = Tensor();
         }
         if (wants(0)) out[0] = d;

@@ -325,8 +325,9 @@ _NETWORK_KIND = {GCNFunction: 0, GCNAggregateFirstFunction: 1, GINFunction: 1, G
 
 def network_loss(convs, spmm_dict, x, labels):
     """Layers ``convs`` with ReLU between them on ``x``, log-softmax and mean NLL loss as one autograd node, or None where
-    some part of it has to run by itself: subclasses and layers with hooks, operators a layer's native form does not take,
-    losses softmax_nll_loss_mean leaves to PyTorch."""
+    some part of it has to run by itself: subclasses, layers with hooks and weights with hooks (one node hands its gradients out
+    together, when the last is formed), operators a layer's native form does not take, losses softmax_nll_loss_mean leaves to
+    PyTorch."""
     if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and labels.is_cuda and labels.dtype == torch.int64
             and labels.dim() == 1 and labels.is_contiguous() and not _module._has_any_global_hook()):
         return None
@@ -334,7 +335,8 @@ def network_loss(convs, spmm_dict, x, labels):
     for conv in convs:
         w = conv.weights
         if (type(conv) not in (GCNConv, GINConv) or conv._forward_hooks or conv._forward_pre_hooks or conv._backward_hooks
-                or conv._backward_pre_hooks or "forward" in conv.__dict__ or w.dtype != torch.float32):
+                or conv._backward_pre_hooks or "forward" in conv.__dict__ or w.dtype != torch.float32
+                or w._backward_hooks or getattr(w, "_post_accumulate_grad_hooks", None)):
             return None
         fn, op = conv.choose(x.shape[0], spmm_dict, bool(kinds))
         kind = _NETWORK_KIND.get(fn)
