@@ -259,27 +259,35 @@ def build_model(net, graph, operators, hidden, num_features, num_classes, num_la
 WINDOW_MIN_LOCAL_SHARE = 0.6
 
 
+def _fastest(ops, X):
+    """The operator of ``ops`` whose product with X takes least (a few launches each, after a cache fill, as inside an epoch).  They
+    take turns and each counts with its best turn: a launch that something else held up would otherwise decide which operator, and
+    with it which order of the sums, a run gets."""
+    best = [float("inf")] * len(ops)
+    for _ in range(3):
+        for i, op in enumerate(ops):
+            best[i] = min(best[i], op.time_ms(X, warmup=1, iters=2, flush_bytes=256 << 20))
+    return ops[best.index(min(best))]
+
+
 def _try_window(graph, dim, op):
     """The windowed layout against ``op`` on this matrix (an addition of this build): when at least
-    WINDOW_MIN_LOCAL_SHARE of the entries have their column within the row's window, both are timed (a few launches each, after a cache fill, as
-    inside an epoch) and the faster one is returned.  The class space of the forests has no such representation, so
-    the choice is made by this measurement instead of by the decider."""
+    WINDOW_MIN_LOCAL_SHARE of the entries have their column within the row's window, both are timed and the faster one is
+    returned.  The class space of the forests has no such representation, so the choice is made by this measurement
+    instead of by the decider."""
     if dim % 4 or graph.csr_data.val.dim() != 1:
         return op
     cand = pcsr_spmm(graph=graph, vec_size=1, if_split=False, CF=0, window=True)
     if cand.window_local_share < WINDOW_MIN_LOCAL_SHARE:
         return op
     X = torch.randn((graph.mtx_nodes + 1) // 2 * 2, dim, device="cuda")
-    ms_op = op.time_ms(X, warmup=2, iters=5, flush_bytes=256 << 20)
-    ms_w = cand.time_ms(X, warmup=2, iters=5, flush_bytes=256 << 20)
-    return cand if ms_w < ms_op else op
+    return _fastest([op, cand], X)
 
 
 def configure_operators(decider, graph, dims, override=None, try_candidates=0, try_window=True):
     """One pcsr_spmm per layer width, configured by the decider (GNN.py:200-209) or by ``override`` =
     (if_split, vec_size, CF, blkWarpNum).  ``try_candidates`` = k > 1 (an addition of this build): the k configurations
-    the forest rates highest are timed on this matrix (a few launches each, after a cache fill, as inside an epoch) and
-    the fastest is kept.  ``try_window``: see _try_window (not with ``override``)."""
+    the forest rates highest are timed on this matrix and the fastest is kept.  ``try_window``: see _try_window (not with ``override``)."""
     ops = {}
     for dim in dims:
         if override is not None or try_candidates <= 1:
@@ -289,13 +297,9 @@ def configure_operators(decider, graph, dims, override=None, try_candidates=0, t
                 ops[dim] = _try_window(graph, dim, ops[dim])
             continue
         X = torch.randn((graph.mtx_nodes + 1) // 2 * 2, dim, device="cuda")  # an even row count serves the 2x1 block formats too
-        best = None
-        for if_split, vec_size, CF, blkWarpNum in decider.candidates_PCSR(graph, dim, try_candidates):
-            op = pcsr_spmm(graph=graph, vec_size=vec_size, if_split=if_split, CF=CF, blkWarpNum=blkWarpNum)
-            ms = op.time_ms(X, warmup=2, iters=5, flush_bytes=256 << 20)
-            if best is None or ms < best[0]:
-                best = (ms, op)
-        ops[dim] = _try_window(graph, dim, best[1]) if try_window else best[1]
+        best = _fastest([pcsr_spmm(graph=graph, vec_size=vec_size, if_split=if_split, CF=CF, blkWarpNum=blkWarpNum)
+                         for if_split, vec_size, CF, blkWarpNum in decider.candidates_PCSR(graph, dim, try_candidates)], X)
+        ops[dim] = _try_window(graph, dim, best) if try_window else best
     return ops
 
 
