@@ -134,7 +134,14 @@ PSP_EXPORT int psp_spmm_plan_for(int N, int CF, int blkWarpNum, psp_spmm_plan *p
         // vectors per lane, so a wavefront carries 8 rows whatever CF is.
         C = std::min(CF, nvec);
         L = 32 / V;
-        while (L > 1 && (L / 2) * C >= nvec) L >>= 1;  // one tile already covers N: no wider than needed
+        // One tile already covers N: no wider than needed -- but four lanes for a width of 5 to 7, whose two pieces would leave two
+        // lanes and two entries in flight.  us at N = 6 with two lanes / four, plain and row-split CSR, plain and row-split 2x1
+        // blocks: 300 000 rows of 21 entries 51 / 34, 54 / 39, 76 / 45, 81 / 49; 200 003 skewed rows of 15 75 / 63, 49 / 41, 88 / 83,
+        // 64 / 44; 20 K rows 10.1 / 8.5, 12.9 / 11.1, 10.8 / 9.7, 13.9 / 11.6; a mesh (five entries a row) loses: 23 / 40, 33 / 51,
+        // 24 / 35, 33 / 42 (a native configuration asks for two lanes).  8- and 4-byte pieces, in the same order: 33, 38, 42, 45;
+        // 61, 39, 79, 43; 8.4, 10.9, 9.0, 11.2; 39, 48, 29, 35.
+        const int least = C == 1 && N > 4 && N < 8 ? 4 : 1;
+        while (L > least && (L / 2) * C >= nvec) L >>= 1;
         U = C == 1 ? 4 : C <= 4 ? 2 : 1;  // feature vectors in flight per lane: U entries x C vectors
         while (U > L) U >>= 1;
     }

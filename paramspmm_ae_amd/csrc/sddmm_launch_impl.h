@@ -38,11 +38,16 @@ int psp_sddmm_launch(const int *rowPtr, const int *colIdx, const float *val, con
     PSP_REQUIRE(!(BCSR && scale), "sddmm: scale is only supported for csr formats");
     PSP_REQUIRE(!(BCSR && row_max), "sddmm: row maxima are only supported for csr formats");
 
-    const int V = psp_vec_width(K);
+    // Widths of 5 to 7: the two pieces of a row would leave lane groups of two.  CSR takes four lanes (two of them idle), blocks a
+    // float per lane on eight.  us at K = 6 with two lanes / so, plain and row-split CSR, plain and row-split 2x1 blocks: 300 000 rows
+    // of 21 entries 77 / 38, 75 / 39, 142 / 50, 141 / 62; 200 003 skewed rows of 15 33 / 33, 47 / 32, 94 / 105, 87 / 48; a mesh 20 / 31,
+    // 21 / 33, 44 / 33, 44 / 31.  8- and 4-byte pieces, in the same order: 45, 46, 76, 77; 35, 37, 103, 54; 38, 39, 25, 26.
+    const bool few = K > 4 && K < 8;
+    const int V = few && BCSR ? 1 : psp_vec_width(K);
     const int nvec = psp_ceil_div(K, V);
     int C = psp_ceil_div(nvec, 16);
     if (C > 4) C = 4;
-    int logL = 0;
+    int logL = few ? 2 : 0;
     while ((C << logL) < nvec) logL++;
     if (logL > 6) return psp_fail(PSP_ERR_RANGE, "sddmm: K = %d is too wide (max %d)", K, 1024);
     if (logL < 4 && C > 1) C = 1;
