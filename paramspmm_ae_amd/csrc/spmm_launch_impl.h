@@ -97,6 +97,7 @@ int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, cons
         PSP_REQUIRE((long long)nrows * NR <= rows_out, "spmm: Y has %d rows, the matrix needs %lld", rows_out,
                     (long long)nrows * NR);
     PSP_REQUIRE(!(row_max && relu_x), "spmm: the softmax-weighted product takes no activation argument");
+    PSP_REQUIRE(!row_max || N % 4 == 0, "spmm softmax: N must be a multiple of 4 (got %d)", N);
     if (nrows > 0) {
         PSP_REQUIRE(rowPtr && X, "spmm: rowPtr / X is null");
         PSP_REQUIRE(!SPLIT || target_row, "spmm: target_row is null");
@@ -104,6 +105,6 @@ int psp_spmm_launch(const int *rowPtr, const int *colIdx, const float *val, cons
     psp_spmm_kernel_t k = psp_spmm_lookup<NR, SPLIT>(plan.coarsen, psp_vec_width(N), plan.unroll, plan.lanes_per_row, row_max != nullptr, relu_x != 0);
     if (!k && nrows > 0)
         return psp_fail(PSP_ERR_ARG, "spmm%s: no kernel for coarsen %d vec %d unroll %d%s", row_max ? " softmax" : "", plan.coarsen,
-                        psp_vec_width(N), plan.unroll, row_max ? " (needs N % 4 == 0 and CF <= 4)" : "");
+                        psp_vec_width(N), plan.unroll, row_max ? " (needs CF <= 4)" : "");
     return psp_spmm_enqueue<NR, SPLIT>(k, plan, rowPtr, colIdx, val, target_row, X, Y, nrows, N, rows_out, stream, row_max, row_sum, relu_x);
 }
