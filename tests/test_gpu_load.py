@@ -1,5 +1,6 @@
 """graph_input.load_from_csr on the device (one native call: transfers, statistics, 2x1 blocks, row splits) against the host
-builders: same arrays bit for bit, same statistics; sizes on both sides of the threaded upload, odd and even row counts."""
+builders: same arrays bit for bit, same statistics; sizes on both sides of the threaded upload and of the upload ring's length, odd and even
+row counts."""
 import numpy as np
 import pytest
 import torch
@@ -60,3 +61,28 @@ def test_native_load_reports_bad_arrays():
         _load((rowPtr, swapped, val), build_on="device")
     g, want = _load((rowPtr, swapped, val)), _load((rowPtr, swapped, val), build_on="host")
     assert torch.equal(g.bcsr_data.colIdx, want.bcsr_data.colIdx) and torch.equal(g.bcsr_data.val, want.bcsr_data.val)
+
+
+@pytest.mark.parametrize("n,row", [(1000003, 40), (4000001, 9)])  # 41 and 38 transfers, the row pointers of them one and two
+def test_slots_of_the_upload_ring_are_used_again(n, row):
+    """Arrays of more than sixteen 8 MB transfers: every slot of the page-locked ring is written again while earlier transfers are
+    under way.  What arrives is what was sent, bit for bit, on the first load and on the next with other values."""
+    rng = np.random.default_rng(n)
+    rowPtr = (np.arange(n + 1, dtype=np.int64) * row).astype(np.int32)
+    nnz = int(rowPtr[-1])
+    # strictly ascending columns: a start per row, steps of 1 to 7
+    start = rng.integers(0, n - 7 * row, n, dtype=np.int32)
+    colIdx = (start[:, None] + np.cumsum(rng.integers(1, 8, (n, row), dtype=np.int32), axis=1, dtype=np.int32)).reshape(-1) - 1
+    assert (rowPtr.nbytes + colIdx.nbytes + 4 * nnz) > 17 * (8 << 20)
+    for turn in range(2):
+        val = rng.random(nnz, dtype=np.float32)
+        print("case", n, row, turn, flush=True)
+        g = _load((rowPtr, colIdx, val), build_on="device")
+        c, b = g.csr_data, g.bcsr_data
+        for name, want in (("rowPtr", rowPtr), ("colIdx", colIdx), ("val", val)):
+            assert torch.equal(c.on_device(name, "cuda").cpu(), torch.from_numpy(want)), name
+        # the blocks that were built from the device arrays meanwhile hold every value once
+        assert int(torch.count_nonzero(b.val)) == int(np.count_nonzero(val))
+        assert abs(float(b.val.double().sum()) - float(val.astype(np.float64).sum())) <= 1e-9 * nnz
+        assert int(b.rowPtr[-1]) == b.colIdx.numel()
+        del g, c, b
