@@ -811,7 +811,7 @@ def main():
             continue
         plan = _capi.spmm_plan(r["dim"], r["CF"], r["blkWarpNum"])
         one_set = plan["register_sets"] == 1
-        sym = "psp_spmm_kernel<%d, %d, %d, %d, %s, false, false, %s, float, psp_plain>" % (plan["coarsen"], plan["vec"], plan["unroll"],
+        sym = "psp_spmm_kernel<%d, %d, %d, %d, %s, false, false, %s, float, psp_plain>" % (plan["coarsen"], plan["load_width"], plan["unroll"],
                                                            2 if r["format"].startswith("bcsr") else 1,
                                                            "true" if "split" in r["format"] else "false",
                                                            "true" if one_set else "false")

@@ -45,8 +45,9 @@ const char *psp_last_error(void);
  *   312: psp_attn_forward_f32 / _backward_f32 (no buffer changed).
  *   313: psp_spmm_window_grad_f32 (no buffer changed).
  *   314: psp_sum_partials_f32, psp_dense_grad_f32 (no buffer changed).
+ *   315: psp_spmm_load_width (no buffer changed).
  * The extension modules and the ctypes loader of this package check it when they are imported. */
-#define PSP_ABI_VERSION 314
+#define PSP_ABI_VERSION 315
 int psp_version(void);
 
 /* How a (N, CF, blkWarpNum) request of the Python layer maps onto the wave64 kernels.
@@ -67,8 +68,8 @@ int psp_version(void);
 #define PSP_CF_PACK(coarsen, log_lanes, log_unroll, segs_sel) \
     (PSP_CF_NATIVE | ((coarsen) - 1) | ((log_lanes) << 3) | ((log_unroll) << 6) | ((segs_sel) << 8))
 typedef struct psp_spmm_plan {
-    int vec;            /* floats every row of X starts at a multiple of: 4 (N%4==0), 2 (N%2==0) or 1.  Loads are 4 floats
-                         * wide from N = 4 on (their alignment is that of one float), 1 float wide below */
+    int vec;            /* floats every row of X starts at a multiple of: 4 (N%4==0), 2 (N%2==0) or 1.  Not the width of the
+                         * kernel's loads, which psp_spmm_load_width(N) gives */
     int coarsen;        /* column vectors per lane (the request's CF, 1..8) */
     int lanes_per_row;  /* power of two, 1..64: lanes that share one sparse row */
     int rows_per_wave;  /* 64 / lanes_per_row */
@@ -85,6 +86,9 @@ int psp_spmm_plan_for(int N, int CF, int blkWarpNum, psp_spmm_plan *plan);
  * is gathered, added, and the next one gathered -- fewer registers, more wavefronts per SIMD; faster wherever at least
  * four entries are in flight, or two with 8 or more lanes per row.  No counterpart in the reference. */
 int psp_spmm_register_sets(int unroll, int lanes_per_row);
+/* Floats per load of a feature row of N (the second argument of the kernel's symbol as a profiler prints it): 4 from N = 4
+ * on, aligned as one float is, 1 below. */
+int psp_spmm_load_width(int N);
 
 /* SpMM and SDDMM entry points (row-wise walks), blkWarpNum | PSP_BW_STRIPE(rows): this launch deals `rows`
  * consecutive rows (segments, block-rows) to one XCD at a time instead of the library option "xcd_stripe_rows".

@@ -46,6 +46,7 @@ SIGNATURES = {
     "psp_get_option": [ctypes.c_char_p],
     "psp_spmm_plan_for": [_i, _i, _i, ctypes.POINTER(SpmmPlan)],
     "psp_spmm_register_sets": [_i, _i],
+    "psp_spmm_load_width": [_i],
     "psp_split_csr_count": [_vp, _i, _i],
     "psp_split_csr": [_vp, _i, _i, _vp, _vp],
     "psp_split_csr_par": [_vp, _vp, _i, _i, _vp, _vp],
@@ -125,7 +126,7 @@ for _name, _args in SIGNATURES.items():
 lib.psp_last_error.argtypes = []
 lib.psp_last_error.restype = ctypes.c_char_p
 
-ABI_VERSION = 314  # PSP_ABI_VERSION of include/paramsp.h: the struct layouts and buffer sizes this module assumes
+ABI_VERSION = 315  # PSP_ABI_VERSION of include/paramsp.h: the struct layouts and buffer sizes this module assumes
 if lib.psp_version() < ABI_VERSION:
     raise ImportError("%s is version %d, this package needs %d: rebuild it (paramspmm_ae_amd/build_param.sh)"
                       % (LIB_PATH, lib.psp_version(), ABI_VERSION))
@@ -192,7 +193,8 @@ def spmm_plan(N, CF, blkWarpNum):
     p = SpmmPlan()
     check(lib.psp_spmm_plan_for(N, CF, blkWarpNum, ctypes.byref(p)))
     d = p.as_dict()
-    d["register_sets"] = lib.psp_spmm_register_sets(p.unroll, p.lanes_per_row)  # which kernel variant the plan launches
+    # which kernel variant the plan launches
+    d["register_sets"], d["load_width"] = lib.psp_spmm_register_sets(p.unroll, p.lanes_per_row), lib.psp_spmm_load_width(N)
     return d
 
 
