@@ -153,7 +153,7 @@ psp_atb_mfma_kernel(const float *__restrict__ A, const float *__restrict__ B, fl
     }
 }
 
-// The 128 x 128 product on the bf16 matrix-core path (option dense_split).  At that shape the fp32 instruction above
+// The 128 x 128 product on the bf16 matrix-core path (option dense_split, from PSP_SPLIT_MIN_ROWS rows on).  At that shape the fp32 instruction above
 // needs as long for its flops as the memory system needs for the two operands; with every fp32 operand taken apart
 // into its three bf16 terms (exact: 8 + 8 + 8 significant bits) and the six term products that matter (error 2^-23 of
 // |a||b| per product) accumulated in fp32 by v_mfma_f32_16x16x32_bf16, the kernel is bound by its traffic again.

@@ -178,7 +178,7 @@ psp_xw_kernel(const float *__restrict__ X, const float *__restrict__ W, float *_
     }
 }
 
-// ---- the 128 x 128 product on the bf16 matrix-core path -----------------------------------------------------------------
+// ---- the 128 x 128 product on the bf16 matrix-core path (option dense_split, from PSP_SPLIT_MIN_ROWS rows on) -----------------
 // At 128 x 128 the fp32 instruction above needs as long for its 32 kflop per row as the memory system needs for the row's
 // 1 KB.  gfx950 multiplies bf16 sixteen times as fast, and an fp32 number is the exact sum of three bf16 numbers
 // (x = hi + mid + lo, 8 + 8 + 8 significant bits), so x w = sum of nine bf16 products, of which the six with at least

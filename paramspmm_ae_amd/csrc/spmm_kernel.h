@@ -35,7 +35,9 @@ typedef float psp_f32x4 __attribute__((ext_vector_type(4)));
 // so a row whose length is no multiple of 4 takes the same 16-byte instructions (`mem` carries the alignment).  Its last
 // piece is moved back to end with the row (psp_vec_col): it repeats up to three columns of the piece in front of it.
 // Widths below 4 use single floats.  Before, widths off the multiples of 4 ran on 8- or 4-byte loads with two and four
-// times the lanes or column tiles: Chung-Lu graph of 200 003 rows and 3.0 M entries, N = 47: 167 us.
+// times the lanes or column tiles: Chung-Lu graph of 200 003 rows and 3.0 M entries, N = 47: 167 us -> 106.  Width 2, which had one
+// 8-byte load, on two lanes of a float each (plain and row-split CSR, plain and row-split 2x1 blocks): SpMM on that graph 61, 47,
+// 95, 74 us -> 54, 36, 62, 46, on a mesh of 10^6 rows 19, 24, 47, 54 -> 22, 28, 19, 24; SDDMM 21, 32, 144, 98 -> 23, 30, 76, 71.
 typedef float psp_f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef double psp_f64x2 __attribute__((ext_vector_type(2)));
 typedef double psp_f64x2_a8 __attribute__((ext_vector_type(2), aligned(8)));

@@ -33,8 +33,8 @@
 // EPI (square layers of 16 or 32 columns, one column tile): the finished row is multiplied by a small dense matrix
 // before it is stored, Y = (A f(X)) W or (A f(X)) W^T -- the dense product of a GCN layer folded into the sparse one.
 // W sits in LDS (transposed on the way in for W^T); a lane group gathers its row of A f(X) with DPP moves and each lane
-// forms its four output columns (N multiply-adds per column).  The row of A f(X) itself can be stored as well (Y_raw:
-// the backward pass needs A dY for the weight gradient and (A dY) W^T for the input gradient).  Measured and dropped:
+// forms its four output columns (N multiply-adds per column).  The row of A f(X) itself can be stored as well (Y_raw, for callers
+// of the C entry that want both; the layers' backward pass forms its weight gradient in KZ and stores no A dY).  Measured and dropped:
 // the same product on the matrix cores, with the block's 64 rows parked in LDS and a barrier (GCN epoch, hidden 16 / 32: 1.71 /
 // 2.60 ms against 1.61 / 2.49) or with a wavefront's own rows and none (92 us against 92 at 16 columns, 156 against 158 at 32).
 // KZ (backward of a layer whose input is Z [M, KZ], KZ = TN or 2 TN, one column tile): the weight gradient f(Z)^T (A X), a KZ x TN

@@ -1,6 +1,7 @@
 // Python module `ParamSpCONV`: the fused GCN layer ops of the reference's SpCONV/SpCONV.cpp:496-512
-// (glue in SpCONV/SpCONV.h:43-193): forward A*(H*W), backward [ (A*dY)*W^T, H^T*(A*dY) ].  The dense
-// products are torch::mm (hipBLASLt / rocBLAS under PyTorch-ROCm); the sparse product is libparamsp_hip.so.
+// (glue in SpCONV/SpCONV.h:43-193): forward A*(H*W), backward [ (A*dY)*W^T, H^T*(A*dY) ]; and this build's layers and losses as
+// autograd nodes.  The sparse products and, for widths that are multiples of 16 up to 128 and 1024 rows or more, the dense
+// ones are libparamsp_hip.so's (but see kept_order_is_ours); torch::mm forms the others.
 #include "glue_common.h"
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -33,14 +34,18 @@ static Tensor aggregate(int fmt, const Tensor &D, const Tensor &rowPtr, const Te
 }
 
 // Rows from which the library's dense kernels are used (PyTorch's GEMM below): they cost one launch with the activation
-// or the mask folded in, where PyTorch needs one for each.
+// or the mask folded in, where PyTorch needs one for each.  us at 1024 rows against PyTorch, relu(Z) W, masked X W^T and weight
+// gradient: 48 x 48 5 / 25, 5 / 27, 10 / 26; 96 x 96 12 / 25, 12 / 27, 20 / 26; 128 x 128 18 / 25, 19 / 27, 13 / 26.  What PyTorch
+// takes is its launches, so the line could lie lower; fewer rows have not been measured.
 constexpr long kDenseRows = 1024;
 
 // Where a product's result is the activation of a ReLU network (GCN, GIN), another order of its sum puts some element on the
 // other side of zero, which drops or adds a whole term of the gradient: a training run would not repeat the figures it gave
 // before.  Those products stay with the order that each shape has always had: the library's (ascending k up to 32 columns,
-// see dense_xw.hip) at the shapes below from 16384 rows on, PyTorch's GEMM elsewhere.  Gradients (X W^T and the weight
-// gradient) and the attention layer have no such step behind them and take the library's kernel at every shape.
+// see dense_xw.hip) at the shapes below from 16384 rows on, PyTorch's GEMM elsewhere.  This is a list of what was the library's
+// before its kernel took every width, not a line that was measured: at the shapes it leaves to PyTorch the kernel is the faster
+// one (48 x 48, 10^6 rows: 81 us against 208).  Gradients (X W^T and the weight gradient) and the attention layer have no such
+// step behind them and take the library's kernel at every shape.
 enum class Order { any, kept };
 static bool kept_order_is_ours(long n, long K1, long K2)
 {
@@ -886,7 +891,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           "nll_loss(log_softmax(layers(x)), labels): (kinds 0 gcn, 1 aggregate first, 2 gcn of relu, 3 aggregate first of relu; operators, x, weights, labels)");
     m.def("split_csr", &pspglue::split_csr, "row split on the host");
     m.def("split_csr_par", &pspglue::split_csr_par, "row split on the host with a precomputed segment prefix");
-    // addition of this build: H^T * G for tall-skinny operands (memory-speed kernel for widths 16..64, else torch::mm)
+    // addition of this build: H^T * G for tall-skinny operands (a kernel of the library's for multiples of 16 up to 128 and 1024
+    // rows or more, else torch::mm)
     m.def("weight_gradient", [](Tensor H, Tensor G) {
         need_gpu(H, "H");
         need_gpu(G, "G");
