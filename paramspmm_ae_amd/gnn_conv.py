@@ -80,6 +80,29 @@ def _native(op, slots=None):
     return k[-1]
 
 
+class _Recorded(torch.autograd.Function):
+    """A native layer or loss as one operation of a trace.  torch.jit.trace records Python functions and ATen operators; of what a
+    native node launches it would record the allocations alone."""
+
+    @staticmethod
+    def forward(ctx, native, front, *inputs):
+        with torch.enable_grad():
+            ctx.inputs = [t.detach().requires_grad_(t.requires_grad) if isinstance(t, torch.Tensor) else t for t in inputs]
+            ctx.out = native(*front, *ctx.inputs)
+        return ctx.out.detach()
+
+    @staticmethod
+    def backward(ctx, grad):
+        at = [i for i, t in enumerate(ctx.inputs) if isinstance(t, torch.Tensor) and t.requires_grad]
+        grads = torch.autograd.grad(ctx.out, [ctx.inputs[i] for i in at], grad, retain_graph=True)
+        return (None, None) + tuple(grads[at.index(i)] if i in at else None for i in range(len(ctx.inputs)))
+
+
+def _run(native, front, *inputs):
+    """``native(*front, *inputs)``; ``front``: what comes before the tensors"""
+    return _Recorded.apply(native, front, *inputs) if torch.jit.is_tracing() else native(*front, *inputs)
+
+
 def nll_loss_mean(logp, labels):
     """``F.nll_loss(logp, labels)`` (mean over the rows, the loss of the reference's training step, GNN.py:131-146)
     through the library's kernels.  PyTorch reduces the whole batch in one workgroup -- 1.7 ms per step forward plus
@@ -88,7 +111,7 @@ def nll_loss_mean(logp, labels):
     int64 labels goes to PyTorch."""
     if (logp.is_cuda and logp.dtype == torch.float32 and logp.dim() == 2 and labels.dtype == torch.int64
             and labels.dim() == 1):
-        return SpCONV.nll_loss_layer(logp.contiguous(), labels.contiguous())
+        return _run(SpCONV.nll_loss_layer, (), logp.contiguous(), labels.contiguous())
     return torch.nn.functional.nll_loss(logp, labels)
 
 
@@ -100,7 +123,7 @@ def softmax_nll_loss_mean(logits, labels):
     operators."""
     if (logits.is_cuda and logits.dtype == torch.float32 and logits.dim() == 2 and labels.dtype == torch.int64
             and labels.dim() == 1 and SpCONV.softmax_nll_supported(int(logits.shape[1]))):
-        return SpCONV.softmax_nll_layer(logits.contiguous(), labels.contiguous())
+        return _run(SpCONV.softmax_nll_layer, (), logits.contiguous(), labels.contiguous())
     return nll_loss_mean(torch.nn.functional.log_softmax(logits, dim=1), labels)
 
 
@@ -109,7 +132,7 @@ class GCNFunction(object):
 
     @staticmethod
     def apply(H, weight, ParamSpMM):
-        return SpCONV.gcn_layer(_native(ParamSpMM), H, weight)
+        return _run(SpCONV.gcn_layer, (_native(ParamSpMM),), H, weight)
 
 
 class GCNAggregateFirstFunction(object):
@@ -121,7 +144,7 @@ class GCNAggregateFirstFunction(object):
 
     @staticmethod
     def apply(H, weight, ParamSpMM):
-        return SpCONV.gcn_aggregate_first_layer(_native(ParamSpMM), H, weight)
+        return _run(SpCONV.gcn_aggregate_first_layer, (_native(ParamSpMM),), H, weight)
 
 
 class GCNReLUInputFunction(object):
@@ -133,7 +156,7 @@ class GCNReLUInputFunction(object):
 
     @staticmethod
     def apply(Z, weight, ParamSpMM):
-        return SpCONV.gcn_relu_layer(_native(ParamSpMM), Z, weight)
+        return _run(SpCONV.gcn_relu_layer, (_native(ParamSpMM),), Z, weight)
 
 
 class _Layer(torch.nn.Module):
@@ -184,7 +207,7 @@ class AGNNFunction(object):
         if _attn_fused(ParamSpMM, X, weights):
             # scores (the head's weight multiplied in) and their aggregation in one launch per direction
             native = _native(ParamSpMM, _slot_columns(ParamSpMM, colIdx))
-            return SpCONV.agnn_layer(native, X, weights, attention_w, bool(relu_input))
+            return _run(SpCONV.agnn_layer, (native,), X, weights, attention_w, bool(relu_input))
         return _AGNNUnfused.apply(X, weights, attention_w, ParamSpMM, colIdx, relu_input)
 
 
@@ -256,7 +279,7 @@ class GINFunction(object):
     @staticmethod
     def apply(X, weight, ParamSpMM):
         if ParamSpMM.vec_size == 1 or (ParamSpMM.vec_size == 2 and X.shape[0] % 2 == 0):
-            return SpCONV.gin_layer(_native(ParamSpMM), X, weight)
+            return _run(SpCONV.gin_layer, (_native(ParamSpMM),), X, weight)
         return _GINOnOperator.apply(X, weight, ParamSpMM)
 
 
@@ -287,7 +310,7 @@ class GINReLUInputFunction(object):
 
     @staticmethod
     def apply(Z, weight, ParamSpMM):
-        return SpCONV.gin_relu_layer(_native(ParamSpMM), Z, weight)
+        return _run(SpCONV.gin_relu_layer, (_native(ParamSpMM),), Z, weight)
 
 
 class GINConv(_Layer):
@@ -328,6 +351,8 @@ def network_loss(convs, spmm_dict, x, labels):
     some part of it has to run by itself: subclasses, layers with hooks and weights with hooks (one node hands its gradients out
     together, when the last is formed), operators a layer's native form does not take, losses softmax_nll_loss_mean leaves to
     PyTorch."""
+    if torch.jit.is_tracing():
+        return None
     if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and labels.is_cuda and labels.dtype == torch.int64
             and labels.dim() == 1 and labels.is_contiguous() and not _module._has_any_global_hook()):
         return None

@@ -69,3 +69,19 @@ def test_tangent_of_a_whole_network_is_refused(graph):
             GNN.loss_of_step(model, labels)
     model.x = x
     GNN.loss_of_step(model, labels).backward()
+
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("window", [False, True])
+def test_traced_functions_compute_what_they_compute_untraced(graph, window):
+    for name, f, at in _layers(graph, window):
+        print("case", name, flush=True)
+        traced = torch.jit.trace(f, at, check_trace=False)
+        other = (at * 0.5 + 0.25).requires_grad_()
+        want = f(other)
+        got = traced(other)
+        assert torch.equal(got, want), name
+        d = torch.randn(want.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+        for a, b in zip(torch.autograd.grad(got, [other], d), torch.autograd.grad(want, [other], d)):
+            # (the windowed attention weight's sum is taken with atomics, in no fixed order)
+            assert torch.allclose(a, b, rtol=1e-4 if window and "attention" in name else 0, atol=0), name
