@@ -85,3 +85,28 @@ def test_traced_functions_compute_what_they_compute_untraced(graph, window):
         for a, b in zip(torch.autograd.grad(got, [other], d), torch.autograd.grad(want, [other], d)):
             # (the windowed attention weight's sum is taken with atomics, in no fixed order)
             assert torch.allclose(a, b, rtol=1e-4 if window and "attention" in name else 0, atol=0), name
+
+
+@pytest.mark.parametrize("window", [False, True])
+def test_saved_tensors_go_through_the_hooks(graph, window):
+    """what a node keeps for its backward pass is packed and unpacked by saved-tensor hooks (here: parked in host memory)"""
+    from paramspmm_ae_amd import GNN
+
+    for name, f, at in _layers(graph, window):
+        print("case", name, flush=True)
+        x, packed = at.clone().requires_grad_(), []
+        want = f(x)
+        d = torch.randn(want.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+        want_grad, = torch.autograd.grad(want, [x], d)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.cuda()):
+            got = f(x)
+        grad, = torch.autograd.grad(got, [x], d)
+        assert packed and torch.equal(got, want)
+        assert torch.allclose(grad, want_grad, rtol=1e-4 if window and "attention" in name else 0, atol=0), name
+    model = GNN.build_model("GCN", graph, _ops(graph, window), 16, 32, 16)
+    labels = torch.randint(0, 16, graph.y.shape, device="cuda")
+    want = torch.autograd.grad(GNN.loss_of_step(model, labels), list(model.parameters()))
+    with torch.autograd.graph.save_on_cpu():
+        loss = GNN.loss_of_step(model, labels)
+    assert type(loss.grad_fn).__name__ == "NetworkLossBackward"
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(loss, list(model.parameters())), want))
